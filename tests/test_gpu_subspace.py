@@ -1,0 +1,103 @@
+"""GPU tests of the SCC's subspace path (k_sub.hip) against the full
+diagonalisation in every iteration (XTBAMD_SUBSPACE=0).
+
+The path stops when max |R| <= 1e-12 max(|A_ii|, 1), the criterion of a
+finished diagonalisation, so density errors are below 1e-12 x 30 eV / gap
+(a few 1e-11 at gaps above 2 eV); the SCC amplifies them by the few units by
+which any rounding is amplified.  Energies (Eh) are second order in them.
+Sizes: occupied and virtual counts at the edges of the 64 x 64 product tiles
+and of the k-blocks of 16, and a molecule with fewer than one tile.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+TOL = {"energy": 1e-9, "charges": 1e-8, "gradient": 1e-8, "wbo": 1e-8, "emo": 1e-7, "hl_gap_ev": 1e-7}
+
+
+def _engine():
+    import xtb_amd
+    if xtb_amd.device_count() < 1:
+        pytest.fail("no GPU visible to the HIP runtime")
+    return xtb_amd
+
+
+def _both(monkeypatch, mols, solvent=None, **kw):
+    xa = _engine()
+    out = []
+    for on in ("0", "1"):
+        monkeypatch.setenv("XTBAMD_SUBSPACE", on)
+        b = xa.Batch(mols, **kw)
+        if solvent:
+            b.set_solvent(solvent, "p16", True)
+        b.run()
+        out.append((b.results(), b.counters()))
+        b.close()
+    return out
+
+
+def _check(a, b, tag):
+    assert a["iterations"] == b["iterations"] and a["converged"] == b["converged"], tag
+    assert a["ihomo"] == b["ihomo"] and np.array_equal(a["focc"], b["focc"]), tag
+    for k, tol in TOL.items():
+        d = float(np.max(np.abs(np.asarray(a[k]) - np.asarray(b[k]))))
+        assert d <= tol, f"{tag} {k}: {d:.2e}"
+
+
+def _halogenated(n, seed):
+    from xtb_amd import workloads as w
+    z, x = w.alkane(n, seed)
+    z, x = z.copy(), x.copy()
+    for h in np.flatnonzero(z == 1)[::5]:
+        c = int(np.argmin(np.linalg.norm(x[:n] - x[h], axis=1)))
+        x[h] = x[c] + (x[h] - x[c]) * (1.77 / 1.09)
+        z[h] = 17
+    return z, x
+
+
+# (H2O)n: 4n occupied, 2n virtual; CnH(2n+2): 3n + 1 of each
+@pytest.mark.parametrize("kind,n", [("water", 1), ("water", 4), ("water", 16), ("water", 17), ("water", 31),
+                                    ("water", 33), ("alkane", 1), ("alkane", 5), ("alkane", 21), ("alkane", 22),
+                                    ("alkane", 42), ("alkane", 43), ("halo", 3), ("halo", 12)])
+def test_subspace_and_full_diagonalisation_agree(monkeypatch, kind, n):
+    from xtb_amd import workloads as w
+    z, x = _halogenated(n, 3) if kind == "halo" else (w.water_cluster if kind == "water" else w.alkane)(n, 3)
+    (full, cf), (sub, cs) = _both(monkeypatch, [(z, x, 0.0, 0)])
+    _check(full[0], sub[0], f"{kind} {n}")
+    if len(x) > 40:   # the path was taken: fewer Jacobi rounds
+        assert cs[1] < cf[1], (cs, cf)
+
+
+@pytest.mark.parametrize("kw,solvent", [({"etemp": 0.0}, None), ({"etemp": 1000.0}, None), ({"etemp": 9000.0}, None),
+                                        ({"guess": "sad"}, None), ({"accuracy": 0.01}, None), ({"maxiter": 3}, None),
+                                        ({}, "water")])
+def test_subspace_options_agree(monkeypatch, kw, solvent):
+    """Smearing (at 9000 K every molecule keeps the full diagonalisation), the
+    SAD guess, tight accuracy, a run cut off before convergence and solvent."""
+    from xtb_amd import workloads as w
+    mols = [w.water_cluster(9, 1), w.alkane(14, 2), w.water_cluster(1, 4), _halogenated(6, 5)]
+    (full, _), (sub, _) = _both(monkeypatch, [(z, x, 0.0, 0) for z, x in mols], solvent, **kw)
+    for k, (a, b) in enumerate(zip(full, sub)):
+        _check(a, b, f"{kw} mol {k}")
+
+
+def test_subspace_small_gaps_ions_and_open_shells(monkeypatch, golden):
+    """Gaps of 0.7 to 3 eV (given up or never taken), charged and open-shell
+    molecules beside gapped ones in one batch."""
+    from xtb_amd import workloads as w
+    mols = []
+    for k in ("mindless01", "mindless02", "mindless05", "mindless07", "mindless09"):
+        g = golden[k]
+        mols.append((np.array(g["numbers"]), np.array(g["positions"]), g["charge"], g["uhf"]))
+    z, x = w.water_cluster(2, 3)
+    mols.append((z[:-1], x[:-1], -1.0, 0))           # HO-(H2O)
+    za, xa = w.alkane(8, 3)
+    mols.append((za[:-1], xa[:-1], 0.0, 1))          # radical
+    mols.append((za[:-1], xa[:-1], 1.0, 0))          # cation
+    mols.append((za, xa, 0.0, 2))                    # triplet
+    mols.append((np.array([2]), np.zeros((1, 3)), 0.0, 0))
+    mols.append((za, xa, 0.0, 0))
+    (full, _), (sub, _) = _both(monkeypatch, mols)
+    for k, (a, b) in enumerate(zip(full, sub)):
+        _check(a, b, f"mol {k}")

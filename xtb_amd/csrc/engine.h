@@ -44,6 +44,7 @@ struct MolState {
   int lastdiag;
   int active;      // still iterating
   int failed;      // error code (0 = fine)
+  int diag;        // full diagonalisation in the current iteration (else the subspace path, k_sub.hip)
   int ihomoa, ihomob, ihomo;
   double eel, eold, egap, ees, eaes, epol, ed, ga, gb, rmsq, efa, efb;
   double eh0;      // Tr(P H0) in eV
@@ -251,7 +252,13 @@ class Batch {
   void setup();
   // returns true while any molecule is active; queue_next: queue the next
   // iteration's first part before waiting for the host's count
-  bool scc_iteration(bool queue_next = false);
+  // subspace: molecules with a gap may take the subspace path (k_sub.hip)
+  // between their first and last diagonalisation; orbitals() must follow
+  // when they have stopped iterating
+  bool scc_iteration(bool queue_next = false, bool subspace = false);
+  // orbitals, orbital energies and occupations of the molecules that stopped
+  // iterating on the subspace path
+  void orbitals();
   void scc_prologue();
   bool prologue_queued_ = false;
   void gradient();
@@ -333,7 +340,7 @@ class Batch {
   int* at = nullptr;
   double *xyz = nullptr, *cn = nullptr, *cn_d4 = nullptr, *cn_eeq = nullptr, *cn_cov = nullptr;
   double *q = nullptr, *dipm = nullptr, *qp = nullptr, *radcn = nullptr;
-  double *vs = nullptr, *vd = nullptr, *vq = nullptr, *ashift = nullptr;
+  double *vs = nullptr, *vd = nullptr, *vq = nullptr;
   double *grad = nullptr, *dhdcn = nullptr, *dedcn = nullptr, *tmp2 = nullptr, *eat = nullptr;
   double *grad_atm = nullptr, *dedcn_atm = nullptr;   // ATM gradient and dE/dCN terms of the set-up
   double *ae01 = nullptr;   // per-atom AES energy partials (3 per atom)
@@ -404,6 +411,22 @@ class Batch {
   // start, to the block-Jacobi lanes
   int eig_blk_iters = 1 << 30;
   int jac_period_ = 1;   // rounds between the lanes' progress tests
+  // the subspace path (k_sub.hip): per-molecule state, residual maxima and
+  // step factors, counts, and its product tiles (a launch's tiles are
+  // [sub_t0[k], sub_t0[k + 1]) of d_sub_tiles); XTBAMD_SUBSPACE=0 turns it off
+  bool subspace_on = true;
+  static constexpr int kSubLists = 8;
+  int sub_t0[kSubLists + 1] = {};
+  long long sub_tiles_cap_ = 0;
+  int4* d_sub_tiles = nullptr;
+  int *sub_ = nullptr, *sub_cnt_ = nullptr;
+  unsigned long long* sub_res_ = nullptr;
+  double* sub_dbl_ = nullptr;
+  int sub_guess_ = 6;   // steps queued before the first count is read
+  void subspace(bool allow);
+  bool final_ = false;      // diagonalise() is orbitals()' one
+  bool need_full_ = true;   // some molecule takes the full diagonalisation
+  void diagonalise();       // of the molecules with MolState::diag: C, emo, occupations
   EigSet eig_;
   void eig_build();
   // the blocked eigensolver on eig_'s problems: A from Am (Jacobi problem
@@ -453,7 +476,7 @@ class Batch {
   unsigned long long* oa_stat = nullptr;
   // sym: the product is symmetric (computed on the b >= a tiles, mirrored)
   void gemm(int kind, const double* a, const double* b, double* c, const double* scale, const int* perm,
-            bool check_active, double alpha = 1.0, const int* mask = nullptr, bool sym = false);
+            bool check_active, double alpha = 1.0, const int* mask = nullptr, bool sym = false, int mask_stride = 1);
   void orthogonalizer();   // C = S^(-1/2) by Newton-Schulz iterations
   void eeq_solve();        // EEQ charges by Gaussian elimination
 

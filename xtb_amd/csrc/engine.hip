@@ -26,6 +26,7 @@
 #include "k_scc.hip"
 #include "k_setup.hip"
 #include "k_solv.hip"
+#include "k_sub.hip"
 
 #define HIPCHECK(x)                                                                              \
   do {                                                                                           \
@@ -771,6 +772,7 @@ void Batch::init_common() {
   trace_rounds = std::getenv("XTBAMD_TRACE_ROUNDS") != nullptr;
   if (const char* r = std::getenv("XTBAMD_JAC_LANES")) jac_lanes = std::min(kMaxLanes, std::max(1, std::atoi(r)));
   if (const char* r = std::getenv("XTBAMD_EIG_BLK_MIN")) eig_blk_min = std::max(65, std::atoi(r));
+  if (const char* r = std::getenv("XTBAMD_SUBSPACE")) subspace_on = std::atoi(r) != 0;
   if (const char* r = std::getenv("XTBAMD_EIG_BLK_ITERS")) eig_blk_iters = std::max(0, std::atoi(r));
   if (on_loan()) {
     // the lender's streams and events (created and kept by the lender)
@@ -828,7 +830,7 @@ void Batch::allocate(const Capacity& c) {
   xyz = alloc<double>(3 * tn);
   cn = alloc<double>(tn); cn_d4 = alloc<double>(tn); cn_eeq = alloc<double>(tn); cn_cov = alloc<double>(tn);
   q = alloc<double>(tn); dipm = alloc<double>(3 * tn); qp = alloc<double>(6 * tn); radcn = alloc<double>(tn);
-  vs = alloc<double>(tn); vd = alloc<double>(3 * tn); vq = alloc<double>(6 * tn); ashift = alloc<double>(tn);
+  vs = alloc<double>(tn); vd = alloc<double>(3 * tn); vq = alloc<double>(6 * tn);
   grad = alloc<double>(3 * tn); dhdcn = alloc<double>(tn); dedcn = alloc<double>(tn);
   grad_atm = alloc<double>(3 * tn); dedcn_atm = alloc<double>(tn);
   tmp2 = alloc<double>(tn); eat = alloc<double>(tn); ae01 = alloc<double>(2 * tn);
@@ -872,6 +874,12 @@ void Batch::allocate(const Capacity& c) {
   G = alloc<double>(tmm);
   jac_nactive = alloc<int>(kMaxLanes);
   d_state_stage = alloc<MolState>(nmol);
+  sub_ = alloc<int>((long long)nmol * kSubInts);
+  HIPCHECK(hipMemset(sub_, 0, (size_t)nmol * kSubInts * sizeof(int)));
+  sub_cnt_ = alloc<int>(4);
+  sub_res_ = alloc<unsigned long long>((long long)nmol * kSubRes);
+  sub_dbl_ = alloc<double>((long long)nmol * kSubDbls);
+  HIPCHECK(hipMemset(sub_dbl_, 0, (size_t)nmol * kSubDbls * sizeof(double)));
   eeq_failed = alloc<int>(nmol);
   eeq_big = alloc<int>(nmol);
   eig_failed = alloc<int>(nmol);
@@ -895,8 +903,8 @@ void Batch::allocate(const Capacity& c) {
   js.offmax = alloc<unsigned long long>(2LL * nmol);   // two sweep-parity buffers
   js.state = alloc<int>((long long)nmol * kJacState);
   js.scale = alloc<double>(nmol);
-  // pivot-factor buffer: at most (nao/64 + 1) pairs per molecule
-  js.qsize = std::max(4096LL, (c.nao / 64 + 2LL * nmol) * 4096LL);
+  // pivot-factor buffer: at most nao / jac_p + 1 pairs of jac_p^2 per molecule
+  js.qsize = std::max(4096LL, (c.nao / jac_p + 2LL * nmol) * (long long)jac_p * jac_p);
   js.qbuf = alloc<double>(js.qsize);
   js.rot = alloc<int>(js.qsize / 1024 + 1);
   js.perm = nullptr;
@@ -1063,6 +1071,41 @@ void Batch::rebuild() {
   grow(d_tiles, tiles_cap_, std::max<long long>(1, ntiles + ntiles_sym));
   if (ntiles)
     HIPCHECK(hipMemcpyAsync(d_tiles, tl.data(), tl.size() * sizeof(int4), hipMemcpyHostToDevice, stream));
+  // product tiles of the subspace path, in the order of its launches
+  {
+    std::vector<int4> st;
+    auto add = [&](int kind, bool sym) {
+      for (int m = 0; m < nmol; ++m) {
+        const MolDesc& d = desc[m];
+        const int o = d.nel / 2, v = d.nao - o;
+        if (!occupied_[m] || d.nopen != 0 || (d.nel & 1) || o < 1 || v < 1) continue;
+        const int rows = kind == kSubR ? v : (kind == kSubB || kind == kSubCY || kind == kSubCYZ || kind == kSubP)
+                                                 ? d.nao : o;
+        const int cols = kind == kSubP ? d.nao : o;
+        for (int a = 0; a < (rows + kTile - 1) / kTile; ++a)
+          for (int b = sym ? a : 0; b < (cols + kTile - 1) / kTile; ++b)
+            st.push_back(make_int4(m, a, b, kind | (sym ? kSubSym : 0)));
+      }
+    };
+    int k = 0;
+    auto launch = [&](std::initializer_list<std::pair<int, bool>> kinds) {
+      sub_t0[k++] = (int)st.size();
+      for (auto& p : kinds) add(p.first, p.second);
+    };
+    launch({{kSubB, false}});
+    launch({{kSubR, false}});
+    launch({{kSubM, true}});
+    launch({{kSubCY, false}, {kSubE1, true}});
+    launch({{kSubZ2, true}, {kSubE, true}});
+    launch({{kSubZ, true}, {kSubE, true}});
+    launch({{kSubCYZ, false}});
+    launch({{kSubP, true}});
+    sub_t0[k] = (int)st.size();
+    grow(d_sub_tiles, sub_tiles_cap_, std::max<long long>(1, (long long)st.size()));
+    if (!st.empty())
+      HIPCHECK(hipMemcpyAsync(d_sub_tiles, st.data(), st.size() * sizeof(int4), hipMemcpyHostToDevice, stream));
+    HIPCHECK(hipStreamSynchronize(stream));   // st goes out of scope
+  }
   // Jacobi problems: dim nao, matrices at m0, eigenvalues at o0
   JacSet& js = jac_n;
   long long qoff = 0;
@@ -1380,7 +1423,7 @@ bool Batch::jacobi(JacSet& js, double* Am, double* Wm, double* evout, bool check
   const bool lanes = rows && !pivot_lds && js.npairs > 0;
   // the largest problems go to the blocked eigensolver on stream3 (after the
   // small ones), beside the lanes
-  const bool blk = rows && !pivot_lds && eig_.np > 0 && iterations_ < eig_blk_iters;
+  const bool blk = rows && !pivot_lds && eig_.np > 0 && (iterations_ < eig_blk_iters || (final_ && eig_blk_iters > 0));
   // the blocked path's problems are marked done for the lanes
   if (blk)
     hipLaunchKernelGGL(k_eig_claim, dim3(1), dim3(256), 0, stream, (const EigProb*)eig_.d_probs, eig_.np, js.state);
@@ -2035,13 +2078,13 @@ void Batch::set_guess(int m, const double* qsh_in, const double* dipm_in, const 
 }
 
 void Batch::gemm(int kind, const double* a, const double* b, double* c, const double* scale_, const int* perm_,
-                 bool check_active, double alpha, const int* mask, bool sym) {
+                 bool check_active, double alpha, const int* mask, bool sym, int mask_stride) {
   const int4* tiles = sym ? d_tiles + ntiles : d_tiles;
   const int nt = sym ? ntiles_sym : ntiles;
   if (nt <= 0) return;
   // SCC-active molecules: the 'active' field of MolState, read with its stride
   const int* m = mask;
-  int ms = 1;
+  int ms = mask_stride;
   if (check_active) {
     m = &d_state[0].active;
     ms = (int)(sizeof(MolState) / sizeof(int));
@@ -2467,14 +2510,71 @@ void Batch::scc_prologue() {
   mixed_here_ = false;
 }
 
-bool Batch::scc_iteration(bool queue_next) {
-  const long long rounds_before = jacobi_rounds_;
-  const Element* el = elements_dev;
-  if (prologue_queued_) prologue_queued_ = false;
-  else scc_prologue();
+// The density of the molecules that may take the subspace path; the others
+// (and those that give up) are left with MolState::diag = 1 and counted into
+// need_full_.  Convergence is decided per molecule on the device; the host
+// queues as many steps as the last iteration took, then the products of the
+// density of whatever converged, and reads the counts while those run.
+void Batch::subspace(bool allow) {
+  allow = allow && subspace_on && !use_ql && oa_max_steps == 0 && !mixed && sub_t0[kSubLists] > 0;
+  const double kt = kBoltzmann * kAutoEV * opt.etemp;
+  hipLaunchKernelGGL(k_sub_begin, dim3(nmol), dim3(256), 0, stream, d_desc, d_state, (const double*)A, ev, sub_,
+                     sub_res_, sub_dbl_, jac_tol, std::max(1.0, opt.etemp > 0.1 ? kSubGapKt * kt : 0.0),
+                     allow ? 1 : 0);
+  need_full_ = true;
+  if (!allow) return;
+  hipLaunchKernelGGL(k_sub_start, dim3(gstride((long long)max_nao * max_nao / 4 + 1), nmol), dim3(256), 0, stream, d_desc,
+                     (const double*)A, (const double*)ev, (const int*)sub_, Sm);
+  const SubBufs bf{A, C, ev, Sm, G, T, W, H, P};
+  auto product = [&](int list, int step, int level) {
+    const int nt = sub_t0[list + 1] - sub_t0[list];
+    if (nt <= 0) return;
+    const int4* tl = d_sub_tiles + sub_t0[list];
+    if (list == 2)
+      hipLaunchKernelGGL((k_sub_gemm<true, false>), dim3(nt), dim3(256), 0, stream, tl, d_desc, bf, (const int*)sub_,
+                         sub_res_, sub_dbl_, step, level);
+    else if (list == 7)
+      hipLaunchKernelGGL((k_sub_gemm<false, true>), dim3(nt), dim3(256), 0, stream, tl, d_desc, bf, (const int*)sub_,
+                         sub_res_, sub_dbl_, step, level);
+    else
+      hipLaunchKernelGGL((k_sub_gemm<false, false>), dim3(nt), dim3(256), 0, stream, tl, d_desc, bf, (const int*)sub_,
+                         sub_res_, sub_dbl_, step, level);
+  };
+  int step = 0, upto = std::min(kSubSteps, std::max(1, sub_guess_));
+  for (;;) {
+    for (; step < upto; ++step) {
+      product(0, step, 0);
+      product(1, step, 0);
+    }
+    hipLaunchKernelGGL(k_sub_outcome, dim3(grid1(nmol, 64)), dim3(64), 0, stream, d_state, nmol, sub_,
+                       (const unsigned long long*)sub_res_, (const double*)sub_dbl_, step);
+    product(2, 0, 0);
+    product(3, 0, 0);
+    product(4, 0, 2);
+    product(5, 0, 3);
+    hipLaunchKernelGGL(k_sub_check, dim3(1), dim3(256), 0, stream, (const MolDesc*)d_desc, d_state, nmol, sub_,
+                       (const unsigned long long*)sub_res_, sub_cnt_);
+    HIPCHECK(hipMemcpyAsync(h_pinned + 8, sub_cnt_, 3 * sizeof(int), hipMemcpyDeviceToHost, stream));
+    HIPCHECK(hipEventRecord(ev_join3, stream));
+    product(5, 0, 4);
+    product(6, 0, 0);
+    product(7, 0, 0);
+    HIPCHECK(hipEventSynchronize(ev_join3));
+    if (h_pinned[8] <= 0 || step >= kSubSteps) break;
+    upto = std::min(kSubSteps, step + 2);
+  }
+  need_full_ = h_pinned[9] > 0;
+  sub_guess_ = std::max(1, h_pinned[10]);
+}
+
+// C, orbital energies and occupations of the molecules with MolState::diag
+// from A = C^T H C
+void Batch::diagonalise() {
   // C holds the previous eigenvectors from the second iteration on: A is
   // nearly diagonal, refine W = I towards its eigenvectors with GEMMs first
   const bool warm = iterations_ > 0 && oa_max_steps > 0;
+  const int* mask = &d_state[0].diag;
+  constexpr int ms = (int)(sizeof(MolState) / sizeof(int));
   if (warm) {
     hipLaunchKernelGGL(k_ident_active, dim3(grid1((long long)max_nao * max_nao, 256), nmol), dim3(256), 0, stream,
                        d_desc, (const MolState*)d_state, W);
@@ -2490,22 +2590,47 @@ bool Batch::scc_iteration(bool queue_next) {
     fold_diag();
     hipLaunchKernelGGL(k_fail_fold, dim3(grid1(nmol, 64)), dim3(64), 0, stream, d_state, nmol,
                        (const int*)eig_failed, 1, kFailDiag, (const int*)nullptr);
-    gemm(4, C, W, T, nullptr, perm, true);    // T = C W(perm, :)^T
+    gemm(4, C, W, T, nullptr, perm, false, 1.0, mask, false, ms);    // T = C W(perm, :)^T
   } else {
     const bool rows = jacobi(jac_n, A, W, emo, true, warm, warm ? banded_passes : 0);
     fold_diag();
     if (rows)
-      gemm(4, C, W, T, nullptr, perm, true);  // T = C W(perm, :)^T
+      gemm(4, C, W, T, nullptr, perm, false, 1.0, mask, false, ms);  // T = C W(perm, :)^T
     else
-      gemm(3, C, W, T, nullptr, perm, true);  // T = C W(:, perm)
+      gemm(3, C, W, T, nullptr, perm, false, 1.0, mask, false, ms);  // T = C W(:, perm)
   }
-  hipLaunchKernelGGL(k_copy_active, dim3(gstride((long long)max_nao * max_nao), nmol), dim3(256), 0, stream,
+  hipLaunchKernelGGL(k_copy_diag, dim3(gstride((long long)max_nao * max_nao), nmol), dim3(256), 0, stream,
                      d_desc, (const MolState*)d_state, (const double*)T, C);
+}
+
+void Batch::orbitals() {
+  if (!subspace_on) return;
+  hipLaunchKernelGGL(k_sub_pending, dim3(1), dim3(256), 0, stream, d_state, nmol, sub_, sub_cnt_);
+  HIPCHECK(hipMemcpyAsync(h_pinned + 8, sub_cnt_, sizeof(int), hipMemcpyDeviceToHost, stream));
+  HIPCHECK(hipStreamSynchronize(stream));
+  if (h_pinned[8] <= 0) return;
+  final_ = true;
+  diagonalise();
+  final_ = false;
   hipLaunchKernelGGL(k_occ_fermi, dim3(nmol), dim3(256), 0, stream, d_desc, d_state, (const double*)emo, focca, foccb,
-                     focc, opt.etemp, (const double*)qsh, (const double*)dipm, (const double*)qp, q_in);
-  mixed_here_ = true;
-  gemm(2, C, C, P, focc, nullptr, true, 1.0, nullptr, true);      // P = C diag(f) C^T (symmetric)
-  mixed_here_ = false;
+                     focc, opt.etemp, (const double*)qsh, (const double*)dipm, (const double*)qp, q_in, 1);
+}
+
+bool Batch::scc_iteration(bool queue_next, bool subspace_ok) {
+  const long long rounds_before = jacobi_rounds_;
+  const Element* el = elements_dev;
+  if (prologue_queued_) prologue_queued_ = false;
+  else scc_prologue();
+  subspace(subspace_ok);
+  if (need_full_) diagonalise();
+  hipLaunchKernelGGL(k_occ_fermi, dim3(nmol), dim3(256), 0, stream, d_desc, d_state, (const double*)emo, focca, foccb,
+                     focc, opt.etemp, (const double*)qsh, (const double*)dipm, (const double*)qp, q_in, 0);
+  if (need_full_) {
+    mixed_here_ = true;
+    gemm(2, C, C, P, focc, nullptr, false, 1.0, &d_state[0].diag, true,
+         (int)(sizeof(MolState) / sizeof(int)));      // P = C diag(f) C^T (symmetric)
+    mixed_here_ = false;
+  }
   hipLaunchKernelGGL(k_population, dim3(grid1(max_nao, 4), nmol), dim3(256), 0, stream, d_desc, (const double*)P,
                      (const double*)S, (const double*)H0, (const double*)D, (const double*)Q, row_q, row_e, row_d,
                      row_qp, (const MolState*)d_state, 0);
@@ -2637,10 +2762,11 @@ void Batch::run() {
   int guard = 0;
   prologue_queued_ = false;
   // (no iteration is queued ahead of the guard's stop)
-  while (scc_iteration(guard + 1 <= opt.maxiter + 2)) {
+  while (scc_iteration(guard + 1 <= opt.maxiter + 2, true)) {
     if (++guard > opt.maxiter + 2) break;
   }
   prologue_queued_ = false;
+  orbitals();
   gradient();
   // the final shell charges and moments of every molecule are on the device
   wfn_valid_ = true;
@@ -2801,7 +2927,7 @@ int Server::step() {
   }
   if (running() == 0) return queued();
   // 2. one SCC iteration of every resident molecule
-  batch.scc_iteration();
+  batch.scc_iteration(false, true);
   // 3. completion: gradient and results of the molecules that stopped iterating
   hipLaunchKernelGGL(k_active_flags, dim3((batch.nmol + 255) / 256), dim3(256), 0, batch.stream,
                      (const MolState*)batch.d_state, batch.nmol, d_active_);
@@ -2812,6 +2938,7 @@ int Server::step() {
   for (int m = 0; m < batch.nmol; ++m)
     if (slot_req_[m] >= 0 && !active_host_[m]) fin.push_back(m);
   if (!fin.empty()) {
+    batch.orbitals();
     batch.select(fin);
     batch.gradient();
     for (int m : fin) {

@@ -902,13 +902,13 @@ __global__ void k_eig_claim(const EigProb* __restrict__ probs, int np, int* jsta
 }
 
 // the problems' matrices into the solver's layout (problems of molecules
-// that no longer iterate are switched off)
+// that are not diagonalised are switched off)
 __global__ void __launch_bounds__(256) k_eig_in(const EigProb* __restrict__ probs, const JacobiProb* __restrict__ jp,
                                                 const MolState* __restrict__ mstate, int* act,
                                                 const double* __restrict__ Asrc, double* Aw) {
   const EigProb p = probs[blockIdx.y];
   const JacobiProb q = jp[p.mol];
-  const bool on = !mstate || mstate[p.mol].active;
+  const bool on = !mstate || mstate[p.mol].diag;
   if (blockIdx.x == 0 && threadIdx.x == 0) act[blockIdx.y] = on ? 1 : 0;
   if (!on) return;
   const int n = p.n;

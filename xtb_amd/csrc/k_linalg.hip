@@ -1780,7 +1780,7 @@ __global__ void __launch_bounds__(256) k_jac_init(const JacobiProb* __restrict__
   __shared__ double sh[4];
   const JacobiProb pr = probs[blockIdx.x];
   int* st = state + blockIdx.x * kJacState;
-  if (mstate && !mstate[blockIdx.x].active) {
+  if (mstate && !mstate[blockIdx.x].diag) {
     if (threadIdx.x == 0) {
       for (int i = 0; i < kJacState; ++i) st[i] = 0;
       st[0] = 1;
@@ -1822,7 +1822,7 @@ __global__ void __launch_bounds__(256) k_jac_init(const JacobiProb* __restrict__
 __global__ void __launch_bounds__(256) k_jac_pad(const JacobiProb* __restrict__ probs, const double* __restrict__ src,
                                                  double* dst, const MolState* __restrict__ mstate, int in) {
   const int p = blockIdx.y;
-  if (mstate && !mstate[p].active) return;
+  if (mstate && !mstate[p].diag) return;
   const JacobiProb pr = probs[p];
   const long long n = pr.dim;
   for (long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < n * n; e += (long long)gridDim.x * blockDim.x) {
@@ -2049,7 +2049,7 @@ __global__ void __launch_bounds__(256) k_tred_ql(const JacobiProb* __restrict__ 
   __shared__ double sc[4];
   __shared__ int ctl[4];
   const int pidx = list[blockIdx.x];
-  if (mstate && !mstate[pidx].active) return;
+  if (mstate && !mstate[pidx].diag) return;
   const JacobiProb pr = probs[pidx];
   const int N = pr.dim;
   // vectors in LDS when they fit, else in the problem's scratch matrix
@@ -2231,7 +2231,7 @@ __global__ void __launch_bounds__(256) k_jac_sort(const JacobiProb* __restrict__
                                                   int max_dim) {
   __shared__ double dg[2048];
   const int p = blockIdx.y;
-  if (mstate && !mstate[p].active) return;
+  if (mstate && !mstate[p].diag) return;
   const JacobiProb pr = probs[p];
   if (pr.dim > max_dim) return;
   const int n = pr.dim, ld = pr.ld;
@@ -2261,7 +2261,7 @@ __global__ void __launch_bounds__(256) k_jac_sort(const JacobiProb* __restrict__
 __global__ void __launch_bounds__(256) k_jac_ident(const JacobiProb* __restrict__ probs, double* W,
                                                    const MolState* __restrict__ mstate) {
   const int p = blockIdx.y;
-  if (mstate && !mstate[p].active) return;
+  if (mstate && !mstate[p].diag) return;
   const JacobiProb pr = probs[p];
   const long long n = pr.dim;
   for (long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < n * n; e += (long long)gridDim.x * blockDim.x) {
@@ -2288,11 +2288,11 @@ __global__ void k_count_active(const MolState* __restrict__ st, int nmol, int* o
   if (threadIdx.x == 0) out[0] = (int)c;
 }
 
-// C <- T for the molecules still iterating
-__global__ void k_copy_active(const MolDesc* __restrict__ desc, const MolState* __restrict__ st,
+// C <- T for the molecules that were diagonalised
+__global__ void k_copy_diag(const MolDesc* __restrict__ desc, const MolState* __restrict__ st,
                               const double* __restrict__ T, double* C) {
   const MolDesc md = desc[blockIdx.y];
-  if (!st[blockIdx.y].active) return;
+  if (!st[blockIdx.y].diag) return;
   const long long n2 = (long long)md.nao * md.nao;
   for (long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x; t < n2; t += (long long)gridDim.x * blockDim.x) C[md.m0 + t] = T[md.m0 + t];
 }

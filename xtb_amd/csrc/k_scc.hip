@@ -239,16 +239,36 @@ __device__ void fermi_channel(int norbs, int nel, double t, const double* eig, d
   s_out = s * kBoltzmann * t;
 }
 
-// occupations, Fermi smearing, HOMO-LUMO gap and the Broyden input vector
+// occupations, Fermi smearing, HOMO-LUMO gap (of the molecules that were
+// diagonalised) and the Broyden input vector (not after the last iteration:
+// final != 0).  A molecule on the subspace path has whole occupations, so
+// its entropy terms vanish.
 __global__ void __launch_bounds__(256) k_occ_fermi(const MolDesc* __restrict__ desc, MolState* state,
                                                    const double* __restrict__ emo, double* focca, double* foccb,
                                                    double* focc, double etemp, const double* __restrict__ qsh,
                                                    const double* __restrict__ dipm, const double* __restrict__ qp,
-                                                   double* q_in) {
+                                                   double* q_in, int final) {
   __shared__ double sh[4];
   const MolDesc md = desc[blockIdx.x];
   MolState& st = state[blockIdx.x];
-  if (!st.active) return;
+  if (final ? !st.diag : !st.active) return;
+  if (!final) {
+    // save the input charges / moments (gfn2broyden_save: src/aespot.F90:1384-1403)
+    double* qi = q_in + md.v0;
+    for (int k = threadIdx.x; k < md.nbr; k += blockDim.x) {
+      double v;
+      if (k < md.nsh) v = qsh[md.s0 + k];
+      else {
+        const int r = k - md.nsh, a = r / 9, c = r % 9;
+        v = c < 3 ? dipm[3 * (md.a0 + a) + c] : qp[6 * (md.a0 + a) + c - 3];
+      }
+      qi[k] = v;
+    }
+    if (!st.diag) {
+      if (threadIdx.x == 0) st.ga = st.gb = 0.0;
+      return;
+    }
+  }
   const int N = md.nao;
   const double* e = emo + md.o0;
   double* fa = focca + md.o0;
@@ -268,17 +288,6 @@ __global__ void __launch_bounds__(256) k_occ_fermi(const MolDesc* __restrict__ d
   }
   __syncthreads();
   for (int i = threadIdx.x; i < N; i += blockDim.x) focc[md.o0 + i] = fa[i] + fb[i];
-  // save the input charges / moments (gfn2broyden_save: src/aespot.F90:1384-1403)
-  double* qi = q_in + md.v0;
-  for (int k = threadIdx.x; k < md.nbr; k += blockDim.x) {
-    double v;
-    if (k < md.nsh) v = qsh[md.s0 + k];
-    else {
-      const int r = k - md.nsh, a = r / 9, c = r % 9;
-      v = c < 3 ? dipm[3 * (md.a0 + a) + c] : qp[6 * (md.a0 + a) + c - 3];
-    }
-    qi[k] = v;
-  }
   if (threadIdx.x == 0) {
     if (st.ihomo + 1 <= N && st.ihomo >= 1) st.egap = e[st.ihomo] - e[st.ihomo - 1];
     st.ga = ga;

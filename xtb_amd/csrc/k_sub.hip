@@ -1,0 +1,453 @@
+// Density of a closed-shell molecule with an orbital gap without a full
+// diagonalisation: between the first and the last SCC iteration only the
+// density is needed, and with every occupation 0 or 2 it depends on the
+// occupied subspace alone, not on the orbitals inside it.
+//
+// C keeps the orbitals of the molecule's last full diagonalisation (o
+// occupied, v virtual columns).  In that basis the Fock matrix A = C^T H C of
+// a later iteration is close to diagonal, and its occupied subspace is the
+// span of Y = [I; X] with the v x o matrix X that solves
+//
+//     R(X) = A_vo + A_vv X - X (A_oo + A_ov X) = 0.
+//
+// X starts from the previous iteration's and takes X -= R / D, D = a_vv - a_oo
+// (element-wise, the diagonals) until max |R| is as small as the off-diagonal
+// elements of a finished diagonalisation (jac_tol max(max |A_ii|, 1)).  A
+// step is two products of 2 N v o and 2 v o^2 flops.  max |R| falls by 20 to
+// 30 times per step for alkanes (gap 11 eV), by 10 for 32 waters (8 eV) and
+// by 2.5 for 700 waters (4 eV); where it falls by less than 6 times, the step
+// becomes one of the second-order Richardson iteration,
+// X' = X_old + w (X - R / D - X_old), with w for the contraction seen (21 ->
+// 13 steps for 700 waters).  The density is
+// P = 2 (C Y) (I + X^T X)^-1 (C Y)^T with the inverse from the product
+// (I - M)(I + M^2)(I + M^4)(I + M^8), M = X^T X, whose neglected part M^16 is
+// bounded below 1e-16.
+//
+// Why a converged X is the occupied subspace: the plain step is X -> X - D^-1
+// T X with T the (symmetrisable) map Z -> A'_vv Z - Z A'_oo of the decoupled
+// blocks.  It contracts by rho < 1 only if D^-1 T has its spectrum in
+// [1 - rho, 1 + rho] (and the second-order one only if that lies above 0), so
+// T is positive definite and every virtual eigenvalue lies above every
+// occupied one by at least (1 - rho) min D.  The path is left unless that is
+// at least kSubGapKt kT: the Fermi occupations of the frontier orbitals are
+// then within 4e-18 of 1 and 0, no entropy term arises, and the density is
+// the one of the full diagonalisation to rounding.
+#pragma once
+#include "device_util.h"
+#include "engine.h"
+
+namespace xtbamd {
+
+constexpr int kSubSteps = 24;        // steps per SCC iteration at most
+// a molecule that gave up gets a fresh basis from its full diagonalisation,
+// which is closer to the next iterations' orbitals (700 waters: given up on
+// the first basis, 8 to 10 steps on the second); after a second time it
+// stays with full diagonalisations
+constexpr int kSubTries = 2;
+constexpr double kSubGapKt = 80.0;   // smallest gap in units of kT
+constexpr double kSubRhoMax = 0.8;   // largest contraction of a plain step
+constexpr double kSubRhoMin = 0.15;  // smallest contraction that takes the second-order step
+constexpr double kSubDrop = 1e-17;   // a factor I + E of the inverse with o max |E| below this is left out
+constexpr double kSubInvMax = 1e-8;  // largest o max |M^8|: the next factor is its square
+// per-molecule integers (kSubInts each)
+constexpr int kSubPhase = 0;   // 0 full diagonalisation, 1 iterating, 2 converged, 3 given up, 4 density formed
+constexpr int kSubPar = 1;     // which of the two X buffers holds X
+constexpr int kSubX = 2;       // X belongs to the current C
+constexpr int kSubOff = 3;     // attempts given up in this run
+constexpr int kSubPend = 4;    // stopped without orbital energies: one diagonalisation to come
+constexpr int kSubFresh = 5;   // X starts from the first-order guess
+constexpr int kSubNext = 6;    // steps taken in this SCC iteration
+constexpr int kSubInts = 8;
+// residual maxima: one per step, then those of E_2 = M^4 and E_3 = M^8
+constexpr int kSubRes = kSubSteps + 2;
+
+// product kinds (the 64 x 64 tiles of a launch name theirs)
+constexpr int kSubSym = 16;   // the tile is one of a symmetric result
+enum SubOp { kSubB = 0, kSubR, kSubM, kSubCY, kSubE1, kSubZ2, kSubE, kSubZ, kSubCYZ, kSubP };
+
+__device__ __forceinline__ int sub_occ(const MolDesc& md) { return md.nel / 2; }
+
+// per-molecule doubles: tolerance of max |R|, the contraction allowed and the
+// contraction seen, then the factor w of each step
+constexpr int kSubTol = 0, kSubLim = 1, kSubRho = 2, kSubW = 3, kSubDbls = kSubW + kSubSteps;
+
+// the contraction of a plain step that explains max |R| falling by r per step
+// of the second-order iteration with factor w (r > sqrt(w - 1))
+__device__ __forceinline__ double sub_mu(double r, double w) { return (r * r + w - 1.0) / (w * r); }
+
+// step s runs unless an earlier one converged, contracted too slowly or met a
+// NaN (a step that did not run leaves its maximum at 0)
+__device__ __forceinline__ bool sub_step_runs(const unsigned long long* __restrict__ res,
+                                              const double* __restrict__ sd, int s) {
+  if (s == 0) return true;
+  const double r1 = __longlong_as_double((long long)res[s - 1]);
+  if (!(r1 > sd[kSubTol])) return false;
+  if (s < 5) return true;
+  // the mean of three steps: max |R| may rise for one step when w sets in
+  const double r = cbrt(r1 / __longlong_as_double((long long)res[s - 4])), w = sd[kSubW + s - 1];
+  return r * r <= w - 1.0 || sub_mu(r, w) <= sd[kSubLim];
+}
+
+// E_k (k = 2, 3) is left out of the inverse
+__device__ __forceinline__ bool sub_dropped(const unsigned long long* __restrict__ res, int o, int k) {
+  return (double)o * __longlong_as_double((long long)res[kSubSteps + k - 2]) < kSubDrop;
+}
+
+// one workgroup per molecule: which path its SCC iteration takes.  MolState's
+// diag = 1: full diagonalisation.
+__global__ void __launch_bounds__(256) k_sub_begin(const MolDesc* __restrict__ desc, MolState* state,
+                                                   const double* __restrict__ A, double* diag, int* sub,
+                                                   unsigned long long* res, double* dbl, double jac_tol,
+                                                   double min_gap, int allow) {
+  __shared__ double sh[4];
+  const int m = blockIdx.x;
+  const MolDesc md = desc[m];
+  MolState& st = state[m];
+  int* si = sub + m * kSubInts;
+  const int active = st.active, first = st.iter == 0;
+  const int o = sub_occ(md), N = md.nao;
+  const bool able = allow && active && !first && si[kSubOff] < kSubTries && md.nopen == 0 && (md.nel & 1) == 0 && md.n > 1 &&
+                    o >= 1 && o < N;
+  __syncthreads();
+  bool on = false;
+  double top = -1e300, low = -1e300, big = 0.0;   // max occupied, -min virtual
+  if (able) {
+    const double* Am = A + md.m0;
+    for (int i = threadIdx.x; i < N; i += blockDim.x) {
+      const double d = Am[(long long)i * N + i];
+      diag[md.o0 + i] = d;
+      if (i < o) top = fmax(top, d);
+      else low = fmax(low, -d);
+      big = fmax(big, fabs(d));
+    }
+    top = block_max<256>(top, sh);
+    low = block_max<256>(low, sh);
+    big = block_max<256>(big, sh);
+    // the contraction that still guarantees the gap, with room for a rate
+    on = (1.0 - kSubRhoMin) * (-low - top) >= min_gap;
+    for (int s = threadIdx.x; s < kSubRes; s += blockDim.x) res[(long long)m * kSubRes + s] = 0ull;
+  }
+  if (threadIdx.x == 0) {
+    if (first && active) si[kSubOff] = 0;
+    if (active) {
+      si[kSubPend] = 0;
+      si[kSubFresh] = on && !si[kSubX];
+      if (!on || si[kSubFresh]) si[kSubPar] = 0;
+      si[kSubX] = on;
+    }
+    si[kSubPhase] = on ? 1 : 0;
+    si[kSubNext] = 0;
+    st.diag = active && !on ? 1 : 0;
+    if (on) {
+      double* sd = dbl + (long long)m * kSubDbls;
+      sd[kSubTol] = jac_tol * fmax(big, 1.0);
+      sd[kSubLim] = fmin(kSubRhoMax, 1.0 - min_gap / (-low - top));
+      sd[kSubRho] = si[kSubFresh] ? 0.0 : 0.9 * sd[kSubRho];
+    }
+  }
+}
+
+// X = -A_vo / D of the molecules without one
+__global__ void __launch_bounds__(256) k_sub_start(const MolDesc* __restrict__ desc, const double* __restrict__ A,
+                                                   const double* __restrict__ diag, const int* __restrict__ sub,
+                                                   double* X) {
+  const int m = blockIdx.y;
+  if (sub[m * kSubInts + kSubPhase] != 1 || !sub[m * kSubInts + kSubFresh]) return;
+  const MolDesc md = desc[m];
+  const int N = md.nao, o = sub_occ(md), v = N - o;
+  const double* Am = A + md.m0;
+  const double* d = diag + md.o0;
+  for (long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x; t < (long long)v * o;
+       t += (long long)gridDim.x * blockDim.x) {
+    const int i = (int)(t / o), j = (int)(t % o);
+    X[md.m0 + t] = -Am[(long long)(o + i) * N + j] / (d[o + i] - d[j]);
+  }
+}
+
+// Buffers of the products (each N x N per molecule at m0): X, X' in Xb, and
+// G, T, W, H, P as scratch (their own contents are dead between the Fock
+// transform and the density).
+struct SubBufs {
+  const double *A, *C, *diag;
+  double *X, *G, *T, *W, *H, *P;
+};
+
+// One 64 x 64 tile of one product of a molecule; tiles (molecule, row tile,
+// column tile, kind).  Operands through two LDS stages (the loads of the next
+// k-block are in flight during the matrix-core work of the current one).
+// Symmetric results (M, its powers E_k = M^(2^k) and the inverse's partial
+// products Z_k commute, P) are formed on the upper tiles and mirrored.
+// Z_2 = (I - M)(I + E_1), Z_(k+1) = Z_k (I + E_k).
+// step: the step of the kinds kSubB and kSubR; level: k of E_k and Z_k.
+// Buffers: M, E_3 in G, E_1, Z_3 in P, E_2 in H, Z_2, Z_4 in W, C Y in T.
+template <bool TA, bool TB>
+__global__ void __launch_bounds__(256) k_sub_gemm(const int4* __restrict__ tiles, const MolDesc* __restrict__ desc,
+                                                  SubBufs bf, const int* __restrict__ sub, unsigned long long* res,
+                                                  double* dbl, int step, int level) {
+  __shared__ double As[2][kBK][kTile + 1];
+  __shared__ double Bs[2][kBK][kTile + 1];
+  const int4 tl = tiles[blockIdx.x];
+  const int m = tl.x, op = tl.w & 15;
+  const bool sym = (tl.w & kSubSym) != 0;
+  const int* si = sub + m * kSubInts;
+  unsigned long long* rs = res + (long long)m * kSubRes;
+  double* sd = dbl + (long long)m * kSubDbls;
+  const MolDesc md = desc[m];
+  const int N = md.nao, o = sub_occ(md), v = N - o;
+  int par = si[kSubPar];
+  if (op <= kSubR) {
+    if (si[kSubPhase] != 1 || !sub_step_runs(rs, sd, step)) return;
+    par = (par + step) & 1;
+    // the first tile's workgroup sets the factor of this step for the second
+    // product's launch
+    if (op == kSubB && tl.y == 0 && tl.z == 0 && threadIdx.x == 0) {
+      double rho = sd[kSubRho], w = 1.0;
+      if (step >= 3) {
+        const double rr = __longlong_as_double((long long)rs[step - 1]) / __longlong_as_double((long long)rs[step - 3]);
+        const double wl = sd[kSubW + step - 1];
+        if (rr > 1.2 * (wl - 1.0)) rho = fmax(rho, fmin(kSubRhoMax, sub_mu(sqrt(rr), wl)));
+        sd[kSubRho] = rho;
+      }
+      // the plain step is better as long as max |R| falls faster than the
+      // second-order iteration's sqrt(w - 1)
+      if (step > 1 && rho >= kSubRhoMin) {
+        const double wo = 2.0 / (1.0 + sqrt(1.0 - rho * rho));
+        const double r1 = __longlong_as_double((long long)rs[step - 1]) / __longlong_as_double((long long)rs[step - 2]);
+        if (sd[kSubW + step - 1] != 1.0 || r1 * r1 > wo - 1.0) w = wo;
+      }
+      sd[kSubW + step] = w;
+    }
+  } else {
+    if (si[kSubPhase] != 2) return;
+  }
+  const long long vo = (long long)v * o;
+  const double* X = bf.X + md.m0 + par * vo;
+  double* G = bf.G + md.m0;
+  double* T = bf.T + md.m0;
+  double* W = bf.W + md.m0;
+  double* H = bf.H + md.m0;
+  double* P = bf.P + md.m0;
+  const bool e2 = !sub_dropped(rs, o, 2), e3 = e2 && !sub_dropped(rs, o, 3);
+  // result (M x Nc) = op(A) (M x K) op(B)
+  const double *Ap, *Bp;
+  int lda = o, ldb = o, M = o, Nc = o, K = o;
+  switch (op) {
+    case kSubB: Ap = bf.A + md.m0 + o; lda = N; Bp = X; M = N; K = v; break;
+    case kSubR: Ap = X; Bp = G; M = v; break;
+    case kSubM: Ap = X; Bp = X; K = v; break;
+    case kSubCY: Ap = bf.C + md.m0 + o; lda = N; Bp = X; M = N; K = v; break;
+    case kSubE1: Ap = G; Bp = G; break;
+    case kSubZ2: Ap = G; Bp = P; break;
+    case kSubE:
+      if (level > 3 || (level == 3 && !e2)) return;   // the list's third launch forms Z_4 only
+      Ap = Bp = level == 2 ? P : H;
+      break;
+    case kSubZ:
+      if (level == 3 ? !e2 : !e3) return;
+      Ap = level == 3 ? W : P;
+      Bp = level == 3 ? H : G;
+      break;
+    case kSubCYZ: Ap = T; Bp = e2 && !e3 ? P : W; M = N; break;
+    default: Ap = G; Bp = T; M = N; Nc = N; break;
+  }
+  const int row0 = tl.y * kTile, col0 = tl.z * kTile;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int wr = w >> 1, wc = w & 1, i16 = lane & 15, k4 = lane >> 4;
+  double ra[4], rb[4];
+  auto fetch = [&](int kb) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int e = tid + 256 * q;
+      const int gi = row0 + (TA ? (e & 63) : (e >> 4)), gk = kb + (TA ? (e >> 6) : (e & 15));
+      const int gj = col0 + (TB ? (e >> 4) : (e & 63)), gk2 = kb + (TB ? (e & 15) : (e >> 6));
+      ra[q] = (gi < M && gk < K) ? (TA ? Ap[(long long)gk * lda + gi] : Ap[(long long)gi * lda + gk]) : 0.0;
+      rb[q] = (gj < Nc && gk2 < K) ? (TB ? Bp[(long long)gj * ldb + gk2] : Bp[(long long)gk2 * ldb + gj]) : 0.0;
+    }
+  };
+  auto stage = [&](int buf) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int e = tid + 256 * q;
+      if (TA) As[buf][e >> 6][e & 63] = ra[q];
+      else As[buf][e & 15][e >> 4] = ra[q];
+      if (TB) Bs[buf][e & 15][e >> 4] = rb[q];
+      else Bs[buf][e >> 6][e & 63] = rb[q];
+    }
+  };
+  v4d acc[2][2];
+#pragma unroll
+  for (int r = 0; r < 2; ++r)
+#pragma unroll
+    for (int c = 0; c < 2; ++c) acc[r][c] = v4d{0.0, 0.0, 0.0, 0.0};
+  fetch(0);
+  stage(0);
+  __syncthreads();
+  int buf = 0;
+  for (int kb = 0; kb < K; kb += kBK) {
+    const bool more = kb + kBK < K;
+    if (more) fetch(kb + kBK);
+#pragma unroll
+    for (int kk = 0; kk < kBK; kk += 4) {
+      double a[2], b[2];
+#pragma unroll
+      for (int r = 0; r < 2; ++r) a[r] = As[buf][kk + k4][32 * wr + 16 * r + i16];
+#pragma unroll
+      for (int c = 0; c < 2; ++c) b[c] = Bs[buf][kk + k4][32 * wc + 16 * c + i16];
+#pragma unroll
+      for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) acc[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[r], b[c], acc[r][c], 0, 0, 0);
+    }
+    if (more) stage(buf ^ 1);
+    __syncthreads();
+    buf ^= 1;
+  }
+  // maxima on the bit patterns: a NaN counts as the largest value
+  unsigned long long big = 0ull;
+  auto see = [&](double x) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(fabs(x));
+    big = big > b ? big : b;
+  };
+  const double* dg = bf.diag + md.o0;
+#pragma unroll
+  for (int r = 0; r < 2; ++r)
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const int gj = col0 + 32 * wc + 16 * c + i16;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int gi = row0 + 32 * wr + 16 * r + k4 + 4 * i;
+        if (gi >= M || gj >= Nc) continue;
+        if (sym && gi > gj) continue;
+        const long long e = (long long)gi * Nc + gj, et = (long long)gj * Nc + gi;
+        const double x = acc[r][c][i];
+        switch (op) {
+          case kSubB: G[e] = bf.A[md.m0 + (long long)gi * N + gj] + x; break;
+          case kSubR: {
+            const double rr = G[(long long)(o + gi) * o + gj] - x;
+            double* xn = bf.X + md.m0 + (par ^ 1) * vo + e;   // holds the X before this one
+            double x1 = X[e] - rr / (dg[o + gi] - dg[gj]);
+            if (step > 0) {
+              const double x0 = *xn, w = sd[kSubW + step];
+              if (w != 1.0) x1 = x0 + w * (x1 - x0);
+            }
+            *xn = x1;
+            see(rr);
+            break;
+          }
+          case kSubM: G[e] = x; G[et] = x; break;
+          case kSubCY: T[e] = bf.C[md.m0 + (long long)gi * N + gj] + x; break;
+          case kSubE1: P[e] = x; P[et] = x; break;
+          case kSubZ2: {
+            const double z = ((gi == gj ? 1.0 : 0.0) - G[e]) + (P[e] - x);
+            W[e] = z;
+            W[et] = z;
+            break;
+          }
+          case kSubE: {
+            double* E = level == 2 ? H : G;
+            E[e] = x;
+            E[et] = x;
+            see(x);
+            break;
+          }
+          case kSubZ: {
+            double* Z = level == 3 ? P : W;
+            const double z = (level == 3 ? W : P)[e] + x;
+            Z[e] = z;
+            Z[et] = z;
+            break;
+          }
+          case kSubCYZ: G[e] = x; break;
+          default: P[e] = 2.0 * x; P[et] = 2.0 * x; break;
+        }
+      }
+    }
+  if (op == kSubR || op == kSubE) {
+#pragma unroll
+    for (int sft = 32; sft > 0; sft >>= 1) {
+      const unsigned long long ob = __shfl_xor(big, sft, 64);
+      big = big > ob ? big : ob;
+    }
+    if (lane == 0 && big) atomicMax(op == kSubR ? &rs[step] : &rs[kSubSteps + level - 2], big);
+  }
+}
+
+// after the steps [0, nstep): converged molecules to phase 2, given up ones
+// to phase 3 with a full diagonalisation; densities formed before to phase 4
+__global__ void k_sub_outcome(MolState* state, int nmol, int* sub, const unsigned long long* __restrict__ res,
+                              const double* __restrict__ dbl, int nstep) {
+  const int m = blockIdx.x * blockDim.x + threadIdx.x;
+  if (m >= nmol) return;
+  int* si = sub + m * kSubInts;
+  if (si[kSubPhase] == 2) si[kSubPhase] = 4;
+  if (si[kSubPhase] != 1) return;
+  const unsigned long long* rs = res + (long long)m * kSubRes;
+  const double* sd = dbl + (long long)m * kSubDbls;
+  int t = 0;
+  while (t < nstep && sub_step_runs(rs, sd, t)) ++t;
+  si[kSubNext] = t;
+  if (__longlong_as_double((long long)rs[t - 1]) <= sd[kSubTol]) {   // each step so far passed sub_step_runs
+    si[kSubPhase] = 2;
+    si[kSubPar] = (si[kSubPar] + t) & 1;
+    si[kSubPend] = 1;
+  } else if (t < nstep || t >= kSubSteps) {
+    si[kSubPhase] = 3;
+    si[kSubOff] += 1;
+    si[kSubX] = 0;
+    state[m].diag = 1;
+  }
+}
+
+// after the powers of M: a molecule whose inverse would need another factor
+// (X too large) takes the full diagonalisation instead.
+// cnt[0]: still iterating, cnt[1]: full diagonalisations, cnt[2]: most steps
+__global__ void __launch_bounds__(256) k_sub_check(const MolDesc* __restrict__ desc, MolState* state, int nmol,
+                                                   int* sub, const unsigned long long* __restrict__ res, int* cnt) {
+  __shared__ double sh[4];
+  double run = 0.0, full = 0.0, most = 0.0;
+  for (int m = threadIdx.x; m < nmol; m += blockDim.x) {
+    int* si = sub + m * kSubInts;
+    if (si[kSubPhase] == 2) {
+      const double e3 = __longlong_as_double((long long)res[(long long)m * kSubRes + kSubSteps + 1]);
+      if (!(sub_occ(desc[m]) * e3 <= kSubInvMax)) {
+        si[kSubPhase] = 3;
+        si[kSubOff] += 1;
+        si[kSubX] = 0;
+        si[kSubPend] = 0;
+        state[m].diag = 1;
+      }
+    }
+    if (si[kSubPhase] == 1) run += 1.0;
+    if (si[kSubPhase] != 0) most = fmax(most, (double)si[kSubNext]);
+    full += state[m].diag ? 1.0 : 0.0;
+  }
+  run = block_sum<256>(run, sh);
+  full = block_sum<256>(full, sh);
+  most = block_max<256>(most, sh);
+  if (threadIdx.x == 0) {
+    cnt[0] = (int)run;
+    cnt[1] = (int)full;
+    cnt[2] = (int)most;
+  }
+}
+
+// molecules that stopped iterating without orbital energies: diag = 1
+__global__ void __launch_bounds__(256) k_sub_pending(MolState* state, int nmol, int* sub, int* cnt) {
+  __shared__ double sh[4];
+  double c = 0.0;
+  for (int m = threadIdx.x; m < nmol; m += blockDim.x) {
+    int* si = sub + m * kSubInts;
+    const bool p = !state[m].active && !state[m].failed && si[kSubPend];
+    state[m].diag = p ? 1 : 0;
+    if (p) {
+      si[kSubPend] = 0;
+      si[kSubX] = 0;
+      c += 1.0;
+    }
+  }
+  c = block_sum<256>(c, sh);
+  if (threadIdx.x == 0) cnt[0] = (int)c;
+}
+
+}  // namespace xtbamd
