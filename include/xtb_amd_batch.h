@@ -80,6 +80,11 @@ int xtbamd_batch_size(xtbamd_batch b);
 /* work counters of the last run: SCC steps launched, block-Jacobi rounds */
 int xtbamd_batch_counters(xtbamd_batch b, int* scc_steps, long long* jacobi_rounds);
 int xtbamd_batch_get(xtbamd_batch b, int m, xtbamd_result* out);
+/* results of all molecules at once: out[m] gets the sizes and scalars of
+ * molecule m; the array pointers of out[0] (any may be NULL; coeff and density
+ * must be) name arrays for the whole batch, the molecules' values
+ * concatenated in order */
+int xtbamd_batch_get_all(xtbamd_batch b, xtbamd_result* out);
 /* current atomic charges [natoms] of molecule m: after xtbamd_batch_setup the
  * initial guess (EEQ, src/eeq_model.f90:678-1015 via newWavefunction,
  * src/xtb/calculator.f90:462-480; SAD; or the restart guess), after an

@@ -278,7 +278,13 @@ class Batch {
   // for a solvent without parameters.  Takes effect at the next setup().
   void set_solvent(const std::string& name, int kernel, bool alpb, int state = 1, double temperature = 298.15);
   bool solvated() const { return solv_on_; }
-  MolResult result(int m, bool matrices = false) const;
+  // arrays: also the result vectors (else sizes, flags and energies only)
+  MolResult result(int m, bool matrices = false, bool arrays = true) const;
+  // every molecule: sizes, flags and energies, and the result vectors of all
+  // molecules concatenated into dst (gradient, q, qsh, dipm, qp, wbo, emo,
+  // focc; a null pointer skips one)
+  std::vector<MolResult> results(double* const dst[8]) const;
+  MolResult result_head(int m, const MolState& st) const;
   // current atomic charges of molecule m (after setup(): the initial guess)
   void charges(int m, double* out) const;
   int size() const { return nmol; }

@@ -23,6 +23,16 @@ class Result(ctypes.Structure):
         [(k, _dp) for k in ("gradient", "charges", "qsh", "dipm", "qp", "wbo", "emo", "focc", "coeff", "density")]
 
 
+_SCALARS = ("natoms", "nshells", "nao", "iterations", "converged", "failed", "ihomo", "energy", "gnorm",
+            "hl_gap_ev", "e_elec", "e_es", "e_aes", "e_axc", "e_disp", "e_rep", "e_atm", "e_solv")
+# the scalar fields of an array of Result
+_SCALAR_DTYPE = np.dtype({"names": _SCALARS + ("dipole",),
+                          "formats": ["i4" if dict(Result._fields_)[k] is ctypes.c_int else "f8" for k in _SCALARS] +
+                          [("f8", (3,))],
+                          "offsets": [getattr(Result, k).offset for k in _SCALARS + ("dipole",)],
+                          "itemsize": ctypes.sizeof(Result)})
+
+
 def library():
     """Load libxtb_amd.so; raises if it has not been built."""
     global _lib
@@ -47,6 +57,8 @@ def library():
     lib.xtbamd_batch_set_guess.restype = ctypes.c_int
     lib.xtbamd_batch_get.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.POINTER(Result)]
     lib.xtbamd_batch_get.restype = ctypes.c_int
+    lib.xtbamd_batch_get_all.argtypes = [ctypes.c_void_p, ctypes.POINTER(Result)]
+    lib.xtbamd_batch_get_all.restype = ctypes.c_int
     lib.xtbamd_batch_charges.argtypes = [ctypes.c_void_p, ctypes.c_int, _dp]
     lib.xtbamd_batch_charges.restype = ctypes.c_int
     lib.xtbamd_batch_free.argtypes = [ctypes.c_void_p]
@@ -213,14 +225,41 @@ class Batch:
         for k, v in out.items():
             setattr(r, k, _ptr(v))
         self._check(lib.xtbamd_batch_get(self._h, m, ctypes.byref(r)))
-        for k in ("natoms", "nshells", "nao", "iterations", "converged", "failed", "ihomo", "energy", "gnorm",
-                  "hl_gap_ev", "e_elec", "e_es", "e_aes", "e_axc", "e_disp", "e_rep", "e_atm", "e_solv"):
+        for k in _SCALARS:
             out[k] = getattr(r, k)
         out["dipole"] = np.array(r.dipole[:])
         return out
 
     def results(self, matrices=False):
-        return [self.result(m, matrices) for m in range(len(self))]
+        if matrices:
+            return [self.result(m, True) for m in range(len(self))]
+        # the arrays of all molecules in one transfer each, handed out as
+        # each molecule's part
+        nmol = len(self)
+        rs = (Result * nmol)()
+        self._check(self._lib.xtbamd_batch_get_all(self._h, rs))   # sizes first
+        tab = np.frombuffer(rs, dtype=_SCALAR_DTYPE)
+        n, nsh, nao = (tab[k].astype(np.int64) for k in ("natoms", "nshells", "nao"))
+        size = {"gradient": 3 * n, "charges": n, "qsh": nsh, "dipm": 3 * n, "qp": 6 * n, "wbo": n * n, "emo": nao,
+                "focc": nao}
+        flat, end = {}, {}
+        for k, c in size.items():
+            flat[k] = np.empty(int(c.sum()))
+            end[k] = np.concatenate([[0], np.cumsum(c)]).tolist()
+            setattr(rs[0], k, _ptr(flat[k]))
+        self._check(self._lib.xtbamd_batch_get_all(self._h, rs))
+        cols = {k: tab[k].tolist() for k in _SCALARS}
+        dip = tab["dipole"].copy()
+        out = []
+        for m in range(nmol):
+            r = {k: flat[k][end[k][m]:end[k][m + 1]] for k in size}
+            for k, w in (("gradient", 3), ("dipm", 3), ("qp", 6), ("wbo", int(n[m]))):
+                r[k] = r[k].reshape(-1, w)
+            for k, c in cols.items():
+                r[k] = c[m]
+            r["dipole"] = dip[m]
+            out.append(r)
+        return out
 
     def close(self):
         if getattr(self, "_h", None):
@@ -245,8 +284,7 @@ def _fetch(lib, get, check):
     for k, v in out.items():
         setattr(r, k, _ptr(v))
     check(get(ctypes.byref(r)))
-    for k in ("natoms", "nshells", "nao", "iterations", "converged", "failed", "ihomo", "energy", "gnorm",
-              "hl_gap_ev", "e_elec", "e_es", "e_aes", "e_axc", "e_disp", "e_rep", "e_atm", "e_solv"):
+    for k in _SCALARS:
         out[k] = getattr(r, k)
     out["dipole"] = np.array(r.dipole[:])
     return out
@@ -363,8 +401,7 @@ def singlepoint_noalloc(numbers, positions, charge=0.0, uhf=0, accuracy=1.0, ete
                                         float(charge), int(uhf), accuracy, etemp, maxiter, ctypes.byref(r))
     if rc < 0:
         raise RuntimeError(_err(lib))
-    for k in ("natoms", "nshells", "nao", "iterations", "converged", "failed", "ihomo", "energy", "gnorm",
-              "hl_gap_ev", "e_elec", "e_es", "e_aes", "e_axc", "e_disp", "e_rep", "e_atm", "e_solv"):
+    for k in _SCALARS:
         out[k] = getattr(r, k)
     out["dipole"] = np.array(r.dipole[:])
     out["qsh"] = out["qsh"][:r.nshells].copy()
