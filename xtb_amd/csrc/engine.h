@@ -421,7 +421,7 @@ class Batch {
   // step factors, counts, and its product tiles (a launch's tiles are
   // [sub_t0[k], sub_t0[k + 1]) of d_sub_tiles); XTBAMD_SUBSPACE=0 turns it off
   bool subspace_on = true;
-  static constexpr int kSubLists = 8;
+  static constexpr int kSubLists = 9;
   int sub_t0[kSubLists + 1] = {};
   long long sub_tiles_cap_ = 0;
   int4* d_sub_tiles = nullptr;
@@ -480,7 +480,9 @@ class Batch {
   int* oa_act = nullptr;
   int* oa_ok = nullptr;
   unsigned long long* oa_stat = nullptr;
-  // sym: the product is symmetric (computed on the b >= a tiles, mirrored)
+  // sym: the product is symmetric (computed on the b >= a tiles, mirrored).
+  // kind kGemmSymLeft: c = a b with a symmetric
+  static constexpr int kGemmSymLeft = 5;
   void gemm(int kind, const double* a, const double* b, double* c, const double* scale, const int* perm,
             bool check_active, double alpha = 1.0, const int* mask = nullptr, bool sym = false, int mask_stride = 1);
   void orthogonalizer();   // C = S^(-1/2) by Newton-Schulz iterations

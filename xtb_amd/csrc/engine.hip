@@ -1029,6 +1029,34 @@ void Batch::release(int m) {
   HIPCHECK(hipStreamSynchronize(stream));
 }
 
+// Appends the tiles of a launch (per molecule) to out in an order that keeps
+// a molecule on one XCD: workgroup b of a launch runs on XCD b mod kXcds, so
+// the matrices of a molecule are fetched by one L2 only.  Molecules go to the
+// least loaded XCD, largest first; one with more than half an XCD's share is
+// spread over all; short queues are filled with skipped entries (x = -1).
+static void xcd_order(const std::vector<std::vector<int4>>& mt, std::vector<int4>& out) {
+  std::vector<int> order;
+  size_t total = 0;
+  for (size_t m = 0; m < mt.size(); ++m)
+    if (!mt[m].empty()) {
+      order.push_back((int)m);
+      total += mt[m].size();
+    }
+  std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return mt[x].size() > mt[y].size(); });
+  std::vector<std::vector<int4>> q(kXcds);
+  for (int m : order) {
+    const bool spread = 2 * kXcds * mt[m].size() > total;
+    size_t x = 0;
+    for (size_t j = 1; j < q.size(); ++j)
+      if (q[j].size() < q[x].size()) x = j;
+    for (size_t j = 0; j < mt[m].size(); ++j) q[spread ? (x + j) % q.size() : x].push_back(mt[m][j]);
+  }
+  size_t len = 0;
+  for (auto& v : q) len = std::max(len, v.size());
+  for (size_t j = 0; j < len; ++j)
+    for (auto& v : q) out.push_back(j < v.size() ? v[j] : make_int4(-1, 0, 0, 0));
+}
+
 // work lists, grid bounds and descriptor table of the occupied slots
 void Batch::rebuild() {
   max_n = max_nsh = max_nao = max_nd4 = max_nbr = 0;
@@ -1056,14 +1084,19 @@ void Batch::rebuild() {
   };
   // GEMM tiles over (molecule, 64x64 tile)
   std::vector<int4> tl, ts;
-  for (int m = 0; m < nmol; ++m) {
-    if (!occupied_[m]) continue;
-    const int nt = (desc[m].nao + 63) / 64;
-    for (int a = 0; a < nt; ++a)
-      for (int b = 0; b < nt; ++b) {
-        tl.push_back(make_int4(m, a, b, 0));
-        if (b >= a) ts.push_back(make_int4(m, a, b, 1));
-      }
+  {
+    std::vector<std::vector<int4>> ml(nmol), ms(nmol);
+    for (int m = 0; m < nmol; ++m) {
+      if (!occupied_[m]) continue;
+      const int nt = (desc[m].nao + 63) / 64;
+      for (int a = 0; a < nt; ++a)
+        for (int b = 0; b < nt; ++b) {
+          ml[m].push_back(make_int4(m, a, b, 0));
+          if (b >= a) ms[m].push_back(make_int4(m, a, b, 1));
+        }
+    }
+    xcd_order(ml, tl);
+    xcd_order(ms, ts);
   }
   ntiles = (int)tl.size();
   ntiles_sym = (int)ts.size();
@@ -1074,28 +1107,28 @@ void Batch::rebuild() {
   // product tiles of the subspace path, in the order of its launches
   {
     std::vector<int4> st;
-    auto add = [&](int kind, bool sym) {
-      for (int m = 0; m < nmol; ++m) {
-        const MolDesc& d = desc[m];
-        const int o = d.nel / 2, v = d.nao - o;
-        if (!occupied_[m] || d.nopen != 0 || (d.nel & 1) || o < 1 || v < 1) continue;
-        const int rows = kind == kSubR ? v : (kind == kSubB || kind == kSubCY || kind == kSubCYZ || kind == kSubP)
-                                                 ? d.nao : o;
-        const int cols = kind == kSubP ? d.nao : o;
-        for (int a = 0; a < (rows + kTile - 1) / kTile; ++a)
-          for (int b = sym ? a : 0; b < (cols + kTile - 1) / kTile; ++b)
-            st.push_back(make_int4(m, a, b, kind | (sym ? kSubSym : 0)));
-      }
-    };
     int k = 0;
     auto launch = [&](std::initializer_list<std::pair<int, bool>> kinds) {
       sub_t0[k++] = (int)st.size();
-      for (auto& p : kinds) add(p.first, p.second);
+      std::vector<std::vector<int4>> mt(nmol);
+      for (auto& p : kinds)
+        for (int m = 0; m < nmol; ++m) {
+          const MolDesc& d = desc[m];
+          const int kind = p.first, o = d.nel / 2, v = d.nao - o;
+          if (!occupied_[m] || d.nopen != 0 || (d.nel & 1) || o < 1 || v < 1) continue;
+          const int rows = kind == kSubR ? v : kind == kSubB || kind == kSubP ? d.nao : o;
+          const int cols = kind == kSubCY || kind == kSubCYZ || kind == kSubP ? d.nao : o;
+          for (int a = 0; a < (rows + kTile - 1) / kTile; ++a)
+            for (int b = p.second ? a : 0; b < (cols + kTile - 1) / kTile; ++b)
+              mt[m].push_back(make_int4(m, a, b, kind | (p.second ? kSubSym : 0)));
+        }
+      xcd_order(mt, st);
     };
     launch({{kSubB, false}});
     launch({{kSubR, false}});
     launch({{kSubM, true}});
-    launch({{kSubCY, false}, {kSubE1, true}});
+    launch({{kSubCY, false}});
+    launch({{kSubE1, true}});
     launch({{kSubZ2, true}, {kSubE, true}});
     launch({{kSubZ, true}, {kSubE, true}});
     launch({{kSubCYZ, false}});
@@ -2092,8 +2125,8 @@ void Batch::gemm(int kind, const double* a, const double* b, double* c, const do
   prof_begin(1);
   // the mixed-precision option: the Fock transforms and the density product
   // (kinds 0-2) on the FP32 matrix cores with the FP64 residual correction
-  if (mixed && mixed_here_ && kind <= 2) {
-    if (kind == 0)
+  if (mixed && mixed_here_ && (kind <= 2 || kind == kGemmSymLeft)) {
+    if (kind == 0 || kind == kGemmSymLeft)
       hipLaunchKernelGGL((k_gemm_mix<false, false, false>), dim3(nt), dim3(256), 0, stream, tiles, d_desc, a, b, c,
                          scale_, alpha, m, ms);
     else if (kind == 1)
@@ -2105,6 +2138,14 @@ void Batch::gemm(int kind, const double* a, const double* b, double* c, const do
     prof_end(1, m, ms);
     return;
   }
+  // L^T B with L symmetric or stored transposed (every product of the default
+  // path but those with C^T on the right)
+  if (use_mfma && (kind == 1 || kind == kGemmSymLeft)) {
+    hipLaunchKernelGGL(k_gemm_tn, dim3(nt), dim3(256), 0, stream, tiles, d_desc, a, b, c, alpha, m, ms);
+    prof_end(1, m, ms);
+    return;
+  }
+  if (kind == kGemmSymLeft) kind = 0;
 #define XTBAMD_GEMM(K, TA, TB, SC, PM)                                                                              \
   case K:                                                                                                          \
     if (use_mfma)                                                                                                  \
@@ -2286,13 +2327,13 @@ void Batch::orthogonalizer() {
   for (int it = 0; it <= maxit; ++it) {
     double *Y = Yb[it & 1], *Z = Zb[it & 1];
     // Y and Z are polynomials in S: they commute, and Z Y, Y T and T Z are symmetric
-    gemm(0, Z, Y, P, nullptr, nullptr, false, 1.0, ns_act, true);     // P = Z Y
+    gemm(kGemmSymLeft, Z, Y, P, nullptr, nullptr, false, 1.0, ns_act, true);     // P = Z Y
     hipLaunchKernelGGL(k_ns_form, gmm, dim3(256), 0, stream, d_sub, (const int*)ns_act, P, ns_res);
     hipLaunchKernelGGL(k_ns_mark, dim3(1), dim3(256), 0, stream, nmol, ns_stage, ns_act, ns_res, it, maxit, ns_failed,
                        jac_nactive, ns_fin);
     HIPCHECK(hipMemcpyAsync(h_pinned + (it & 1), jac_nactive, sizeof(int), hipMemcpyDeviceToHost, stream));
-    gemm(0, Y, P, Yb[(it + 1) & 1], nullptr, nullptr, false, 1.0, ns_act, true);   // Y T
-    gemm(0, P, Z, Zb[(it + 1) & 1], nullptr, nullptr, false, 1.0, ns_act, true);   // T Z
+    gemm(kGemmSymLeft, Y, P, Yb[(it + 1) & 1], nullptr, nullptr, false, 1.0, ns_act, true);   // Y T
+    gemm(kGemmSymLeft, P, Z, Zb[(it + 1) & 1], nullptr, nullptr, false, 1.0, ns_act, true);   // T Z
     if (it > 0) {
       HIPCHECK(hipEventSynchronize(ev_join3));   // iteration it - 1's count is on the host
       if (h_pinned[(it - 1) & 1] <= 0) break;
@@ -2505,7 +2546,7 @@ void Batch::scc_prologue() {
                      D, Q, shift, vs, vd, vq, ao_sh, ao_at, thr2, H, (const MolState*)d_state);
   // generalized eigenproblem in the current orbital basis C (S-orthonormal)
   mixed_here_ = true;   // the Fock transforms and the density product may run mixed
-  gemm(0, H, C, T, nullptr, nullptr, true);   // T = H C
+  gemm(kGemmSymLeft, H, C, T, nullptr, nullptr, true);   // T = H C
   gemm(1, C, T, A, nullptr, nullptr, true, 1.0, nullptr, true);   // A = C^T H C (symmetric)
   mixed_here_ = false;
 }
@@ -2530,15 +2571,12 @@ void Batch::subspace(bool allow) {
     const int nt = sub_t0[list + 1] - sub_t0[list];
     if (nt <= 0) return;
     const int4* tl = d_sub_tiles + sub_t0[list];
-    if (list == 2)
-      hipLaunchKernelGGL((k_sub_gemm<true, false>), dim3(nt), dim3(256), 0, stream, tl, d_desc, bf, (const int*)sub_,
-                         sub_res_, sub_dbl_, step, level);
-    else if (list == 7)
-      hipLaunchKernelGGL((k_sub_gemm<false, true>), dim3(nt), dim3(256), 0, stream, tl, d_desc, bf, (const int*)sub_,
-                         sub_res_, sub_dbl_, step, level);
+    if (list == 3)   // C Y
+      hipLaunchKernelGGL(k_sub_gemm<true>, dim3(nt), dim3(256), 0, stream, tl, d_desc, bf, d_state, sub_, sub_res_,
+                         sub_dbl_, step, level);
     else
-      hipLaunchKernelGGL((k_sub_gemm<false, false>), dim3(nt), dim3(256), 0, stream, tl, d_desc, bf, (const int*)sub_,
-                         sub_res_, sub_dbl_, step, level);
+      hipLaunchKernelGGL(k_sub_gemm<false>, dim3(nt), dim3(256), 0, stream, tl, d_desc, bf, d_state, sub_, sub_res_,
+                         sub_dbl_, step, level);
   };
   int step = 0, upto = std::min(kSubSteps, std::max(1, sub_guess_));
   for (;;) {
@@ -2550,15 +2588,16 @@ void Batch::subspace(bool allow) {
                        (const unsigned long long*)sub_res_, (const double*)sub_dbl_, step);
     product(2, 0, 0);
     product(3, 0, 0);
-    product(4, 0, 2);
-    product(5, 0, 3);
+    product(4, 0, 0);
+    product(5, 0, 2);
+    product(6, 0, 3);
     hipLaunchKernelGGL(k_sub_check, dim3(1), dim3(256), 0, stream, (const MolDesc*)d_desc, d_state, nmol, sub_,
                        (const unsigned long long*)sub_res_, sub_cnt_);
     HIPCHECK(hipMemcpyAsync(h_pinned + 8, sub_cnt_, 3 * sizeof(int), hipMemcpyDeviceToHost, stream));
     HIPCHECK(hipEventRecord(ev_join3, stream));
-    product(5, 0, 4);
-    product(6, 0, 0);
+    product(6, 0, 4);
     product(7, 0, 0);
+    product(8, 0, 0);
     HIPCHECK(hipEventSynchronize(ev_join3));
     if (h_pinned[8] <= 0 || step >= kSubSteps) break;
     upto = std::min(kSubSteps, step + 2);
@@ -2739,13 +2778,13 @@ void Batch::gradient() {
   }
   // bond orders from P S; open-shell molecules from the spin densities
   // Pa = C fa C^T and Pb = C fb C^T (src/scf_module.F90:856-873)
-  gemm(0, P, S, A, nullptr, nullptr, false, 1.0, phase_act);
+  gemm(kGemmSymLeft, P, S, A, nullptr, nullptr, false, 1.0, phase_act);
   hipLaunchKernelGGL(k_wbo, dim3(grid1((long long)sub_max_n * sub_max_n, 256), ns), dim3(256), 0, stream, d_sub, xyz,
                      at_ao0, at, el, (const double*)A, wbo, 0, (const int*)nullptr);
   if (nsub_open > 0)
     for (int spin = 0; spin < 2; ++spin) {
       gemm(2, C, C, T, spin ? foccb : focca, nullptr, false, 1.0, open_act, true);   // spin density
-      gemm(0, T, S, A, nullptr, nullptr, false, 1.0, open_act);
+      gemm(kGemmSymLeft, T, S, A, nullptr, nullptr, false, 1.0, open_act);
       hipLaunchKernelGGL(k_wbo, dim3(grid1((long long)sub_max_n * sub_max_n, 256), ns), dim3(256), 0, stream, d_sub,
                          xyz, at_ao0, at, el, (const double*)A, wbo, 1 + spin, (const int*)open_act);
     }

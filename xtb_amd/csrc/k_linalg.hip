@@ -29,7 +29,7 @@ __global__ void __launch_bounds__(256) k_gemm(const int4* __restrict__ tiles, co
   __shared__ double As[kBK][kTile + 1];
   __shared__ double Bs[kBK][kTile + 1];
   const int4 tl = tiles[blockIdx.x];
-  if (mask && !mask[(long long)tl.x * mstride]) return;
+  if (tl.x < 0 || (mask && !mask[(long long)tl.x * mstride])) return;
   const MolDesc md = desc[tl.x];
   const int N = md.nao;
   const double* Am = A + md.m0;
@@ -106,6 +106,116 @@ __global__ void __launch_bounds__(256) k_gemm(const int4* __restrict__ tiles, co
 // column lane%16.
 typedef double v4d __attribute__((ext_vector_type(4)));
 
+// One wave's 32 x 32 block (rows row0.., columns col0..) of L^T R, L (K x M)
+// and R (K x Nc) with row strides ldl and ldr; RMINOR: R is stored Nc x K.
+// The operands go from global memory straight into the lane layout of
+// v_mfma_f64_16x16x4f64 (four rows of 16 consecutive doubles per load), the
+// loads of the next 16 rows in flight during the 16 matrix instructions of
+// the current ones: no LDS and no barrier, so waves of different problems and
+// sizes share a compute unit freely.  Rows and columns outside the result
+// read a valid element instead and are not written by the callers.
+template <bool RMINOR>
+__device__ __forceinline__ void wave_mm(const double* __restrict__ L, int ldl, int M, const double* __restrict__ R,
+                                        int ldr, int Nc, int K, int row0, int col0, v4d (&acc)[2][2]) {
+  const int lane = threadIdx.x & 63, i16 = lane & 15, k4 = lane >> 4;
+  const double *lp[2], *rp[2];
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    lp[r] = L + (long long)k4 * ldl + min(row0 + 16 * r + i16, M - 1);
+    const int cj = min(col0 + 16 * r + i16, Nc - 1);
+    rp[r] = RMINOR ? R + (long long)cj * ldr + k4 : R + (long long)k4 * ldr + cj;
+  }
+  const long long sl = 4LL * ldl, sr = RMINOR ? 4 : 4LL * ldr;
+#pragma unroll
+  for (int r = 0; r < 2; ++r)
+#pragma unroll
+    for (int c = 0; c < 2; ++c) acc[r][c] = v4d{0.0, 0.0, 0.0, 0.0};
+  const int nfull = K >> 4;
+  double a[4][2], b[4][2];
+  auto load = [&](double (&x)[4][2], double (&y)[4][2]) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int r = 0; r < 2; ++r) {
+        x[u][r] = lp[r][u * sl];
+        y[u][r] = rp[r][u * sr];
+      }
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      lp[r] += 4 * sl;
+      rp[r] += 4 * sr;
+    }
+  };
+  auto mul = [&](const double (&x)[2], const double (&y)[2]) {
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+      for (int c = 0; c < 2; ++c) acc[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[r], y[c], acc[r][c], 0, 0, 0);
+  };
+  if (nfull > 0) load(a, b);
+  for (int q = 0; q < nfull; ++q) {
+    double a2[4][2], b2[4][2];
+    if (q + 1 < nfull) load(a2, b2);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) mul(a[u], b[u]);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int r = 0; r < 2; ++r) {
+        a[u][r] = a2[u][r];
+        b[u][r] = b2[u][r];
+      }
+  }
+  // the last K mod 16 rows; rows from K on count as zero
+  const int rest = K & 15;
+  double at[4][2], bt[4][2];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const bool in = 4 * u + k4 < rest;
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      at[u][r] = in ? lp[r][u * sl] : 0.0;
+      bt[u][r] = in ? rp[r][u * sr] : 0.0;
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+    if (4 * u < rest) mul(at[u], bt[u]);
+}
+
+// Symmetric-left and transposed-left products of the batch on wave_mm: C = L^T
+// B per molecule, all N x N (L symmetric: L B), a 64 x 64 tile per workgroup.
+// sym tiles (w != 0): the result is symmetric, formed on the upper tiles.
+__global__ void __launch_bounds__(256) k_gemm_tn(const int4* __restrict__ tiles, const MolDesc* __restrict__ desc,
+                                                 const double* __restrict__ L, const double* __restrict__ B, double* C,
+                                                 double alpha, const int* __restrict__ mask, int mstride) {
+  const int4 tl = tiles[blockIdx.x];
+  if (tl.x < 0 || (mask && !mask[(long long)tl.x * mstride])) return;
+  const MolDesc md = desc[tl.x];
+  const int N = md.nao;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, i16 = lane & 15, k4 = lane >> 4;
+  const int row0 = tl.y * kTile + 32 * (w >> 1), col0 = tl.z * kTile + 32 * (w & 1);
+  const bool sym = tl.w != 0;
+  if (row0 >= N || col0 >= N || (sym && row0 > col0)) return;
+  v4d acc[2][2];
+  wave_mm<false>(L + md.m0, N, N, B + md.m0, N, N, N, row0, col0, acc);
+  double* Cm = C + md.m0;
+#pragma unroll
+  for (int r = 0; r < 2; ++r)
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const int gj = col0 + 16 * c + i16;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int gi = row0 + 16 * r + k4 + 4 * i;
+        if (gi >= N || gj >= N || (sym && gi > gj)) continue;
+        const double x = alpha * acc[r][c][i];
+        Cm[(long long)gi * N + gj] = x;
+        if (sym) Cm[(long long)gj * N + gi] = x;
+      }
+    }
+}
+
 template <bool TA, bool TB, bool SCALE, bool PERM>
 __global__ void __launch_bounds__(256) k_gemm_mfma(const int4* __restrict__ tiles, const MolDesc* __restrict__ desc,
                                                    const double* __restrict__ A, const double* __restrict__ B,
@@ -117,7 +227,7 @@ __global__ void __launch_bounds__(256) k_gemm_mfma(const int4* __restrict__ tile
   __shared__ double As[2][kBK][kTile + 1];
   __shared__ double Bs[2][kBK][kTile + 1];
   const int4 tl = tiles[blockIdx.x];
-  if (mask && !mask[(long long)tl.x * mstride]) return;
+  if (tl.x < 0 || (mask && !mask[(long long)tl.x * mstride])) return;
   const MolDesc md = desc[tl.x];
   const int N = md.nao;
   const double* Am = A + md.m0;
@@ -226,7 +336,7 @@ __global__ void __launch_bounds__(256) k_gemm_mix(const int4* __restrict__ tiles
   __shared__ double As[kBK][kTile + 1];
   __shared__ double Bs[kBK][kTile + 1];
   const int4 tl = tiles[blockIdx.x];
-  if (mask && !mask[(long long)tl.x * mstride]) return;
+  if (tl.x < 0 || (mask && !mask[(long long)tl.x * mstride])) return;
   const MolDesc md = desc[tl.x];
   const int N = md.nao;
   const double* Am = A + md.m0;

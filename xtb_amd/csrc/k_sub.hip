@@ -75,17 +75,52 @@ constexpr int kSubTol = 0, kSubLim = 1, kSubRho = 2, kSubW = 3, kSubDbls = kSubW
 // of the second-order iteration with factor w (r > sqrt(w - 1))
 __device__ __forceinline__ double sub_mu(double r, double w) { return (r * r + w - 1.0) / (w * r); }
 
-// step s runs unless an earlier one converged, contracted too slowly or met a
-// NaN (a step that did not run leaves its maximum at 0)
-__device__ __forceinline__ bool sub_step_runs(const unsigned long long* __restrict__ res,
+// step s is not needed: an earlier one converged (a step that did not run
+// leaves its maximum at 0)
+__device__ __forceinline__ bool sub_step_done(const unsigned long long* __restrict__ res,
                                               const double* __restrict__ sd, int s) {
-  if (s == 0) return true;
-  const double r1 = __longlong_as_double((long long)res[s - 1]);
-  if (!(r1 > sd[kSubTol])) return false;
-  if (s < 5) return true;
-  // the mean of three steps: max |R| may rise for one step when w sets in
-  const double r = cbrt(r1 / __longlong_as_double((long long)res[s - 4])), w = sd[kSubW + s - 1];
-  return r * r <= w - 1.0 || sub_mu(r, w) <= sd[kSubLim];
+  return s > 0 && __longlong_as_double((long long)res[s - 1]) <= sd[kSubTol];
+}
+
+// the full diagonalisation takes the molecule over
+__device__ __forceinline__ void sub_give_up(int* si, MolState* st) {
+  si[kSubPhase] = 3;
+  si[kSubOff] += 1;
+  si[kSubX] = 0;
+  si[kSubPend] = 0;
+  st->diag = 1;
+}
+
+// one thread: the factor w of step s, or the end where max |R| is a NaN or
+// falls too slowly (the mean of three steps: it may rise for one when w sets in)
+__device__ __forceinline__ void sub_rate(const unsigned long long* __restrict__ res, double* sd, int* si,
+                                         MolState* st, int s) {
+  auto at = [&](int k) { return __longlong_as_double((long long)res[k]); };
+  double rho = sd[kSubRho], w = 1.0;
+  if (s > 0) {
+    const double wl = sd[kSubW + s - 1];
+    bool slow = !(at(s - 1) < 1e300);
+    if (s >= 5) {
+      const double r = cbrt(at(s - 1) / at(s - 4));
+      slow = slow || !(r * r <= wl - 1.0 || sub_mu(r, wl) <= sd[kSubLim]);
+    }
+    if (slow) {
+      sub_give_up(si, st);
+      return;
+    }
+    if (s >= 3) {
+      const double rr = at(s - 1) / at(s - 3);
+      if (rr > 1.2 * (wl - 1.0)) rho = fmax(rho, fmin(kSubRhoMax, sub_mu(sqrt(rr), wl)));
+      sd[kSubRho] = rho;
+    }
+    // the plain step is better as long as max |R| falls faster than the
+    // second-order iteration's sqrt(w - 1)
+    if (s > 1 && rho >= kSubRhoMin) {
+      const double wo = 2.0 / (1.0 + sqrt(1.0 - rho * rho)), r1 = at(s - 1) / at(s - 2);
+      if (wl != 1.0 || r1 * r1 > wo - 1.0) w = wo;
+    }
+  }
+  sd[kSubW + s] = w;
 }
 
 // E_k (k = 2, 3) is left out of the inverse
@@ -160,148 +195,89 @@ __global__ void __launch_bounds__(256) k_sub_start(const MolDesc* __restrict__ d
   for (long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x; t < (long long)v * o;
        t += (long long)gridDim.x * blockDim.x) {
     const int i = (int)(t / o), j = (int)(t % o);
-    X[md.m0 + t] = -Am[(long long)(o + i) * N + j] / (d[o + i] - d[j]);
+    const double x = -Am[(long long)(o + i) * N + j] / (d[o + i] - d[j]);
+    X[md.m0 + t] = x;
+    X[md.m0 + 2LL * v * o + (long long)j * v + i] = x;
   }
 }
 
-// Buffers of the products (each N x N per molecule at m0): X, X' in Xb, and
-// G, T, W, H, P as scratch (their own contents are dead between the Fock
+// Buffers of the products (each N x N per molecule at m0): X holds X and its
+// transpose twice (4 v o <= N^2: X of parity 0 and 1, then X^T of both); G,
+// T, W, H, P are scratch (their own contents are dead between the Fock
 // transform and the density).
 struct SubBufs {
   const double *A, *C, *diag;
   double *X, *G, *T, *W, *H, *P;
 };
 
-// One 64 x 64 tile of one product of a molecule; tiles (molecule, row tile,
-// column tile, kind).  Operands through two LDS stages (the loads of the next
-// k-block are in flight during the matrix-core work of the current one).
-// Symmetric results (M, its powers E_k = M^(2^k) and the inverse's partial
-// products Z_k commute, P) are formed on the upper tiles and mirrored.
+// One 64 x 64 tile of one product of a molecule, a wave per 32 x 32 quarter
+// (wave_mm: no LDS, no barrier, a quarter outside the result ends at once);
+// tiles (molecule, row tile, column tile, kind).  Every operand but C is kept
+// so that the product runs down its rows: A, the powers of M and the partial
+// products Z are symmetric, X is kept with its transpose, C Y and C Y Z are
+// formed transposed (o x N).  Symmetric results (M, E_k = M^(2^k), Z_k, P) are
+// formed on the upper tiles and mirrored.
 // Z_2 = (I - M)(I + E_1), Z_(k+1) = Z_k (I + E_k).
 // step: the step of the kinds kSubB and kSubR; level: k of E_k and Z_k.
-// Buffers: M, E_3 in G, E_1, Z_3 in P, E_2 in H, Z_2, Z_4 in W, C Y in T.
-template <bool TA, bool TB>
+// Buffers: M, E_3 in G, E_1, Z_3 in P, E_2 in H, Z_2, Z_4 in W, (C Y)^T in T.
+template <bool RMINOR>
 __global__ void __launch_bounds__(256) k_sub_gemm(const int4* __restrict__ tiles, const MolDesc* __restrict__ desc,
-                                                  SubBufs bf, const int* __restrict__ sub, unsigned long long* res,
+                                                  SubBufs bf, MolState* state, int* sub, unsigned long long* res,
                                                   double* dbl, int step, int level) {
-  __shared__ double As[2][kBK][kTile + 1];
-  __shared__ double Bs[2][kBK][kTile + 1];
   const int4 tl = tiles[blockIdx.x];
   const int m = tl.x, op = tl.w & 15;
+  if (m < 0) return;
   const bool sym = (tl.w & kSubSym) != 0;
-  const int* si = sub + m * kSubInts;
+  int* si = sub + m * kSubInts;
+  if (si[kSubPhase] != (op <= kSubR ? 1 : 2)) return;
   unsigned long long* rs = res + (long long)m * kSubRes;
   double* sd = dbl + (long long)m * kSubDbls;
   const MolDesc md = desc[m];
   const int N = md.nao, o = sub_occ(md), v = N - o;
   int par = si[kSubPar];
   if (op <= kSubR) {
-    if (si[kSubPhase] != 1 || !sub_step_runs(rs, sd, step)) return;
+    if (sub_step_done(rs, sd, step)) return;
     par = (par + step) & 1;
     // the first tile's workgroup sets the factor of this step for the second
-    // product's launch
-    if (op == kSubB && tl.y == 0 && tl.z == 0 && threadIdx.x == 0) {
-      double rho = sd[kSubRho], w = 1.0;
-      if (step >= 3) {
-        const double rr = __longlong_as_double((long long)rs[step - 1]) / __longlong_as_double((long long)rs[step - 3]);
-        const double wl = sd[kSubW + step - 1];
-        if (rr > 1.2 * (wl - 1.0)) rho = fmax(rho, fmin(kSubRhoMax, sub_mu(sqrt(rr), wl)));
-        sd[kSubRho] = rho;
-      }
-      // the plain step is better as long as max |R| falls faster than the
-      // second-order iteration's sqrt(w - 1)
-      if (step > 1 && rho >= kSubRhoMin) {
-        const double wo = 2.0 / (1.0 + sqrt(1.0 - rho * rho));
-        const double r1 = __longlong_as_double((long long)rs[step - 1]) / __longlong_as_double((long long)rs[step - 2]);
-        if (sd[kSubW + step - 1] != 1.0 || r1 * r1 > wo - 1.0) w = wo;
-      }
-      sd[kSubW + step] = w;
-    }
-  } else {
-    if (si[kSubPhase] != 2) return;
+    // product's launch, or gives the molecule up
+    if (op == kSubB && tl.y == 0 && tl.z == 0 && threadIdx.x == 0) sub_rate(rs, sd, si, state + m, step);
   }
   const long long vo = (long long)v * o;
-  const double* X = bf.X + md.m0 + par * vo;
+  double* Xm = bf.X + md.m0;
+  const double* X = Xm + par * vo;
   double* G = bf.G + md.m0;
   double* T = bf.T + md.m0;
   double* W = bf.W + md.m0;
   double* H = bf.H + md.m0;
   double* P = bf.P + md.m0;
   const bool e2 = !sub_dropped(rs, o, 2), e3 = e2 && !sub_dropped(rs, o, 3);
-  // result (M x Nc) = op(A) (M x K) op(B)
-  const double *Ap, *Bp;
-  int lda = o, ldb = o, M = o, Nc = o, K = o;
+  // result (M x Nc) = L^T R with L (K x M), R (K x Nc), or R (Nc x K) for C
+  const double *Lp, *Rp;
+  int ldl = o, ldr = o, M = o, Nc = o, K = o;
   switch (op) {
-    case kSubB: Ap = bf.A + md.m0 + o; lda = N; Bp = X; M = N; K = v; break;
-    case kSubR: Ap = X; Bp = G; M = v; break;
-    case kSubM: Ap = X; Bp = X; K = v; break;
-    case kSubCY: Ap = bf.C + md.m0 + o; lda = N; Bp = X; M = N; K = v; break;
-    case kSubE1: Ap = G; Bp = G; break;
-    case kSubZ2: Ap = G; Bp = P; break;
+    case kSubB: Lp = bf.A + md.m0 + (long long)o * N; ldl = N; Rp = X; M = N; K = v; break;
+    case kSubR: Lp = X + 2 * vo; ldl = v; Rp = G; M = v; break;
+    case kSubM: Lp = X; Rp = X; K = v; break;
+    case kSubCY: Lp = X; Rp = bf.C + md.m0 + o; ldr = N; Nc = N; K = v; break;
+    case kSubE1: Lp = G; Rp = G; break;
+    case kSubZ2: Lp = G; Rp = P; break;
     case kSubE:
       if (level > 3 || (level == 3 && !e2)) return;   // the list's third launch forms Z_4 only
-      Ap = Bp = level == 2 ? P : H;
+      Lp = Rp = level == 2 ? P : H;
       break;
     case kSubZ:
       if (level == 3 ? !e2 : !e3) return;
-      Ap = level == 3 ? W : P;
-      Bp = level == 3 ? H : G;
+      Lp = level == 3 ? W : P;
+      Rp = level == 3 ? H : G;
       break;
-    case kSubCYZ: Ap = T; Bp = e2 && !e3 ? P : W; M = N; break;
-    default: Ap = G; Bp = T; M = N; Nc = N; break;
+    case kSubCYZ: Lp = e2 && !e3 ? P : W; Rp = T; ldr = N; Nc = N; break;
+    default: Lp = G; ldl = N; Rp = T; ldr = N; M = Nc = N; break;
   }
-  const int row0 = tl.y * kTile, col0 = tl.z * kTile;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int wr = w >> 1, wc = w & 1, i16 = lane & 15, k4 = lane >> 4;
-  double ra[4], rb[4];
-  auto fetch = [&](int kb) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int e = tid + 256 * q;
-      const int gi = row0 + (TA ? (e & 63) : (e >> 4)), gk = kb + (TA ? (e >> 6) : (e & 15));
-      const int gj = col0 + (TB ? (e >> 4) : (e & 63)), gk2 = kb + (TB ? (e & 15) : (e >> 6));
-      ra[q] = (gi < M && gk < K) ? (TA ? Ap[(long long)gk * lda + gi] : Ap[(long long)gi * lda + gk]) : 0.0;
-      rb[q] = (gj < Nc && gk2 < K) ? (TB ? Bp[(long long)gj * ldb + gk2] : Bp[(long long)gk2 * ldb + gj]) : 0.0;
-    }
-  };
-  auto stage = [&](int buf) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int e = tid + 256 * q;
-      if (TA) As[buf][e >> 6][e & 63] = ra[q];
-      else As[buf][e & 15][e >> 4] = ra[q];
-      if (TB) Bs[buf][e & 15][e >> 4] = rb[q];
-      else Bs[buf][e >> 6][e & 63] = rb[q];
-    }
-  };
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, i16 = lane & 15, k4 = lane >> 4;
+  const int row0 = tl.y * kTile + 32 * (w >> 1), col0 = tl.z * kTile + 32 * (w & 1);
+  if (row0 >= M || col0 >= Nc || (sym && row0 > col0)) return;
   v4d acc[2][2];
-#pragma unroll
-  for (int r = 0; r < 2; ++r)
-#pragma unroll
-    for (int c = 0; c < 2; ++c) acc[r][c] = v4d{0.0, 0.0, 0.0, 0.0};
-  fetch(0);
-  stage(0);
-  __syncthreads();
-  int buf = 0;
-  for (int kb = 0; kb < K; kb += kBK) {
-    const bool more = kb + kBK < K;
-    if (more) fetch(kb + kBK);
-#pragma unroll
-    for (int kk = 0; kk < kBK; kk += 4) {
-      double a[2], b[2];
-#pragma unroll
-      for (int r = 0; r < 2; ++r) a[r] = As[buf][kk + k4][32 * wr + 16 * r + i16];
-#pragma unroll
-      for (int c = 0; c < 2; ++c) b[c] = Bs[buf][kk + k4][32 * wc + 16 * c + i16];
-#pragma unroll
-      for (int r = 0; r < 2; ++r)
-#pragma unroll
-        for (int c = 0; c < 2; ++c) acc[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[r], b[c], acc[r][c], 0, 0, 0);
-    }
-    if (more) stage(buf ^ 1);
-    __syncthreads();
-    buf ^= 1;
-  }
+  wave_mm<RMINOR>(Lp, ldl, M, Rp, ldr, Nc, K, row0, col0, acc);
   // maxima on the bit patterns: a NaN counts as the largest value
   unsigned long long big = 0ull;
   auto see = [&](double x) {
@@ -309,14 +285,15 @@ __global__ void __launch_bounds__(256) k_sub_gemm(const int4* __restrict__ tiles
     big = big > b ? big : b;
   };
   const double* dg = bf.diag + md.o0;
+  const double ws = op == kSubR && step > 0 ? sd[kSubW + step] : 1.0;
 #pragma unroll
   for (int r = 0; r < 2; ++r)
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
-      const int gj = col0 + 32 * wc + 16 * c + i16;
+      const int gj = col0 + 16 * c + i16;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int gi = row0 + 32 * wr + 16 * r + k4 + 4 * i;
+        const int gi = row0 + 16 * r + k4 + 4 * i;
         if (gi >= M || gj >= Nc) continue;
         if (sym && gi > gj) continue;
         const long long e = (long long)gi * Nc + gj, et = (long long)gj * Nc + gi;
@@ -325,18 +302,19 @@ __global__ void __launch_bounds__(256) k_sub_gemm(const int4* __restrict__ tiles
           case kSubB: G[e] = bf.A[md.m0 + (long long)gi * N + gj] + x; break;
           case kSubR: {
             const double rr = G[(long long)(o + gi) * o + gj] - x;
-            double* xn = bf.X + md.m0 + (par ^ 1) * vo + e;   // holds the X before this one
+            double* xn = Xm + (par ^ 1) * vo;   // holds the X before this one
             double x1 = X[e] - rr / (dg[o + gi] - dg[gj]);
-            if (step > 0) {
-              const double x0 = *xn, w = sd[kSubW + step];
-              if (w != 1.0) x1 = x0 + w * (x1 - x0);
+            if (ws != 1.0) {
+              const double x0 = xn[e];
+              x1 = x0 + ws * (x1 - x0);
             }
-            *xn = x1;
+            xn[e] = x1;
+            xn[2 * vo + (long long)gj * v + gi] = x1;
             see(rr);
             break;
           }
           case kSubM: G[e] = x; G[et] = x; break;
-          case kSubCY: T[e] = bf.C[md.m0 + (long long)gi * N + gj] + x; break;
+          case kSubCY: T[e] = bf.C[md.m0 + (long long)gj * N + gi] + x; break;
           case kSubE1: P[e] = x; P[et] = x; break;
           case kSubZ2: {
             const double z = ((gi == gj ? 1.0 : 0.0) - G[e]) + (P[e] - x);
@@ -369,7 +347,9 @@ __global__ void __launch_bounds__(256) k_sub_gemm(const int4* __restrict__ tiles
       const unsigned long long ob = __shfl_xor(big, sft, 64);
       big = big > ob ? big : ob;
     }
-    if (lane == 0 && big) atomicMax(op == kSubR ? &rs[step] : &rs[kSubSteps + level - 2], big);
+    // (most waves of a large molecule find a larger maximum there already)
+    unsigned long long* to = op == kSubR ? &rs[step] : &rs[kSubSteps + level - 2];
+    if (lane == 0 && big > __atomic_load_n(to, __ATOMIC_RELAXED)) atomicMax(to, big);
   }
 }
 
@@ -385,17 +365,14 @@ __global__ void k_sub_outcome(MolState* state, int nmol, int* sub, const unsigne
   const unsigned long long* rs = res + (long long)m * kSubRes;
   const double* sd = dbl + (long long)m * kSubDbls;
   int t = 0;
-  while (t < nstep && sub_step_runs(rs, sd, t)) ++t;
+  while (t < nstep && !sub_step_done(rs, sd, t)) ++t;
   si[kSubNext] = t;
-  if (__longlong_as_double((long long)rs[t - 1]) <= sd[kSubTol]) {   // each step so far passed sub_step_runs
+  if (sub_step_done(rs, sd, t)) {
     si[kSubPhase] = 2;
     si[kSubPar] = (si[kSubPar] + t) & 1;
     si[kSubPend] = 1;
-  } else if (t < nstep || t >= kSubSteps) {
-    si[kSubPhase] = 3;
-    si[kSubOff] += 1;
-    si[kSubX] = 0;
-    state[m].diag = 1;
+  } else if (t >= kSubSteps) {
+    sub_give_up(si, state + m);
   }
 }
 
@@ -411,11 +388,7 @@ __global__ void __launch_bounds__(256) k_sub_check(const MolDesc* __restrict__ d
     if (si[kSubPhase] == 2) {
       const double e3 = __longlong_as_double((long long)res[(long long)m * kSubRes + kSubSteps + 1]);
       if (!(sub_occ(desc[m]) * e3 <= kSubInvMax)) {
-        si[kSubPhase] = 3;
-        si[kSubOff] += 1;
-        si[kSubX] = 0;
-        si[kSubPend] = 0;
-        state[m].diag = 1;
+        sub_give_up(si, state + m);
       }
     }
     if (si[kSubPhase] == 1) run += 1.0;
