@@ -381,7 +381,7 @@ class Batch {
   int* jac_nactive = nullptr;
   int* perm = nullptr;
   int* eeq_failed = nullptr;
-  int* eeq_big = nullptr;        // sub-list indices of EEQ systems factorised column by column
+  int* eeq_bad = nullptr;        // EEQ matrices that are not positive definite
   // implicit solvation: device model, Born radii and chain factors, surface
   // (per atom and per grid point), H-bond weights, potential, dE/dbrad, the
   // interaction matrix (n x n at p0) and per-molecule surface energy, shape

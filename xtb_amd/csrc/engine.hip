@@ -60,35 +60,43 @@ __global__ void k_copy(const double* a, double* b, long long n) {
   if (i < n) b[i] = a[i];
 }
 
-// EEQ systems with at least this many unknowns are factorised column by column
-// across the whole device instead of inside one workgroup
-constexpr int kEeqBigNe = 256;
+// shell charges from the atomic ones (iniqshell: src/scc_core.f90:1475-1506)
+__device__ __forceinline__ void eeq_shells(const MolDesc& md, const Element* __restrict__ el,
+                                           const int* __restrict__ at, const int* __restrict__ at_sh0, const double* q,
+                                           double* qsh, const double* __restrict__ zsh) {
+  for (int i = threadIdx.x; i < md.n; i += blockDim.x) {
+    const Element& e = el[at[md.a0 + i]];
+    for (int s = 0; s < e.nsh; ++s) {
+      const int k = md.s0 + at_sh0[md.a0 + i] + s;
+      qsh[k] = (zsh[k] / e.zval) * q[md.a0 + i];
+    }
+  }
+}
 
-// EEQ charges: Gaussian elimination with partial pivoting of the constrained
-// (n+1) x (n+1) system E y = x in place (the reference solves it with dsysv,
-// src/eeq_model.f90:678-1015), then the shell charges (iniqshell:
-// src/scc_core.f90:1475-1506); uniform charges if the solve fails
-// (src/xtb/calculator.f90:479-484).  One workgroup per molecule.
-// Systems of at least big_ne unknowns arrive factorised by k_eeq_lu_pivot /
-// k_eeq_lu_update (the same elimination spread over the whole device); this
-// kernel then only substitutes.
+// EEQ charges of the molecules whose charge-interaction matrix is not
+// positive definite (bad): Gaussian elimination with partial pivoting of the
+// constrained (n+1) x (n+1) system E y = x in place (the reference solves it
+// with dsysv, src/eeq_model.f90:678-1015); uniform charges if the solve fails
+// (src/xtb/calculator.f90:479-484).  One workgroup per molecule; every other
+// molecule takes the Cholesky path below.
 __global__ void __launch_bounds__(256) k_eeq_gesv(const MolDesc* __restrict__ desc, const Element* __restrict__ el,
                                                   const int* __restrict__ at, const int* __restrict__ at_sh0, double* E,
                                                   double* xE, double* yE, double* q, double* qsh,
-                                                  const double* __restrict__ zsh, int* failed, int big_ne) {
+                                                  const double* __restrict__ zsh, int* failed,
+                                                  const int* __restrict__ bad) {
   __shared__ double sh[4];
   __shared__ double shv[4];
   __shared__ int shi[4];
   __shared__ int piv;
   const MolDesc md = desc[blockIdx.x];
+  if (!bad[md.mol]) return;
   const int ne = md.ne, n = md.n;
   double* M = E + md.e0;
   double* b = xE + md.y0;
   double* y = yE + md.y0;
   const int tid = threadIdx.x;
-  const bool factored = ne >= big_ne;
-  bool ok = !(factored && failed[md.mol]);
-  for (int k = 0; k < (factored ? 0 : ne); ++k) {
+  bool ok = true;
+  for (int k = 0; k < ne; ++k) {
     // pivot: largest |M[i][k]|, i >= k, smallest index on ties
     double best = -1.0;
     int bi = k;
@@ -157,18 +165,220 @@ __global__ void __launch_bounds__(256) k_eeq_gesv(const MolDesc* __restrict__ de
     if (tid == 0) failed[md.mol] = 1;
   }
   __syncthreads();
-  for (int i = tid; i < n; i += blockDim.x) {
-    const Element& e = el[at[md.a0 + i]];
-    for (int s = 0; s < e.nsh; ++s) {
-      const int k = md.s0 + at_sh0[md.a0 + i] + s;
-      qsh[k] = (zsh[k] / e.zval) * q[md.a0 + i];
-    }
-  }
+  eeq_shells(md, el, at, at_sh0, q, qsh, zsh);
 }
 
-__global__ void k_eeq_reset(const MolDesc* __restrict__ desc, int ns, int* failed) {
+__device__ __forceinline__ double lane_value(double x, int lane) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(x);
+  const unsigned lo = __builtin_amdgcn_readlane((unsigned)b, lane);
+  const unsigned hi = __builtin_amdgcn_readlane((unsigned)(b >> 32), lane);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// EEQ charges by Cholesky: with J the n x n charge-interaction block (a
+// Coulomb matrix of Gaussian charges, positive definite in practice),
+// J q + lambda 1 = b and sum q = Q give lambda = (z2 z1 - Q) / z2 z2 and
+// q = L^-T (z1 - lambda z2), z1 = L^-1 b, z2 = L^-1 1.  The vectors 1 (row n
+// of E) and b ride along as rows n and n + 1 of the factorisation, so the
+// forward substitutions come with it.  Two launches per 32 columns for all
+// molecules (the pivoted elimination was 15 us per column inside one
+// workgroup and 28 us per column over the device): 2.9 -> 0.2 ms for 194
+// atoms, 58 -> 5 ms for 2100.
+// A molecule whose pivot is not positive is flagged in bad.
+constexpr int kEeqNb = 32;
+
+// Block column kb: every workgroup factors the 32 x 32 diagonal block (one
+// wave, a row per lane, in registers) and solves 256 rows below it, one per
+// thread.  The diagonal block's factor goes, transposed, to the block's upper
+// triangle, which no workgroup of this launch reads, and its inverse diagonal
+// to yE.
+__global__ void __launch_bounds__(256) k_eeq_panel(const MolDesc* __restrict__ desc, int kb, double* E, double* xE,
+                                                   double* yE, int* bad) {
+  __shared__ double Ls[kEeqNb][kEeqNb + 1];
+  __shared__ double inv[kEeqNb];
+  __shared__ int fine;
+  const MolDesc md = desc[blockIdx.y];
+  const int n = md.n, ne = md.ne, k0 = kb * kEeqNb;
+  if (k0 >= n || bad[md.mol]) return;
+  const int nb = min(kEeqNb, n - k0), below = n + 2 - (k0 + nb);
+  if ((int)blockIdx.x * 256 >= below) return;
+  double* M = E + md.e0;
+  double* b = xE + md.y0;
+  const int tid = threadIdx.x;
+  for (int e = tid; e < kEeqNb * kEeqNb; e += 256) {
+    const int r = e / kEeqNb, c = e % kEeqNb;
+    Ls[r][c] = r < nb && c <= r ? M[(long long)(k0 + r) * ne + k0 + c] : (r == c ? 1.0 : 0.0);
+  }
+  __syncthreads();
+  if (tid < 64) {
+    const int row = tid & 31;
+    double a[kEeqNb];
+    bool ok = true;
+#pragma unroll
+    for (int c = 0; c < kEeqNb; ++c) a[c] = Ls[row][c];
+#pragma unroll
+    for (int c = 0; c < kEeqNb; ++c) {
+      const double d = lane_value(a[c], c);
+      ok = ok && d > 0.0;
+      const double s = 1.0 / sqrt(d);
+      a[c] *= s;
+      if (tid == c) inv[c] = s;
+#pragma unroll
+      for (int j = c + 1; j < kEeqNb; ++j) a[j] -= a[c] * lane_value(a[c], j);
+    }
+    if (tid < 32) {
+#pragma unroll
+      for (int c = 0; c < kEeqNb; ++c) Ls[row][c] = c <= row ? a[c] : 0.0;
+    }
+    if (tid == 0) fine = ok ? 1 : 0;
+  }
+  __syncthreads();
+  if (!fine) {
+    if (tid == 0) bad[md.mol] = 1;
+    return;
+  }
+  if (blockIdx.x == 0) {
+    for (int e = tid; e < kEeqNb * kEeqNb; e += 256) {
+      const int r = e / kEeqNb, c = e % kEeqNb;
+      if (r < nb && c < r) M[(long long)(k0 + c) * ne + k0 + r] = Ls[r][c];
+    }
+    if (tid < nb) yE[md.y0 + k0 + tid] = inv[tid];
+  }
+  const int i = k0 + nb + blockIdx.x * 256 + tid;
+  if (i >= n + 2) return;
+  double* p = i <= n ? M + (long long)i * ne + k0 : b + k0;
+  double x[kEeqNb];
+#pragma unroll
+  for (int c = 0; c < kEeqNb; ++c) x[c] = c < nb ? p[c] : 0.0;
+#pragma unroll
+  for (int c = 0; c < kEeqNb; ++c) {
+    double s = x[c];
+#pragma unroll
+    for (int t = 0; t < c; ++t) s -= x[t] * Ls[c][t];
+    x[c] = s * inv[c];
+  }
+#pragma unroll
+  for (int c = 0; c < kEeqNb; ++c)
+    if (c < nb) p[c] = x[c];
+}
+
+// trailing update after block column kb (32 columns): rows i of the lower
+// triangle and the two vector rows, 64 x 64 tiles
+__global__ void __launch_bounds__(256) k_eeq_update(const MolDesc* __restrict__ desc, int kb, double* E, double* xE,
+                                                    const int* __restrict__ bad) {
+  __shared__ double Ri[64][kEeqNb + 1], Rj[64][kEeqNb + 1];
+  const MolDesc md = desc[blockIdx.z];
+  const int n = md.n, ne = md.ne, k0 = kb * kEeqNb, k1 = k0 + kEeqNb;
+  const int i0 = k1 + 64 * blockIdx.y, j0 = k1 + 64 * blockIdx.x;
+  if (blockIdx.x > blockIdx.y || j0 >= n || i0 >= n + 2 || bad[md.mol]) return;
+  double* M = E + md.e0;
+  double* b = xE + md.y0;
+  const int tid = threadIdx.x;
+  for (int e = tid; e < 64 * kEeqNb; e += 256) {
+    const int r = e / kEeqNb, c = e % kEeqNb, i = i0 + r, j = j0 + r;
+    Ri[r][c] = i <= n ? M[(long long)i * ne + k0 + c] : (i == n + 1 ? b[k0 + c] : 0.0);
+    Rj[r][c] = j < n ? M[(long long)j * ne + k0 + c] : 0.0;
+  }
+  __syncthreads();
+  const int tx = tid & 15, ty = tid >> 4;
+  double acc[4][4] = {};
+#pragma unroll 4
+  for (int c = 0; c < kEeqNb; ++c) {
+    double x[4], y[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      x[u] = Ri[ty + 16 * u][c];
+      y[u] = Rj[tx + 16 * u][c];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int w = 0; w < 4; ++w) acc[u][w] += x[u] * y[w];
+  }
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const int i = i0 + ty + 16 * u, j = j0 + tx + 16 * w;
+      if (i >= n + 2 || j >= n || (i < n && j > i)) continue;
+      if (i <= n) M[(long long)i * ne + j] -= acc[u][w];
+      else b[j] -= acc[u][w];
+    }
+}
+
+// multiplier, back substitution (one workgroup per molecule, 32 unknowns at a
+// time, the last first) and the shell charges
+__global__ void __launch_bounds__(256) k_eeq_solve(const MolDesc* __restrict__ desc, const Element* __restrict__ el,
+                                                   const int* __restrict__ at, const int* __restrict__ at_sh0,
+                                                   const double* __restrict__ E, double* xE,
+                                                   const double* __restrict__ yE, double* q, double* qsh,
+                                                   const double* __restrict__ zsh, int* bad) {
+  __shared__ double sh[4];
+  __shared__ double part[8][kEeqNb];
+  __shared__ double Ls[kEeqNb][kEeqNb + 1];
+  const MolDesc md = desc[blockIdx.x];
+  if (bad[md.mol]) return;
+  const int n = md.n, ne = md.ne, tid = threadIdx.x;
+  const double* M = E + md.e0;
+  const double* z2 = M + (long long)n * ne;
+  double* z = xE + md.y0;
+  double* x = q + md.a0;
+  double d1 = 0.0, d2 = 0.0;
+  for (int i = tid; i < n; i += 256) {
+    d1 += z2[i] * z[i];
+    d2 += z2[i] * z2[i];
+  }
+  d1 = block_sum<256>(d1, sh);
+  d2 = block_sum<256>(d2, sh);
+  const double lam = (d1 - md.charge) / d2;
+  for (int k0 = (n - 1) / kEeqNb * kEeqNb; k0 >= 0; k0 -= kEeqNb) {
+    const int nb = min(kEeqNb, n - k0), k1 = k0 + nb;
+    const int c = tid & 31, g = tid >> 5;
+    for (int e = tid; e < kEeqNb * kEeqNb; e += 256) {
+      const int r = e / kEeqNb, t = e % kEeqNb;   // L[t][r], t > r, from the block's upper triangle
+      Ls[r][t] = t < nb && r < t ? M[(long long)(k0 + r) * ne + k0 + t] : 0.0;
+    }
+    double s[4] = {0.0, 0.0, 0.0, 0.0};
+    if (c < nb) {
+      int i = k1 + g;
+      for (; i + 24 < n; i += 32)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) s[u] += M[(long long)(i + 8 * u) * ne + k0 + c] * x[i + 8 * u];
+      for (; i < n; i += 8) s[0] += M[(long long)i * ne + k0 + c] * x[i];
+    }
+    part[g][c] = (s[0] + s[1]) + (s[2] + s[3]);
+    __syncthreads();
+    if (tid < 64) {
+      double r = 0.0, di = 0.0;
+      if (c < nb) {
+        r = z[k0 + c] - lam * z2[k0 + c];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) r -= part[u][c];
+        di = yE[md.y0 + k0 + c];
+      }
+      for (int t = kEeqNb - 1; t >= 0; --t) {
+        const double xt = __shfl(r * di, t, 64);
+        r -= Ls[c][t] * xt;   // zero for t <= c
+      }
+      if (tid < nb) x[k0 + tid] = r * di;
+    }
+    __syncthreads();
+  }
+  double tot = 0.0;
+  for (int i = tid; i < n; i += 256) tot += x[i];
+  tot = block_sum<256>(tot, sh);
+  if (!(fabs(tot - md.charge) <= 1.e-6)) {
+    if (tid == 0) bad[md.mol] = 1;
+    return;
+  }
+  eeq_shells(md, el, at, at_sh0, q, qsh, zsh);
+}
+
+__global__ void k_eeq_reset(const MolDesc* __restrict__ desc, int ns, int* failed, int* bad) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < ns) failed[desc[k].mol] = 0;
+  if (k >= ns) return;
+  failed[desc[k].mol] = 0;
+  if (bad) bad[desc[k].mol] = 0;
 }
 
 // Failure codes of MolState::failed (0 = fine).
@@ -187,76 +397,6 @@ __global__ void k_fail_fold(MolState* st, int nmol, const int* __restrict__ flag
   if (m >= nmol || (sel && !sel[m]) || !flags[(long long)m * stride]) return;
   if (!st[m].failed) st[m].failed = code;
   st[m].active = 0;
-}
-
-// Column k of the LU factorisation with partial pivoting of large EEQ systems
-// (one workgroup per listed molecule): pivot search with the same tie rule as
-// k_eeq_gesv, row swap, multipliers and the right-hand-side update.
-__global__ void __launch_bounds__(256) k_eeq_lu_pivot(const MolDesc* __restrict__ desc, const int* __restrict__ list,
-                                                      int k, double* E, double* xE, int* failed) {
-  __shared__ double shv[4];
-  __shared__ int shi[4];
-  __shared__ int piv;
-  const MolDesc md = desc[list[blockIdx.x]];
-  const int ne = md.ne;
-  if (k >= ne || failed[md.mol]) return;
-  double* M = E + md.e0;
-  double* b = xE + md.y0;
-  const int tid = threadIdx.x;
-  double best = -1.0;
-  int bi = k;
-  for (int i = k + tid; i < ne; i += blockDim.x) {
-    const double v = fabs(M[(long long)i * ne + k]);
-    if (v > best) { best = v; bi = i; }
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const double ov = __shfl_xor(best, o, 64);
-    const int oi = __shfl_xor(bi, o, 64);
-    if (ov > best || (ov == best && oi < bi)) { best = ov; bi = oi; }
-  }
-  if ((tid & 63) == 0) { shv[tid >> 6] = best; shi[tid >> 6] = bi; }
-  __syncthreads();
-  if (tid == 0) {
-    double bv = shv[0];
-    int bx = shi[0];
-    for (int w = 1; w < 4; ++w)
-      if (shv[w] > bv || (shv[w] == bv && shi[w] < bx)) { bv = shv[w]; bx = shi[w]; }
-    piv = (bv > 0.0) ? bx : -1;
-    if (piv < 0) failed[md.mol] = 1;
-  }
-  __syncthreads();
-  const int p = piv;
-  if (p < 0) return;
-  if (p != k) {
-    for (int j = tid; j < ne; j += blockDim.x) {
-      const double t = M[(long long)k * ne + j];
-      M[(long long)k * ne + j] = M[(long long)p * ne + j];
-      M[(long long)p * ne + j] = t;
-    }
-    if (tid == 0) { const double t = b[k]; b[k] = b[p]; b[p] = t; }
-    __syncthreads();
-  }
-  const double dkk = M[(long long)k * ne + k], bk = b[k];
-  for (int i = k + 1 + tid; i < ne; i += blockDim.x) {
-    const double l = M[(long long)i * ne + k] / dkk;
-    M[(long long)i * ne + k] = l;
-    b[i] -= l * bk;
-  }
-}
-
-// rank-1 update of the trailing block after column k: one workgroup per row
-__global__ void __launch_bounds__(256) k_eeq_lu_update(const MolDesc* __restrict__ desc, const int* __restrict__ list,
-                                                       int k, double* E, const int* __restrict__ failed) {
-  const MolDesc md = desc[list[blockIdx.y]];
-  const int ne = md.ne;
-  const int i = k + 1 + blockIdx.x;
-  if (i >= ne || failed[md.mol]) return;
-  double* M = E + md.e0;
-  const double l = M[(long long)i * ne + k];
-  double* Mi = M + (long long)i * ne;
-  const double* Mk = M + (long long)k * ne;
-  for (int j = k + 1 + threadIdx.x; j < ne; j += blockDim.x) Mi[j] -= l * Mk[j];
 }
 
 // zero the atomic dipoles and quadrupoles (or the gradient) of the selected molecules
@@ -881,7 +1021,7 @@ void Batch::allocate(const Capacity& c) {
   sub_dbl_ = alloc<double>((long long)nmol * kSubDbls);
   HIPCHECK(hipMemset(sub_dbl_, 0, (size_t)nmol * kSubDbls * sizeof(double)));
   eeq_failed = alloc<int>(nmol);
-  eeq_big = alloc<int>(nmol);
+  eeq_bad = alloc<int>(nmol);
   eig_failed = alloc<int>(nmol);
   HIPCHECK(hipMemset(eig_failed, 0, nmol * sizeof(int)));
   d_sub = alloc<MolDesc>(nmol);
@@ -2396,7 +2536,7 @@ void Batch::setup() {
                      el, at, xyz, cn, radcn, gab3, gab5);
   // implicit solvent: Born radii, surface, H-bond weights, shape, matrix B
   if (solv_on_ && sub_max_n > 0) {
-    hipLaunchKernelGGL(k_eeq_reset, dim3(grid1(ns, 64)), dim3(64), 0, s4, d_sub, ns, sv_failed);
+    hipLaunchKernelGGL(k_eeq_reset, dim3(grid1(ns, 64)), dim3(64), 0, s4, d_sub, ns, sv_failed, (int*)nullptr);
     hipLaunchKernelGGL(k_solv_born, dim3(grid1(sub_max_n, 64), ns), dim3(64), 0, s4, d_sub,
                        (const SolvDev*)d_solv, at, xyz, sv_brad, sv_dpsi);
     hipLaunchKernelGGL(k_solv_sasa, dim3(sub_max_n, ns), dim3(64), 0, s4, d_sub, (const SolvDev*)d_solv, at, xyz,
@@ -2446,36 +2586,31 @@ void Batch::setup() {
   // initial charges: EEQ (default) or SAD.  The EEQ solve runs on stream2
   // beside the integrals and S^(-1/2) (it reads only CN, zsh and geometry,
   // writes only its own system and the charges); joined below.
-  std::vector<int> big;
   if (resident) {
-    hipLaunchKernelGGL(k_eeq_reset, dim3(grid1(ns, 64)), dim3(64), 0, stream, d_sub, ns, eeq_failed);
+    hipLaunchKernelGGL(k_eeq_reset, dim3(grid1(ns, 64)), dim3(64), 0, stream, d_sub, ns, eeq_failed, eeq_bad);
     hipLaunchKernelGGL(k_q_from_qsh, dim3(grid1(sub_max_n, 64), ns), dim3(64), 0, stream, d_sub, sh_at,
                        (const double*)qsh, q);
   } else if (eeq) {
     const long long ne = sub_max_n + 1;
-    hipLaunchKernelGGL(k_eeq_matrix, dim3(grid1(ne * ne, 256), ns), dim3(256), 0, stream2, d_sub, el, at, xyz,
-                       cn_eeq, E, xE);
-    hipLaunchKernelGGL(k_eeq_reset, dim3(grid1(ns, 64)), dim3(64), 0, stream2, d_sub, ns, eeq_failed);
-    // large systems: one launch pair per column over the whole device
-    int big_max = 0;
-    for (int k = 0; k < ns; ++k)
-      if (desc[sel_[k]].ne >= kEeqBigNe) {
-        big.push_back(k);
-        big_max = std::max(big_max, desc[sel_[k]].ne);
-      }
-    if (!big.empty()) {
-      HIPCHECK(hipMemcpyAsync(eeq_big, big.data(), big.size() * sizeof(int), hipMemcpyHostToDevice, stream2));
-      const int nb = (int)big.size();
-      for (int k = 0; k < big_max; ++k) {
-        hipLaunchKernelGGL(k_eeq_lu_pivot, dim3(nb), dim3(256), 0, stream2, d_sub, (const int*)eeq_big, k, E, xE,
-                           eeq_failed);
-        if (big_max - k - 1 > 0)
-          hipLaunchKernelGGL(k_eeq_lu_update, dim3(big_max - k - 1, nb), dim3(256), 0, stream2, d_sub,
-                             (const int*)eeq_big, k, E, (const int*)eeq_failed);
-      }
+    const dim3 gm(grid1(ne * ne, 256), ns);
+    hipLaunchKernelGGL(k_eeq_reset, dim3(grid1(ns, 64)), dim3(64), 0, stream2, d_sub, ns, eeq_failed, eeq_bad);
+    hipLaunchKernelGGL(k_eeq_matrix, gm, dim3(256), 0, stream2, d_sub, el, at, xyz, cn_eeq, E, xE,
+                       (const int*)nullptr);
+    for (int kb = 0; kb * kEeqNb < sub_max_n; ++kb) {
+      const int rest = sub_max_n + 2 - kb * kEeqNb;
+      hipLaunchKernelGGL(k_eeq_panel, dim3(grid1(rest, 256), ns), dim3(256), 0, stream2, d_sub, kb, E, xE, yE,
+                         eeq_bad);
+      if (rest - 2 > kEeqNb)
+        hipLaunchKernelGGL(k_eeq_update, dim3(grid1(rest - 2 - kEeqNb, 64), grid1(rest - kEeqNb, 64), ns), dim3(256),
+                           0, stream2, d_sub, kb, E, xE, (const int*)eeq_bad);
     }
+    hipLaunchKernelGGL(k_eeq_solve, dim3(ns), dim3(256), 0, stream2, d_sub, el, at, at_sh0, (const double*)E, xE,
+                       (const double*)yE, q, qsh, (const double*)zsh, eeq_bad);
+    // not positive definite: the matrix again, then the pivoted elimination
+    hipLaunchKernelGGL(k_eeq_matrix, gm, dim3(256), 0, stream2, d_sub, el, at, xyz, cn_eeq, E, xE,
+                       (const int*)eeq_bad);
     hipLaunchKernelGGL(k_eeq_gesv, dim3(ns), dim3(256), 0, stream2, d_sub, el, at, at_sh0, E, xE, yE, q, qsh,
-                       (const double*)zsh, eeq_failed, kEeqBigNe);
+                       (const double*)zsh, eeq_failed, (const int*)eeq_bad);
   } else {
     hipLaunchKernelGGL(k_sad_guess, dim3(grid1(sub_max_n, 64), ns), dim3(64), 0, stream, d_sub, el, at, at_sh0, q,
                        qsh, (const double*)zsh);
@@ -2537,7 +2672,7 @@ void Batch::scc_prologue() {
     hipLaunchKernelGGL(k_solv_pot, dim3(max_n, nmol), dim3(64), 0, stream, d_desc, (const double*)sv_B,
                        (const double*)q, sv_pot, (const MolState*)d_state);
   hipLaunchKernelGGL(k_shift_final, dim3(grid1(max_nsh, 64), nmol), dim3(64), 0, stream, d_desc, el, at, sh_at,
-                     (const double*)d4dum, (const double*)dzv, solv_on_ ? (const double*)sv_pot : nullptr, shift,
+                     (const int*)d4_at, (const double*)d4dum, (const double*)dzv, solv_on_ ? (const double*)sv_pot : nullptr, shift,
                      (const MolState*)d_state);
   HIPCHECK(hipEventRecord(ev_join, stream2));
   HIPCHECK(hipStreamWaitEvent(stream, ev_join, 0));
@@ -2695,7 +2830,7 @@ bool Batch::scc_iteration(bool queue_next, bool subspace_ok) {
   hipLaunchKernelGGL(k_scc_control, dim3(nmol), dim3(256), 0, stream, d_desc, d_state, (const double*)jq,
                      (const double*)shgam, (const double*)row_e, (const double*)ae01, (const double*)zv,
                      (const double*)d4dum, solv_on_ ? (const double*)sv_qbq : nullptr, (const double*)sv_gsasa,
-                     sv_gshift, sh_at, qsh, q, dipm, qp, q_in, dq, qlast, dqlast, bdf, bu, ba, bomega, scfconv, qconv);
+                     sv_gshift, at_sh0, qsh, q, dipm, qp, q_in, dq, qlast, dqlast, bdf, bu, ba, bomega, scfconv, qconv);
   HIPCHECK(hipGetLastError());
   iterations_ += 1;
   if (trace_rounds)

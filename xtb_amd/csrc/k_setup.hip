@@ -418,8 +418,9 @@ __global__ void k_dispmat(const MolDesc* __restrict__ desc, const Element* __res
 // src/eeq_model.f90:60-80,678-860)
 __global__ void k_eeq_matrix(const MolDesc* __restrict__ desc, const Element* __restrict__ el,
                              const int* __restrict__ at, const double* __restrict__ xyz, const double* __restrict__ cn_eeq,
-                             double* E, double* xE) {
+                             double* E, double* xE, const int* __restrict__ only) {
   const MolDesc md = desc[blockIdx.y];
+  if (only && !only[md.mol]) return;
   const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   const long long ne = md.ne;
   if (t >= ne * ne) return;

@@ -30,7 +30,7 @@
 // T is positive definite and every virtual eigenvalue lies above every
 // occupied one by at least (1 - rho) min D.  The path is left unless that is
 // at least kSubGapKt kT: the Fermi occupations of the frontier orbitals are
-// then within 4e-18 of 1 and 0, no entropy term arises, and the density is
+// then within 9e-17 of 1 and 0 (half a unit in the last place), no entropy term arises, and the density is
 // the one of the full diagonalisation to rounding.
 #pragma once
 #include "device_util.h"
@@ -44,7 +44,7 @@ constexpr int kSubSteps = 24;        // steps per SCC iteration at most
 // the first basis, 8 to 10 steps on the second); after a second time it
 // stays with full diagonalisations
 constexpr int kSubTries = 2;
-constexpr double kSubGapKt = 80.0;   // smallest gap in units of kT
+constexpr double kSubGapKt = 74.0;   // smallest gap in units of kT
 constexpr double kSubRhoMax = 0.8;   // largest contraction of a plain step
 constexpr double kSubRhoMin = 0.15;  // smallest contraction that takes the second-order step
 constexpr double kSubDrop = 1e-17;   // a factor I + E of the inverse with o max |E| below this is left out
