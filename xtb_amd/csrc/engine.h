@@ -108,9 +108,11 @@ struct JacobiProb {
   int ev_off;                 // eigenvalue offset
   int group;                  // lane (stream) of the two-lane round schedule
   int ld;                     // row stride of the problem's A and W (dim, or dim rounded up to 16)
-  long long src_off;          // the matrix in the caller's packed layout (row stride dim)
+  long long src_off;          // the matrix in the caller's layout (row stride src_ld)
   int maxsw;                  // sweeps before the problem is given up (failed)
-  int pad_;
+  int mol;                    // batch slot
+  int src_ld;
+  int row0;                   // first row of the problem in the molecule's matrix (a diagonal block)
 };
 
 // stream lanes of the block-Jacobi rounds (at most)
@@ -124,6 +126,10 @@ constexpr int kProfLines = 64, kProfLineU64 = 16;
 // A set of Jacobi problems (one per molecule) with its device work lists.
 struct JacSet {
   std::vector<JacobiProb> probs;
+  int nprob = 0;              // 1 or (half) 2 per slot
+  bool half = false;          // the occupied and the virtual block of every subspace molecule
+  bool shared = false;        // ja, jw and qbuf belong to another set
+  long long small_cap = 0, pairs_cap = 0, ta_cap = 0, tw_cap = 0, to_cap = 0, big_cap = 0, xp_cap = 0, xt_cap = 0;
   JacobiProb* d_probs = nullptr;
   int nsmall = 0, npairs = 0, nta = 0, ntw = 0, max_rounds = 0;
   int max_rounds_lanes = 0;   // the same without the blocked eigensolver's problems
@@ -334,8 +340,7 @@ class Batch {
   std::vector<char> occupied_;
   std::vector<HostMol> hmol_;
   std::vector<char> elem_present_;
-  long long tiles_cap_ = 0, small_cap_ = 0, pairs_cap_ = 0, ta_cap_ = 0, tw_cap_ = 0, to_cap_ = 0, big_cap_ = 0;
-  long long xp_cap_ = 0, xt_cap_ = 0;
+  long long tiles_cap_ = 0;
   void allocate(const Capacity& c);
   void init_common();
   void place(int m, const MolDesc& d, const HostMol& hm, const MolState& st, bool upload);
@@ -378,6 +383,12 @@ class Batch {
   int2* pair_list = nullptr;   // the molecules' HostMol::pairs at p0   // per atom pair H0 gradient terms: 5 doubles at 5 * (p0 + i n + j)
   // Jacobi bookkeeping
   JacSet jac_n;
+  JacSet jac_h;                // the diagonal blocks of the last diagonalisation (k_sub.hip)
+  void jac_alloc(JacSet& js, int nprob);
+  void jac_lists(JacSet& js);  // problems and work lists of the occupied slots
+  // ptr holds at least need elements (cap: its capacity)
+  template <class T_>
+  void grow(T_*& ptr, long long& cap, long long need);
   int* jac_nactive = nullptr;
   int* perm = nullptr;
   int* eeq_failed = nullptr;
@@ -421,7 +432,7 @@ class Batch {
   // step factors, counts, and its product tiles (a launch's tiles are
   // [sub_t0[k], sub_t0[k + 1]) of d_sub_tiles); XTBAMD_SUBSPACE=0 turns it off
   bool subspace_on = true;
-  static constexpr int kSubLists = 9;
+  static constexpr int kSubLists = 15;
   int sub_t0[kSubLists + 1] = {};
   long long sub_tiles_cap_ = 0;
   int4* d_sub_tiles = nullptr;
@@ -430,6 +441,7 @@ class Batch {
   double* sub_dbl_ = nullptr;
   int sub_guess_ = 6;   // steps queued before the first count is read
   void subspace(bool allow);
+  bool split_ok() const { return jac_p == 32 && !apply_lds && !pivot_lds; }
   bool final_ = false;      // diagonalise() is orbitals()' one
   bool need_full_ = true;   // some molecule takes the full diagonalisation
   void diagonalise();       // of the molecules with MolState::diag: C, emo, occupations

@@ -1036,18 +1036,20 @@ void Batch::allocate(const Capacity& c) {
   ns_fin = alloc<int>(nmol);
   ns_act = alloc<int>(nmol);
   ns_failed = alloc<int>(nmol);
-  // Jacobi set: per-slot problem table and state; work lists grow on demand
+  jac_alloc(jac_n, nmol);
   JacSet& js = jac_n;
-  js.probs.assign(nmol, JacobiProb());
-  js.d_probs = alloc<JacobiProb>(nmol);
-  js.offmax = alloc<unsigned long long>(2LL * nmol);   // two sweep-parity buffers
-  js.state = alloc<int>((long long)nmol * kJacState);
-  js.scale = alloc<double>(nmol);
   // pivot-factor buffer: at most nao / jac_p + 1 pairs of jac_p^2 per molecule
   js.qsize = std::max(4096LL, (c.nao / jac_p + 2LL * nmol) * (long long)jac_p * jac_p);
   js.qbuf = alloc<double>(js.qsize);
   js.rot = alloc<int>(js.qsize / 1024 + 1);
   js.perm = nullptr;
+  if (subspace_on && split_ok()) {
+    jac_h.half = true;
+    jac_alloc(jac_h, 2 * nmol);
+    jac_h.qsize = js.qsize;
+    jac_h.qbuf = js.qbuf;
+    jac_h.rot = js.rot;
+  }
   Element* d_el = alloc<Element>(XTB_MAX_Z + 1);
   HIPCHECK(hipMemcpy(d_el, host_elements(), (XTB_MAX_Z + 1) * sizeof(Element), hipMemcpyHostToDevice));
   elements_dev = d_el;
@@ -1169,6 +1171,24 @@ void Batch::release(int m) {
   HIPCHECK(hipStreamSynchronize(stream));
 }
 
+template <class T_>
+void Batch::grow(T_*& ptr, long long& capv, long long need) {
+  if (need <= capv && ptr) return;
+  if (ptr) {
+    HIPCHECK(hipStreamSynchronize(stream));
+    auto it = std::find(allocs_.begin(), allocs_.end(), (void*)ptr);
+    if (it != allocs_.end()) allocs_.erase(it);
+    if (!on_loan()) HIPCHECK(hipFree(ptr));   // a loan's pieces are never released
+  }
+  capv = std::max<long long>(need, 2 * capv);
+  ptr = alloc<T_>(capv);
+}
+
+// closed shells with occupied and virtual orbitals
+static bool sub_able(const MolDesc& d) {
+  return d.n > 1 && d.nopen == 0 && (d.nel & 1) == 0 && d.nel >= 2 && d.nel / 2 < d.nao;
+}
+
 // Appends the tiles of a launch (per molecule) to out in an order that keeps
 // a molecule on one XCD: workgroup b of a launch runs on XCD b mod kXcds, so
 // the matrices of a molecule are fetched by one L2 only.  Molecules go to the
@@ -1210,18 +1230,6 @@ void Batch::rebuild() {
     max_nbr = std::max(max_nbr, d.nbr);
   }
   HIPCHECK(hipMemcpyAsync(d_desc, desc.data(), nmol * sizeof(MolDesc), hipMemcpyHostToDevice, stream));
-  auto grow = [&](auto*& ptr, long long& capv, long long need) {
-    using T_ = typename std::remove_reference<decltype(*ptr)>::type;
-    if (need <= capv && ptr) return;
-    if (ptr) {
-      HIPCHECK(hipStreamSynchronize(stream));
-      auto it = std::find(allocs_.begin(), allocs_.end(), (void*)ptr);
-      if (it != allocs_.end()) allocs_.erase(it);
-      if (!on_loan()) HIPCHECK(hipFree(ptr));   // a loan's pieces are never released
-    }
-    capv = std::max<long long>(need, 2 * capv);
-    ptr = alloc<T_>(capv);
-  };
   // GEMM tiles over (molecule, 64x64 tile)
   std::vector<int4> tl, ts;
   {
@@ -1248,64 +1256,93 @@ void Batch::rebuild() {
   {
     std::vector<int4> st;
     int k = 0;
-    auto launch = [&](std::initializer_list<std::pair<int, bool>> kinds) {
+    // a product: its kind and flags, rows and columns (0: N, 1: occupied, 2: virtual)
+    struct Kind {
+      int w, rows, cols;
+    };
+    auto launch = [&](const std::vector<Kind>& kinds) {
       sub_t0[k++] = (int)st.size();
       std::vector<std::vector<int4>> mt(nmol);
-      for (auto& p : kinds)
+      for (const Kind& kd : kinds)
         for (int m = 0; m < nmol; ++m) {
           const MolDesc& d = desc[m];
-          const int kind = p.first, o = d.nel / 2, v = d.nao - o;
-          if (!occupied_[m] || d.nopen != 0 || (d.nel & 1) || o < 1 || v < 1) continue;
-          const int rows = kind == kSubR ? v : kind == kSubB || kind == kSubP ? d.nao : o;
-          const int cols = kind == kSubCY || kind == kSubCYZ || kind == kSubP ? d.nao : o;
-          for (int a = 0; a < (rows + kTile - 1) / kTile; ++a)
-            for (int b = p.second ? a : 0; b < (cols + kTile - 1) / kTile; ++b)
-              mt[m].push_back(make_int4(m, a, b, kind | (p.second ? kSubSym : 0)));
+          if (!occupied_[m] || !sub_able(d)) continue;
+          const int dims[3] = {d.nao, d.nel / 2, d.nao - d.nel / 2};
+          for (int a = 0; a < (dims[kd.rows] + kTile - 1) / kTile; ++a)
+            for (int b = kd.w & kSubSym ? a : 0; b < (dims[kd.cols] + kTile - 1) / kTile; ++b)
+              mt[m].push_back(make_int4(m, a, b, kd.w));
         }
       xcd_order(mt, st);
     };
-    launch({{kSubB, false}});
-    launch({{kSubR, false}});
-    launch({{kSubM, true}});
-    launch({{kSubCY, false}});
-    launch({{kSubE1, true}});
-    launch({{kSubZ2, true}, {kSubE, true}});
-    launch({{kSubZ, true}, {kSubE, true}});
-    launch({{kSubCYZ, false}});
-    launch({{kSubP, true}});
+    launch({{kSubB, 0, 1}});
+    launch({{kSubR, 2, 1}});
+    launch({{kSubM | kSubSym, 1, 1}});
+    launch({{kSubCY, 1, 0}});
+    launch({{kSubE1 | kSubSym, 1, 1}});
+    launch({{kSubZ2 | kSubSym, 1, 1}, {kSubE | kSubSym, 1, 1}});
+    launch({{kSubZ | kSubSym, 1, 1}, {kSubE | kSubSym, 1, 1}});
+    launch({{kSubCYZ, 1, 0}});
+    launch({{kSubP | kSubSym, 0, 0}});
+    for (int kind = kRotM; kind < kRotU; ++kind)
+      launch({{kind | kSubSym, 1, 1}, {kind | kRotVirt | kSubSym, 2, 2}});
+    launch({{kRotU, 2, 1}});
     sub_t0[k] = (int)st.size();
     grow(d_sub_tiles, sub_tiles_cap_, std::max<long long>(1, (long long)st.size()));
     if (!st.empty())
       HIPCHECK(hipMemcpyAsync(d_sub_tiles, st.data(), st.size() * sizeof(int4), hipMemcpyHostToDevice, stream));
     HIPCHECK(hipStreamSynchronize(stream));   // st goes out of scope
   }
-  // Jacobi problems: dim nao, matrices at m0, eigenvalues at o0
-  JacSet& js = jac_n;
+  jac_lists(jac_n);
+  if (subspace_on && split_ok()) jac_lists(jac_h);
+}
+
+// per-slot problem table and state of a set; the work lists grow on demand
+void Batch::jac_alloc(JacSet& js, int nprob) {
+  js.nprob = nprob;
+  js.probs.assign(nprob, JacobiProb());
+  js.d_probs = alloc<JacobiProb>(nprob);
+  js.offmax = alloc<unsigned long long>(2LL * nprob);   // two sweep-parity buffers
+  js.state = alloc<int>((long long)nprob * kJacState);
+  js.scale = alloc<double>(nprob);
+}
+
+void Batch::jac_lists(JacSet& js) {
   long long qoff = 0;
   std::vector<int> small, big, blk;
   std::vector<int2> pairs;
   std::vector<int4> ta, tw, to;
   // the blocked eigensolver takes the largest problems on the register path
-  const bool blk_path = jac_padded && jac_p == 32 && !use_ql;
+  const bool blk_path = jac_padded && jac_p == 32 && !use_ql && !js.half;
   js.max_rounds = 0;
   js.max_rounds_lanes = 0;
   js.big_max_dim = 0;
   js.big_max_ld = 0;
   long long poff = 0;
-  for (int m = 0; m < nmol; ++m) {
+  // problems: the whole matrix (dim nao, at m0, eigenvalues at o0), or its
+  // occupied and virtual diagonal blocks
+  for (int m = 0; m < js.nprob; ++m) {
     JacobiProb& p = js.probs[m];
     std::memset(&p, 0, sizeof(p));
-    if (!occupied_[m]) continue;
-    p.dim = desc[m].nao;
+    const int mol = js.half ? m / 2 : m;
+    p.mol = mol;
+    if (!occupied_[mol]) continue;
+    const MolDesc& d = desc[mol];
+    if (js.half && !sub_able(d)) continue;
+    p.dim = d.nao;
+    if (js.half) {
+      p.row0 = m & 1 ? d.nel / 2 : 0;
+      p.dim = m & 1 ? d.nao - d.nel / 2 : d.nel / 2;
+    }
     p.nb = (p.dim + jac_p / 2 - 1) / (jac_p / 2);
     p.nbp = p.nb + (p.nb & 1);
     p.rounds = std::max(1, p.nbp - 1);
-    p.src_off = desc[m].m0;
-    p.ld = jac_padded ? (p.dim + 15) / 16 * 16 : p.dim;
-    p.a_off = jac_padded ? poff : desc[m].m0;
+    p.src_ld = d.nao;
+    p.src_off = d.m0 + (long long)p.row0 * (d.nao + 1);
+    p.ld = jac_padded ? (p.dim + 15) / 16 * 16 : d.nao;
+    p.a_off = jac_padded ? poff : p.src_off;
     p.w_off = p.a_off;
     if (jac_padded) poff += (long long)p.ld * p.ld;
-    p.ev_off = desc[m].o0;
+    p.ev_off = d.o0 + p.row0;
     p.q_off = qoff;
     p.maxsw = jac_max_sweeps;
     js.big_max_ld = std::max(js.big_max_ld, p.ld);
@@ -1419,31 +1456,37 @@ void Batch::rebuild() {
   }
   js.gxp[kMaxLanes] = (int)xp.size();
   js.gxt[kMaxLanes] = (int)xt.size();
-  grow(js.d_xp, xp_cap_, std::max<long long>(1, (long long)xp.size()));
-  grow(js.d_xt, xt_cap_, std::max<long long>(1, (long long)xt.size()));
+  grow(js.d_xp, js.xp_cap, std::max<long long>(1, (long long)xp.size()));
+  grow(js.d_xt, js.xt_cap, std::max<long long>(1, (long long)xt.size()));
   if (!xp.empty()) HIPCHECK(hipMemcpyAsync(js.d_xp, xp.data(), xp.size() * sizeof(int2), hipMemcpyHostToDevice, stream));
   if (!xt.empty()) HIPCHECK(hipMemcpyAsync(js.d_xt, xt.data(), xt.size() * sizeof(int4), hipMemcpyHostToDevice, stream));
   if (qoff > js.qsize) throw std::runtime_error("Jacobi pivot buffer too small");
   if (jac_padded) {
-    long long c0 = js.jcap;
-    grow(js.ja, c0, std::max<long long>(1, poff));
-    grow(js.jw, js.jcap, std::max<long long>(1, poff));
+    // the working copies are those of jac_n for both sets
+    JacSet& own = jac_n;
+    long long c0 = own.jcap;
+    grow(own.ja, c0, std::max<long long>(1, poff));
+    grow(own.jw, own.jcap, std::max<long long>(1, poff));
+    js.ja = own.ja;
+    js.jw = own.jw;
   }
-  HIPCHECK(hipMemcpyAsync(js.d_probs, js.probs.data(), nmol * sizeof(JacobiProb), hipMemcpyHostToDevice, stream));
+  HIPCHECK(hipMemcpyAsync(js.d_probs, js.probs.data(), js.nprob * sizeof(JacobiProb), hipMemcpyHostToDevice, stream));
   js.nsmall = (int)small.size();
   js.npairs = (int)pairs.size();
   js.nta = (int)ta.size();
   js.ntw = (int)tw.size();
   js.nto = (int)to.size();
-  grow(js.d_small, small_cap_, std::max<long long>(1, js.nsmall));
-  grow(js.d_pairs, pairs_cap_, std::max<long long>(1, js.npairs));
-  grow(js.d_ta, ta_cap_, std::max<long long>(1, js.nta));
-  grow(js.d_tw, tw_cap_, std::max<long long>(1, js.ntw));
-  grow(js.d_to, to_cap_, std::max<long long>(1, js.nto));
-  eig_.mols = blk;
-  eig_build();
+  grow(js.d_small, js.small_cap, std::max<long long>(1, js.nsmall));
+  grow(js.d_pairs, js.pairs_cap, std::max<long long>(1, js.npairs));
+  grow(js.d_ta, js.ta_cap, std::max<long long>(1, js.nta));
+  grow(js.d_tw, js.tw_cap, std::max<long long>(1, js.ntw));
+  grow(js.d_to, js.to_cap, std::max<long long>(1, js.nto));
+  if (!js.half) {
+    eig_.mols = blk;
+    eig_build();
+  }
   js.nbig = (int)big.size();
-  grow(js.d_big, big_cap_, std::max<long long>(1, js.nbig));
+  grow(js.d_big, js.big_cap, std::max<long long>(1, js.nbig));
   if (!big.empty()) HIPCHECK(hipMemcpyAsync(js.d_big, big.data(), big.size() * sizeof(int), hipMemcpyHostToDevice, stream));
   if (!small.empty())
     HIPCHECK(hipMemcpyAsync(js.d_small, small.data(), small.size() * sizeof(int), hipMemcpyHostToDevice, stream));
@@ -1571,7 +1614,7 @@ Batch::~Batch() {
 
 // ---------------------------------------------------------------------------
 bool Batch::jacobi(JacSet& js, double* Am, double* Wm, double* evout, bool check_active, bool keep_w, int banded) {
-  const int nb = nmol;
+  const int nb = js.nprob;
   const bool rows = jac_p == 32 && !apply_lds && !keep_w && banded == 0;
   const MolState* act = check_active ? (const MolState*)d_state : (const MolState*)nullptr;
   double* Wout = Wm;
@@ -1596,7 +1639,8 @@ bool Batch::jacobi(JacSet& js, double* Am, double* Wm, double* evout, bool check
   const bool lanes = rows && !pivot_lds && js.npairs > 0;
   // the largest problems go to the blocked eigensolver on stream3 (after the
   // small ones), beside the lanes
-  const bool blk = rows && !pivot_lds && eig_.np > 0 && (iterations_ < eig_blk_iters || (final_ && eig_blk_iters > 0));
+  const bool blk = rows && !pivot_lds && !js.half && eig_.np > 0 &&
+                   (iterations_ < eig_blk_iters || (final_ && eig_blk_iters > 0));
   // the blocked path's problems are marked done for the lanes
   if (blk)
     hipLaunchKernelGGL(k_eig_claim, dim3(1), dim3(256), 0, stream, (const EigProb*)eig_.d_probs, eig_.np, js.state);
@@ -2092,7 +2136,7 @@ void Batch::jacobi_lanes(JacSet& js, double* Am, double* Wm) {
     const int nto = js.gto[g + 1] - js.gto[g];
     if (live[g] && nto > 0)
       hipLaunchKernelGGL(k_jac_offmax, dim3(nto), dim3(256), 0, ls[g], js.d_probs, js.d_to + js.gto[g],
-                         (const double*)Am, (const int*)js.state, js.offmax + nmol, 0);
+                         (const double*)Am, (const int*)js.state, js.offmax + js.nprob, 0);
   }
   const int period = std::max(1, jac_period_);
   const int rmax = (jac_max_sweeps + 1) * js.max_rounds;
@@ -2113,11 +2157,11 @@ void Batch::jacobi_lanes(JacSet& js, double* Am, double* Wm) {
       if (jac_cross)
         hipLaunchKernelGGL(k_jac_pairsR<true>, dim3(js.gxp[g + 1] - js.gxp[g]), dim3(64), 0, ls[g], js.d_probs,
                            js.d_xp + js.gxp[g], rr, (const double*)Am, js.qbuf, js.rot, (const double*)js.scale,
-                           js.state, inner_sweeps, sample ? jw : nullptr, jac_tol, js.offmax, nmol, pts);
+                           js.state, inner_sweeps, sample ? jw : nullptr, jac_tol, js.offmax, js.nprob, pts);
       else
         hipLaunchKernelGGL(k_jac_pairsR<false>, dim3(js.gxp[g + 1] - js.gxp[g]), dim3(64), 0, ls[g], js.d_probs,
                            js.d_xp + js.gxp[g], rr, (const double*)Am, js.qbuf, js.rot, (const double*)js.scale,
-                           js.state, inner_sweeps, sample ? jw : nullptr, jac_tol, js.offmax, nmol, pts);
+                           js.state, inner_sweeps, sample ? jw : nullptr, jac_tol, js.offmax, js.nprob, pts);
       if (sample) prof_end(2, nullptr, 0, ls[g]);
     }
   };
@@ -2140,7 +2184,7 @@ void Batch::jacobi_lanes(JacSet& js, double* Am, double* Wm) {
     if (r % period == 0 && pending < 0) {
       for (int g = 0; g < kMaxLanes; ++g) {
         if (!live[g]) continue;
-        hipLaunchKernelGGL(k_jac_count, dim3(1), dim3(256), 0, ls[g], js.d_probs, nmol, (const int*)js.state, g,
+        hipLaunchKernelGGL(k_jac_count, dim3(1), dim3(256), 0, ls[g], js.d_probs, js.nprob, (const int*)js.state, g,
                            jac_nactive + g);
         HIPCHECK(hipMemcpyAsync(h_pinned + g, jac_nactive + g, sizeof(int), hipMemcpyDeviceToHost, ls[g]));
         HIPCHECK(hipEventRecord(lane_ev[g], ls[g]));
@@ -2158,7 +2202,7 @@ void Batch::jacobi_lanes(JacSet& js, double* Am, double* Wm) {
         ts = prof_ts_ + (size_t)kProfSlotU64 * (kProfTsSlots + prof_ts_used_[1]++);
       hipLaunchKernelGGL(k_jac_apply_R, dim3(js.gxt[g + 1] - js.gxt[g]), dim3(64), 0, ls[g], js.d_probs,
                          js.d_xt + js.gxt[g], r, Am, Wm, (const double*)js.qbuf, (const int*)js.rot,
-                         (const int*)js.state, js.offmax, nmol, tw, ts);
+                         (const int*)js.state, js.offmax, js.nprob, tw, ts);
       if (sample) prof_end(3, nullptr, 0, ls[g]);
     }
     jacobi_rounds_ += 1;
@@ -2784,7 +2828,40 @@ void Batch::orbitals() {
   HIPCHECK(hipStreamSynchronize(stream));
   if (h_pinned[8] <= 0) return;
   final_ = true;
-  diagonalise();
+  if (split_ok()) {
+    // rotate the orbitals so that A falls into its occupied and virtual
+    // blocks, then diagonalise those
+    const dim3 gm(gstride((long long)max_nao * max_nao), nmol);
+    const int* mask = &d_state[0].diag;
+    constexpr int ms = (int)(sizeof(MolState) / sizeof(int));
+    auto rot = [&](int list, int level) {
+      const int nt = sub_t0[list + 1] - sub_t0[list];
+      if (nt > 0)
+        hipLaunchKernelGGL(k_rot_gemm, dim3(nt), dim3(256), 0, stream, d_sub_tiles + sub_t0[list], d_desc,
+                           SubBufs{A, C, ev, Sm, G, T, W, H, P}, (const MolState*)d_state, (const int*)sub_,
+                           (const unsigned long long*)sub_res_, level);
+    };
+    rot(9, 0);
+    rot(10, 0);
+    for (int level = 0; level < 2; ++level)
+      for (int k = 11; k < 14; ++k) rot(k, level);
+    rot(14, 0);
+    hipLaunchKernelGGL(k_rot_diag, gm, dim3(256), 0, stream, d_desc, (const MolState*)d_state,
+                       (const unsigned long long*)sub_res_, (const double*)W, (const double*)H, G);
+    gemm(kGemmSymLeft, A, G, T, nullptr, nullptr, false, 1.0, mask, false, ms);   // A U
+    gemm(0, C, G, W, nullptr, nullptr, false, 1.0, mask, false, ms);              // C U
+    gemm(1, G, T, H, nullptr, nullptr, false, 1.0, mask, true, ms);               // U^T A U
+    hipLaunchKernelGGL(k_copy_diag, gm, dim3(256), 0, stream, d_desc, (const MolState*)d_state, (const double*)W, C);
+    hipLaunchKernelGGL(k_zero_diag, gm, dim3(256), 0, stream, d_desc, (const MolState*)d_state, W);
+    jacobi(jac_h, H, W, emo, true);
+    for (int b = 0; b < 2; ++b)
+      hipLaunchKernelGGL(k_fail_fold, dim3(grid1(nmol, 64)), dim3(64), 0, stream, d_state, nmol,
+                         (const int*)jac_h.state + b * kJacState + 1, 2 * kJacState, kFailDiag, (const int*)nullptr);
+    gemm(4, C, W, T, nullptr, perm, false, 1.0, mask, false, ms);                 // T = C W(perm, :)^T
+    hipLaunchKernelGGL(k_copy_diag, gm, dim3(256), 0, stream, d_desc, (const MolState*)d_state, (const double*)T, C);
+  } else {
+    diagonalise();
+  }
   final_ = false;
   hipLaunchKernelGGL(k_occ_fermi, dim3(nmol), dim3(256), 0, stream, d_desc, d_state, (const double*)emo, focca, foccb,
                      focc, opt.etemp, (const double*)qsh, (const double*)dipm, (const double*)qp, q_in, 1);

@@ -477,7 +477,7 @@ __global__ void __launch_bounds__(256) k_dc_leaf(const EigProb* __restrict__ pro
     q[u * kLd + v] = (u == v) ? 1.0 : 0.0;
   }
   __syncthreads();
-  jacobi64(a, q, 1e-15 * fmax(scl, 1e-300), 40, cs, pq, flags, red);
+  jacobi64(a, q, m, 1e-15 * fmax(scl, 1e-300), 40, cs, pq, flags, red);
   __syncthreads();
   // ascending order of the leaf's eigenvalues (ties by index)
   for (int u = threadIdx.x; u < m; u += blockDim.x) {

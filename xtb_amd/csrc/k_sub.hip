@@ -423,4 +423,116 @@ __global__ void __launch_bounds__(256) k_sub_pending(MolState* state, int nmol, 
   if (threadIdx.x == 0) cnt[0] = (int)c;
 }
 
+// ---------------------------------------------------------------------------
+// The last diagonalisation of a molecule on the subspace path: with X known,
+//
+//     U = [ Qo  -(X Qo)^T ]      Qo = (I + X^T X)^(-1/2)
+//         [ X Qo     Qv   ]      Qv = (I + X X^T)^(-1/2)   (X Qo = Qv X)
+//
+// is orthogonal and U^T A U falls into an occupied and a virtual block (what
+// couples them is R, below the tolerance of a finished diagonalisation), so
+// two problems of about half the size are left: half the rounds per sweep
+// and a quarter of the elements per round each.
+// The inverse square roots start from I - M / 2 + 3 M^2 / 8 (error 5 M^3 / 16)
+// and take one step Q <- Q (3 I - Q^2 (I + M)) / 2 (error e -> 3 e^2 / 4), a
+// second one where M^6 is not below rounding.
+constexpr int kRotVirt = 8;   // a kind + kRotVirt: the same for the virtual block (not kRotU)
+enum RotOp { kRotM = 0, kRotQ1, kRotS, kRotG, kRotQ, kRotU };
+constexpr double kRotOne = 1e-10;   // o max |M^4| up to which one step is enough
+
+__device__ __forceinline__ bool rot_two(const unsigned long long* __restrict__ res, int o) {
+  return !((double)o * __longlong_as_double((long long)res[kSubSteps]) < kRotOne);
+}
+
+// M in G, the Q of level 0 in W and of level 1 in H (both blocks in one N x N
+// buffer: o x o, then v x v); U replaces M in G
+__global__ void __launch_bounds__(256) k_rot_gemm(const int4* __restrict__ tiles, const MolDesc* __restrict__ desc,
+                                                  SubBufs bf, const MolState* __restrict__ state,
+                                                  const int* __restrict__ sub,
+                                                  const unsigned long long* __restrict__ res, int level) {
+  const int4 tl = tiles[blockIdx.x];
+  const int m = tl.x, op = tl.w & 7;
+  if (m < 0 || !state[m].diag) return;
+  const bool virt = (tl.w & kRotVirt) != 0, sym = (tl.w & kSubSym) != 0;
+  const MolDesc md = desc[m];
+  const int N = md.nao, o = sub_occ(md), v = N - o;
+  const bool two = rot_two(res + (long long)m * kSubRes, o);
+  if (level > 0 && !two) return;
+  const long long vo = (long long)v * o, off = md.m0 + (virt ? (long long)o * o : 0);
+  const double* X = bf.X + md.m0 + sub[m * kSubInts + kSubPar] * vo;
+  double* Mb = bf.G + off;
+  double* T = bf.T + off;
+  double* cur = (level & 1 ? bf.H : bf.W) + off;
+  double* oth = (level & 1 ? bf.W : bf.H) + off;
+  const int nb = virt ? v : o;
+  const double *Lp = cur, *Rp = cur;
+  int ldl = nb, M = nb, K = nb;
+  switch (op) {
+    case kRotM: Lp = Rp = virt ? X + 2 * vo : X; K = N - nb; break;
+    case kRotQ1: Lp = Rp = Mb; break;
+    case kRotS: break;
+    case kRotG: Lp = oth; Rp = Mb; break;
+    case kRotQ: Rp = T; break;
+    default: Lp = X + 2 * vo; ldl = v; M = v; Rp = (two ? bf.W : bf.H) + md.m0; break;
+  }
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, i16 = lane & 15, k4 = lane >> 4;
+  const int row0 = tl.y * kTile + 32 * (w >> 1), col0 = tl.z * kTile + 32 * (w & 1);
+  if (row0 >= M || col0 >= nb || (sym && row0 > col0)) return;
+  v4d acc[2][2];
+  wave_mm<false>(Lp, ldl, M, Rp, nb, nb, K, row0, col0, acc);
+  double* U = bf.G + md.m0;
+#pragma unroll
+  for (int r = 0; r < 2; ++r)
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const int gj = col0 + 16 * c + i16;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int gi = row0 + 16 * r + k4 + 4 * i;
+        if (gi >= M || gj >= nb || (sym && gi > gj)) continue;
+        const long long e = (long long)gi * nb + gj, et = (long long)gj * nb + gi;
+        const double x = acc[r][c][i], one = gi == gj ? 1.0 : 0.0;
+        switch (op) {
+          case kRotM: Mb[e] = x; Mb[et] = x; break;
+          case kRotQ1: {
+            const double y = one - 0.5 * Mb[e] + 0.375 * x;
+            cur[e] = y;
+            cur[et] = y;
+            break;
+          }
+          case kRotS: oth[e] = x; oth[et] = x; break;
+          case kRotG: {
+            const double y = 1.5 * one - 0.5 * (oth[e] + x);
+            T[e] = y;
+            T[et] = y;
+            break;
+          }
+          case kRotQ: oth[e] = x; oth[et] = x; break;
+          default:
+            U[(long long)(o + gi) * N + gj] = x;
+            U[(long long)gj * N + o + gi] = -x;
+            break;
+        }
+      }
+    }
+}
+
+// the diagonal blocks of U
+__global__ void __launch_bounds__(256) k_rot_diag(const MolDesc* __restrict__ desc, const MolState* __restrict__ state,
+                                                  const unsigned long long* __restrict__ res,
+                                                  const double* __restrict__ W, const double* __restrict__ H,
+                                                  double* U) {
+  const int m = blockIdx.y;
+  if (!state[m].diag) return;
+  const MolDesc md = desc[m];
+  const int N = md.nao, o = sub_occ(md), v = N - o;
+  const double* Q = (rot_two(res + (long long)m * kSubRes, o) ? W : H) + md.m0;
+  const long long oo = (long long)o * o, all = oo + (long long)v * v;
+  for (long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x; t < all; t += (long long)gridDim.x * blockDim.x) {
+    const long long u = t < oo ? t : t - oo;
+    const int nb = t < oo ? o : v, r0 = t < oo ? 0 : o;
+    U[md.m0 + (r0 + u / nb) * N + r0 + u % nb] = Q[t];
+  }
+}
+
 }  // namespace xtbamd
