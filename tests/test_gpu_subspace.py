@@ -39,7 +39,11 @@ def _both(monkeypatch, mols, solvent=None, **kw):
 
 def _check(a, b, tag):
     assert a["iterations"] == b["iterations"] and a["converged"] == b["converged"], tag
-    assert a["ihomo"] == b["ihomo"] and np.array_equal(a["focc"], b["focc"]), tag
+    assert a["ihomo"] == b["ihomo"], tag
+    # both come from a diagonalisation of the same matrix to within TOL["emo"]
+    # (and its Fermi level): |df| <= 2 spins x (2 x 1e-7 eV) / (4 kT), kT = 0.0259 eV
+    # at 300 K (the lowest temperature here with fractional occupations)
+    assert float(np.max(np.abs(a["focc"] - b["focc"]))) <= 4 * TOL["emo"] / (4 * 0.02585), tag
     for k, tol in TOL.items():
         d = float(np.max(np.abs(np.asarray(a[k]) - np.asarray(b[k]))))
         assert d <= tol, f"{tag} {k}: {d:.2e}"

@@ -30,8 +30,9 @@
 // T is positive definite and every virtual eigenvalue lies above every
 // occupied one by at least (1 - rho) min D.  The path is left unless that is
 // at least kSubGapKt kT: the Fermi occupations of the frontier orbitals are
-// then within 9e-17 of 1 and 0 (half a unit in the last place), no entropy term arises, and the density is
-// the one of the full diagonalisation to rounding.
+// then within e^-26 = 5e-12 of 1 and 0, the size of the density error that the
+// tolerance of R admits, and far below the 1e-9 from which entropy counts.
+// The occupations handed back are those of the last diagonalisation.
 #pragma once
 #include "device_util.h"
 #include "engine.h"
@@ -44,7 +45,7 @@ constexpr int kSubSteps = 24;        // steps per SCC iteration at most
 // the first basis, 8 to 10 steps on the second); after a second time it
 // stays with full diagonalisations
 constexpr int kSubTries = 2;
-constexpr double kSubGapKt = 74.0;   // smallest gap in units of kT
+constexpr double kSubGapKt = 52.0;   // smallest gap in units of kT
 constexpr double kSubRhoMax = 0.8;   // largest contraction of a plain step
 constexpr double kSubRhoMin = 0.15;  // smallest contraction that takes the second-order step
 constexpr double kSubDrop = 1e-17;   // a factor I + E of the inverse with o max |E| below this is left out
@@ -100,21 +101,20 @@ __device__ __forceinline__ void sub_rate(const unsigned long long* __restrict__ 
   if (s > 0) {
     const double wl = sd[kSubW + s - 1];
     bool slow = !(at(s - 1) < 1e300);
-    if (s >= 5) {
-      const double r = cbrt(at(s - 1) / at(s - 4));
-      slow = slow || !(r * r <= wl - 1.0 || sub_mu(r, wl) <= sd[kSubLim]);
+    double r = 0.0;
+    if (s >= 4) {
+      r = cbrt(at(s - 1) / at(s - 4));
+      slow = slow || (s >= 5 && !(r * r <= wl - 1.0 || sub_mu(r, wl) <= sd[kSubLim]));
     }
     if (slow) {
       sub_give_up(si, st);
       return;
     }
-    if (s >= 3) {
-      const double rr = at(s - 1) / at(s - 3);
-      if (rr > 1.2 * (wl - 1.0)) rho = fmax(rho, fmin(kSubRhoMax, sub_mu(sqrt(rr), wl)));
-      sd[kSubRho] = rho;
-    }
+    if (r * r > 1.1 * (wl - 1.0)) rho = fmax(rho, fmin(kSubRhoMax, sub_mu(r, wl)));
+    sd[kSubRho] = rho;
     // the plain step is better as long as max |R| falls faster than the
     // second-order iteration's sqrt(w - 1)
+    rho = fmin(rho, 0.95 * sd[kSubLim]);   // so that the optimal rate is not taken for a contraction over the limit
     if (s > 1 && rho >= kSubRhoMin) {
       const double wo = 2.0 / (1.0 + sqrt(1.0 - rho * rho)), r1 = at(s - 1) / at(s - 2);
       if (wl != 1.0 || r1 * r1 > wo - 1.0) w = wo;
