@@ -180,14 +180,16 @@ __device__ __forceinline__ double lane_value(double x, int lane) {
 // J q + lambda 1 = b and sum q = Q give lambda = (z2 z1 - Q) / z2 z2 and
 // q = L^-T (z1 - lambda z2), z1 = L^-1 b, z2 = L^-1 1.  The vectors 1 (row n
 // of E) and b ride along as rows n and n + 1 of the factorisation, so the
-// forward substitutions come with it.  Two launches per 32 columns for all
+// forward substitutions come with it.  Two launches per 16 columns for all
 // molecules (the pivoted elimination was 15 us per column inside one
 // workgroup and 28 us per column over the device): 2.9 -> 0.2 ms for 194
 // atoms, 58 -> 5 ms for 2100.
 // A molecule whose pivot is not positive is flagged in bad.
-constexpr int kEeqNb = 32;
+// (16 columns: the rows of a block fit the registers without spills; at 32
+// the panel kernel took 110 us instead of 10)
+constexpr int kEeqNb = 16;
 
-// Block column kb: every workgroup factors the 32 x 32 diagonal block (one
+// Block column kb: every workgroup factors the 16 x 16 diagonal block (one
 // wave, a row per lane, in registers) and solves 256 rows below it, one per
 // thread.  The diagonal block's factor goes, transposed, to the block's upper
 // triangle, which no workgroup of this launch reads, and its inverse diagonal
@@ -211,7 +213,7 @@ __global__ void __launch_bounds__(256) k_eeq_panel(const MolDesc* __restrict__ d
   }
   __syncthreads();
   if (tid < 64) {
-    const int row = tid & 31;
+    const int row = tid & (kEeqNb - 1);
     double a[kEeqNb];
     bool ok = true;
 #pragma unroll
@@ -226,7 +228,7 @@ __global__ void __launch_bounds__(256) k_eeq_panel(const MolDesc* __restrict__ d
 #pragma unroll
       for (int j = c + 1; j < kEeqNb; ++j) a[j] -= a[c] * lane_value(a[c], j);
     }
-    if (tid < 32) {
+    if (tid < kEeqNb) {
 #pragma unroll
       for (int c = 0; c < kEeqNb; ++c) Ls[row][c] = c <= row ? a[c] : 0.0;
     }
@@ -249,20 +251,19 @@ __global__ void __launch_bounds__(256) k_eeq_panel(const MolDesc* __restrict__ d
   double* p = i <= n ? M + (long long)i * ne + k0 : b + k0;
   double x[kEeqNb];
 #pragma unroll
-  for (int c = 0; c < kEeqNb; ++c) x[c] = c < nb ? p[c] : 0.0;
+  for (int c = 0; c < kEeqNb; ++c) x[c] = p[min(c, nb - 1)];
 #pragma unroll
   for (int c = 0; c < kEeqNb; ++c) {
-    double s = x[c];
+    x[c] *= inv[c];
 #pragma unroll
-    for (int t = 0; t < c; ++t) s -= x[t] * Ls[c][t];
-    x[c] = s * inv[c];
+    for (int t = c + 1; t < kEeqNb; ++t) x[t] -= x[c] * Ls[t][c];
   }
 #pragma unroll
   for (int c = 0; c < kEeqNb; ++c)
     if (c < nb) p[c] = x[c];
 }
 
-// trailing update after block column kb (32 columns): rows i of the lower
+// trailing update after block column kb: rows i of the lower
 // triangle and the two vector rows, 64 x 64 tiles
 __global__ void __launch_bounds__(256) k_eeq_update(const MolDesc* __restrict__ desc, int kb, double* E, double* xE,
                                                     const int* __restrict__ bad) {
@@ -306,7 +307,7 @@ __global__ void __launch_bounds__(256) k_eeq_update(const MolDesc* __restrict__ 
     }
 }
 
-// multiplier, back substitution (one workgroup per molecule, 32 unknowns at a
+// multiplier, back substitution (one workgroup per molecule, 16 unknowns at a
 // time, the last first) and the shell charges
 __global__ void __launch_bounds__(256) k_eeq_solve(const MolDesc* __restrict__ desc, const Element* __restrict__ el,
                                                    const int* __restrict__ at, const int* __restrict__ at_sh0,
@@ -314,7 +315,8 @@ __global__ void __launch_bounds__(256) k_eeq_solve(const MolDesc* __restrict__ d
                                                    const double* __restrict__ yE, double* q, double* qsh,
                                                    const double* __restrict__ zsh, int* bad) {
   __shared__ double sh[4];
-  __shared__ double part[8][kEeqNb];
+  constexpr int kGroups = 256 / kEeqNb;
+  __shared__ double part[kGroups][kEeqNb];
   __shared__ double Ls[kEeqNb][kEeqNb + 1];
   const MolDesc md = desc[blockIdx.x];
   if (bad[md.mol]) return;
@@ -333,7 +335,7 @@ __global__ void __launch_bounds__(256) k_eeq_solve(const MolDesc* __restrict__ d
   const double lam = (d1 - md.charge) / d2;
   for (int k0 = (n - 1) / kEeqNb * kEeqNb; k0 >= 0; k0 -= kEeqNb) {
     const int nb = min(kEeqNb, n - k0), k1 = k0 + nb;
-    const int c = tid & 31, g = tid >> 5;
+    const int c = tid & (kEeqNb - 1), g = tid / kEeqNb;
     for (int e = tid; e < kEeqNb * kEeqNb; e += 256) {
       const int r = e / kEeqNb, t = e % kEeqNb;   // L[t][r], t > r, from the block's upper triangle
       Ls[r][t] = t < nb && r < t ? M[(long long)(k0 + r) * ne + k0 + t] : 0.0;
@@ -341,10 +343,10 @@ __global__ void __launch_bounds__(256) k_eeq_solve(const MolDesc* __restrict__ d
     double s[4] = {0.0, 0.0, 0.0, 0.0};
     if (c < nb) {
       int i = k1 + g;
-      for (; i + 24 < n; i += 32)
+      for (; i + 3 * kGroups < n; i += 4 * kGroups)
 #pragma unroll
-        for (int u = 0; u < 4; ++u) s[u] += M[(long long)(i + 8 * u) * ne + k0 + c] * x[i + 8 * u];
-      for (; i < n; i += 8) s[0] += M[(long long)i * ne + k0 + c] * x[i];
+        for (int u = 0; u < 4; ++u) s[u] += M[(long long)(i + kGroups * u) * ne + k0 + c] * x[i + kGroups * u];
+      for (; i < n; i += kGroups) s[0] += M[(long long)i * ne + k0 + c] * x[i];
     }
     part[g][c] = (s[0] + s[1]) + (s[2] + s[3]);
     __syncthreads();
@@ -353,7 +355,7 @@ __global__ void __launch_bounds__(256) k_eeq_solve(const MolDesc* __restrict__ d
       if (c < nb) {
         r = z[k0 + c] - lam * z2[k0 + c];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) r -= part[u][c];
+        for (int u = 0; u < kGroups; ++u) r -= part[u][c];
         di = yE[md.y0 + k0 + c];
       }
       for (int t = kEeqNb - 1; t >= 0; --t) {

@@ -240,9 +240,25 @@ __global__ void __launch_bounds__(256) k_trd_col(const EigProb* __restrict__ pro
   const double* a = V + (long long)kVy * ld;
   double* Xp = X + p.x_off;
   double* Yp = Xp + (long long)2 * kEigNb * ld;
+  // the first 512 elements of this wave's row and of a are in flight while
+  // the workgroup forms the reflector, which only scales the product
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int r = j + 1 + blockIdx.x * 4 + wv;
+  const double* Ar = A + p.m_off + (long long)min(r, n - 1) * ld;
+  double fr[8], fa[8];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const int c = j + 2 + lane + 64 * q;
+    const bool in = c < n;
+    fr[q] = in ? Ar[c] : 0.0;
+    fa[q] = in ? a[c] : 0.0;
+  }
+  const double ar1 = Ar[j + 1], ar = a[min(r, n - 1)];
+  // the panel corrections' operand: lane t < i takes W(r, t), lane i + t V(r, t)
+  double xv = 0.0;
+  if (lane < 2 * i) xv = Xp[(long long)(lane < i ? kEigNb + lane : lane - i) * ld + min(r, n - 1)];
   double beta, tau, scale;
   trd_reflector(a, part2 + p.p_off2, Xp, ld, n, j, i, beta, tau, scale, y);
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   if (blockIdx.x == 0) {
     // publish column j: d, e, tau and v (Vh row j, panel buffers)
     if (tid == 0) {
@@ -261,33 +277,26 @@ __global__ void __launch_bounds__(256) k_trd_col(const EigProb* __restrict__ pro
   // w = tau (A22 v - W y1 - V y2) for this wave's row: the row product with
   // four independent partial sums per lane, the 2i panel corrections one per
   // lane, both reduced across the wave
-  const int r = j + 1 + blockIdx.x * 4 + wv;
   double wvdot = 0.0;
   if (r < n) {
-    const double* Ar = A + p.m_off + (long long)r * ld;
     // eight independent partial sums per lane: eight loads of the row in
     // flight per lane (the product is bound by memory latency, not issue)
     double sp[8];
 #pragma unroll
-    for (int q = 0; q < 8; ++q) sp[q] = 0.0;
-    int c = j + 2 + lane;
+    for (int q = 0; q < 8; ++q) sp[q] = fr[q] * fa[q];
+    int c = j + 2 + lane + 512;
 #pragma unroll 2
     for (; c + 448 < n; c += 512)
 #pragma unroll
       for (int q = 0; q < 8; ++q) sp[q] = fma(Ar[c + 64 * q], a[c + 64 * q], sp[q]);
     for (; c < n; c += 64) sp[0] = fma(Ar[c], a[c], sp[0]);
     double s = scale * (((sp[0] + sp[1]) + (sp[2] + sp[3])) + ((sp[4] + sp[5]) + (sp[6] + sp[7])));
-    if (lane == 0) s += Ar[j + 1];   // v[j+1] = 1
-    // corrections: lane t < i takes W(r, t) y1[t], lane i + t takes V(r, t) y2[t]
-    if (lane < 2 * i) {
-      const int t = lane < i ? lane : lane - i;
-      const double xv = lane < i ? Xp[(long long)(kEigNb + t) * ld + r] : Xp[(long long)t * ld + r];
-      s -= xv * y[lane];
-    }
+    if (lane == 0) s += ar1;   // v[j+1] = 1
+    if (lane < 2 * i) s -= xv * y[lane];
     s = tau * wave_sum(s);
     if (lane == 0) {
       V[(long long)kVw * ld + r] = s;
-      const double vr = r == j + 1 ? 1.0 : a[r] * scale;
+      const double vr = r == j + 1 ? 1.0 : ar * scale;
       wvdot = s * vr;
     }
   }
@@ -295,33 +304,75 @@ __global__ void __launch_bounds__(256) k_trd_col(const EigProb* __restrict__ pro
   if (tid == 0) V[(long long)kVrc * ld + blockIdx.x] = wvdot;
 }
 
+// Sums over the wave's 64 lanes of 64 values per lane, value l to lane l: each
+// step hands half of the values to the lane across and keeps the sums of the
+// other half, 63 exchanges instead of 6 per value.
+template <int H>
+__device__ __forceinline__ void wave_sums_step(double (&x)[64], int lane) {
+  const bool up = (lane & H) != 0;
+#pragma unroll
+  for (int q = 0; q < H; ++q) {
+    const double keep = up ? x[q + H] : x[q], send = up ? x[q] : x[q + H];
+    x[q] = keep + __shfl_xor(send, H, 64);
+  }
+}
+__device__ __forceinline__ double wave_sums64(double (&x)[64]) {
+  const int lane = threadIdx.x & 63;
+  wave_sums_step<32>(x, lane);
+  wave_sums_step<16>(x, lane);
+  wave_sums_step<8>(x, lane);
+  wave_sums_step<4>(x, lane);
+  wave_sums_step<2>(x, lane);
+  wave_sums_step<1>(x, lane);
+  return x[0];
+}
+
 // finish >= 0: w of column finish gets alpha v (alpha = -tau (w . v) / 2 from
 // k_trd_col's partials) and goes to the panel buffers.  next >= 0: the
 // corrected row a = A(next, next:n) minus the panel's first next - j0 vector
 // pairs, and this workgroup's partial sums for next's reflector; at
-// next = n - 1 only the last diagonal entry.  One thread per row.
+// next = n - 1 only the last diagonal entry.  One thread per row, its 64
+// panel elements in registers from the correction to the partial sums, all
+// loads issued before the first use: the launch is one chain of memory
+// latencies (12.5 -> 7 us at 1024 rows with the sums taken from registers by
+// exchanges instead of a second pass over the panel).
 __global__ void __launch_bounds__(256) k_trd_row(const EigProb* __restrict__ probs, const int* __restrict__ act,
                                                  const double* __restrict__ A, double* X, double* vec, double* part2,
                                                  int finish, int next, int j0) {
   __shared__ double sh[4];
-  __shared__ double cw[2 * kEigNb + 2];
-  __shared__ double ra[256];   // this workgroup's rows of the corrected row a (0 outside the tail)
-  __shared__ double rw[256];   // and of the just finished w (t = i)
-  if (!act[blockIdx.y]) return;
+  __shared__ double cw[2 * kEigNb];
+  __shared__ double red[4][kTrdPart];
   const EigProb p = probs[blockIdx.y];
-  const int n = p.n, ld = p.ld, tid = threadIdx.x;
+  if (!act[blockIdx.y]) return;
+  const int n = p.n, ld = p.ld, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int first = next >= 0 ? next : finish + 1;   // rows [first, n)
   if (first >= n || (int)blockIdx.x * 256 >= n - first) return;
   double* V = vec + p.v_off;
   double* Xp = X + p.x_off;
   double* Yp = Xp + (long long)2 * kEigNb * ld;
-  const int r0 = first + blockIdx.x * 256;
-  const int r = r0 + tid;
+  const int r = first + blockIdx.x * 256 + tid;
+  const int rc = min(r, n - 1);
+  const bool fin = finish >= 0 && finish < n - 1;
+  const bool row = next >= 0 && next < n;
+  const int jn = row ? next : 0, ni = row ? jn - j0 : 0;   // pairs 0..ni-1 correct the row (ni = i + 1 after a finish)
+  const int i = fin ? finish - j0 : -1;
+  // all kEigNb pairs take part with fixed trip counts: the panel rows t >= ni
+  // are still zero (cleared at the panel start) and so are their coefficients
+  double x[64], ar = 0.0, cv = 0.0, cwv = 0.0;
+  if (row) {
+#pragma unroll
+    for (int t = 0; t < 2 * kEigNb; ++t) x[t] = Xp[(long long)t * ld + rc];
+    ar = A[p.m_off + (long long)jn * ld + rc];
+    if (tid < kEigNb) {
+      cv = Xp[(long long)tid * ld + jn];                 // v_t[jn]
+      cwv = Xp[(long long)(kEigNb + tid) * ld + jn];     // w_t[jn]
+    }
+  }
   double alpha = 0.0, wi = 0.0;
-  int i = -1;
-  if (finish >= 0 && finish < n - 1) {
+  if (fin) {
     const int j = finish;
-    i = j - j0;
+    const double vi = Xp[(long long)i * ld + rc], w0 = V[(long long)kVw * ld + rc];
+    const double wjn = row ? V[(long long)kVw * ld + jn] : 0.0, tau = V[(long long)kVtau * ld + j];
     const int nw = (n - 1 - j + 3) / 4;   // k_trd_col workgroups
     const double* pw = V + (long long)kVrc * ld;
     double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
@@ -333,81 +384,42 @@ __global__ void __launch_bounds__(256) k_trd_row(const EigProb* __restrict__ pro
       s3 += pw[w + 768];
     }
     for (; w < nw; w += 256) s0 += pw[w];
-    const double s = sum256((s0 + s1) + (s2 + s3), sh);
-    alpha = -0.5 * V[(long long)kVtau * ld + j] * s;
+    alpha = -0.5 * tau * sum256((s0 + s1) + (s2 + s3), sh);
     if (r < n && r > j) {
-      wi = fma(alpha, Xp[(long long)i * ld + r], V[(long long)kVw * ld + r]);
+      wi = fma(alpha, vi, w0);
       Xp[(long long)(kEigNb + i) * ld + r] = wi;
       Yp[(long long)i * ld + r] = wi;
     }
+    // w_i[jn] is completed here, not yet visible in X
+    if (tid == i) cwv = fma(alpha, cv, wjn);
   }
-  if (next < 0 || next >= n) return;
-  const int jn = next, ni = jn - j0;   // pairs 0..ni-1 correct the row (ni = i + 1 after a finish)
-  // all kEigNb pairs take part with fixed trip counts, so that every load is
-  // issued before the sums need it: the panel rows t >= ni are still zero
-  // (cleared at the panel start) and so are their coefficients here
+  if (!row) return;
   if (tid < kEigNb) {
-    const bool on = tid < ni;
-    cw[tid] = on ? Xp[(long long)tid * ld + jn] : 0.0;   // v_t[jn]
-    // w_t[jn]; the pair just finished is completed here, not yet visible in X
-    cw[kEigNb + tid] = !on ? 0.0
-                       : tid == i ? fma(alpha, Xp[(long long)tid * ld + jn], V[(long long)kVw * ld + jn])
-                                  : Xp[(long long)(kEigNb + tid) * ld + jn];
+    cw[tid] = tid < ni ? cv : 0.0;
+    cw[kEigNb + tid] = tid < ni ? cwv : 0.0;
   }
   __syncthreads();
-  double ar = 0.0;
+#pragma unroll
+  for (int t = 0; t < kEigNb; ++t) {
+    if (t == i) x[kEigNb + t] = wi;
+    ar -= cw[t] * x[kEigNb + t] + cw[kEigNb + t] * x[t];
+  }
   if (r < n) {
-    ar = A[p.m_off + (long long)jn * ld + r];
-    double vt[kEigNb], wt[kEigNb];
-#pragma unroll
-    for (int t = 0; t < kEigNb; ++t) {
-      vt[t] = Xp[(long long)t * ld + r];
-      wt[t] = t == i ? wi : Xp[(long long)(kEigNb + t) * ld + r];
-    }
-#pragma unroll
-    for (int t = 0; t < kEigNb; ++t) ar -= cw[t] * wt[t] + cw[kEigNb + t] * vt[t];
     V[(long long)kVy * ld + r] = ar;
     if (jn == n - 1) V[(long long)kVd * ld + jn] = ar;
   }
-  // partial sums over rows jn + 2..n-1: |a|^2, v_t . a, w_t . a (products
-  // k = 0, 1 + t, 1 + kEigNb + t; zero for t >= ni); wave wv takes the
-  // products k = wv (mod 4), each lane four of the workgroup's 256 rows, all
-  // loads of a wave issued before its sums
-  const bool tail = r < n && r >= jn + 2;
-  ra[tid] = tail ? ar : 0.0;
-  rw[tid] = wi;
+  // partial sums over rows jn + 2..n-1: |a|^2, v_t . a, w_t . a (zero for t >= ni)
+  const double at = r < n && r >= jn + 2 ? ar : 0.0;
+#pragma unroll
+  for (int t = 0; t < 2 * kEigNb; ++t) x[t] *= at;
+  const double ss = wave_sum(at * at);
+  const double st = wave_sums64(x);
+  red[wv][1 + lane] = st;
+  if (lane == 0) red[wv][0] = ss;
   __syncthreads();
-  const int lane = tid & 63, wv = tid >> 6;
-  const int rows = min(256, n - r0);
-  double* pr = part2 + p.p_off2 + (long long)blockIdx.x * kTrdPart;
-  constexpr int kPerWave = (kTrdPart + 3) / 4;
-  double au[4];
-#pragma unroll
-  for (int q = 0; q < 4; ++q) au[q] = ra[lane + 64 * q];
-  double acc[kPerWave];
-#pragma unroll
-  for (int c = 0; c < kPerWave; ++c) {
-    const int k = wv + 4 * c;
-    double x = 0.0;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int u = lane + 64 * q;
-      double o = 0.0;
-      if (k < kTrdPart && u < rows) {
-        if (k == 0) o = au[q];
-        else if (k < 1 + kEigNb) o = Xp[(long long)(k - 1) * ld + r0 + u];
-        else o = (k - 1 - kEigNb) == i ? rw[u] : Xp[(long long)(k - 1) * ld + r0 + u];
-      }
-      x = fma(o, au[q], x);
-    }
-    acc[c] = x;
-  }
-#pragma unroll
-  for (int c = 0; c < kPerWave; ++c) {
-    const int k = wv + 4 * c;
-    const double x = wave_sum(acc[c]);
-    if (lane == 0 && k < kTrdPart) pr[k] = x;
-  }
+  if (tid < kTrdPart)
+    part2[p.p_off2 + (long long)blockIdx.x * kTrdPart + tid] =
+        (red[0][tid] + red[1][tid]) + (red[2][tid] + red[3][tid]);
 }
 
 // the tridiagonal form as it leaves the tridiagonalisation (kept beside the
