@@ -439,6 +439,10 @@ class Batch {
   int *sub_ = nullptr, *sub_cnt_ = nullptr;
   unsigned long long* sub_res_ = nullptr;
   double* sub_dbl_ = nullptr;
+  // molecules of at most sub_wg orbitals take the path in one workgroup each
+  int sub_wg = 64;
+  int sub_nwg_ = 0;
+  int* d_sub_wg = nullptr;
   int sub_guess_ = 6;   // steps queued before the first count is read
   void subspace(bool allow);
   bool split_ok() const { return jac_p == 32 && !apply_lds && !pivot_lds; }

@@ -915,6 +915,7 @@ void Batch::init_common() {
   if (const char* r = std::getenv("XTBAMD_JAC_LANES")) jac_lanes = std::min(kMaxLanes, std::max(1, std::atoi(r)));
   if (const char* r = std::getenv("XTBAMD_EIG_BLK_MIN")) eig_blk_min = std::max(65, std::atoi(r));
   if (const char* r = std::getenv("XTBAMD_SUBSPACE")) subspace_on = std::atoi(r) != 0;
+  if (const char* r = std::getenv("XTBAMD_SUB_WG")) sub_wg = std::atoi(r);
   if (const char* r = std::getenv("XTBAMD_EIG_BLK_ITERS")) eig_blk_iters = std::max(0, std::atoi(r));
   if (on_loan()) {
     // the lender's streams and events (created and kept by the lender)
@@ -1019,6 +1020,7 @@ void Batch::allocate(const Capacity& c) {
   sub_ = alloc<int>((long long)nmol * kSubInts);
   HIPCHECK(hipMemset(sub_, 0, (size_t)nmol * kSubInts * sizeof(int)));
   sub_cnt_ = alloc<int>(4);
+  d_sub_wg = alloc<int>(nmol);
   sub_res_ = alloc<unsigned long long>((long long)nmol * kSubRes);
   sub_dbl_ = alloc<double>((long long)nmol * kSubDbls);
   HIPCHECK(hipMemset(sub_dbl_, 0, (size_t)nmol * kSubDbls * sizeof(double)));
@@ -1268,11 +1270,11 @@ void Batch::rebuild() {
       for (const Kind& kd : kinds)
         for (int m = 0; m < nmol; ++m) {
           const MolDesc& d = desc[m];
-          if (!occupied_[m] || !sub_able(d)) continue;
+          if (!occupied_[m] || !sub_able(d) || (d.nao <= sub_wg && (kd.w & 32) == 0)) continue;
           const int dims[3] = {d.nao, d.nel / 2, d.nao - d.nel / 2};
           for (int a = 0; a < (dims[kd.rows] + kTile - 1) / kTile; ++a)
             for (int b = kd.w & kSubSym ? a : 0; b < (dims[kd.cols] + kTile - 1) / kTile; ++b)
-              mt[m].push_back(make_int4(m, a, b, kd.w));
+              mt[m].push_back(make_int4(m, a, b, kd.w & 31));
         }
       xcd_order(mt, st);
     };
@@ -1285,14 +1287,23 @@ void Batch::rebuild() {
     launch({{kSubZ | kSubSym, 1, 1}, {kSubE | kSubSym, 1, 1}});
     launch({{kSubCYZ, 1, 0}});
     launch({{kSubP | kSubSym, 0, 0}});
+    // the rotation of the last diagonalisation: molecules of every size (32)
     for (int kind = kRotM; kind < kRotU; ++kind)
-      launch({{kind | kSubSym, 1, 1}, {kind | kRotVirt | kSubSym, 2, 2}});
-    launch({{kRotU, 2, 1}});
+      launch({{kind | kSubSym | 32, 1, 1}, {kind | kRotVirt | kSubSym | 32, 2, 2}});
+    launch({{kRotU | 32, 2, 1}});
     sub_t0[k] = (int)st.size();
+    // the molecules that k_sub_wg takes, largest first
+    std::vector<int> wg;
+    for (int m = 0; m < nmol; ++m)
+      if (occupied_[m] && sub_able(desc[m]) && desc[m].nao <= sub_wg) wg.push_back(m);
+    std::stable_sort(wg.begin(), wg.end(), [&](int x, int y) { return desc[x].nao > desc[y].nao; });
+    sub_nwg_ = (int)wg.size();
+    if (sub_nwg_)
+      HIPCHECK(hipMemcpyAsync(d_sub_wg, wg.data(), wg.size() * sizeof(int), hipMemcpyHostToDevice, stream));
     grow(d_sub_tiles, sub_tiles_cap_, std::max<long long>(1, (long long)st.size()));
     if (!st.empty())
       HIPCHECK(hipMemcpyAsync(d_sub_tiles, st.data(), st.size() * sizeof(int4), hipMemcpyHostToDevice, stream));
-    HIPCHECK(hipStreamSynchronize(stream));   // st goes out of scope
+    HIPCHECK(hipStreamSynchronize(stream));   // st and wg go out of scope
   }
   jac_lists(jac_n);
   if (subspace_on && split_ok()) jac_lists(jac_h);
@@ -2745,9 +2756,22 @@ void Batch::subspace(bool allow) {
                      allow ? 1 : 0);
   need_full_ = true;
   if (!allow) return;
-  hipLaunchKernelGGL(k_sub_start, dim3(gstride((long long)max_nao * max_nao / 4 + 1), nmol), dim3(256), 0, stream, d_desc,
-                     (const double*)A, (const double*)ev, (const int*)sub_, Sm);
+  const bool wide = sub_t0[1] > sub_t0[0];
+  if (wide) {
+    hipLaunchKernelGGL(k_sub_start, dim3(gstride((long long)max_nao * max_nao / 4 + 1), nmol), dim3(256), 0, stream, d_desc,
+                     (const double*)A, (const double*)ev, (const int*)sub_, Sm, sub_wg);
+  }
   const SubBufs bf{A, C, ev, Sm, G, T, W, H, P};
+  // the small molecules, one workgroup each, beside the products of the others
+  if (sub_nwg_ > 0) {
+    if (wide) {
+      HIPCHECK(hipEventRecord(ev_fork, stream));
+      HIPCHECK(hipStreamWaitEvent(stream2, ev_fork, 0));
+    }
+    hipLaunchKernelGGL(k_sub_wg, dim3(sub_nwg_), dim3(512), 0, wide ? stream2 : stream, (const int*)d_sub_wg, d_desc,
+                       bf, d_state, sub_, sub_res_, sub_dbl_);
+    if (wide) HIPCHECK(hipEventRecord(ev_join, stream2));
+  }
   auto product = [&](int list, int step, int level) {
     const int nt = sub_t0[list + 1] - sub_t0[list];
     if (nt <= 0) return;
@@ -2759,23 +2783,33 @@ void Batch::subspace(bool allow) {
       hipLaunchKernelGGL(k_sub_gemm<false>, dim3(nt), dim3(256), 0, stream, tl, d_desc, bf, d_state, sub_, sub_res_,
                          sub_dbl_, step, level);
   };
+  auto counts = [&]() {
+    hipLaunchKernelGGL(k_sub_check, dim3(1), dim3(256), 0, stream, (const MolDesc*)d_desc, d_state, nmol, sub_,
+                       (const unsigned long long*)sub_res_, sub_wg, sub_cnt_);
+    HIPCHECK(hipMemcpyAsync(h_pinned + 8, sub_cnt_, 3 * sizeof(int), hipMemcpyDeviceToHost, stream));
+    HIPCHECK(hipEventRecord(ev_join3, stream));
+  };
+  if (!wide) {
+    counts();
+    HIPCHECK(hipEventSynchronize(ev_join3));
+    need_full_ = h_pinned[9] > 0;
+    return;
+  }
   int step = 0, upto = std::min(kSubSteps, std::max(1, sub_guess_));
-  for (;;) {
+  for (bool joined = false;; joined = true) {
     for (; step < upto; ++step) {
       product(0, step, 0);
       product(1, step, 0);
     }
     hipLaunchKernelGGL(k_sub_outcome, dim3(grid1(nmol, 64)), dim3(64), 0, stream, d_state, nmol, sub_,
-                       (const unsigned long long*)sub_res_, (const double*)sub_dbl_, step);
+                       (const unsigned long long*)sub_res_, (const double*)sub_dbl_, (const MolDesc*)d_desc, sub_wg, step);
     product(2, 0, 0);
     product(3, 0, 0);
     product(4, 0, 0);
     product(5, 0, 2);
     product(6, 0, 3);
-    hipLaunchKernelGGL(k_sub_check, dim3(1), dim3(256), 0, stream, (const MolDesc*)d_desc, d_state, nmol, sub_,
-                       (const unsigned long long*)sub_res_, sub_cnt_);
-    HIPCHECK(hipMemcpyAsync(h_pinned + 8, sub_cnt_, 3 * sizeof(int), hipMemcpyDeviceToHost, stream));
-    HIPCHECK(hipEventRecord(ev_join3, stream));
+    if (sub_nwg_ > 0 && !joined) HIPCHECK(hipStreamWaitEvent(stream, ev_join, 0));
+    counts();
     product(6, 0, 4);
     product(7, 0, 0);
     product(8, 0, 0);

@@ -110,8 +110,8 @@ typedef double v4d __attribute__((ext_vector_type(4)));
 // and R (K x Nc) with row strides ldl and ldr; RMINOR: R is stored Nc x K.
 // The operands go from global memory straight into the lane layout of
 // v_mfma_f64_16x16x4f64 (four rows of 16 consecutive doubles per load), the
-// loads of the next 16 rows in flight during the 16 matrix instructions of
-// the current ones: no LDS and no barrier, so waves of different problems and
+// loads of the next 32 rows in flight during the 16 matrix instructions of
+// the current 16 (a load takes about twice as long as those): no LDS and no barrier, so waves of different problems and
 // sizes share a compute unit freely.  Rows and columns outside the result
 // read a valid element instead and are not written by the callers.
 template <bool RMINOR>
@@ -130,57 +130,57 @@ __device__ __forceinline__ void wave_mm(const double* __restrict__ L, int ldl, i
   for (int r = 0; r < 2; ++r)
 #pragma unroll
     for (int c = 0; c < 2; ++c) acc[r][c] = v4d{0.0, 0.0, 0.0, 0.0};
-  const int nfull = K >> 4;
-  double a[4][2], b[4][2];
-  auto load = [&](double (&x)[4][2], double (&y)[4][2]) {
+  // blocks of 16 rows (the last one filled up with zeros) in three register
+  // sets, two blocks in flight behind the one at work
+  const int nq = (K + 15) >> 4;
+  double a[3][4][2], b[3][4][2];
+  auto load = [&](double (&x)[4][2], double (&y)[4][2], int q) {
+    if (16 * q + 16 <= K) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+      for (int u = 0; u < 4; ++u)
 #pragma unroll
-      for (int r = 0; r < 2; ++r) {
-        x[u][r] = lp[r][u * sl];
-        y[u][r] = rp[r][u * sr];
+        for (int r = 0; r < 2; ++r) {
+          x[u][r] = lp[r][u * sl];
+          y[u][r] = rp[r][u * sr];
+        }
+    } else {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const bool in = 16 * q + 4 * u + k4 < K;
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+          x[u][r] = in ? lp[r][u * sl] : 0.0;
+          y[u][r] = in ? rp[r][u * sr] : 0.0;
+        }
       }
+    }
 #pragma unroll
     for (int r = 0; r < 2; ++r) {
       lp[r] += 4 * sl;
       rp[r] += 4 * sr;
     }
   };
-  auto mul = [&](const double (&x)[2], const double (&y)[2]) {
-#pragma unroll
-    for (int r = 0; r < 2; ++r)
-#pragma unroll
-      for (int c = 0; c < 2; ++c) acc[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[r], y[c], acc[r][c], 0, 0, 0);
-  };
-  if (nfull > 0) load(a, b);
-  for (int q = 0; q < nfull; ++q) {
-    double a2[4][2], b2[4][2];
-    if (q + 1 < nfull) load(a2, b2);
-#pragma unroll
-    for (int u = 0; u < 4; ++u) mul(a[u], b[u]);
+  auto mul = [&](const double (&x)[4][2], const double (&y)[4][2]) {
 #pragma unroll
     for (int u = 0; u < 4; ++u)
 #pragma unroll
-      for (int r = 0; r < 2; ++r) {
-        a[u][r] = a2[u][r];
-        b[u][r] = b2[u][r];
+      for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+          acc[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[u][r], y[u][c], acc[r][c], 0, 0, 0);
+  };
+#pragma unroll
+  for (int t = 0; t < 3; ++t)
+    if (t < nq) load(a[t], b[t], t);
+  for (int q = 0; q < nq; q += 3) {
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+      if (q + t < nq) {
+        mul(a[t], b[t]);
+        if (q + t + 3 < nq) load(a[t], b[t], q + t + 3);
       }
-  }
-  // the last K mod 16 rows; rows from K on count as zero
-  const int rest = K & 15;
-  double at[4][2], bt[4][2];
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const bool in = 4 * u + k4 < rest;
-#pragma unroll
-    for (int r = 0; r < 2; ++r) {
-      at[u][r] = in ? lp[r][u * sl] : 0.0;
-      bt[u][r] = in ? rp[r][u * sr] : 0.0;
     }
   }
-#pragma unroll
-  for (int u = 0; u < 4; ++u)
-    if (4 * u < rest) mul(at[u], bt[u]);
 }
 
 // Symmetric-left and transposed-left products of the batch on wave_mm: C = L^T

@@ -185,10 +185,10 @@ __global__ void __launch_bounds__(256) k_sub_begin(const MolDesc* __restrict__ d
 // X = -A_vo / D of the molecules without one
 __global__ void __launch_bounds__(256) k_sub_start(const MolDesc* __restrict__ desc, const double* __restrict__ A,
                                                    const double* __restrict__ diag, const int* __restrict__ sub,
-                                                   double* X) {
+                                                   double* X, int sub_wg) {
   const int m = blockIdx.y;
-  if (sub[m * kSubInts + kSubPhase] != 1 || !sub[m * kSubInts + kSubFresh]) return;
   const MolDesc md = desc[m];
+  if (md.nao <= sub_wg || sub[m * kSubInts + kSubPhase] != 1 || !sub[m * kSubInts + kSubFresh]) return;
   const int N = md.nao, o = sub_occ(md), v = N - o;
   const double* Am = A + md.m0;
   const double* d = diag + md.o0;
@@ -210,38 +210,34 @@ struct SubBufs {
   double *X, *G, *T, *W, *H, *P;
 };
 
-// One 64 x 64 tile of one product of a molecule, a wave per 32 x 32 quarter
-// (wave_mm: no LDS, no barrier, a quarter outside the result ends at once);
-// tiles (molecule, row tile, column tile, kind).  Every operand but C is kept
-// so that the product runs down its rows: A, the powers of M and the partial
-// products Z are symmetric, X is kept with its transpose, C Y and C Y Z are
-// formed transposed (o x N).  Symmetric results (M, E_k = M^(2^k), Z_k, P) are
-// formed on the upper tiles and mirrored.
-// Z_2 = (I - M)(I + E_1), Z_(k+1) = Z_k (I + E_k).
-// step: the step of the kinds kSubB and kSubR; level: k of E_k and Z_k.
+// One wave's 32 x 32 block (row0, col0) of one product of a molecule
+// (wave_mm).  Every operand but C is kept so that the product runs down its
+// rows: A, the powers of M and the partial products Z are symmetric, X is
+// kept with its transpose, C Y and C Y Z are formed transposed (o x N).
+// Symmetric results (M, E_k = M^(2^k), Z_k, P) are formed on the upper blocks
+// and mirrored.  Z_2 = (I - M)(I + E_1), Z_(k+1) = Z_k (I + E_k).
+// par: the parity of X; ws: the factor w of the step (kSubR); level: k of E_k
+// and Z_k; e2, e3: E_2, E_3 take part.  big: maximum (bit pattern) of |R|, |E|.
 // Buffers: M, E_3 in G, E_1, Z_3 in P, E_2 in H, Z_2, Z_4 in W, (C Y)^T in T.
-template <bool RMINOR>
-__global__ void __launch_bounds__(256) k_sub_gemm(const int4* __restrict__ tiles, const MolDesc* __restrict__ desc,
-                                                  SubBufs bf, MolState* state, int* sub, unsigned long long* res,
-                                                  double* dbl, int step, int level) {
-  const int4 tl = tiles[blockIdx.x];
-  const int m = tl.x, op = tl.w & 15;
-  if (m < 0) return;
-  const bool sym = (tl.w & kSubSym) != 0;
-  int* si = sub + m * kSubInts;
-  if (si[kSubPhase] != (op <= kSubR ? 1 : 2)) return;
-  unsigned long long* rs = res + (long long)m * kSubRes;
-  double* sd = dbl + (long long)m * kSubDbls;
-  const MolDesc md = desc[m];
-  const int N = md.nao, o = sub_occ(md), v = N - o;
-  int par = si[kSubPar];
-  if (op <= kSubR) {
-    if (sub_step_done(rs, sd, step)) return;
-    par = (par + step) & 1;
-    // the first tile's workgroup sets the factor of this step for the second
-    // product's launch, or gives the molecule up
-    if (op == kSubB && tl.y == 0 && tl.z == 0 && threadIdx.x == 0) sub_rate(rs, sd, si, state + m, step);
+struct SubShape {
+  int rows, cols;
+};
+__device__ __forceinline__ SubShape sub_shape(int op, int N, int o) {
+  const int v = N - o;
+  switch (op) {
+    case kSubB: return {N, o};
+    case kSubR: return {v, o};
+    case kSubCY:
+    case kSubCYZ: return {o, N};
+    case kSubP: return {N, N};
+    default: return {o, o};
   }
+}
+
+template <bool RMINOR>
+__device__ __forceinline__ void sub_block(int op, int level, bool sym, const MolDesc& md, const SubBufs& bf, int par,
+                                          double ws, bool e2, bool e3, int row0, int col0, unsigned long long& big) {
+  const int N = md.nao, o = sub_occ(md), v = N - o;
   const long long vo = (long long)v * o;
   double* Xm = bf.X + md.m0;
   const double* X = Xm + par * vo;
@@ -250,7 +246,6 @@ __global__ void __launch_bounds__(256) k_sub_gemm(const int4* __restrict__ tiles
   double* W = bf.W + md.m0;
   double* H = bf.H + md.m0;
   double* P = bf.P + md.m0;
-  const bool e2 = !sub_dropped(rs, o, 2), e3 = e2 && !sub_dropped(rs, o, 3);
   // result (M x Nc) = L^T R with L (K x M), R (K x Nc), or R (Nc x K) for C
   const double *Lp, *Rp;
   int ldl = o, ldr = o, M = o, Nc = o, K = o;
@@ -273,19 +268,16 @@ __global__ void __launch_bounds__(256) k_sub_gemm(const int4* __restrict__ tiles
     case kSubCYZ: Lp = e2 && !e3 ? P : W; Rp = T; ldr = N; Nc = N; break;
     default: Lp = G; ldl = N; Rp = T; ldr = N; M = Nc = N; break;
   }
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, i16 = lane & 15, k4 = lane >> 4;
-  const int row0 = tl.y * kTile + 32 * (w >> 1), col0 = tl.z * kTile + 32 * (w & 1);
   if (row0 >= M || col0 >= Nc || (sym && row0 > col0)) return;
+  const int lane = threadIdx.x & 63, i16 = lane & 15, k4 = lane >> 4;
   v4d acc[2][2];
   wave_mm<RMINOR>(Lp, ldl, M, Rp, ldr, Nc, K, row0, col0, acc);
   // maxima on the bit patterns: a NaN counts as the largest value
-  unsigned long long big = 0ull;
   auto see = [&](double x) {
     const unsigned long long b = (unsigned long long)__double_as_longlong(fabs(x));
     big = big > b ? big : b;
   };
   const double* dg = bf.diag + md.o0;
-  const double ws = op == kSubR && step > 0 ? sd[kSubW + step] : 1.0;
 #pragma unroll
   for (int r = 0; r < 2; ++r)
 #pragma unroll
@@ -341,6 +333,35 @@ __global__ void __launch_bounds__(256) k_sub_gemm(const int4* __restrict__ tiles
         }
       }
     }
+}
+
+// A 64 x 64 tile of a product per workgroup, a wave per quarter; tiles
+// (molecule, row tile, column tile, kind).  For the molecules above sub_wg.
+template <bool RMINOR>
+__global__ void __launch_bounds__(256) k_sub_gemm(const int4* __restrict__ tiles, const MolDesc* __restrict__ desc,
+                                                  SubBufs bf, MolState* state, int* sub, unsigned long long* res,
+                                                  double* dbl, int step, int level) {
+  const int4 tl = tiles[blockIdx.x];
+  const int m = tl.x, op = tl.w & 15;
+  if (m < 0) return;
+  int* si = sub + m * kSubInts;
+  if (si[kSubPhase] != (op <= kSubR ? 1 : 2)) return;
+  unsigned long long* rs = res + (long long)m * kSubRes;
+  double* sd = dbl + (long long)m * kSubDbls;
+  const MolDesc md = desc[m];
+  int par = si[kSubPar];
+  if (op <= kSubR) {
+    if (sub_step_done(rs, sd, step)) return;
+    par = (par + step) & 1;
+    // the first tile's workgroup sets the factor of this step for the second
+    // product's launch, or gives the molecule up
+    if (op == kSubB && tl.y == 0 && tl.z == 0 && threadIdx.x == 0) sub_rate(rs, sd, si, state + m, step);
+  }
+  const bool e2 = !sub_dropped(rs, sub_occ(md), 2), e3 = e2 && !sub_dropped(rs, sub_occ(md), 3);
+  const int w = threadIdx.x >> 6;
+  unsigned long long big = 0ull;
+  sub_block<RMINOR>(op, level, (tl.w & kSubSym) != 0, md, bf, par, op == kSubR && step > 0 ? sd[kSubW + step] : 1.0,
+                    e2, e3, tl.y * kTile + 32 * (w >> 1), tl.z * kTile + 32 * (w & 1), big);
   if (op == kSubR || op == kSubE) {
 #pragma unroll
     for (int sft = 32; sft > 0; sft >>= 1) {
@@ -349,16 +370,135 @@ __global__ void __launch_bounds__(256) k_sub_gemm(const int4* __restrict__ tiles
     }
     // (most waves of a large molecule find a larger maximum there already)
     unsigned long long* to = op == kSubR ? &rs[step] : &rs[kSubSteps + level - 2];
-    if (lane == 0 && big > __atomic_load_n(to, __ATOMIC_RELAXED)) atomicMax(to, big);
+    if ((threadIdx.x & 63) == 0 && big > __atomic_load_n(to, __ATOMIC_RELAXED)) atomicMax(to, big);
+  }
+}
+
+// The whole of an SCC iteration's subspace path of one molecule in one
+// workgroup of 8 waves (a wave takes every eighth 32 x 32 block of a
+// product): up to sub_wg orbitals a product is shorter than a launch, and a
+// batch has a molecule for every compute unit.  One call site of the product
+// (two with the row-minor C Y) in a loop over the sequence of kinds.
+__global__ void __launch_bounds__(512) k_sub_wg(const int* __restrict__ list, const MolDesc* __restrict__ desc,
+                                                SubBufs bf, MolState* state, int* sub, unsigned long long* res,
+                                                double* dbl) {
+  __shared__ unsigned long long top;
+  __shared__ int phase, more;
+  const int m = list[blockIdx.x];
+  int* si = sub + m * kSubInts;
+  if (si[kSubPhase] != 1) return;
+  unsigned long long* rs = res + (long long)m * kSubRes;
+  double* sd = dbl + (long long)m * kSubDbls;
+  const MolDesc md = desc[m];
+  const int N = md.nao, o = sub_occ(md), v = N - o;
+  const int tid = threadIdx.x, w = tid >> 6;
+  const int par0 = si[kSubPar];
+  if (si[kSubFresh]) {
+    const double* Am = bf.A + md.m0;
+    const double* d = bf.diag + md.o0;
+    double* X = bf.X + md.m0;
+    for (int t = tid; t < v * o; t += 512) {
+      const int i = t / o, j = t % o;
+      const double x = -Am[(long long)(o + i) * N + j] / (d[o + i] - d[j]);
+      X[t] = x;
+      X[2LL * v * o + (long long)j * v + i] = x;
+    }
+  }
+  if (tid == 0) {
+    top = 0ull;
+    phase = 1;
+  }
+  int op = kSubB, step = 0, level = 0;
+  bool e2 = false, e3 = false;
+  for (;;) {
+    if (op == kSubB && tid == 0) {
+      sub_rate(rs, sd, si, state + m, step);
+      phase = si[kSubPhase];
+    }
+    __syncthreads();
+    if (phase != 1) return;   // given up
+    const int par = (par0 + step) & 1;
+    const bool sym = op == kSubM || op == kSubE1 || op == kSubZ2 || op == kSubE || op == kSubZ || op == kSubP;
+    const SubShape sh = sub_shape(op, N, o);
+    const int nr = (sh.rows + 31) / 32, nc = (sh.cols + 31) / 32;
+    const double ws = op == kSubR && step > 0 ? sd[kSubW + step] : 1.0;
+    unsigned long long big = 0ull;
+    if (op == kSubCY) {
+      for (int t = w; t < nr * nc; t += 8)
+        sub_block<true>(op, level, sym, md, bf, par, ws, e2, e3, 32 * (t / nc), 32 * (t % nc), big);
+    } else {
+      // (the two kinds that share a launch run one after the other here)
+      for (int t = w; t < nr * nc; t += 8)
+        sub_block<false>(op, level, sym, md, bf, par, ws, e2, e3, 32 * (t / nc), 32 * (t % nc), big);
+    }
+    if (op == kSubR || op == kSubE) {
+#pragma unroll
+      for (int sft = 32; sft > 0; sft >>= 1) {
+        const unsigned long long ob = __shfl_xor(big, sft, 64);
+        big = big > ob ? big : ob;
+      }
+      if ((tid & 63) == 0) atomicMax(&top, big);
+    }
+    __syncthreads();
+    if (tid == 0) {
+      more = 1;
+      if (op == kSubR) {
+        rs[step] = top;
+        if (sub_step_done(rs, sd, step + 1)) more = 0;
+        else if (step + 1 >= kSubSteps) sub_give_up(si, state + m);
+      } else if (op == kSubE) {
+        rs[kSubSteps + level - 2] = top;
+        if (level == 3 && !((double)o * __longlong_as_double((long long)top) <= kSubInvMax)) sub_give_up(si, state + m);
+      }
+      top = 0ull;
+      phase = si[kSubPhase];
+    }
+    __syncthreads();
+    if (phase != 1) return;
+    // the next product
+    if (op == kSubB) op = kSubR;
+    else if (op == kSubR) {
+      ++step;
+      op = more ? kSubB : kSubM;
+    } else if (op == kSubM) op = kSubCY;
+    else if (op == kSubCY) op = kSubE1;
+    else if (op == kSubE1) op = kSubZ2;
+    else if (op == kSubZ2) {
+      op = kSubE;
+      level = 2;
+    } else if (op == kSubE) {
+      if (level == 2) e2 = !sub_dropped(rs, o, 2);
+      else e3 = e2 && !sub_dropped(rs, o, 3);
+      // E_2, Z_3, E_3, Z_4
+      if (level == 2 && e2) {
+        op = kSubZ;
+        level = 3;
+      } else if (level == 3 && e3) {
+        op = kSubZ;
+        level = 4;
+      } else {
+        op = kSubCYZ;
+      }
+    } else if (op == kSubZ) {
+      op = level == 3 ? kSubE : kSubCYZ;
+    } else if (op == kSubCYZ) op = kSubP;
+    else break;
+  }
+  if (tid == 0) {
+    si[kSubPar] = (par0 + step) & 1;
+    si[kSubNext] = step;
+    si[kSubPend] = 1;
+    si[kSubPhase] = 4;
   }
 }
 
 // after the steps [0, nstep): converged molecules to phase 2, given up ones
 // to phase 3 with a full diagonalisation; densities formed before to phase 4
 __global__ void k_sub_outcome(MolState* state, int nmol, int* sub, const unsigned long long* __restrict__ res,
-                              const double* __restrict__ dbl, int nstep) {
+                              const double* __restrict__ dbl, const MolDesc* __restrict__ desc, int sub_wg,
+                              int nstep) {
   const int m = blockIdx.x * blockDim.x + threadIdx.x;
-  if (m >= nmol) return;
+  if (m >= nmol || desc[m].nao <= sub_wg) return;
   int* si = sub + m * kSubInts;
   if (si[kSubPhase] == 2) si[kSubPhase] = 4;
   if (si[kSubPhase] != 1) return;
@@ -379,8 +519,10 @@ __global__ void k_sub_outcome(MolState* state, int nmol, int* sub, const unsigne
 // after the powers of M: a molecule whose inverse would need another factor
 // (X too large) takes the full diagonalisation instead.
 // cnt[0]: still iterating, cnt[1]: full diagonalisations, cnt[2]: most steps
+// (of the molecules above sub_wg)
 __global__ void __launch_bounds__(256) k_sub_check(const MolDesc* __restrict__ desc, MolState* state, int nmol,
-                                                   int* sub, const unsigned long long* __restrict__ res, int* cnt) {
+                                                   int* sub, const unsigned long long* __restrict__ res, int sub_wg,
+                                                   int* cnt) {
   __shared__ double sh[4];
   double run = 0.0, full = 0.0, most = 0.0;
   for (int m = threadIdx.x; m < nmol; m += blockDim.x) {
@@ -392,7 +534,7 @@ __global__ void __launch_bounds__(256) k_sub_check(const MolDesc* __restrict__ d
       }
     }
     if (si[kSubPhase] == 1) run += 1.0;
-    if (si[kSubPhase] != 0) most = fmax(most, (double)si[kSubNext]);
+    if (si[kSubPhase] != 0 && desc[m].nao > sub_wg) most = fmax(most, (double)si[kSubNext]);
     full += state[m].diag ? 1.0 : 0.0;
   }
   run = block_sum<256>(run, sh);
