@@ -169,7 +169,7 @@ struct GemmJob;
 // the product job lists, built by Batch::rebuild().
 struct EigSet {
   int np = 0, maxn = 0, npanel = 0, maxdepth = 0;
-  std::vector<int> mols;                 // batch slot of each problem
+  std::vector<int> mols;                 // Jacobi problem (batch slot) of each problem
   std::vector<int> zfin;                 // buffer (0/1) of each problem's final eigenvectors
   std::vector<long long> v_off;          // each problem's vector block in vec
   std::vector<int> ld;                   // each problem's row stride
@@ -227,8 +227,9 @@ struct EigMem {
   virtual ~EigMem() = default;
 };
 // work arrays, trees and product job lists of es's problems (es.mols set,
-// dims their dimensions)
-void eig_set_build(EigSet& es, const std::vector<int>& dims, EigMem& mem);
+// dims their dimensions); the n x ld arrays that fit are those of lend (a set
+// that is never solved at the same time and is rebuilt before es only)
+void eig_set_build(EigSet& es, const std::vector<int>& dims, EigMem& mem, const EigSet* lend = nullptr);
 // the blocked eigensolver on es's problems: problem k's matrix is read from
 // Am at jprobs[es.mols[k]] (a_off, ld), its eigenvalues are written to Am's
 // diagonal and its eigenvectors as rows of Wm (w_off, ld); jstate gets the
@@ -449,11 +450,12 @@ class Batch {
   bool final_ = false;      // diagonalise() is orbitals()' one
   bool need_full_ = true;   // some molecule takes the full diagonalisation
   void diagonalise();       // of the molecules with MolState::diag: C, emo, occupations
-  EigSet eig_;
-  void eig_build();
-  // the blocked eigensolver on eig_'s problems: A from Am (Jacobi problem
+  EigSet eig_;     // whole matrices (jac_n's problems)
+  EigSet eig_h_;   // occupied and virtual blocks (jac_h's), in eig_'s work arrays
+  void eig_build(EigSet& es, const JacSet& js);
+  // the blocked eigensolver on the set's problems: A from Am (Jacobi problem
   // layout), eigenvalues onto Am's diagonal, eigenvector rows into Wm
-  void eig_blocked(const JacSet& js, double* Am, double* Wm, bool check_active, hipStream_t s);
+  void eig_blocked(EigSet& es, const JacSet& js, double* Am, double* Wm, bool check_active, hipStream_t s);
   // returns true when W comes out as rows (row j = eigenvector j)
   void jacobi_lanes(JacSet& js, double* Am, double* Wm);
   bool jacobi(JacSet& js, double* Am, double* Wm, double* evout, bool check_active, bool keep_w = false,

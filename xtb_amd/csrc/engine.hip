@@ -1325,7 +1325,8 @@ void Batch::jac_lists(JacSet& js) {
   std::vector<int2> pairs;
   std::vector<int4> ta, tw, to;
   // the blocked eigensolver takes the largest problems on the register path
-  const bool blk_path = jac_padded && jac_p == 32 && !use_ql && !js.half;
+  // (not the blocks of a molecule on lent memory, whose size is fixed)
+  const bool blk_path = jac_padded && jac_p == 32 && !use_ql && !(js.half && on_loan());
   js.max_rounds = 0;
   js.max_rounds_lanes = 0;
   js.big_max_dim = 0;
@@ -1494,10 +1495,9 @@ void Batch::jac_lists(JacSet& js) {
   grow(js.d_ta, js.ta_cap, std::max<long long>(1, js.nta));
   grow(js.d_tw, js.tw_cap, std::max<long long>(1, js.ntw));
   grow(js.d_to, js.to_cap, std::max<long long>(1, js.nto));
-  if (!js.half) {
-    eig_.mols = blk;
-    eig_build();
-  }
+  EigSet& es = js.half ? eig_h_ : eig_;
+  es.mols = blk;
+  eig_build(es, js);
   js.nbig = (int)big.size();
   grow(js.d_big, js.big_cap, std::max<long long>(1, js.nbig));
   if (!big.empty()) HIPCHECK(hipMemcpyAsync(js.d_big, big.data(), big.size() * sizeof(int), hipMemcpyHostToDevice, stream));
@@ -1605,6 +1605,7 @@ Batch::~Batch() {
   for (auto& v : prof_ev_)
     for (hipEvent_t e : v) (void)hipEventDestroy(e);
   if (eig_.graph) (void)hipGraphExecDestroy(eig_.graph);
+  if (eig_h_.graph) (void)hipGraphExecDestroy(eig_h_.graph);
   if (on_loan()) {
     // the lender owns the memory, streams and events; only wait for the work
     (void)hipStreamSynchronize(stream);
@@ -1652,11 +1653,12 @@ bool Batch::jacobi(JacSet& js, double* Am, double* Wm, double* evout, bool check
   const bool lanes = rows && !pivot_lds && js.npairs > 0;
   // the largest problems go to the blocked eigensolver on stream3 (after the
   // small ones), beside the lanes
-  const bool blk = rows && !pivot_lds && !js.half && eig_.np > 0 &&
+  EigSet& es = js.half ? eig_h_ : eig_;
+  const bool blk = rows && !pivot_lds && es.np > 0 &&
                    (iterations_ < eig_blk_iters || (final_ && eig_blk_iters > 0));
   // the blocked path's problems are marked done for the lanes
   if (blk)
-    hipLaunchKernelGGL(k_eig_claim, dim3(1), dim3(256), 0, stream, (const EigProb*)eig_.d_probs, eig_.np, js.state);
+    hipLaunchKernelGGL(k_eig_claim, dim3(1), dim3(256), 0, stream, (const EigProb*)es.d_probs, es.np, js.state);
   // the lanes test their progress once per period of their largest problem
   jac_period_ = blk ? std::max(1, js.max_rounds_lanes) : js.max_rounds;
   const bool forked = lanes || blk;
@@ -1671,7 +1673,7 @@ bool Batch::jacobi(JacSet& js, double* Am, double* Wm, double* evout, bool check
   if (js.nsmall)
     hipLaunchKernelGGL(k_jac_small, dim3(js.nsmall), dim3(256), 0, forked ? stream3 : stream, js.d_probs, js.d_small,
                        Am, Wm, (const double*)js.scale, js.state, keep_w ? 1 : 0, rows ? 1 : 0, jac_tol);
-  if (blk) eig_blocked(js, Am, Wm, check_active, stream3);
+  if (blk) eig_blocked(es, js, Am, Wm, check_active, stream3);
   if (forked) {
     if (lanes) jacobi_lanes(js, Am, Wm);
     HIPCHECK(hipEventRecord(ev_join, stream2));
@@ -1756,9 +1758,9 @@ bool Batch::jacobi(JacSet& js, double* Am, double* Wm, double* evout, bool check
 }
 
 // ---------------------------------------------------------------------------
-// blocked eigensolver: work arrays, trees and product job lists of eig_'s
+// blocked eigensolver: work arrays, trees and product job lists of a set's
 // problems (built once per rebuild; the device addresses are fixed)
-void Batch::eig_build() {
+void Batch::eig_build(EigSet& es, const JacSet& js) {
   // device memory of the batch (a loan's pieces are never released)
   struct BatchMem : EigMem {
     Batch* b;
@@ -1771,13 +1773,13 @@ void Batch::eig_build() {
     }
   } mem(this);
   std::vector<int> dims;
-  for (int m : eig_.mols) dims.push_back(desc[m].nao);
-  eig_set_build(eig_, dims, mem);
+  for (int m : es.mols) dims.push_back(js.probs[m].dim);
+  eig_set_build(es, dims, mem, &es == &eig_ ? nullptr : &eig_);
   // captured on stream3 (the null stream of a loan cannot be captured)
-  eig_.use_graph = eig_graph && !on_loan();
+  es.use_graph = eig_graph && !on_loan();
 }
 
-void eig_set_build(EigSet& es, const std::vector<int>& dims, EigMem& mem) {
+void eig_set_build(EigSet& es, const std::vector<int>& dims, EigMem& mem, const EigSet* lend) {
   if (es.graph) {
     // the captured launches name the old work arrays
     HIPCHECK(hipGraphExecDestroy(es.graph));
@@ -1794,6 +1796,16 @@ void eig_set_build(EigSet& es, const std::vector<int>& dims, EigMem& mem) {
     }
     capv = std::max<long long>(need, capv);
     ptr = (T_*)mem.get((size_t)std::max(1LL, capv) * sizeof(T_));
+  };
+  // the n x ld arrays, written before they are read in every solve, may be
+  // lent; capacity 0 marks a lent one: looked at again in the next build
+  auto work = [&](auto*& ptr, int k, auto* lent, long long need) {
+    if (lend && es.cap[k] == 0 && need <= lend->cap[k]) {
+      ptr = lent;
+      return;
+    }
+    if (es.cap[k] == 0) ptr = nullptr;
+    grow(ptr, es.cap[k], need);
   };
   std::vector<EigProb> probs(es.np);
   long long mat = 0, vv = 0, iv = 0, xx = 0, pp = 0, pp2 = 0, tt = 0, gg = 0;
@@ -1835,16 +1847,16 @@ void eig_set_build(EigSet& es, const std::vector<int>& dims, EigMem& mem) {
   }
   es.npanel = (es.maxn - 1 + kEigNb - 1) / kEigNb;
   es.nblk = (es.maxn - 1 + kBtNb - 1) / kBtNb;
-  grow(es.Aw, es.cap[0], mat);
-  grow(es.Vh, es.cap[1], mat);
-  grow(es.Z0, es.cap[2], mat);
-  grow(es.Z1, es.cap[3], mat);
-  grow(es.U, es.cap[4], mat);
+  work(es.Aw, 0, lend ? lend->Aw : nullptr, mat);
+  work(es.Vh, 1, lend ? lend->Vh : nullptr, mat);
+  work(es.Z0, 2, lend ? lend->Z0 : nullptr, mat);
+  work(es.Z1, 3, lend ? lend->Z1 : nullptr, mat);
+  work(es.U, 4, lend ? lend->U : nullptr, mat);
   grow(es.vec, es.cap[5], vv);
   grow(es.ivec, es.cap[6], iv);
   grow(es.X, es.cap[7], xx);
   grow(es.P, es.cap[8], pp);
-  grow(es.P2, es.cap[9], pp);
+  work(es.P2, 9, lend ? lend->P2 : nullptr, pp);
   grow(es.Tf, es.cap[10], tt);
   grow(es.d_probs, es.cap[11], es.np);
   grow(es.act, es.cap[12], es.np);
@@ -2018,8 +2030,8 @@ void eig_set_build(EigSet& es, const std::vector<int>& dims, EigMem& mem) {
   HIPCHECK(hipMemset(es.P, 0, (size_t)std::max(1LL, pp) * sizeof(double)));
 }
 
-void Batch::eig_blocked(const JacSet& js, double* Am, double* Wm, bool check_active, hipStream_t s) {
-  eig_set_run(eig_, js.d_probs, js.state, check_active ? (const MolState*)d_state : (const MolState*)nullptr, Am, Wm,
+void Batch::eig_blocked(EigSet& es, const JacSet& js, double* Am, double* Wm, bool check_active, hipStream_t s) {
+  eig_set_run(es, js.d_probs, js.state, check_active ? (const MolState*)d_state : (const MolState*)nullptr, Am, Wm,
               s);
 }
 
@@ -2574,9 +2586,10 @@ void Batch::setup() {
     hipLaunchKernelGGL(k_d4_refweights, dim3(grid1(sub_max_n, 64), ns), dim3(64), 0, stream3, d_sub, el, at, cn_cov,
                        (const double*)nullptr, zetavec, zerovec, zetadcn, zerodcn);
     hipLaunchKernelGGL(k_d4_c6<1>, dim3(gstride((long long)sub_max_n * (sub_max_n + 1) / 2), ns), dim3(256), 0,
-                       stream3, d_sub, el, at, c6ref, zetavec, zerovec, zetadcn, zerodcn, c6, dc6, c60, dc60);
-    hipLaunchKernelGGL(k_d4_atm, dim3(sub_max_n, ns), dim3(256), 0, stream3, d_sub, el, at, xyz, (const double*)c60,
-                       (const double*)dc60, grad_atm, dedcn_atm, eat);
+                       stream3, d_sub, el, at, c6ref, zetavec, zerovec, zetadcn, zerodcn, (const double*)xyz, c6, dc6,
+                       c60, dc60);
+    hipLaunchKernelGGL(k_d4_atm, dim3(sub_max_n, ns), dim3(256), 0, stream3, d_sub, (const double*)xyz,
+                       (const double*)c60, (const double*)dc60, (const double*)c6, grad_atm, dedcn_atm, eat);
     if (fork) HIPCHECK(hipEventRecord(ev_atm, stream3));
   }
   // the matrices and factors that depend on the geometry and CN only
@@ -2998,7 +3011,7 @@ void Batch::gradient() {
   hipLaunchKernelGGL(k_d4_refweights, dim3(grid1(sub_max_n, 64), ns), dim3(64), 0, stream, d_sub, el, at, cn_cov, q,
                      zetavec, zerovec, zetadcn, zerodcn);
   hipLaunchKernelGGL(k_d4_c6<2>, dim3(gstride((long long)sub_max_n * (sub_max_n + 1) / 2), ns), dim3(256), 0, stream,
-                     d_sub, el, at, c6ref, zetavec, zerovec, zetadcn, zerodcn, c6, dc6, c60, dc60);
+                     d_sub, el, at, c6ref, zetavec, zerovec, zetadcn, zerodcn, (const double*)xyz, c6, dc6, c60, dc60);
   hipLaunchKernelGGL(k_d4_grad2, gat, dim3(64), 0, stream, d_sub, el, at, xyz, (const double*)c6, (const double*)dc6,
                      grad, dedcn);
   hipLaunchKernelGGL(k_add_atm, dim3(grid1(sub_max_n, 64), ns), dim3(64), 0, stream, d_sub,

@@ -920,7 +920,7 @@ __global__ void __launch_bounds__(256) k_eig_in(const EigProb* __restrict__ prob
                                                 const double* __restrict__ Asrc, double* Aw) {
   const EigProb p = probs[blockIdx.y];
   const JacobiProb q = jp[p.mol];
-  const bool on = !mstate || mstate[p.mol].diag;
+  const bool on = !mstate || mstate[q.mol].diag;
   if (blockIdx.x == 0 && threadIdx.x == 0) act[blockIdx.y] = on ? 1 : 0;
   if (!on) return;
   const int n = p.n;

@@ -298,14 +298,17 @@ __global__ void __launch_bounds__(64) k_grad_h0(const MolDesc* __restrict__ desc
 
 // atomic C6 and dC6/dCN for atom pairs (get_atomic_c6: src/disp/dftd4.F90:1069-1147),
 // for the charge-scaled (c6, dc6) and the zero-charge (c60, dc60) weights
-// PART 1: the zero-charge C6 and its CN derivatives (c60, dc60), PART 2:
-// those at the SCC charges (c6, dc6)
+// PART 1: the pair factors of the three-body term from the zero-charge C6:
+// sqrt(C6) in c60, dC6/dCN / (2 C6) in dc60 and the damping factor
+// (R0 / r)^(16/3) in c6 (whose own values PART 2 writes later);
+// PART 2: C6 and dC6/dCN at the SCC charges (c6, dc6)
 template <int PART>
 __global__ void __launch_bounds__(256) k_d4_c6(const MolDesc* __restrict__ desc, const Element* __restrict__ el,
                                                const int* __restrict__ at,
                         const double* __restrict__ c6ref, const double* __restrict__ zetavec,
                         const double* __restrict__ zerovec, const double* __restrict__ zetadcn,
-                        const double* __restrict__ zerodcn, double* c6, double* dc6, double* c60, double* dc60) {
+                        const double* __restrict__ zerodcn, const double* __restrict__ xyz, double* c6, double* dc6,
+                        double* c60, double* dc60) {
   // one atom pair i >= j per thread (grid-stride over the lower triangle):
   // C6 is symmetric, its CN derivatives are formed for both atoms of the pair
   const MolDesc md = desc[blockIdx.y];
@@ -345,12 +348,31 @@ __global__ void __launch_bounds__(256) k_d4_c6(const MolDesc* __restrict__ desc,
         dj = fma(zI[r], zdJ[q] * rc, dj);
       }
     const long long ij = md.p0 + (long long)i * n + j, ji = md.p0 + (long long)j * n + i;
-    double* cc = PART == 1 ? c60 : c6;
-    double* dc = PART == 1 ? dc60 : dc6;
-    cc[ij] = s1;
-    cc[ji] = s1;
-    dc[ij] = di;   // dC6(i,j)/dCN_i
-    dc[ji] = dj;   // dC6(j,i)/dCN_j
+    if (PART == 1) {
+      const double s = sqrt(s1), h = 0.5 / s1;
+      double damp = 0.0;
+      if (i != j) {
+        const double* xi = xyz + 3 * (md.a0 + i);
+        const double* xj = xyz + 3 * (md.a0 + j);
+        const double dx = xi[0] - xj[0], dy = xi[1] - xj[1], dz = xi[2] - xj[2];
+        // damping radius of the pair over its distance, to the power alp / 3
+        static_assert(kD4alp == 16, "ATM damping exponent");
+        const double r0 = kD4a1 * sqrt(3.0 * el[zi].sqrtzr4r2 * el[zj].sqrtzr4r2) + kD4a2;
+        const double u = r0 / sqrt(dx * dx + dy * dy + dz * dz), u2 = u * u;
+        damp = u2 * u2 * u * cbrt(u);
+      }
+      c60[ij] = s;
+      c60[ji] = s;
+      dc60[ij] = di * h;
+      dc60[ji] = dj * h;
+      c6[ij] = damp;
+      c6[ji] = damp;
+    } else {
+      c6[ij] = s1;
+      c6[ji] = s1;
+      dc6[ij] = di;   // dC6(i,j)/dCN_i
+      dc6[ji] = dj;   // dC6(j,i)/dCN_j
+    }
   }
 }
 
@@ -392,82 +414,111 @@ __global__ void __launch_bounds__(64) k_d4_grad2(const MolDesc* __restrict__ des
   }
 }
 
+// 1 / x and 1 / sqrt(x), x > 0, from the hardware approximations by two
+// Newton steps each
+__device__ __forceinline__ double quick_rcp(double x) {
+  double y = __builtin_amdgcn_rcp(x);
+  y = fma(y, fma(-x, y, 1.0), y);
+  return fma(y, fma(-x, y, 1.0), y);
+}
+__device__ __forceinline__ double quick_rsqrt(double x) {
+  double y = __builtin_amdgcn_rsq(x);
+  y = fma(0.5 * y, fma(-x * y, y, 1.0), y);
+  return fma(0.5 * y, fma(-x * y, y, 1.0), y);
+}
+
 // ATM three-body term with zero-charge C6 (atm_gradient_latp, molecular branch:
 // src/disp/dftd4.F90:2121-2174, deriv_atm_triple :2354-2433): the triples of atom a;
 // writes atom a's gradient, dE/dCN and energy terms (no accumulation: it runs
-// beside the SCC, and the gradient adds them later)
-constexpr int kAtmLds = 4096;   // molecules up to this size keep per-atom factors in LDS
+// beside the SCC, and the gradient adds them later).
+// Bound by FP64 arithmetic, n^3 / 2 triples per molecule and three visits
+// each: everything that belongs to a pair (sqrt(C6), the damping power and
+// the CN ratio, from k_d4_c6<1>; the distance to a, in LDS) is formed once
+// per pair, so that a triple takes one 1 / sqrt, one 1 / x and products (the
+// square and cube roots and seven divisions per triple took 51 ms for 2100
+// atoms and 4.7 ms for the 512-molecule batch).  A lane per atom c, the atoms
+// b < c shared out over the four waves.
+constexpr int kAtmB = 128;   // atoms b per LDS block
 
-__global__ void __launch_bounds__(256) k_d4_atm(const MolDesc* __restrict__ desc, const Element* __restrict__ el,
-                                                const int* __restrict__ at, const double* __restrict__ xyz,
-                                                const double* __restrict__ c6, const double* __restrict__ dc6,
-                                                double* grad, double* dedcn, double* eatm) {
+__global__ void __launch_bounds__(256) k_d4_atm(const MolDesc* __restrict__ desc, const double* __restrict__ xyz,
+                                                const double* __restrict__ sc6, const double* __restrict__ dcr,
+                                                const double* __restrict__ damp, double* grad, double* dedcn,
+                                                double* eatm) {
   __shared__ double sh[4];
-  __shared__ double sq[kAtmLds];   // sqrt of each atom's sqrt(Z) <r4>/<r2> factor
+  // of the pairs (a, b): vector, r^2, 1 / r, sqrt(C6), damping, CN ratio
+  __shared__ double pb[kAtmB][8];
   const MolDesc md = desc[blockIdx.y];
   const int a = blockIdx.x;
   if (a >= md.n) return;
-  const int n = md.n;
+  const int n = md.n, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const double* x = xyz + 3 * md.a0;
-  const double* C = c6 + md.p0;
-  const double* dC = dc6 + md.p0;
+  const double* S = sc6 + md.p0;
+  const double* F = damp + md.p0;
+  const double* Da = dcr + md.p0 + (long long)a * n;
   const double cut2 = 1600.0;
-  const bool cached = n <= kAtmLds;
-  if (cached)
-    for (int b = threadIdx.x; b < n; b += blockDim.x) sq[b] = sqrt(el[at[md.a0 + b]].sqrtzr4r2);
-  __syncthreads();
-  // damping radius of a pair: a1 sqrt(3 s_i s_j) + a2 = a1 sqrt(3) sqrt(s_i) sqrt(s_j) + a2
-  auto rad = [&](int i, int j, double si, double sj) {
-    return cached ? kD4a1 * 1.7320508075688772 * sq[i] * sq[j] + kD4a2 : kD4a1 * sqrt(3.0 * si * sj) + kD4a2;
-  };
   const double ra[3] = {x[3 * a], x[3 * a + 1], x[3 * a + 2]};
-  const double sa = el[at[md.a0 + a]].sqrtzr4r2;
   double g[3] = {0, 0, 0}, e = 0.0, dcn = 0.0;
-  const long long npair = (long long)n * (n - 1) / 2;
-  for (long long t = threadIdx.x; t < npair; t += blockDim.x) {
-    int b, c;
-    tri_index(t, b, c);  // b > c
-    if (b == a || c == a) continue;
-    const double rij[3] = {x[3 * b] - ra[0], x[3 * b + 1] - ra[1], x[3 * b + 2] - ra[2]};
-    const double r2ij = rij[0] * rij[0] + rij[1] * rij[1] + rij[2] * rij[2];
-    if (r2ij > cut2) continue;
-    const double rik[3] = {x[3 * c] - ra[0], x[3 * c + 1] - ra[1], x[3 * c + 2] - ra[2]};
-    const double r2ik = rik[0] * rik[0] + rik[1] * rik[1] + rik[2] * rik[2];
-    if (r2ik > cut2) continue;
-    const double rjk[3] = {x[3 * c] - x[3 * b], x[3 * c + 1] - x[3 * b + 1], x[3 * c + 2] - x[3 * b + 2]};
-    const double r2jk = rjk[0] * rjk[0] + rjk[1] * rjk[1] + rjk[2] * rjk[2];
-    if (r2jk > cut2) continue;
-    const double sb = el[at[md.a0 + b]].sqrtzr4r2, sc = el[at[md.a0 + c]].sqrtzr4r2;
-    const double cij = rad(a, b, sa, sb);
-    const double cik = rad(a, c, sa, sc);
-    const double cjk = rad(b, c, sb, sc);
-    const double c6ij = C[(long long)a * n + b], c6ik = C[(long long)a * n + c], c6jk = C[(long long)b * n + c];
-    const double c9 = -sqrt(c6ij * c6ik * c6jk);
-    const double ccc1 = cij * cjk * cik;
-    const double rrr2 = r2ij * r2jk * r2ik;
-    const double rrr1 = sqrt(rrr2);
-    const double rrr3 = rrr1 * rrr2;
-    const double ang_fact = 0.375 / (rrr2 * rrr3);
-    const double ang = ang_fact * (r2ij + r2jk - r2ik) * (r2ij - r2jk + r2ik) * (-r2ij + r2jk + r2ik) + 1.0 / rrr3;
-    // (ccc1 / rrr1)^(alp / 3) with alp = 16: x^5 cbrt(x)
-    static_assert(kD4alp == 16, "ATM damping exponent");
-    const double qd = ccc1 / rrr1, qd2 = qd * qd;
-    const double cralp = qd2 * qd2 * qd * cbrt(qd);
-    const double fdmp = 1.0 / (1.0 + 6.0 * cralp);
-    const double dfdmp = -(2.0 * kD4alp * cralp) * fdmp * fdmp;
-    const double dE = -fdmp * ang * c9;
-    double dang = -ang_fact * (r2ij * r2ij * r2ij + r2ij * r2ij * (r2jk + r2ik) +
-                               r2ij * (3.0 * r2jk * r2jk + 2.0 * r2jk * r2ik + 3.0 * r2ik * r2ik) -
-                               5.0 * (r2jk - r2ik) * (r2jk - r2ik) * (r2jk + r2ik));
-    const double dGr1 = (-dang * c9 * fdmp + dfdmp * c9 * ang) / r2ij;
-    dang = -ang_fact * (r2ik * r2ik * r2ik + r2ik * r2ik * (r2jk + r2ij) +
-                        r2ik * (3.0 * r2jk * r2jk + 2.0 * r2jk * r2ij + 3.0 * r2ij * r2ij) -
-                        5.0 * (r2jk - r2ij) * (r2jk - r2ij) * (r2jk + r2ij));
-    const double dGr2 = (-dang * c9 * fdmp + dfdmp * c9 * ang) / r2ik;
-    for (int k = 0; k < 3; ++k) g[k] += (-dGr1 * rij[k] - dGr2 * rik[k]) * kD4s9;
-    const double dc9 = 0.5 * c9 * (dC[(long long)a * n + b] / c6ij + dC[(long long)a * n + c] / c6ik);
-    dcn += -ang * fdmp * dc9 * kD4s9;
-    e += dE * kD4s9 / 3.0;
+  for (int b0 = 0; b0 < n; b0 += kAtmB) {
+    __syncthreads();
+    if ((int)threadIdx.x < kAtmB) {
+      const int b = b0 + threadIdx.x;
+      double v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+      if (b < n && b != a) {
+        for (int k = 0; k < 3; ++k) v[k] = x[3 * b + k] - ra[k];
+        v[3] = v[0] * v[0] + v[1] * v[1] + v[2] * v[2];
+        v[4] = quick_rsqrt(v[3]);
+        v[5] = S[(long long)a * n + b];
+        v[6] = F[(long long)a * n + b];
+        v[7] = Da[b];
+      }
+      for (int k = 0; k < 8; ++k) pb[threadIdx.x][k] = v[k];
+    }
+    __syncthreads();
+    for (int c0 = b0 / 64 * 64; c0 < n; c0 += 64) {
+      const int c = c0 + lane;
+      double rik[3] = {0, 0, 0}, r2ik = 0.0, ivik = 0.0, sik = 0.0, fik = 0.0, dik = 0.0;
+      bool on = c < n && c != a;
+      if (on) {
+        for (int k = 0; k < 3; ++k) rik[k] = x[3 * c + k] - ra[k];
+        r2ik = rik[0] * rik[0] + rik[1] * rik[1] + rik[2] * rik[2];
+        ivik = quick_rsqrt(r2ik);
+        sik = S[(long long)a * n + c];
+        fik = F[(long long)a * n + c];
+        dik = Da[c];
+        on = r2ik <= cut2;
+      }
+      const int bend = min(min(b0 + kAtmB, n), c0 + 64);   // b < c
+      for (int b = b0 + w; b < bend; b += 4) {
+        const double* v = pb[b - b0];
+        const double r2ij = v[3];
+        if (b == a || r2ij > cut2) continue;
+        const double d0 = rik[0] - v[0], d1 = rik[1] - v[1], d2 = rik[2] - v[2];
+        const double r2jk = d0 * d0 + d1 * d1 + d2 * d2;
+        if (!on || b >= c || r2jk > cut2) continue;
+        const double sjk = S[(long long)b * n + c], fjk = F[(long long)b * n + c];
+        const double ivij = v[4];
+        const double c9 = -(v[5] * sik) * sjk;
+        const double inv1 = (ivij * ivik) * quick_rsqrt(r2jk), inv2 = inv1 * inv1, inv3 = inv1 * inv2;   // 1 / (r r r)^k
+        const double ang_fact = 0.375 * inv2 * inv3;
+        const double ang = ang_fact * (r2ij + r2jk - r2ik) * (r2ij - r2jk + r2ik) * (-r2ij + r2jk + r2ik) + inv3;
+        const double cralp = (v[6] * fik) * fjk;
+        const double fdmp = quick_rcp(1.0 + 6.0 * cralp);
+        const double dfdmp = -(2.0 * kD4alp * cralp) * fdmp * fdmp;
+        const double da = dfdmp * c9 * ang, cf = ang_fact * c9 * fdmp;
+        const double g1 = r2ij * r2ij * r2ij + r2ij * r2ij * (r2jk + r2ik) +
+                          r2ij * (3.0 * r2jk * r2jk + 2.0 * r2jk * r2ik + 3.0 * r2ik * r2ik) -
+                          5.0 * (r2jk - r2ik) * (r2jk - r2ik) * (r2jk + r2ik);
+        const double g2 = r2ik * r2ik * r2ik + r2ik * r2ik * (r2jk + r2ij) +
+                          r2ik * (3.0 * r2jk * r2jk + 2.0 * r2jk * r2ij + 3.0 * r2ij * r2ij) -
+                          5.0 * (r2jk - r2ij) * (r2jk - r2ij) * (r2jk + r2ij);
+        const double dGr1 = (cf * g1 + da) * (ivij * ivij);
+        const double dGr2 = (cf * g2 + da) * (ivik * ivik);
+        for (int k = 0; k < 3; ++k) g[k] += (-dGr1 * v[k] - dGr2 * rik[k]) * kD4s9;
+        const double ce = c9 * (ang * fdmp) * kD4s9;
+        dcn -= ce * (v[7] + dik);
+        e -= ce / 3.0;
+      }
+    }
   }
   for (int k = 0; k < 3; ++k) g[k] = block_sum<256>(g[k], sh);
   dcn = block_sum<256>(dcn, sh);
