@@ -105,3 +105,37 @@ def test_subspace_small_gaps_ions_and_open_shells(monkeypatch, golden):
     (full, _), (sub, _) = _both(monkeypatch, mols)
     for k, (a, b) in enumerate(zip(full, sub)):
         _check(a, b, f"mol {k}")
+
+
+@pytest.mark.parametrize("blk_min", [65, 96])
+def test_blocks_on_the_blocked_eigensolver(monkeypatch, blk_min):
+    """Last diagonalisation with the blocks of at least blk_min rows on the
+    blocked eigensolver (both, one or neither block of a molecule)."""
+    from xtb_amd import workloads as w
+    monkeypatch.setenv("XTBAMD_EIG_BLK_MIN", str(blk_min))
+    mols = [w.alkane(n, 3) for n in (20, 27, 33, 40)] + [w.water_cluster(k, 5) for k in (14, 23, 40)]
+    (a, _), (b, _) = _both(monkeypatch, mols)
+    for (z, _), x, y in zip(mols, a, b):
+        _check(x, y, f"{len(z)} atoms")
+
+
+def test_orthogonalisation_over_the_spectrum():
+    """S^(-1/2) from S = I (two atoms far apart: every eigenvalue at one end of
+    the interval that the scaled steps expect) to eigenvalues far below it
+    (compressed molecules); the oracle diagonalises the generalised problem.
+    Energies agree to cond(S) eps x 30 Eh, below 1e-9 Eh up to cond(S) = 1e5."""
+    xa = _engine()
+    from oracle import pyoracle as po
+    h4 = np.array([[0.0, 0.0, 0.9 * k] for k in range(4)])
+    mols = [(np.array([2, 2]), np.array([[0.0, 0.0, 0.0], [0.0, 0.0, 40.0]])),
+            (np.array([1, 1]), np.array([[0.0, 0.0, 0.0], [0.0, 0.0, 0.7]])),
+            (np.array([1, 1, 1, 1]), h4),
+            (np.array([6, 6, 1, 1]), np.array([[0, 0, 0], [0, 0, 1.8], [0, 0, -1.6], [0, 0, 3.4]], dtype=float))]
+    b = xa.Batch(mols)
+    b.run()
+    res = b.results()
+    b.close()
+    for (z, x), r in zip(mols, res):
+        o = po.singlepoint(z, x)
+        assert r["iterations"] == o["iterations"], z
+        assert abs(r["energy"] - o["e_total"]) <= 1e-9, (z, r["energy"], o["e_total"])

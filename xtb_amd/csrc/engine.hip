@@ -442,7 +442,7 @@ __global__ void k_ns_begin(int nmol, const int* __restrict__ sel, int* stage, in
   const int m = blockIdx.x * blockDim.x + threadIdx.x;
   if (m >= nmol) return;
   stage[m] = sel[m] ? 0 : 2;
-  act[m] = sel[m] ? 1 : 0;
+  act[m] = act[nmol + m] = sel[m] ? 1 : 0;
   if (sel[m]) {
     failed[m] = 0;
     cbound[m] = 0.0;
@@ -469,6 +469,16 @@ __global__ void k_sad_guess(const MolDesc* __restrict__ desc, const Element* __r
 // --- Newton-Schulz iteration for S^(-1/2) (coupled form, Higham, "Functions
 // of Matrices", 2008, eq. 6.35): Y0 = S/c, Z0 = I,
 // T = (3I - Z Y)/2, Y <- Y T, Z <- T Z; Z -> (S/c)^(-1/2).
+// The first kNsScaled steps take m Y and m Z for Y and Z, with the m that maps
+// the ends of the expected spectrum to one value (Chen and Chow, "A stable
+// scaling of Newton-Schulz for improving the sign function computation of a
+// Hermitian matrix", Argonne ANL/MCS-P5059-0114, 2014).  With the singular
+// values of Y0^(1/2) in [kNsLow, sqrt 2] six steps are enough where plain ones
+// take eight or nine; smaller ones still grow faster than by plain steps and take
+// one or two more.  Bound by the products (700 waters: 30 of 1.4 ms before,
+// 18 now: the first step needs one, the last only Z's); the error of
+// S^(-1/2) is no larger (max |X S X - I| at 400 rows, condition 30 to 1500:
+// 0.9 to 5.3e-14, plain steps 0.9 to 5.5e-14).
 // c = max row sum |S_ij| bounds the spectrum of S from above.
 // grid (row chunks of 64, molecules); half the maximum over
 // the molecule's rows by an atomic max on the bit patterns of cbound (cleared
@@ -501,19 +511,22 @@ __global__ void __launch_bounds__(256) k_ns_bound(const MolDesc* __restrict__ de
     atomicMax((unsigned long long*)&cbound[md.mol], (unsigned long long)__double_as_longlong(0.5 * m));
 }
 
+constexpr int kNsScaled = 5;      // scaled steps
+constexpr double kNsLow = 0.2;    // lower end of the expected interval
+
 __global__ void k_ns_init(const MolDesc* __restrict__ desc, const double* __restrict__ S,
-                          const double* __restrict__ cbound, double* Y, double* Z) {
+                          const double* __restrict__ cbound, double* Y) {
   const MolDesc md = desc[blockIdx.y];
   const long long N = md.nao;
-  for (long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x; t < N * N; t += (long long)gridDim.x * blockDim.x) {
+  for (long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x; t < N * N; t += (long long)gridDim.x * blockDim.x)
     Y[md.m0 + t] = S[md.m0 + t] / cbound[md.mol];
-    Z[md.m0 + t] = (t / N == t % N) ? 1.0 : 0.0;
-  }
 }
 
-// T = (3I - P)/2 with P = Z Y, and max |I - P| per molecule
+// T = m (3I - m^2 P)/2 with P = Z Y, and max |I - P| per molecule; the first
+// step (Z = I) takes P = Y from src and leaves Z <- T in Z too
 __global__ void __launch_bounds__(256) k_ns_form(const MolDesc* __restrict__ desc, const int* __restrict__ act,
-                                                 double* P, unsigned long long* res) {
+                                                 const double* src, double* P, double* Z, double mu,
+                                                 unsigned long long* res) {
   __shared__ double sh[4];
   const MolDesc md = desc[blockIdx.y];
   if (!act[md.mol]) return;
@@ -522,17 +535,21 @@ __global__ void __launch_bounds__(256) k_ns_form(const MolDesc* __restrict__ des
   double r = 0.0;
   for (long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x; t < N * N; t += (long long)gridDim.x * blockDim.x) {
     const double d = (t / N == t % N) ? 1.0 : 0.0;
-    const double p = P[md.m0 + t];
+    const double p = src[md.m0 + t];
     r = fmax(r, fabs(d - p));
-    P[md.m0 + t] = 0.5 * (3.0 * d - p);
+    const double f = 0.5 * mu * (3.0 * d - mu * mu * p);
+    P[md.m0 + t] = f;
+    if (Z) Z[md.m0 + t] = f;
   }
   r = block_max<256>(r, sh);
   if (threadIdx.x == 0 && r > 0.0) atomicMax(&res[md.mol], (unsigned long long)__double_as_longlong(r));
 }
 
-// per-molecule convergence: residual < 1e-10, then one more update (quadratic
-// convergence takes it to rounding level); act = 0 once done, and fin = the
-// parity of the iteration whose buffers hold the molecule's final Y, Z
+// per-molecule convergence: residual < 1e-10 after the scaled steps, then one
+// more update of Z (quadratic convergence takes it to rounding level); act = 0
+// once done, act[nmol + m] = 0 from the last update on (which needs no new
+// Y, and no P = Z Y after it), and fin = the parity of the iteration whose
+// buffers hold the molecule's final Z
 __global__ void __launch_bounds__(256) k_ns_mark(int nmol, int* stage, int* act, unsigned long long* res, int iter,
                                                  int maxiter, int* failed, int* nactive, int* fin) {
   __shared__ double sh[4];
@@ -542,10 +559,11 @@ __global__ void __launch_bounds__(256) k_ns_mark(int nmol, int* stage, int* act,
     res[m] = 0ull;
     const int before = stage[m];
     if (stage[m] == 1) stage[m] = 2;
-    else if (stage[m] == 0 && r < 1e-10) stage[m] = 1;
+    else if (stage[m] == 0 && iter >= kNsScaled && r < 1e-10) stage[m] = 1;
     if (stage[m] == 0 && iter >= maxiter) { stage[m] = 2; failed[m] = 1; }
     if (before < 2 && stage[m] == 2) fin[m] = iter & 1;
     act[m] = stage[m] < 2 ? 1 : 0;
+    act[nmol + m] = stage[m] == 0 ? 1 : 0;
     c += act[m];
   }
   c = block_sum<256>(c, sh);
@@ -1038,7 +1056,7 @@ void Batch::allocate(const Capacity& c) {
   ns_res = alloc<unsigned long long>(nmol);
   ns_stage = alloc<int>(nmol);
   ns_fin = alloc<int>(nmol);
-  ns_act = alloc<int>(nmol);
+  ns_act = alloc<int>(2 * nmol);
   ns_failed = alloc<int>(nmol);
   jac_alloc(jac_n, nmol);
   JacSet& js = jac_n;
@@ -2522,7 +2540,7 @@ void Batch::orthogonalizer() {
                      ns_act, ns_failed, ns_res, ns_c);
   hipLaunchKernelGGL(k_ns_bound, dim3(grid1(sub_max_nao, 64), nsub), dim3(256), 0, stream, d_sub, (const double*)S,
                      ns_c);
-  hipLaunchKernelGGL(k_ns_init, gmm, dim3(256), 0, stream, d_sub, (const double*)S, (const double*)ns_c, A, W);
+  hipLaunchKernelGGL(k_ns_init, gmm, dim3(256), 0, stream, d_sub, (const double*)S, (const double*)ns_c, A);
   const int maxit = 60;
   // Y and Z alternate between two buffers each (A/H and W/T) by iteration
   // parity; a molecule's final pair is at the parity recorded when it stops
@@ -2533,16 +2551,25 @@ void Batch::orthogonalizer() {
   // has stopped changes nothing.  The host therefore reads iteration it's
   // count of running molecules only after iteration it + 1 is queued: the GPU
   // never waits for the host's read.
+  const int* more = ns_act + nmol;   // molecules before their last update
+  double lo = kNsLow, hi = sqrt(2.0);
   for (int it = 0; it <= maxit; ++it) {
+    double mu = 1.0;
+    if (it < kNsScaled) {
+      mu = sqrt(3.0 / (hi * hi + hi * lo + lo * lo));
+      lo = 0.5 * mu * lo * (3.0 - mu * mu * lo * lo);
+      hi = 1.0;
+    }
     double *Y = Yb[it & 1], *Z = Zb[it & 1];
     // Y and Z are polynomials in S: they commute, and Z Y, Y T and T Z are symmetric
-    gemm(kGemmSymLeft, Z, Y, P, nullptr, nullptr, false, 1.0, ns_act, true);     // P = Z Y
-    hipLaunchKernelGGL(k_ns_form, gmm, dim3(256), 0, stream, d_sub, (const int*)ns_act, P, ns_res);
+    if (it > 0) gemm(kGemmSymLeft, Z, Y, P, nullptr, nullptr, false, 1.0, more, true);     // P = Z Y
+    hipLaunchKernelGGL(k_ns_form, gmm, dim3(256), 0, stream, d_sub, more, it ? (const double*)P : (const double*)Y, P,
+                       it ? (double*)nullptr : Zb[1], mu, ns_res);
     hipLaunchKernelGGL(k_ns_mark, dim3(1), dim3(256), 0, stream, nmol, ns_stage, ns_act, ns_res, it, maxit, ns_failed,
                        jac_nactive, ns_fin);
     HIPCHECK(hipMemcpyAsync(h_pinned + (it & 1), jac_nactive, sizeof(int), hipMemcpyDeviceToHost, stream));
-    gemm(kGemmSymLeft, Y, P, Yb[(it + 1) & 1], nullptr, nullptr, false, 1.0, ns_act, true);   // Y T
-    gemm(kGemmSymLeft, P, Z, Zb[(it + 1) & 1], nullptr, nullptr, false, 1.0, ns_act, true);   // T Z
+    gemm(kGemmSymLeft, Y, P, Yb[(it + 1) & 1], nullptr, nullptr, false, 1.0, more, true);   // Y T
+    if (it > 0) gemm(kGemmSymLeft, P, Z, Zb[(it + 1) & 1], nullptr, nullptr, false, 1.0, ns_act, true);   // T Z
     if (it > 0) {
       HIPCHECK(hipEventSynchronize(ev_join3));   // iteration it - 1's count is on the host
       if (h_pinned[(it - 1) & 1] <= 0) break;
