@@ -139,3 +139,23 @@ def test_orthogonalisation_over_the_spectrum():
         o = po.singlepoint(z, x)
         assert r["iterations"] == o["iterations"], z
         assert abs(r["energy"] - o["e_total"]) <= 1e-9, (z, r["energy"], o["e_total"])
+
+
+@pytest.mark.parametrize("maxiter", [31, 33, 34, 36])
+def test_mixing_history_around_the_lds_limit(maxiter):
+    """Broyden histories of 30, 32 (the largest whose inverse is taken in LDS),
+    33 and 35 earlier iterations: an accuracy that no iteration reaches keeps
+    the SCC going.  Both sides are converged to rounding long before, so the
+    energies agree to a few ulp of 30 Eh times the SCC's amplification."""
+    xa = _engine()
+    from oracle import pyoracle as po
+    from xtb_amd import workloads as w
+    mols = [w.water_cluster(2, 3), w.alkane(4, 3)]
+    b = xa.Batch(mols, accuracy=1e-11, maxiter=maxiter)
+    b.run()
+    res = b.results()
+    b.close()
+    for (z, x), r in zip(mols, res):
+        o = po.singlepoint(z, x, accuracy=1e-11, maxiter=maxiter)
+        assert r["iterations"] >= maxiter - 1 and r["iterations"] == o["iterations"], (r["iterations"], o["iterations"])
+        assert abs(r["energy"] - o["e_total"]) <= 1e-10, (z, r["energy"], o["e_total"])

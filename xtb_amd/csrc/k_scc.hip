@@ -395,6 +395,13 @@ __global__ void k_pop_reduce(const MolDesc* __restrict__ desc, const Element* __
 
 // Energy, convergence test and charge mixing of one molecule (one workgroup):
 // src/scc_core.f90:523-632 with broyden (src/broyden.f90:37-153).
+// Bound by latency: the mixing's dot products over the history and the inverse
+// of its it1 x it1 matrix.  Up to kBroydLds earlier iterations the inverse is
+// taken in LDS by all threads; in global memory with a thread per row (which
+// the longer histories keep: 2 x 33^2 doubles and more) every element of the
+// elimination waits a memory round trip.
+constexpr int kBroydLds = 32;
+constexpr int kBroydPer = kBroydLds / 4;   // rows per thread (256 threads: 4 rows of 2 kBroydLds = 64 columns)
 __global__ void __launch_bounds__(256) k_scc_control(
     const MolDesc* __restrict__ desc, MolState* state, const double* __restrict__ jq, const double* __restrict__ gam,
     const double* __restrict__ row_e, const double* __restrict__ ae, const double* __restrict__ zv,
@@ -404,6 +411,7 @@ __global__ void __launch_bounds__(256) k_scc_control(
     double scfconv, double qconv) {
   __shared__ double sh[4];
   __shared__ double red[8];
+  __shared__ double gj[kBroydLds][2 * kBroydLds + 1];
   const MolDesc md = desc[blockIdx.x];
   MolState& st = state[blockIdx.x];
   if (!st.active) return;
@@ -512,10 +520,22 @@ __global__ void __launch_bounds__(256) k_scc_control(
     // one wave per earlier iteration, no barrier between them
     for (int i = tid >> 6; i < it1; i += 4) {
       const double* dfk = df + (long long)i * nbr;
+      // eight elements per lane and pass: the loads of a pass are in flight together
       double s1 = 0.0, s2 = 0.0;
-      for (int k = tid & 63; k < nbr; k += 64) {
-        s1 += dfk[k] * dfi[k];
-        s2 += dfk[k] * dqv[k];
+      for (int k0 = tid & 63; k0 < nbr; k0 += 512) {
+        double x[8], y[8], z[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int k = k0 + 64 * e;
+          x[e] = k < nbr ? dfk[k] : 0.0;
+          y[e] = k < nbr ? dfi[k] : 0.0;
+          z[e] = k < nbr ? dqv[k] : 0.0;
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          s1 += x[e] * y[e];
+          s2 += x[e] * z[e];
+        }
       }
       s1 = wave_sum(s1);
       s2 = wave_sum(s2);
@@ -526,62 +546,112 @@ __global__ void __launch_bounds__(256) k_scc_control(
       }
     }
     __syncthreads();
-    for (int e = tid; e < it1 * it1; e += blockDim.x) {
-      const int i = e / it1, j = e % it1;
-      double v = om[j] * om[i] * a[(long long)j * mx + i];
-      if (i == j) v += 0.01 * 0.01;
-      beta[e] = v;
-    }
-    __syncthreads();
-    // Gauss-Jordan inverse of beta (matinv: src/broyden.f90:158-184), in place with an identity copy in gmm area
-    double* inv_m = gmm + mx;
-    for (int e = tid; e < it1 * it1; e += blockDim.x) inv_m[e] = (e / it1 == e % it1) ? 1.0 : 0.0;
-    __syncthreads();
-    for (int k = 0; k < it1; ++k) {
-      if (tid == 0) {
+    const bool small = it1 <= kBroydLds;
+    if (small) {
+      // beta and its inverse by Gauss-Jordan in LDS, one thread per element:
+      // the same operations on every element as below
+      const int wd = 2 * it1, gr = tid >> 6, gc = tid & 63;   // this thread's rows gr + 4 x, its column
+      for (int e = tid; e < it1 * it1; e += blockDim.x) {
+        const int i = e / it1, j = e % it1;
+        double v = om[j] * om[i] * a[(long long)j * mx + i];
+        if (i == j) v += 0.01 * 0.01;
+        gj[i][j] = v;
+        gj[i][it1 + j] = i == j ? 1.0 : 0.0;
+      }
+      __syncthreads();
+      for (int k = 0; k < it1; ++k) {
         int p = k;
         for (int i = k + 1; i < it1; ++i)
-          if (fabs(beta[(long long)i * it1 + k]) > fabs(beta[(long long)p * it1 + k])) p = i;
-        red[0] = p;
-      }
-      __syncthreads();
-      const int p = (int)red[0];
-      if (p != k)
-        for (int j = tid; j < it1; j += blockDim.x) {
-          double t = beta[(long long)k * it1 + j];
-          beta[(long long)k * it1 + j] = beta[(long long)p * it1 + j];
-          beta[(long long)p * it1 + j] = t;
-          t = inv_m[(long long)k * it1 + j];
-          inv_m[(long long)k * it1 + j] = inv_m[(long long)p * it1 + j];
-          inv_m[(long long)p * it1 + j] = t;
+          if (fabs(gj[i][k]) > fabs(gj[p][k])) p = i;
+        double row = 0.0, other = 0.0;
+        if (tid < wd) {
+          row = gj[p][tid];
+          other = gj[k][tid];
         }
-      __syncthreads();
-      const double piv = beta[(long long)k * it1 + k];
-      __syncthreads();
+        const double piv = gj[p][k];
+        __syncthreads();
+        if (tid < wd) {
+          if (p != k) gj[p][tid] = other;
+          gj[k][tid] = row / piv;
+        }
+        __syncthreads();
+        // column k is read by every thread before any of them changes it
+        double f[kBroydPer];
+#pragma unroll
+        for (int x = 0; x < kBroydPer; ++x) f[x] = gr + 4 * x < it1 ? gj[gr + 4 * x][k] : 0.0;
+        const double gk = gc < wd ? gj[k][gc] : 0.0;
+        __syncthreads();
+#pragma unroll
+        for (int x = 0; x < kBroydPer; ++x) {
+          const int i = gr + 4 * x;
+          if (i < it1 && gc < wd && i != k && f[x] != 0.0) gj[i][gc] -= f[x] * gk;
+        }
+        __syncthreads();
+      }
       for (int j = tid; j < it1; j += blockDim.x) {
-        beta[(long long)k * it1 + j] /= piv;
-        inv_m[(long long)k * it1 + j] /= piv;
+        double s = 0.0;
+        for (int i = 0; i < it1; ++i) s += c[i] * gj[i][it1 + j];
+        gmm[j] = s;
       }
       __syncthreads();
-      // eliminate column k: each thread owns full rows i
-      for (int i = tid; i < it1; i += blockDim.x) {
-        if (i == k) continue;
-        const double f = beta[(long long)i * it1 + k];
-        if (f == 0.0) continue;
-        for (int j = 0; j < it1; ++j) {
-          beta[(long long)i * it1 + j] -= f * beta[(long long)k * it1 + j];
-          inv_m[(long long)i * it1 + j] -= f * inv_m[(long long)k * it1 + j];
+    } else {
+      for (int e = tid; e < it1 * it1; e += blockDim.x) {
+        const int i = e / it1, j = e % it1;
+        double v = om[j] * om[i] * a[(long long)j * mx + i];
+        if (i == j) v += 0.01 * 0.01;
+        beta[e] = v;
+      }
+      __syncthreads();
+      // Gauss-Jordan inverse of beta (matinv: src/broyden.f90:158-184), in place with an identity copy in gmm area
+      double* inv_m = gmm + mx;
+      for (int e = tid; e < it1 * it1; e += blockDim.x) inv_m[e] = (e / it1 == e % it1) ? 1.0 : 0.0;
+      __syncthreads();
+      for (int k = 0; k < it1; ++k) {
+        if (tid == 0) {
+          int p = k;
+          for (int i = k + 1; i < it1; ++i)
+            if (fabs(beta[(long long)i * it1 + k]) > fabs(beta[(long long)p * it1 + k])) p = i;
+          red[0] = p;
         }
+        __syncthreads();
+        const int p = (int)red[0];
+        if (p != k)
+          for (int j = tid; j < it1; j += blockDim.x) {
+            double t = beta[(long long)k * it1 + j];
+            beta[(long long)k * it1 + j] = beta[(long long)p * it1 + j];
+            beta[(long long)p * it1 + j] = t;
+            t = inv_m[(long long)k * it1 + j];
+            inv_m[(long long)k * it1 + j] = inv_m[(long long)p * it1 + j];
+            inv_m[(long long)p * it1 + j] = t;
+          }
+        __syncthreads();
+        const double piv = beta[(long long)k * it1 + k];
+        __syncthreads();
+        for (int j = tid; j < it1; j += blockDim.x) {
+          beta[(long long)k * it1 + j] /= piv;
+          inv_m[(long long)k * it1 + j] /= piv;
+        }
+        __syncthreads();
+        // eliminate column k: each thread owns full rows i
+        for (int i = tid; i < it1; i += blockDim.x) {
+          if (i == k) continue;
+          const double f = beta[(long long)i * it1 + k];
+          if (f == 0.0) continue;
+          for (int j = 0; j < it1; ++j) {
+            beta[(long long)i * it1 + j] -= f * beta[(long long)k * it1 + j];
+            inv_m[(long long)i * it1 + j] -= f * inv_m[(long long)k * it1 + j];
+          }
+        }
+        __syncthreads();
+      }
+      // gamma(j) = sum_i c(i) beta^-1(i, j)
+      for (int j = tid; j < it1; j += blockDim.x) {
+        double s = 0.0;
+        for (int i = 0; i < it1; ++i) s += c[i] * inv_m[(long long)i * it1 + j];
+        gmm[j] = s;
       }
       __syncthreads();
     }
-    // gamma(j) = sum_i c(i) beta^-1(i, j)
-    for (int j = tid; j < it1; j += blockDim.x) {
-      double s = 0.0;
-      for (int i = 0; i < it1; ++i) s += c[i] * inv_m[(long long)i * it1 + j];
-      gmm[j] = s;
-    }
-    __syncthreads();
     double* ui = u + (long long)i1 * nbr;
     for (int k = tid; k < nbr; k += blockDim.x) {
       ui[k] = alpha * dfi[k] + inv * (qi[k] - ql[k]);
@@ -591,6 +661,7 @@ __global__ void __launch_bounds__(256) k_scc_control(
     __syncthreads();
     for (int k = tid; k < nbr; k += blockDim.x) {
       double v = qi[k] + alpha * dqv[k];
+#pragma unroll 4
       for (int i = 0; i < it1; ++i) v = v - om[i] * gmm[i] * u[(long long)i * nbr + k];
       qi[k] = v;
     }
