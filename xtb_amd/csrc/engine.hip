@@ -2662,9 +2662,9 @@ void Batch::setup() {
     hipLaunchKernelGGL(k_sdqh0<1>, dim3(grid1(sub_max_psp, 64), ns), dim3(64), 0, stream, d_sub, el, at, xyz, at_sh0,
                        at_ao0, selfe, intcut, (const int2*)pair_list, S, H0, H0n, D, Q);
   if (sub_max_pd > 0)
-    hipLaunchKernelGGL(k_sdqh0<2>, dim3(grid1(sub_max_pd, 64), ns), dim3(64), 0, stream, d_sub, el, at, xyz, at_sh0,
+    hipLaunchKernelGGL(k_sdqh0<2>, dim3(grid1(sub_max_pd, 64), ns, kDWaves), dim3(64), 0, stream, d_sub, el, at, xyz, at_sh0,
                        at_ao0, selfe, intcut, (const int2*)pair_list, S, H0, H0n, D, Q);
-  hipLaunchKernelGGL(k_sdq_onsite, dim3(grid1(sub_max_n, 64), ns), dim3(64), 0, stream, d_sub, el, at, xyz, at_sh0,
+  hipLaunchKernelGGL(k_sdq_onsite, dim3(grid1(sub_max_n, 64), ns, kDWaves), dim3(64), 0, stream, d_sub, el, at, xyz, at_sh0,
                      at_ao0, selfe, intcut, S, H0, H0n, D, Q);
   {
     // the integral kernels wrote the lower triangles: mirror them, S first
@@ -3027,7 +3027,7 @@ void Batch::gradient() {
                        (const double*)T, (const double*)H0n, (const double*)S, (const double*)shift, (const double*)vs,
                        (const double*)vd, (const double*)vq, intcut, (const int2*)pair_list, gpair);
   if (sub_max_pd > 0)
-    hipLaunchKernelGGL(k_grad_h0_pairs<2>, dim3(grid1(sub_max_pd, 64), ns), dim3(64), 0, stream2, d_sub, el, at, xyz,
+    hipLaunchKernelGGL(k_grad_h0_pairs<2>, dim3(grid1(sub_max_pd, 64), ns), dim3(64 * kDWaves), 0, stream2, d_sub, el, at, xyz,
                        at_sh0, at_ao0, (const double*)selfe, (const double*)dsedcn, (const double*)P,
                        (const double*)T, (const double*)H0n, (const double*)S, (const double*)shift, (const double*)vs,
                        (const double*)vd, (const double*)vq, intcut, (const int2*)pair_list, gpair);

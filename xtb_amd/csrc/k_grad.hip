@@ -182,8 +182,10 @@ __device__ void grad_dispatch(int li, int lj, const Element& ei, int is, const E
 // added to i and subtracted from j) and the dE/dCN sums of either side,
 // stored at gpair[5 * (p0 + i n + j)].  k_grad_h0 then gives atom a (one
 // workgroup, thread = partner b) the sum over its pairs in a fixed order.
+// Pairs with d shells: kDWaves waves per 64 pairs, a wave per share of the
+// shell pairs (d_wave), summed in LDS in wave order.
 template <int LMAX>
-__global__ void __launch_bounds__(64) k_grad_h0_pairs(const MolDesc* __restrict__ desc, const Element* __restrict__ el,
+__global__ void __launch_bounds__(LMAX < 2 ? 64 : 64 * kDWaves) k_grad_h0_pairs(const MolDesc* __restrict__ desc, const Element* __restrict__ el,
                                                       const int* __restrict__ at, const double* __restrict__ xyz,
                                                       const int* __restrict__ at_sh0, const int* __restrict__ at_ao0,
                                                       const double* __restrict__ selfe,
@@ -195,8 +197,11 @@ __global__ void __launch_bounds__(64) k_grad_h0_pairs(const MolDesc* __restrict_
                                                       const int2* __restrict__ pairs, double* gpair) {
   const MolDesc md = desc[blockIdx.y];
   // LMAX 1 takes the pair list's leading s/p-only pairs, LMAX 2 the rest
-  const long long t = (LMAX < 2 ? 0 : md.npsp) + (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (LMAX < 2 ? (long long)md.npsp : (long long)md.n * (md.n - 1) / 2)) return;
+  const int lane = threadIdx.x & 63, wave = LMAX < 2 ? 0 : threadIdx.x >> 6;
+  const long long t0 = (LMAX < 2 ? 0 : md.npsp) + (long long)blockIdx.x * 64;
+  const long long t1 = LMAX < 2 ? (long long)md.npsp : (long long)md.n * (md.n - 1) / 2;
+  if (t0 >= t1) return;   // the whole workgroup
+  const long long t = min(t0 + lane, t1 - 1);
   const int2 pr = pairs[md.p0 + t];   // grouped by element pair: one code path per wave
   const int iat = pr.x, jat = pr.y;
   const int N = md.nao;
@@ -205,7 +210,7 @@ __global__ void __launch_bounds__(64) k_grad_h0_pairs(const MolDesc* __restrict_
   const double* rj = x + 3 * jat;
   const double rij[3] = {ri[0] - rj[0], ri[1] - rj[1], ri[2] - rj[2]};
   const double rij2 = rij[0] * rij[0] + rij[1] * rij[1] + rij[2] * rij[2];
-  if (rij2 > 1600.0) return;
+  const bool on = t0 + lane < t1 && rij2 <= 1600.0;
   const Element& ei = el[at[md.a0 + iat]];
   const Element& ej = el[at[md.a0 + jat]];
   GradPairIn in;
@@ -217,12 +222,16 @@ __global__ void __launch_bounds__(64) k_grad_h0_pairs(const MolDesc* __restrict_
   const double t14 = sqrt(rr), t17 = 1.0 / rij2;
   double gp[3] = {0, 0, 0}, dcn_i = 0.0, dcn_j = 0.0;
   int aoi = at_ao0[md.a0 + iat];
-  for (int is = 0; is < ei.nsh; ++is) {
+  for (int is = 0; on && is < ei.nsh; ++is) {
     const int li = ei.l[is];
     const int shi = md.s0 + at_sh0[md.a0 + iat] + is;
     int aoj = at_ao0[md.a0 + jat];
     for (int js = 0; js < ej.nsh; ++js) {
       const int lj = ej.l[js];
+      if (LMAX > 1 && d_wave(li, lj) != wave) {
+        aoj += 2 * lj + 1;
+        continue;
+      }
       const int shj = md.s0 + at_sh0[md.a0 + jat] + js;
       const double k1 = ei.shpoly[li] * 0.01, k2 = ej.shpoly[lj] * 0.01;
       const double t15 = k1 * t14, t23 = k2 * t14;
@@ -247,6 +256,22 @@ __global__ void __launch_bounds__(64) k_grad_h0_pairs(const MolDesc* __restrict_
     }
     aoi += 2 * li + 1;
   }
+  if (LMAX > 1) {
+    __shared__ double part[kDWaves - 1][5][64];
+    if (wave > 0) {
+      for (int k = 0; k < 3; ++k) part[wave - 1][k][lane] = gp[k];
+      part[wave - 1][3][lane] = dcn_i;
+      part[wave - 1][4][lane] = dcn_j;
+    }
+    __syncthreads();
+    if (wave > 0) return;
+    for (int w = 0; w < kDWaves - 1; ++w) {
+      for (int k = 0; k < 3; ++k) gp[k] += part[w][k][lane];
+      dcn_i += part[w][3][lane];
+      dcn_j += part[w][4][lane];
+    }
+  }
+  if (!on) return;
   double* o = gpair + 5 * (md.p0 + (long long)iat * md.n + jat);
   o[0] = gp[0];
   o[1] = gp[1];

@@ -200,7 +200,7 @@ __device__ void pair_dispatch(int li, int lj, const Element& ei, int is, const E
 
 // one thread per atom pair (i > j), pairs taken from the molecule's list
 // grouped by element pair (one code path per wave); LMAX 1 takes the list's
-// leading s/p-only pairs, LMAX 2 the rest
+// leading s/p-only pairs, LMAX 2 the rest (blockIdx.z = d_wave)
 template <int LMAX>
 __global__ void __launch_bounds__(64) k_sdqh0(const MolDesc* __restrict__ desc, const Element* __restrict__ el, const int* __restrict__ at,
                         const double* __restrict__ xyz, const int* __restrict__ at_sh0, const int* __restrict__ at_ao0,
@@ -235,6 +235,10 @@ __global__ void __launch_bounds__(64) k_sdqh0(const MolDesc* __restrict__ desc, 
     int aoj = at_ao0[md.a0 + j];
     for (int js = 0; js < ej.nsh; ++js) {
       const int lj = ej.l[js];
+      if (LMAX > 1 && d_wave(li, lj) != (int)blockIdx.z) {
+        aoj += 2 * lj + 1;
+        continue;
+      }
       const double hii = selfe[md.s0 + at_sh0[md.a0 + i] + is];
       const double hjj = selfe[md.s0 + at_sh0[md.a0 + j] + js];
       const double zi = ei.zeta[is], zj = ej.zeta[js];
@@ -258,7 +262,9 @@ __global__ void __launch_bounds__(64) k_sdqh0(const MolDesc* __restrict__ desc, 
 
 // on-site blocks: S = 1, H0 = self energy, dipole/quadrupole moments of the
 // atom's own shell pairs about the origin (build_SDQH0 :298-369); atoms
-// without d shells take the s/p-only code (no d-shell temporaries)
+// without d shells take the s/p-only code (no d-shell temporaries).
+// blockIdx.z = d_wave of the shell pair (the pp pair of an atom without d
+// shells with z = 0), the squares of S and H0 with z = 1
 __global__ void __launch_bounds__(64) k_sdq_onsite(const MolDesc* __restrict__ desc, const Element* __restrict__ el,
                              const int* __restrict__ at, const double* __restrict__ xyz, const int* __restrict__ at_sh0,
                              const int* __restrict__ at_ao0, const double* __restrict__ selfe, double intcut, double* S,
@@ -276,37 +282,45 @@ __global__ void __launch_bounds__(64) k_sdq_onsite(const MolDesc* __restrict__ d
   double* Dm = D + 3 * md.m0;
   double* Qm = Q + 6 * md.m0;
   const int ao0 = at_ao0[md.a0 + i];
-  // zero the whole on-site square first (S and H0 stay zero off the diagonal)
-  int nao_at = 0;
-  for (int s = 0; s < e.nsh; ++s) nao_at += 2 * e.l[s] + 1;
-  for (int u = 0; u < nao_at; ++u)
-    for (int v = 0; v < nao_at; ++v) {
-      const long long p = (long long)(ao0 + u) * N + ao0 + v;
-      Sm[p] = (u == v) ? 1.0 : 0.0;
-      H0m[p] = 0.0;
-      Hnm[p] = 0.0;
+  const int z = blockIdx.z;
+  // S and H0 stay zero off the diagonal
+  if (z == 1) {
+    int nao_at = 0;
+    for (int s = 0; s < e.nsh; ++s) nao_at += 2 * e.l[s] + 1;
+    for (int u = 0; u < nao_at; ++u)
+      for (int v = 0; v < nao_at; ++v) {
+        const long long p = (long long)(ao0 + u) * N + ao0 + v;
+        Sm[p] = (u == v) ? 1.0 : 0.0;
+        H0m[p] = 0.0;
+        Hnm[p] = 0.0;
+      }
+    int aoi = ao0;
+    for (int is = 0; is < e.nsh; ++is) {
+      const double se = selfe[md.s0 + at_sh0[md.a0 + i] + is];
+      for (int k = 0; k < 2 * e.l[is] + 1; ++k, ++aoi) {
+        const long long p = (long long)aoi * N + aoi;
+        H0m[p] = se;
+        Hnm[p] = se;
+      }
     }
+  }
   bool has_d = false;
   for (int s = 0; s < e.nsh; ++s) has_d = has_d || e.l[s] > 1;
   int aoi = ao0;
   for (int is = 0; is < e.nsh; ++is) {
-    const double se = selfe[md.s0 + at_sh0[md.a0 + i] + is];
-    for (int k = 0; k < 2 * e.l[is] + 1; ++k) {
-      const long long p = (long long)(aoi + k) * N + aoi + k;
-      H0m[p] = se;
-      Hnm[p] = se;
-    }
     int aoj = ao0;
     for (int js = 0; js < e.nsh; ++js) {
-      if (js <= is) {
+      const int li = e.l[is], lj = e.l[js];
+      const int home = !has_d && li + lj == 2 ? 0 : d_wave(li, lj);
+      if (js <= is && home == z) {
         if (has_d)
-          pair_dispatch<2>(e.l[is], e.l[js], e, is, e, js, ri, ri, intcut, 0.0, aoi, aoj, N, NN, nullptr, nullptr,
-                           nullptr, Dm, Qm);
+          pair_dispatch<2>(li, lj, e, is, e, js, ri, ri, intcut, 0.0, aoi, aoj, N, NN, nullptr, nullptr, nullptr, Dm,
+                           Qm);
         else
-          pair_dispatch<1>(e.l[is], e.l[js], e, is, e, js, ri, ri, intcut, 0.0, aoi, aoj, N, NN, nullptr, nullptr,
-                           nullptr, Dm, Qm);
+          pair_dispatch<1>(li, lj, e, is, e, js, ri, ri, intcut, 0.0, aoi, aoj, N, NN, nullptr, nullptr, nullptr, Dm,
+                           Qm);
       }
-      aoj += 2 * e.l[js] + 1;
+      aoj += 2 * lj + 1;
     }
     aoi += 2 * e.l[is] + 1;
   }
