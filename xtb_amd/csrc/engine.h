@@ -446,6 +446,13 @@ class Batch {
   int* d_sub_wg = nullptr;
   int sub_guess_ = 6;   // steps queued before the first count is read
   void subspace(bool allow);
+  // The AES kernels of an SCC iteration go to a second stream from kAesFork
+  // atom pairs (slots x largest n^2) on.  Below, the two forks and joins of an
+  // iteration cost more than the kernels (one water 3.5 -> 3.25 ms on one
+  // stream, halogenated 23-carbon chain 13.2 -> 12.6 ms, 6 us each for 194 atoms);
+  // above, the kernels take 50 us (512-molecule batch) beside as long ones.
+  static constexpr long long kAesFork = 1 << 17;
+  bool aes_fork() const { return (long long)nmol * max_n * max_n > kAesFork; }
   bool split_ok() const { return jac_p == 32 && !apply_lds && !pivot_lds; }
   bool final_ = false;      // diagonalise() is orbitals()' one
   bool need_full_ = true;   // some molecule takes the full diagonalisation

@@ -1682,24 +1682,28 @@ bool Batch::jacobi(JacSet& js, double* Am, double* Wm, double* evout, bool check
   const bool forked = lanes || blk;
   // the problems of dimension <= 64 (one workgroup each, k_jac_small) run
   // on stream3 beside the lanes
-  if (forked) {
-    HIPCHECK(hipEventRecord(ev_fork, stream));
-    HIPCHECK(hipStreamWaitEvent(stream2, ev_fork, 0));
-    HIPCHECK(hipStreamWaitEvent(stream3, ev_fork, 0));
-    HIPCHECK(hipStreamWaitEvent(stream4, ev_fork, 0));
-  }
+  // (only the streams that get work are forked and joined: one molecule's
+  // rounds stay on the main stream)
+  static_assert(kMaxLanes == 3, "a stream per lane");
+  const bool f2 = lanes && js.gpairs[1] < js.gpairs[2], f4 = lanes && js.gpairs[2] < js.gpairs[3];
+  const bool f3 = forked && (js.nsmall > 0 || blk);
+  if (f2 || f3 || f4) HIPCHECK(hipEventRecord(ev_fork, stream));
+  if (f2) HIPCHECK(hipStreamWaitEvent(stream2, ev_fork, 0));
+  if (f3) HIPCHECK(hipStreamWaitEvent(stream3, ev_fork, 0));
+  if (f4) HIPCHECK(hipStreamWaitEvent(stream4, ev_fork, 0));
   if (js.nsmall)
     hipLaunchKernelGGL(k_jac_small, dim3(js.nsmall), dim3(256), 0, forked ? stream3 : stream, js.d_probs, js.d_small,
                        Am, Wm, (const double*)js.scale, js.state, keep_w ? 1 : 0, rows ? 1 : 0, jac_tol);
   if (blk) eig_blocked(es, js, Am, Wm, check_active, stream3);
   if (forked) {
     if (lanes) jacobi_lanes(js, Am, Wm);
-    HIPCHECK(hipEventRecord(ev_join, stream2));
-    HIPCHECK(hipStreamWaitEvent(stream, ev_join, 0));
-    HIPCHECK(hipEventRecord(ev_join3, stream3));
-    HIPCHECK(hipStreamWaitEvent(stream, ev_join3, 0));
-    HIPCHECK(hipEventRecord(ev_join4, stream4));
-    HIPCHECK(hipStreamWaitEvent(stream, ev_join4, 0));
+    auto join = [&](hipEvent_t ev, hipStream_t s) {
+      HIPCHECK(hipEventRecord(ev, s));
+      HIPCHECK(hipStreamWaitEvent(stream, ev, 0));
+    };
+    if (f2) join(ev_join, stream2);
+    if (f3) join(ev_join3, stream3);
+    if (f4) join(ev_join4, stream4);
   } else if (js.npairs) {
     // banded rounds first (neighbouring blocks only), then cyclic sweeps;
     // every round starts with the convergence test of the problems at a
@@ -2754,10 +2758,14 @@ void Batch::scc_prologue() {
   const Element* el = elements_dev;
   const double thr2 = neglect * 1.0e-2;
   // the AES potentials (read only charges and moments, write only vs, vd,
-  // vq) on stream2 beside the shell and D4 potentials; joined before the Fock build
-  HIPCHECK(hipEventRecord(ev_fork, stream));
-  HIPCHECK(hipStreamWaitEvent(stream2, ev_fork, 0));
-  hipLaunchKernelGGL(k_aes_pot, dim3(std::max(1, max_n), nmol), dim3(64), 0, stream2, d_desc, el, at, xyz, q, dipm, qp,
+  // vq) on stream2 beside the shell and D4 potentials, joined before the Fock
+  // build, where they take longer than the fork and the join (aes_fork)
+  const hipStream_t s2 = aes_fork() ? stream2 : stream;
+  if (s2 != stream) {
+    HIPCHECK(hipEventRecord(ev_fork, stream));
+    HIPCHECK(hipStreamWaitEvent(stream2, ev_fork, 0));
+  }
+  hipLaunchKernelGGL(k_aes_pot, dim3(std::max(1, max_n), nmol), dim3(64), 0, s2, d_desc, el, at, xyz, q, dipm, qp,
                      gab3, gab5, 1, vs, vd, vq, (const MolState*)d_state);
   hipLaunchKernelGGL(k_shell_pot, dim3(grid1(max_nsh, 4), nmol), dim3(256), 0, stream, d_desc, (const double*)J,
                      (const double*)qsh, (const double*)shgam, shift, 1, (const MolState*)d_state);
@@ -2771,8 +2779,10 @@ void Batch::scc_prologue() {
   hipLaunchKernelGGL(k_shift_final, dim3(grid1(max_nsh, 64), nmol), dim3(64), 0, stream, d_desc, el, at, sh_at,
                      (const int*)d4_at, (const double*)d4dum, (const double*)dzv, solv_on_ ? (const double*)sv_pot : nullptr, shift,
                      (const MolState*)d_state);
-  HIPCHECK(hipEventRecord(ev_join, stream2));
-  HIPCHECK(hipStreamWaitEvent(stream, ev_join, 0));
+  if (s2 != stream) {
+    HIPCHECK(hipEventRecord(ev_join, stream2));
+    HIPCHECK(hipStreamWaitEvent(stream, ev_join, 0));
+  }
   hipLaunchKernelGGL(k_fock, dim3(std::max(1, ((max_nao + 31) / 32) * ((max_nao + 31) / 32 + 1) / 2), nmol), dim3(256),
                      0, stream, d_desc, S, H0,
                      D, Q, shift, vs, vd, vq, ao_sh, ao_at, thr2, H, (const MolState*)d_state);
@@ -2964,10 +2974,14 @@ bool Batch::scc_iteration(bool queue_next, bool subspace_ok) {
   hipLaunchKernelGGL(k_pop_reduce, dim3(grid1(max_n, 64), nmol), dim3(64), 0, stream, d_desc, el, at, xyz, at_sh0,
                      at_ao0, (const double*)zsh, (const double*)row_q, (const double*)row_d, (const double*)row_qp,
                      qsh, q, dipm, qp, (const MolState*)d_state, 0);
-  // the AES energy terms on stream2 beside the shell and D4 energy terms
-  HIPCHECK(hipEventRecord(ev_fork, stream));
-  HIPCHECK(hipStreamWaitEvent(stream2, ev_fork, 0));
-  hipLaunchKernelGGL(k_aes_energy, dim3(std::max(1, max_n), nmol), dim3(64), 0, stream2, d_desc, el, at, xyz, q, dipm,
+  // the AES energy terms on stream2 beside the shell and D4 energy terms (as
+  // the potentials, where that pays)
+  const hipStream_t s2 = aes_fork() ? stream2 : stream;
+  if (s2 != stream) {
+    HIPCHECK(hipEventRecord(ev_fork, stream));
+    HIPCHECK(hipStreamWaitEvent(stream2, ev_fork, 0));
+  }
+  hipLaunchKernelGGL(k_aes_energy, dim3(std::max(1, max_n), nmol), dim3(64), 0, s2, d_desc, el, at, xyz, q, dipm,
                      qp, gab3, gab5, ae01, (const MolState*)d_state);
   hipLaunchKernelGGL(k_shell_pot, dim3(grid1(max_nsh, 4), nmol), dim3(256), 0, stream, d_desc, (const double*)J,
                      (const double*)qsh, (const double*)shgam, jq, 0, (const MolState*)d_state);
@@ -2978,8 +2992,10 @@ bool Batch::scc_iteration(bool queue_next, bool subspace_ok) {
   if (solv_on_)
     hipLaunchKernelGGL(k_solv_energy, dim3(nmol), dim3(256), 0, stream, d_desc, (const double*)sv_B, (const double*)q,
                        sv_qbq, (const MolState*)d_state);
-  HIPCHECK(hipEventRecord(ev_join, stream2));
-  HIPCHECK(hipStreamWaitEvent(stream, ev_join, 0));
+  if (s2 != stream) {
+    HIPCHECK(hipEventRecord(ev_join, stream2));
+    HIPCHECK(hipStreamWaitEvent(stream, ev_join, 0));
+  }
   hipLaunchKernelGGL(k_scc_control, dim3(nmol), dim3(256), 0, stream, d_desc, d_state, (const double*)jq,
                      (const double*)shgam, (const double*)row_e, (const double*)ae01, (const double*)zv,
                      (const double*)d4dum, solv_on_ ? (const double*)sv_qbq : nullptr, (const double*)sv_gsasa,
