@@ -334,7 +334,7 @@ __device__ __forceinline__ double wave_sums64(double (&x)[64]) {
 // next = n - 1 only the last diagonal entry.  One thread per row, its 64
 // panel elements in registers from the correction to the partial sums, all
 // loads issued before the first use: the launch is one chain of memory
-// latencies (12.5 -> 7 us at 1024 rows with the sums taken from registers by
+// latencies (12.5 -> 8.8 us at 1000 rows with the sums taken from registers by
 // exchanges instead of a second pass over the panel).
 __global__ void __launch_bounds__(256) k_trd_row(const EigProb* __restrict__ probs, const int* __restrict__ act,
                                                  const double* __restrict__ A, double* X, double* vec, double* part2,

@@ -461,8 +461,8 @@ __device__ __forceinline__ double quick_rsqrt(double x) {
 // the CN ratio, from k_d4_c6<1>; the distance to a, in LDS) is formed once
 // per pair, so that a triple takes one 1 / sqrt, one 1 / x and products (the
 // square and cube roots and seven divisions per triple took 51 ms for 2100
-// atoms and 4.7 ms for the 512-molecule batch).  A lane per atom c, the atoms
-// b < c shared out over the four waves.
+// atoms, this takes 15.5; 1.9 ms for the 512-molecule batch).  A lane per atom
+// c, the atoms b < c shared out over the four waves.
 constexpr int kAtmB = 128;   // atoms b per LDS block
 
 __global__ void __launch_bounds__(256) k_d4_atm(const MolDesc* __restrict__ desc, const double* __restrict__ xyz,

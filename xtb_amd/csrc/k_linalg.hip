@@ -110,9 +110,10 @@ typedef double v4d __attribute__((ext_vector_type(4)));
 // and R (K x Nc) with row strides ldl and ldr; RMINOR: R is stored Nc x K.
 // The operands go from global memory straight into the lane layout of
 // v_mfma_f64_16x16x4f64 (four rows of 16 consecutive doubles per load), the
-// loads of the next 32 rows in flight during the 16 matrix instructions of
-// the current 16 (a load takes about twice as long as those): no LDS and no barrier, so waves of different problems and
-// sizes share a compute unit freely.  Rows and columns outside the result
+// loads of the next 32 rows in flight during the 16 matrix instructions
+// of the current 16 (a load takes about twice as long as those): no LDS and
+// no barrier, so waves of different problems and sizes share a compute unit
+// freely.  Rows and columns outside the result
 // read a valid element instead and are not written by the callers.
 template <bool RMINOR>
 __device__ __forceinline__ void wave_mm(const double* __restrict__ L, int ldl, int M, const double* __restrict__ R,
@@ -453,7 +454,7 @@ template __global__ void k_gemm_mfma<false, false, false, true>(const int4*, con
 // off-diagonal magnitude; the solve stops when it is <= tol or after maxsweep
 // sweeps.  Returns the number of rounds that applied a rotation.  A matrix of
 // dimension n < 64 (zero beyond) pairs its own n rows only: n - 1 rounds per
-// sweep instead of 63 (6 AOs: 71 -> 20 us, 26 AOs: 360 -> 180 us).
+// sweep instead of 63 (6 AOs: 71 -> 17 to 48 us, 26 AOs: 360 -> 330 us).
 constexpr int kLd = 65;
 
 __device__ int jacobi64(double* a, double* q, int n, double tol, int maxsweep, double* cs, int* pq, int* flags,
