@@ -276,13 +276,13 @@ def main():
     }
     ql = os.environ.get("XTBAMD_EIG") == "ql"
     lds = os.environ.get("XTBAMD_PIVOT_KERNEL") == "lds"
-    names = {"gemm": "k_gemm_mfma (batched FP64 GEMM on the matrix cores)",
+    names = {"gemm": "k_gemm_tn (batched FP64 products on the matrix cores)",
              "jacobi": ql and "k_tred_ql (tridiagonalisation + QL eigensolver, one workgroup per molecule)" or
              lds and "k_jac_pairsP (32x32 pivot problems of the block-Jacobi eigensolver, in LDS)" or
              "k_jac_pairsR (register-resident Jacobi sweep of each 32x32 pivot problem, one wave)",
              "apply": "k_jac_apply_R (A and W tile updates of a block-Jacobi round, FP64 MFMA, one wave per "
                       "32x32 tile)"}
-    short = {"gemm": "k_gemm_mfma", "jacobi": ql and "k_tred_ql" or lds and "k_jac_pairsP" or "k_jac_pairsR",
+    short = {"gemm": "k_gemm_tn", "jacobi": ql and "k_tred_ql" or lds and "k_jac_pairsP" or "k_jac_pairsR",
              "apply": "k_jac_apply_R"}
     # HBM bytes per launch from the FETCH_SIZE / WRITE_SIZE counter runs of this
     # workload (copy-calibrated) and the GPU-time shares of its kernel-trace
