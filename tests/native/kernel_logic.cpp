@@ -1,0 +1,92 @@
+// Host runs of the bookkeeping of single kernels (one lane, see
+// hip/hip_runtime.h beside this file).  kernel_logic CHECK: exit status 0 if
+// the check holds.
+#include <hip/hip_runtime.h>
+#include <sys/mman.h>
+#include <unistd.h>
+
+#include <cstdio>
+#include <cstdlib>
+#include <string>
+#include <vector>
+
+#include "k_linalg.hip"
+#include "k_sub.hip"
+
+using namespace xtbamd;
+namespace xtbamd {
+thread_local double lds[1];   // the dynamic LDS of a kernel that is not run here
+}
+
+// an array whose end is the end of a readable page: a read behind it faults
+template <class T>
+T* guarded(size_t n) {
+  const size_t page = (size_t)sysconf(_SC_PAGESIZE), bytes = n * sizeof(T), room = (bytes + page - 1) / page * page;
+  char* p = (char*)mmap(nullptr, room + page, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS, -1, 0);
+  if (p == MAP_FAILED || mprotect(p + room, page, PROT_NONE) != 0) std::abort();
+  return (T*)(p + room - bytes);
+}
+
+static int failures = 0;
+#define EXPECT(c)                                                     \
+  do {                                                                \
+    if (!(c)) {                                                       \
+      std::printf("%s:%d: %s\n", __FILE__, __LINE__, #c);             \
+      ++failures;                                                     \
+    }                                                                 \
+  } while (0)
+
+// one closed-shell molecule of N orbitals, o of them occupied, on the subspace path
+struct One {
+  MolDesc md;
+  MolState st;
+  int* si = guarded<int>(kSubInts);
+  unsigned long long* res = guarded<unsigned long long>(kSubRes);
+  double* sd = guarded<double>(kSubDbls);
+  std::vector<double> A, C, ev, X, G, T, W, H, P;
+  One(int N, int o) {
+    std::memset(&md, 0, sizeof(md));
+    std::memset(&st, 0, sizeof(st));
+    md.n = 2;
+    md.nao = N;
+    md.nel = 2 * o;
+    st.active = 1;
+    for (auto* v : {&A, &C, &X, &G, &T, &W, &H, &P}) v->assign((size_t)N * N, 0.0);
+    for (int i = 0; i < N; ++i) ev.push_back(i < o ? -10.0 : 5.0);
+  }
+  SubBufs bufs() { return SubBufs{A.data(), C.data(), ev.data(), X.data(), G.data(), T.data(), W.data(), H.data(), P.data()}; }
+};
+
+// every product launch of an iteration stays inside the molecule's residuals
+// and factors, those of the last molecule of the batch too
+static void sub_products() {
+  One m(80, 30);
+  const int steps[] = {0, 1, kSubSteps - 1};
+  const int dens[][2] = {{kSubM, 0}, {kSubCY, 0}, {kSubE1, 0}, {kSubZ2, 2}, {kSubE, 2}, {kSubZ, 3},
+                         {kSubE, 3}, {kSubZ, 4},  {kSubE, 4},  {kSubCYZ, 0}, {kSubP, 0}};
+  for (int s : steps)
+    for (int op : {(int)kSubB, (int)kSubR}) {
+      m.si[kSubPhase] = 1;
+      m.sd[kSubTol] = -1.0;
+      int4 tile{0, 0, 0, op};
+      k_sub_gemm<false>(&tile, &m.md, m.bufs(), &m.st, m.si, m.res, m.sd, s, 0);
+    }
+  for (auto& d : dens) {
+    m.si[kSubPhase] = 2;
+    m.res[kSubSteps] = m.res[kSubSteps + 1] = (unsigned long long)__double_as_longlong(1e-3);
+    std::printf("product %d level %d\n", d[0], d[1]);
+    std::fflush(stdout);
+    int4 tile{0, 0, 0, d[0] == kSubCY || d[0] == kSubCYZ ? d[0] : d[0] | kSubSym};
+    if (d[0] == kSubCY)
+      k_sub_gemm<true>(&tile, &m.md, m.bufs(), &m.st, m.si, m.res, m.sd, 0, d[1]);
+    else
+      k_sub_gemm<false>(&tile, &m.md, m.bufs(), &m.st, m.si, m.res, m.sd, 0, d[1]);
+  }
+}
+
+int main(int argc, char** argv) {
+  const std::string what = argc > 1 ? argv[1] : "";
+  if (what == "sub_products") sub_products();
+  else return 2;
+  return failures ? 1 : 0;
+}

@@ -257,7 +257,7 @@ __device__ __forceinline__ void sub_block(int op, int level, bool sym, const Mol
     case kSubE1: Lp = G; Rp = G; break;
     case kSubZ2: Lp = G; Rp = P; break;
     case kSubE:
-      if (level > 3 || (level == 3 && !e2)) return;   // the list's third launch forms Z_4 only
+      if (level == 3 && !e2) return;
       Lp = Rp = level == 2 ? P : H;
       break;
     case kSubZ:
@@ -343,7 +343,9 @@ __global__ void __launch_bounds__(256) k_sub_gemm(const int4* __restrict__ tiles
                                                   double* dbl, int step, int level) {
   const int4 tl = tiles[blockIdx.x];
   const int m = tl.x, op = tl.w & 15;
-  if (m < 0) return;
+  // (the last launch of the list of Z and E tiles forms Z_4 only: there is no
+  // E_4, and no residual slot for its maximum)
+  if (m < 0 || (op == kSubE && level > 3)) return;
   int* si = sub + m * kSubInts;
   if (si[kSubPhase] != (op <= kSubR ? 1 : 2)) return;
   unsigned long long* rs = res + (long long)m * kSubRes;
