@@ -406,19 +406,16 @@ __global__ void __launch_bounds__(512) k_sub_wg(const int* __restrict__ list, co
       X[2LL * v * o + (long long)j * v + i] = x;
     }
   }
+  // thread 0 decides between the two barriers after each product, when no wave
+  // reads the shared words
   if (tid == 0) {
     top = 0ull;
-    phase = 1;
+    sub_rate(rs, sd, si, state + m, 0);
   }
   int op = kSubB, step = 0, level = 0;
   bool e2 = false, e3 = false;
+  __syncthreads();
   for (;;) {
-    if (op == kSubB && tid == 0) {
-      sub_rate(rs, sd, si, state + m, step);
-      phase = si[kSubPhase];
-    }
-    __syncthreads();
-    if (phase != 1) return;   // given up
     const int par = (par0 + step) & 1;
     const bool sym = op == kSubM || op == kSubE1 || op == kSubZ2 || op == kSubE || op == kSubZ || op == kSubP;
     const SubShape sh = sub_shape(op, N, o);
@@ -448,6 +445,7 @@ __global__ void __launch_bounds__(512) k_sub_wg(const int* __restrict__ list, co
         rs[step] = top;
         if (sub_step_done(rs, sd, step + 1)) more = 0;
         else if (step + 1 >= kSubSteps) sub_give_up(si, state + m);
+        else sub_rate(rs, sd, si, state + m, step + 1);
       } else if (op == kSubE) {
         rs[kSubSteps + level - 2] = top;
         if (level == 3 && !((double)o * __longlong_as_double((long long)top) <= kSubInvMax)) sub_give_up(si, state + m);
@@ -456,7 +454,7 @@ __global__ void __launch_bounds__(512) k_sub_wg(const int* __restrict__ list, co
       phase = si[kSubPhase];
     }
     __syncthreads();
-    if (phase != 1) return;
+    if (phase != 1) return;   // given up
     // the next product
     if (op == kSubB) op = kSubR;
     else if (op == kSubR) {
