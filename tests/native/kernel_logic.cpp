@@ -84,9 +84,54 @@ static void sub_products() {
   }
 }
 
+// a lane's count and marks take every problem of the lane that k_jac_small
+// does not solve, whatever its size; a problem that left the rounds
+// unfinished fails its molecule
+static void jacobi_unfinished() {
+  const int n = 5;
+  JacobiProb pr[n];
+  MolState st[n];
+  std::memset(pr, 0, sizeof(pr));
+  std::memset(st, 0, sizeof(st));
+  int state[n * kJacState] = {}, active = -1;
+  double scale[n];
+  unsigned long long off[2 * n] = {};
+  const int dim[n] = {48, 80, 48, 20, 0}, small[n] = {0, 0, 0, 1, 1};
+  for (int p = 0; p < n; ++p) {
+    pr[p].dim = dim[p];
+    pr[p].small = small[p];
+    pr[p].mol = p;
+    pr[p].nb = (dim[p] + 15) / 16;
+    pr[p].nbp = pr[p].nb + (pr[p].nb & 1);
+    pr[p].rounds = std::max(1, pr[p].nbp - 1);
+    pr[p].maxsw = 40;
+    scale[p] = 1.0;
+    st[p].active = st[p].diag = 1;
+    off[p] = (unsigned long long)__double_as_longlong(p == 2 ? 1e-15 : 1.0);
+  }
+  pr[1].group = 1;
+  state[3 * kJacState] = 1;   // k_jac_small's
+  k_jac_count(pr, n, state, 0, &active);
+  EXPECT(active == 2);
+  k_jac_count(pr, n, state, 1, &active);
+  EXPECT(active == 1);
+  k_jac_mark(pr, n, scale, state, off, 0, &active, 1e-12, -1);
+  EXPECT(active == 2 && state[2 * kJacState] == 1 && state[0] == 0);
+  state[1 * kJacState] = state[1 * kJacState + 1] = 1;   // given up
+  for (unsigned p = 0; p < n + 1; ++p) {
+    blockIdx.x = p;
+    k_jac_fold(pr, n, state, st, 3);
+  }
+  blockIdx.x = 0;
+  EXPECT(st[0].failed == 3 && st[0].active == 0);   // unfinished
+  EXPECT(st[1].failed == 3 && st[1].active == 0);
+  for (int p = 2; p < n; ++p) EXPECT(st[p].failed == 0 && st[p].active == 1);
+}
+
 int main(int argc, char** argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "sub_products") sub_products();
+  else if (what == "jacobi_unfinished") jacobi_unfinished();
   else return 2;
   return failures ? 1 : 0;
 }

@@ -7,6 +7,8 @@
   from the host with XTBAMD_JAC_MAX_SWEEPS=1; every kernel still ends
   normally) fails its molecule: result["failed"] is the eigensolver's code,
   singlepoint raises, and the other molecules of the batch are untouched.
+* Problems of 33 to 64 rows give the same results on the rounds
+  (XTBAMD_JAC_SMALL=32) as in the one-workgroup solver.
 * The server refuses a request that can never fit its budget at submit time.
 """
 import numpy as np
@@ -69,6 +71,42 @@ def test_diagonalization_that_gives_up_fails_the_molecule(monkeypatch):
     for r in b.results():
         assert r["converged"] and r["failed"] == 0
     b.close()
+
+
+def test_problems_of_33_to_64_rows_on_the_rounds(monkeypatch, golden):
+    """Whole matrices and occupied / virtual blocks on either side of 32 rows,
+    alone (a lane that holds nothing else) and together.  Both solvers stop at
+    |A_ij| <= 1e-12 max |A_ii|: energies agree to rounding (1e-9 Eh, as for the
+    subspace path), charges and gradients to 1e-8."""
+    xa = _engine()
+    from xtb_amd import workloads as w
+    mols = []
+    for k in ("mindless01", "mindless02", "mindless07"):
+        g = golden[k]
+        mols.append((np.array(g["numbers"]), np.array(g["positions"]), g["charge"], g["uhf"]))
+    for n in (4, 5, 6, 7, 10, 11):                # 24 to 66 AOs, 16 to 44 occupied
+        z, x = w.water_cluster(n, 3)
+        mols.append((z, x, 0.0, 0))
+    z, x = w.alkane(9, 2)
+    mols.append((z[:-1], x[:-1], 0.0, 1))         # open shell: whole matrices only
+
+    def run(batch):
+        b = xa.Batch(batch).run()
+        r = b.results()
+        b.close()
+        return r
+
+    ref = run(mols)
+    monkeypatch.setenv("XTBAMD_JAC_SMALL", "32")
+    got = run(mols)
+    alone = [run([m])[0] for m in mols]
+    for k, (a, b, c) in enumerate(zip(ref, got, alone)):
+        print(f"mol {k} nao={a['nao']} dE={b['energy'] - a['energy']:.1e}", flush=True)
+        assert a["failed"] == b["failed"] == 0 and a["iterations"] == b["iterations"], k
+        assert abs(a["energy"] - b["energy"]) <= 1e-9, k
+        for key in ("charges", "gradient"):
+            assert float(np.max(np.abs(a[key] - b[key]))) <= 1e-8, (k, key)
+        _same(b, c, f"mol {k} alone")
 
 
 def test_server_refuses_request_beyond_budget():

@@ -113,6 +113,7 @@ struct JacobiProb {
   int mol;                    // batch slot
   int src_ld;
   int row0;                   // first row of the problem in the molecule's matrix (a diagonal block)
+  int small;                  // solved by k_jac_small (or nothing to solve): not in the rounds
 };
 
 // stream lanes of the block-Jacobi rounds (at most)
@@ -488,6 +489,9 @@ class Batch {
   // finite-difference Hessians beyond the reference's test tolerances.
   double jac_tol_mid = 1e-8;
   double jac_tol_q = 0.0;
+  // problems of at most this dimension (XTBAMD_JAC_SMALL, 32 to the 64 of its
+  // LDS matrix) go to k_jac_small, larger ones to the rounds
+  int jac_small = 64;
   int jac_max_sweeps = 40;   // sweeps before a Jacobi problem is given up (the molecule fails)
   int jac_cross = 1;   // most outer rounds' pivots rotate only the pairs across their two blocks
   bool trace_rounds = false;   // print the Jacobi rounds of each SCC iteration to stderr

@@ -932,6 +932,7 @@ void Batch::init_common() {
   if (const char* r = std::getenv("XTBAMD_JAC_MAX_SWEEPS")) jac_max_sweeps = std::min(40, std::max(1, std::atoi(r)));
   trace_rounds = std::getenv("XTBAMD_TRACE_ROUNDS") != nullptr;
   if (const char* r = std::getenv("XTBAMD_JAC_LANES")) jac_lanes = std::min(kMaxLanes, std::max(1, std::atoi(r)));
+  if (const char* r = std::getenv("XTBAMD_JAC_SMALL")) jac_small = std::min(64, std::max(32, std::atoi(r)));
   if (const char* r = std::getenv("XTBAMD_EIG_BLK_MIN")) eig_blk_min = std::max(65, std::atoi(r));
   if (const char* r = std::getenv("XTBAMD_SUBSPACE")) subspace_on = std::atoi(r) != 0;
   if (const char* r = std::getenv("XTBAMD_SUB_WG")) sub_wg = std::atoi(r);
@@ -1358,6 +1359,7 @@ void Batch::jac_lists(JacSet& js) {
     std::memset(&p, 0, sizeof(p));
     const int mol = js.half ? m / 2 : m;
     p.mol = mol;
+    p.small = 1;
     if (!occupied_[mol]) continue;
     const MolDesc& d = desc[mol];
     if (js.half && !sub_able(d)) continue;
@@ -1379,10 +1381,11 @@ void Batch::jac_lists(JacSet& js) {
     p.q_off = qoff;
     p.maxsw = jac_max_sweeps;
     js.big_max_ld = std::max(js.big_max_ld, p.ld);
-    if (p.dim <= 64) {
+    if (p.dim <= jac_small) {
       small.push_back(m);
       continue;
     }
+    p.small = 0;
     // the largest problems also go to the blocked eigensolver, which takes
     // them for the first eig_blk_iters SCC iterations (the lanes after)
     const bool to_blk = blk_path && p.dim >= eig_blk_min;
@@ -1681,7 +1684,7 @@ bool Batch::jacobi(JacSet& js, double* Am, double* Wm, double* evout, bool check
   // the lanes test their progress once per period of their largest problem
   jac_period_ = blk ? std::max(1, js.max_rounds_lanes) : js.max_rounds;
   const bool forked = lanes || blk;
-  // the problems of dimension <= 64 (one workgroup each, k_jac_small) run
+  // the small problems (one workgroup each, k_jac_small) run
   // on stream3 beside the lanes
   // (only the streams that get work are forked and joined: one molecule's
   // rounds stay on the main stream)
@@ -2284,7 +2287,7 @@ void Batch::eigh_rows(JacSet& js, double* Am, double* Wm, double* evout) {
     hipLaunchKernelGGL(k_jac_small, dim3(js.nsmall), dim3(256), 0, stream, js.d_probs, js.d_small, Am, Wm,
                        (const double*)js.scale, js.state, 0, 1, jac_tol);
     hipLaunchKernelGGL(k_jac_sort, dim3(1, nmol), dim3(256), 0, stream, js.d_probs, (const double*)Am, evout, perm, st,
-                       64);
+                       jac_small);
   }
   if (js.nbig) {
     const int cap = std::min(js.big_max_dim, 1600);
@@ -2886,19 +2889,17 @@ void Batch::diagonalise() {
     refine(A, W);
   }
   // a molecule whose eigensolve gave up fails and stops iterating here
-  auto fold_diag = [&]() {
-    hipLaunchKernelGGL(k_fail_fold, dim3(grid1(nmol, 64)), dim3(64), 0, stream, d_state, nmol,
-                       (const int*)jac_n.state + 1, kJacState, kFailDiag, (const int*)nullptr);
-  };
   if (use_ql && !warm) {
     eigh_rows(jac_n, A, W, emo);
-    fold_diag();
+    hipLaunchKernelGGL(k_fail_fold, dim3(grid1(nmol, 64)), dim3(64), 0, stream, d_state, nmol,
+                       (const int*)jac_n.state + 1, kJacState, kFailDiag, (const int*)nullptr);
     hipLaunchKernelGGL(k_fail_fold, dim3(grid1(nmol, 64)), dim3(64), 0, stream, d_state, nmol,
                        (const int*)eig_failed, 1, kFailDiag, (const int*)nullptr);
     gemm(4, C, W, T, nullptr, perm, false, 1.0, mask, false, ms);    // T = C W(perm, :)^T
   } else {
     const bool rows = jacobi(jac_n, A, W, emo, true, warm, warm ? banded_passes : 0);
-    fold_diag();
+    hipLaunchKernelGGL(k_jac_fold, dim3(grid1(jac_n.nprob, 64)), dim3(64), 0, stream,
+                       (const JacobiProb*)jac_n.d_probs, jac_n.nprob, (const int*)jac_n.state, d_state, kFailDiag);
     if (rows)
       gemm(4, C, W, T, nullptr, perm, false, 1.0, mask, false, ms);  // T = C W(perm, :)^T
     else
@@ -2941,9 +2942,8 @@ void Batch::orbitals() {
     hipLaunchKernelGGL(k_copy_diag, gm, dim3(256), 0, stream, d_desc, (const MolState*)d_state, (const double*)W, C);
     hipLaunchKernelGGL(k_zero_diag, gm, dim3(256), 0, stream, d_desc, (const MolState*)d_state, W);
     jacobi(jac_h, H, W, emo, true);
-    for (int b = 0; b < 2; ++b)
-      hipLaunchKernelGGL(k_fail_fold, dim3(grid1(nmol, 64)), dim3(64), 0, stream, d_state, nmol,
-                         (const int*)jac_h.state + b * kJacState + 1, 2 * kJacState, kFailDiag, (const int*)nullptr);
+    hipLaunchKernelGGL(k_jac_fold, dim3(grid1(jac_h.nprob, 64)), dim3(64), 0, stream,
+                       (const JacobiProb*)jac_h.d_probs, jac_h.nprob, (const int*)jac_h.state, d_state, kFailDiag);
     gemm(4, C, W, T, nullptr, perm, false, 1.0, mask, false, ms);                 // T = C W(perm, :)^T
     hipLaunchKernelGGL(k_copy_diag, gm, dim3(256), 0, stream, d_desc, (const MolState*)d_state, (const double*)T, C);
   } else {

@@ -601,7 +601,7 @@ __device__ __forceinline__ bool jac_boundary(int rounds, int r) {
 }
 
 // state per problem: [0] done, [1] failed, [5] outer sweeps (block path) or
-// inner rounds with rotations (dim <= 64)
+// inner rounds with rotations (k_jac_small)
 constexpr int kJacState = 8;
 // XCDs of the gfx950 part (MI355X): workgroup b of a launch runs on XCD b mod kXcds
 constexpr int kXcds = 8;
@@ -1983,7 +1983,7 @@ __global__ void __launch_bounds__(256) k_jac_mark(const JacobiProb* __restrict__
   double c = 0.0;
   for (int p = threadIdx.x; p < nprob; p += blockDim.x) {
     const JacobiProb pr = probs[p];
-    if (pr.dim <= 64) continue;   // solved by k_jac_small
+    if (pr.small) continue;
     if (group >= 0 && pr.group != group) continue;
     int* st = state + p * kJacState;
     if (st[0]) continue;
@@ -2016,11 +2016,25 @@ __global__ void __launch_bounds__(256) k_jac_count(const JacobiProb* __restrict_
   double c = 0.0;
   for (int p = threadIdx.x; p < nprob; p += blockDim.x) {
     const JacobiProb pr = probs[p];
-    if (pr.dim <= 64 || pr.group != group) continue;
+    if (pr.small || pr.group != group) continue;
     if (!state[p * kJacState]) c += 1.0;
   }
   c = block_sum<256>(c, sh);
   if (threadIdx.x == 0) nactive[0] = (int)c;
+}
+
+// A molecule with a problem that gave up, or that left the solver unfinished,
+// gets the code and stops iterating, like the early return of the reference's
+// SCC after a failed diagonalization (src/scc_core.f90:475-480)
+__global__ void k_jac_fold(const JacobiProb* __restrict__ probs, int nprob, const int* __restrict__ state,
+                           MolState* mstate, int code) {
+  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= nprob) return;
+  const int* st = state + p * kJacState;
+  MolState& ms = mstate[probs[p].mol];
+  if (probs[p].dim == 0 || !ms.diag || (st[0] && !st[1])) return;
+  if (!ms.failed) ms.failed = code;
+  ms.active = 0;
 }
 
 // ---------------------------------------------------------------------------
