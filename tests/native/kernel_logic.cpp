@@ -128,10 +128,51 @@ static void jacobi_unfinished() {
   for (int p = 2; p < n; ++p) EXPECT(st[p].failed == 0 && st[p].active == 1);
 }
 
+// a molecule that converges within few steps is held to the contraction that
+// its gap allows, too
+static void sub_contraction() {
+  // residuals, allowed contraction, carried one, factor of the later steps; stays on the path
+  struct {
+    std::vector<double> r;
+    double lim, rho, w;
+    bool stays;
+  } cases[] = {
+      {{2e-11}, 0.3, 0.0, 1.0, true},
+      {{2e-11}, 0.3, 0.5, 1.0, false},
+      {{1e-9, 2e-11}, 0.3, 0.2, 1.0, true},
+      {{1e-9, 2e-11}, 0.01, 0.0, 1.0, false},
+      {{6e-11, 2.5e-11}, 0.3, 0.0, 1.0, false},
+      {{1e-10, 7e-11, 4.9e-11, 2.9e-11}, 0.3, 0.0, 1.0, false},
+      {{1e-10, 7e-11, 4.9e-11, 2.9e-11}, 0.8, 0.0, 1.0, true},
+      {{1e-3, 1e-4, 1e-5, 1e-6, 1e-7, 1e-11}, 0.3, 0.0, 1.0, true},
+      {{1e-9, 1e-10, 6e-11, 5e-11, 4e-11, 2.9e-11}, 0.3, 0.0, 1.0, false},
+      // second-order steps: falling by sqrt(w - 1) is their optimum
+      {{1e-9, 4e-10, 2e-10, 9e-11, 5e-11, 2.5e-11}, 0.8, 0.6, 1.2, true},
+  };
+  for (auto& c : cases) {
+    One m(80, 30);
+    const int t = (int)c.r.size();
+    m.si[kSubPhase] = 1;
+    m.sd[kSubTol] = 3e-11;
+    m.sd[kSubLim] = c.lim;
+    m.sd[kSubRho] = c.rho;
+    for (int s = 0; s < t; ++s) {
+      m.res[s] = (unsigned long long)__double_as_longlong(c.r[s]);
+      m.sd[kSubW + s] = s > 1 ? c.w : 1.0;
+    }
+    k_sub_outcome(&m.st, 1, m.si, m.res, m.sd, &m.md, 64, kSubSteps);
+    std::printf("%d steps, limit %g: phase %d\n", t, c.lim, m.si[kSubPhase]);
+    EXPECT(m.si[kSubNext] == t);
+    EXPECT(m.si[kSubPhase] == (c.stays ? 2 : 3));
+    EXPECT(m.st.diag == (c.stays ? 0 : 1) && m.si[kSubOff] == (c.stays ? 0 : 1));
+  }
+}
+
 int main(int argc, char** argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "sub_products") sub_products();
   else if (what == "jacobi_unfinished") jacobi_unfinished();
+  else if (what == "sub_contraction") sub_contraction();
   else return 2;
   return failures ? 1 : 0;
 }

@@ -86,6 +86,24 @@ def test_subspace_options_agree(monkeypatch, kw, solvent):
         _check(a, b, f"{kw} mol {k}")
 
 
+@pytest.mark.parametrize("ratio", [0.4, 0.7, 0.8, 0.84, 0.86, 0.95, 1.05, 1.4])
+def test_subspace_at_temperatures_around_the_gap_bound(monkeypatch, ratio):
+    """Electronic temperatures at which 52 kT is `ratio` times the gap: on the
+    path with room, at the edge where its diagonal estimate (0.85 of the gap)
+    or the contraction decides, and above, where every molecule keeps the full
+    diagonalisation.  The density error of whole occupations is e^-26 at the
+    bound itself, so the tolerances are those of every other temperature."""
+    from xtb_amd import workloads as w
+    xa = _engine()
+    for z, x in (w.water_cluster(9, 1), w.alkane(14, 2), w.water_cluster(30, 4)):
+        gap = xa.singlepoint(z, x)["hl_gap_ev"]
+        t = ratio * gap / (52 * 8.617333e-5)
+        (full, cf), (sub, cs) = _both(monkeypatch, [(z, x, 0.0, 0)], etemp=t)
+        _check(full[0], sub[0], f"{len(z)} atoms, {t:.0f} K")
+        if ratio > 1.0:
+            assert cs == cf, (cs, cf)
+
+
 def test_subspace_small_gaps_ions_and_open_shells(monkeypatch, golden):
     """Gaps of 0.7 to 3 eV (given up or never taken), charged and open-shell
     molecules beside gapped ones in one batch."""

@@ -29,7 +29,8 @@
 // [1 - rho, 1 + rho] (and the second-order one only if that lies above 0), so
 // T is positive definite and every virtual eigenvalue lies above every
 // occupied one by at least (1 - rho) min D.  The path is left unless that is
-// at least kSubGapKt kT: the Fermi occupations of the frontier orbitals are
+// at least kSubGapKt kT, rho being the contraction seen over the last steps
+// (sub_rate during the steps, sub_gap_kept at convergence): the Fermi occupations of the frontier orbitals are
 // then within e^-26 = 5e-12 of 1 and 0, the size of the density error that the
 // tolerance of R admits, and far below the 1e-9 from which entropy counts.
 // The occupations handed back are those of the last diagonalisation.
@@ -92,6 +93,26 @@ __device__ __forceinline__ void sub_give_up(int* si, MolState* st) {
   st->diag = 1;
 }
 
+// max |R| fell too slowly over the three steps before step s >= 5
+__device__ __forceinline__ bool sub_slow(const unsigned long long* __restrict__ res, const double* __restrict__ sd,
+                                         int s) {
+  auto at = [&](int k) { return __longlong_as_double((long long)res[k]); };
+  const double wl = sd[kSubW + s - 1], r = cbrt(at(s - 1) / at(s - 4));
+  return !(r * r <= wl - 1.0 || sub_mu(r, wl) <= sd[kSubLim]);
+}
+
+// A molecule that converged with t residuals did so at a contraction that
+// keeps the gap: of the last three steps, of the first one or two (which are
+// plain) where there are fewer, of the SCC iteration before where X needed
+// one step only
+__device__ __forceinline__ bool sub_gap_kept(const unsigned long long* __restrict__ res,
+                                             const double* __restrict__ sd, int t) {
+  if (t >= 5) return !sub_slow(res, sd, t);
+  if (t < 2) return sd[kSubRho] <= sd[kSubLim];
+  const double r = __longlong_as_double((long long)res[min(t - 1, 2)]) / __longlong_as_double((long long)res[0]);
+  return (t == 2 ? r : sqrt(r)) <= sd[kSubLim];
+}
+
 // one thread: the factor w of step s, or the end where max |R| is a NaN or
 // falls too slowly (the mean of three steps: it may rise for one when w sets in)
 __device__ __forceinline__ void sub_rate(const unsigned long long* __restrict__ res, double* sd, int* si,
@@ -100,16 +121,11 @@ __device__ __forceinline__ void sub_rate(const unsigned long long* __restrict__ 
   double rho = sd[kSubRho], w = 1.0;
   if (s > 0) {
     const double wl = sd[kSubW + s - 1];
-    bool slow = !(at(s - 1) < 1e300);
-    double r = 0.0;
-    if (s >= 4) {
-      r = cbrt(at(s - 1) / at(s - 4));
-      slow = slow || (s >= 5 && !(r * r <= wl - 1.0 || sub_mu(r, wl) <= sd[kSubLim]));
-    }
-    if (slow) {
+    if (!(at(s - 1) < 1e300) || (s >= 5 && sub_slow(res, sd, s))) {
       sub_give_up(si, st);
       return;
     }
+    const double r = s >= 4 ? cbrt(at(s - 1) / at(s - 4)) : 0.0;
     if (r * r > 1.1 * (wl - 1.0)) rho = fmax(rho, fmin(kSubRhoMax, sub_mu(r, wl)));
     sd[kSubRho] = rho;
     // the plain step is better as long as max |R| falls faster than the
@@ -443,8 +459,10 @@ __global__ void __launch_bounds__(512) k_sub_wg(const int* __restrict__ list, co
       more = 1;
       if (op == kSubR) {
         rs[step] = top;
-        if (sub_step_done(rs, sd, step + 1)) more = 0;
-        else if (step + 1 >= kSubSteps) sub_give_up(si, state + m);
+        if (sub_step_done(rs, sd, step + 1)) {
+          more = 0;
+          if (!sub_gap_kept(rs, sd, step + 1)) sub_give_up(si, state + m);
+        } else if (step + 1 >= kSubSteps) sub_give_up(si, state + m);
         else sub_rate(rs, sd, si, state + m, step + 1);
       } else if (op == kSubE) {
         rs[kSubSteps + level - 2] = top;
@@ -508,6 +526,10 @@ __global__ void k_sub_outcome(MolState* state, int nmol, int* sub, const unsigne
   while (t < nstep && !sub_step_done(rs, sd, t)) ++t;
   si[kSubNext] = t;
   if (sub_step_done(rs, sd, t)) {
+    if (!sub_gap_kept(rs, sd, t)) {
+      sub_give_up(si, state + m);
+      return;
+    }
     si[kSubPhase] = 2;
     si[kSubPar] = (si[kSubPar] + t) & 1;
     si[kSubPend] = 1;
