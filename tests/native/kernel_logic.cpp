@@ -168,11 +168,43 @@ static void sub_contraction() {
   }
 }
 
+// who may take the path in the next iteration: not the molecules that gave up,
+// open shells, filled bases and gaps far below the bound
+static void sub_next() {
+  struct {
+    int active, off, nopen, nel, nao, phase;
+    double gap;
+    bool may;
+  } cases[] = {{1, 0, 0, 8, 6, 0, 4.0, true},  {1, 0, 0, 8, 6, 0, 1.0, false}, {1, 0, 0, 8, 6, 2, 1.0, true},
+               {1, 0, 0, 8, 6, 4, 1.0, true},  {1, 1, 0, 8, 6, 3, 4.0, true},  {1, 2, 0, 8, 6, 3, 4.0, false},
+               {0, 0, 0, 8, 6, 4, 4.0, false}, {1, 0, 1, 7, 6, 0, 4.0, false}, {1, 0, 0, 12, 6, 0, 4.0, false}};
+  for (auto& c : cases) {
+    MolDesc md;
+    MolState st;
+    std::memset(&md, 0, sizeof(md));
+    std::memset(&st, 0, sizeof(st));
+    md.n = 3;
+    md.nao = c.nao;
+    md.nel = c.nel;
+    md.nopen = c.nopen;
+    st.active = c.active;
+    int* si = guarded<int>(kSubInts);
+    int* cnt = guarded<int>(2);
+    double* e = guarded<double>(c.nao);
+    si[kSubOff] = c.off;
+    si[kSubPhase] = c.phase;
+    for (int i = 0; i < c.nao; ++i) e[i] = i < c.nel / 2 ? -12.0 : -12.0 + c.gap;
+    k_sub_next(&md, &st, 1, si, e, 1.344, cnt);
+    EXPECT(cnt[0] == c.active && cnt[1] == (c.may ? 1 : 0) && si[kSubMay] == cnt[1]);
+  }
+}
+
 int main(int argc, char** argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "sub_products") sub_products();
   else if (what == "jacobi_unfinished") jacobi_unfinished();
   else if (what == "sub_contraction") sub_contraction();
+  else if (what == "sub_next") sub_next();
   else return 2;
   return failures ? 1 : 0;
 }

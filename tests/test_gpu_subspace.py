@@ -104,6 +104,39 @@ def test_subspace_at_temperatures_around_the_gap_bound(monkeypatch, ratio):
             assert cs == cf, (cs, cf)
 
 
+def test_subspace_launches_only_where_a_molecule_can_use_them(monkeypatch, capfd):
+    """Steps queued per SCC iteration (XTBAMD_TRACE_ROUNDS): none in the first
+    one, whose orbitals the path needs; none at all for open shells, for gaps
+    far below 52 kT (9000 K) and once every molecule has given up; the second
+    iteration starts with the steps of a cold start."""
+    from xtb_amd import workloads as w
+    xa = _engine()
+    monkeypatch.setenv("XTBAMD_TRACE_ROUNDS", "1")
+
+    def steps(mols, **kw):
+        capfd.readouterr()
+        b = xa.Batch(mols, **kw)
+        out = []
+        for _ in range(2):   # a batch run again starts anew
+            b.run()
+            out.append([int(ln.split()[-3]) for ln in capfd.readouterr().err.splitlines() if "subspace steps" in ln])
+        b.close()
+        assert len(out[0]) > 3 and out[0] == out[1], out
+        return out[0]
+
+    zw, xw = w.water_cluster(20, 3)
+    za, xa_ = w.alkane(14, 3)
+    s = steps([(zw, xw, 0.0, 0), (za, xa_, 0.0, 0)])
+    print(s, flush=True)
+    assert s[0] == 0 and s[1] >= 6 and all(k > 0 for k in s[1:]), s
+    assert not any(steps([(za[:-1], xa_[:-1], 0.0, 1)]))
+    assert not any(steps([(zw, xw, 0.0, 0)], etemp=9000.0))
+    small = w.water_cluster(3, 3) + (0.0, 0)
+    s = steps([small])
+    assert s[0] == 0 and any(s[1:]), s
+    assert not any(steps([small], etemp=9000.0))
+
+
 def test_subspace_small_gaps_ions_and_open_shells(monkeypatch, golden):
     """Gaps of 0.7 to 3 eV (given up or never taken), charged and open-shell
     molecules beside gapped ones in one batch."""

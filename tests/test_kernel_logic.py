@@ -23,7 +23,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("check", ["sub_products", "jacobi_unfinished", "sub_contraction"])
+@pytest.mark.parametrize("check", ["sub_products", "jacobi_unfinished", "sub_contraction", "sub_next"])
 def test_kernel_logic(program, check):
     r = subprocess.run([program, check], capture_output=True, text=True)
     assert r.returncode == 0, f"status {r.returncode}\n{r.stdout}{r.stderr}"

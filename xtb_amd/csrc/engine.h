@@ -445,7 +445,12 @@ class Batch {
   int sub_wg = 64;
   int sub_nwg_ = 0;
   int* d_sub_wg = nullptr;
-  int sub_guess_ = 6;   // steps queued before the first count is read
+  static constexpr int kSubCold = 6;   // steps queued for a cold start
+  int sub_guess_ = kSubCold;   // steps queued before the first count is read
+  int sub_may_ = 0;            // molecules that may take the path in the next SCC iteration
+  bool sub_used_ = false;      // some molecule may have stopped on it
+  double sub_min_gap() const;
+  int sub_steps_ = 0;   // steps queued in the last SCC iteration
   void subspace(bool allow);
   // The AES kernels of an SCC iteration go to a second stream from kAesFork
   // atom pairs (slots x largest n^2) on.  Below, the two forks and joins of an

@@ -2797,19 +2797,27 @@ void Batch::scc_prologue() {
   mixed_here_ = false;
 }
 
+// smallest gap of the subspace path at this electronic temperature [eV]
+double Batch::sub_min_gap() const {
+  return std::max(1.0, opt.etemp > 0.1 ? kSubGapKt * kBoltzmann * kAutoEV * opt.etemp : 0.0);
+}
+
 // The density of the molecules that may take the subspace path; the others
 // (and those that give up) are left with MolState::diag = 1 and counted into
 // need_full_.  Convergence is decided per molecule on the device; the host
 // queues as many steps as the last iteration took, then the products of the
-// density of whatever converged, and reads the counts while those run.
+// density of whatever converged, and reads the counts while those run.  Where
+// no molecule may take the path (the last iteration's count) nothing but the
+// flags is queued.
 void Batch::subspace(bool allow) {
-  allow = allow && subspace_on && !use_ql && oa_max_steps == 0 && !mixed && sub_t0[kSubLists] > 0;
-  const double kt = kBoltzmann * kAutoEV * opt.etemp;
+  allow = allow && subspace_on && !use_ql && oa_max_steps == 0 && !mixed && sub_t0[kSubLists] > 0 && sub_may_ > 0;
   hipLaunchKernelGGL(k_sub_begin, dim3(nmol), dim3(256), 0, stream, d_desc, d_state, (const double*)A, ev, sub_,
-                     sub_res_, sub_dbl_, jac_tol, std::max(1.0, opt.etemp > 0.1 ? kSubGapKt * kt : 0.0),
-                     allow ? 1 : 0);
+                     sub_res_, sub_dbl_, jac_tol, sub_min_gap(), allow ? 1 : 0);
   need_full_ = true;
+  sub_steps_ = 0;
   if (!allow) return;
+  sub_used_ = true;
+  sub_steps_ = 1;   // at least
   const bool wide = sub_t0[1] > sub_t0[0];
   if (wide) {
     hipLaunchKernelGGL(k_sub_start, dim3(gstride((long long)max_nao * max_nao / 4 + 1), nmol), dim3(256), 0, stream, d_desc,
@@ -2872,7 +2880,8 @@ void Batch::subspace(bool allow) {
     upto = std::min(kSubSteps, step + 2);
   }
   need_full_ = h_pinned[9] > 0;
-  sub_guess_ = std::max(1, h_pinned[10]);
+  sub_steps_ = step;
+  if (h_pinned[10] > 0) sub_guess_ = h_pinned[10];
 }
 
 // C, orbital energies and occupations of the molecules with MolState::diag
@@ -2910,7 +2919,7 @@ void Batch::diagonalise() {
 }
 
 void Batch::orbitals() {
-  if (!subspace_on) return;
+  if (!sub_used_) return;
   hipLaunchKernelGGL(k_sub_pending, dim3(1), dim3(256), 0, stream, d_state, nmol, sub_, sub_cnt_);
   HIPCHECK(hipMemcpyAsync(h_pinned + 8, sub_cnt_, sizeof(int), hipMemcpyDeviceToHost, stream));
   HIPCHECK(hipStreamSynchronize(stream));
@@ -3004,10 +3013,12 @@ bool Batch::scc_iteration(bool queue_next, bool subspace_ok) {
   HIPCHECK(hipGetLastError());
   iterations_ += 1;
   if (trace_rounds)
-    std::fprintf(stderr, "scc iteration %d: %lld Jacobi rounds\n", iterations_, jacobi_rounds_ - rounds_before);
+    std::fprintf(stderr, "scc iteration %d: %lld Jacobi rounds, %d subspace steps\n", iterations_,
+                 jacobi_rounds_ - rounds_before, sub_steps_);
   // any molecule still active?
-  hipLaunchKernelGGL(k_count_active, dim3(1), dim3(256), 0, stream, (const MolState*)d_state, nmol, jac_nactive);
-  HIPCHECK(hipMemcpyAsync(h_pinned, jac_nactive, sizeof(int), hipMemcpyDeviceToHost, stream));
+  hipLaunchKernelGGL(k_sub_next, dim3(1), dim3(256), 0, stream, (const MolDesc*)d_desc, (const MolState*)d_state, nmol,
+                     sub_, (const double*)emo, sub_min_gap(), jac_nactive);
+  HIPCHECK(hipMemcpyAsync(h_pinned, jac_nactive, 2 * sizeof(int), hipMemcpyDeviceToHost, stream));
   if (queue_next) {
     // the next iteration's first part keeps the GPU busy while the host
     // waits for the count (it changes nothing if no molecule is active)
@@ -3018,6 +3029,7 @@ bool Batch::scc_iteration(bool queue_next, bool subspace_ok) {
   } else {
     HIPCHECK(hipStreamSynchronize(stream));
   }
+  sub_may_ = h_pinned[1];
   return h_pinned[0] > 0;
 }
 
@@ -3105,6 +3117,9 @@ void Batch::run() {
   setup();
   int guard = 0;
   prologue_queued_ = false;
+  sub_used_ = false;
+  sub_may_ = 0;
+  sub_guess_ = kSubCold;
   // (no iteration is queued ahead of the guard's stop)
   while (scc_iteration(guard + 1 <= opt.maxiter + 2, true)) {
     if (++guard > opt.maxiter + 2) break;

@@ -2405,14 +2405,6 @@ __global__ void k_state_scatter(const MolDesc* __restrict__ desc, const MolState
   if (k < n) st[desc[k].mol] = stage[k];
 }
 
-__global__ void k_count_active(const MolState* __restrict__ st, int nmol, int* out) {
-  __shared__ double sh[4];
-  double c = 0.0;
-  for (int m = threadIdx.x; m < nmol; m += blockDim.x) c += st[m].active ? 1.0 : 0.0;
-  c = block_sum<256>(c, sh);
-  if (threadIdx.x == 0) out[0] = (int)c;
-}
-
 // T <- 0 for the molecules that are diagonalised
 __global__ void k_zero_diag(const MolDesc* __restrict__ desc, const MolState* __restrict__ st, double* T) {
   const MolDesc md = desc[blockIdx.y];

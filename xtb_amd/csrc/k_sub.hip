@@ -59,7 +59,13 @@ constexpr int kSubOff = 3;     // attempts given up in this run
 constexpr int kSubPend = 4;    // stopped without orbital energies: one diagonalisation to come
 constexpr int kSubFresh = 5;   // X starts from the first-order guess
 constexpr int kSubNext = 6;    // steps taken in this SCC iteration
+constexpr int kSubMay = 7;     // may take the path in the next SCC iteration
 constexpr int kSubInts = 8;
+// the gap of the last orbitals, in units of the one that k_sub_begin asks of
+// the diagonal, from which a molecule off the path may take it next: the
+// diagonal moves by a few percent per iteration.  Below it the iteration would
+// queue the path's launches and wait for their counts for nothing
+constexpr double kSubMayGap = 0.9;
 // residual maxima: one per step, then those of E_2 = M^4 and E_3 = M^8
 constexpr int kSubRes = kSubSteps + 2;
 
@@ -157,8 +163,7 @@ __global__ void __launch_bounds__(256) k_sub_begin(const MolDesc* __restrict__ d
   int* si = sub + m * kSubInts;
   const int active = st.active, first = st.iter == 0;
   const int o = sub_occ(md), N = md.nao;
-  const bool able = allow && active && !first && si[kSubOff] < kSubTries && md.nopen == 0 && (md.nel & 1) == 0 && md.n > 1 &&
-                    o >= 1 && o < N;
+  const bool able = allow && active && !first && si[kSubMay];
   __syncthreads();
   bool on = false;
   double top = -1e300, low = -1e300, big = 0.0;   // max occupied, -min virtual
@@ -566,6 +571,36 @@ __global__ void __launch_bounds__(256) k_sub_check(const MolDesc* __restrict__ d
     cnt[0] = (int)run;
     cnt[1] = (int)full;
     cnt[2] = (int)most;
+  }
+}
+
+// after an SCC iteration, cnt[0]: molecules still iterating, cnt[1]: those of
+// them that may take the path in the next one (kSubMay; closed shells with
+// occupied and virtual orbitals, on the path now or with a gap that comes near)
+__global__ void __launch_bounds__(256) k_sub_next(const MolDesc* __restrict__ desc, const MolState* __restrict__ state,
+                                                  int nmol, int* sub, const double* __restrict__ emo, double min_gap,
+                                                  int* cnt) {
+  __shared__ double sh[4];
+  double run = 0.0, may = 0.0;
+  for (int m = threadIdx.x; m < nmol; m += blockDim.x) {
+    const MolDesc& md = desc[m];
+    int* si = sub + m * kSubInts;
+    const int o = sub_occ(md);
+    bool on = state[m].active && si[kSubOff] < kSubTries && md.nopen == 0 && (md.nel & 1) == 0 && md.n > 1 && o >= 1 &&
+              o < md.nao;
+    if (on && si[kSubPhase] != 2 && si[kSubPhase] != 4) {
+      const double* e = emo + md.o0;
+      on = (1.0 - kSubRhoMin) * (e[o] - e[o - 1]) >= kSubMayGap * min_gap;
+    }
+    si[kSubMay] = on ? 1 : 0;
+    run += state[m].active ? 1.0 : 0.0;
+    may += on ? 1.0 : 0.0;
+  }
+  run = block_sum<256>(run, sh);
+  may = block_sum<256>(may, sh);
+  if (threadIdx.x == 0) {
+    cnt[0] = (int)run;
+    cnt[1] = (int)may;
   }
 }
 
