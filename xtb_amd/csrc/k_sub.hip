@@ -61,11 +61,6 @@ constexpr int kSubFresh = 5;   // X starts from the first-order guess
 constexpr int kSubNext = 6;    // steps taken in this SCC iteration
 constexpr int kSubMay = 7;     // may take the path in the next SCC iteration
 constexpr int kSubInts = 8;
-// the gap of the last orbitals, in units of the one that k_sub_begin asks of
-// the diagonal, from which a molecule off the path may take it next: the
-// diagonal moves by a few percent per iteration.  Below it the iteration would
-// queue the path's launches and wait for their counts for nothing
-constexpr double kSubMayGap = 0.9;
 // residual maxima: one per step, then those of E_2 = M^4 and E_3 = M^8
 constexpr int kSubRes = kSubSteps + 2;
 
@@ -576,7 +571,10 @@ __global__ void __launch_bounds__(256) k_sub_check(const MolDesc* __restrict__ d
 
 // after an SCC iteration, cnt[0]: molecules still iterating, cnt[1]: those of
 // them that may take the path in the next one (kSubMay; closed shells with
-// occupied and virtual orbitals, on the path now or with a gap that comes near)
+// occupied and virtual orbitals, on the path now or with a gap of the last
+// orbitals that k_sub_begin would ask of the diagonal: below it the iteration
+// would queue the path's launches and wait for their counts for nothing, 8.9
+// instead of 8.2 ms for a polyene of 20 carbons, gap 1.45 eV)
 __global__ void __launch_bounds__(256) k_sub_next(const MolDesc* __restrict__ desc, const MolState* __restrict__ state,
                                                   int nmol, int* sub, const double* __restrict__ emo, double min_gap,
                                                   int* cnt) {
@@ -590,7 +588,7 @@ __global__ void __launch_bounds__(256) k_sub_next(const MolDesc* __restrict__ de
               o < md.nao;
     if (on && si[kSubPhase] != 2 && si[kSubPhase] != 4) {
       const double* e = emo + md.o0;
-      on = (1.0 - kSubRhoMin) * (e[o] - e[o - 1]) >= kSubMayGap * min_gap;
+      on = (1.0 - kSubRhoMin) * (e[o] - e[o - 1]) >= min_gap;
     }
     si[kSubMay] = on ? 1 : 0;
     run += state[m].active ? 1.0 : 0.0;
