@@ -138,8 +138,8 @@ def test_alkane_c64():
 
 
 def test_water96_device_wide_eeq():
-    """96 H2O (288 atoms, 576 AOs): the 289-unknown EEQ system is factorised
-    column by column across the device rather than in one workgroup."""
+    """96 H2O (288 atoms, 576 AOs): an EEQ system of 18 panels, whose trailing
+    updates are spread over the device."""
     xa = _engine()
     from xtb_amd import workloads as w
     z, x = w.water_cluster(96, 5)

@@ -8,9 +8,10 @@
   requests submitted in waves while others iterate; each result bitwise the
   same as the molecule alone, and against the oracle's values in
   tests/golden/serve_oracle.npz.
-* The device EEQ guess (one workgroup per molecule below 256 unknowns, column
-  by column across the device above) against the oracle's om_eeq_guess and
-  the reference's EEQ golden value for water (test/unit/test_eeq.f90:43-136).
+* The device EEQ guess (blocked Cholesky over all molecules; pivoted
+  elimination of the molecules whose matrix is not positive definite) against
+  the oracle's om_eeq_guess and the reference's EEQ golden value for water
+  (test/unit/test_eeq.f90:43-136).
 
 Tolerances: energy 1e-6 Eh, charges 1e-5 e, gradient 1e-5 Eh/bohr; iteration
 counts exact.
@@ -113,7 +114,7 @@ def test_device_eeq_guess(golden):
     g = golden["eeq_water"]
     cases = [("eeq_water", (np.array(g["numbers"]), np.array(g["positions"])), 0.0),
              ("water32", w.water_cluster(32, 0), 0.0), ("alkane20", w.alkane(20, 6), 0.0),
-             ("water96 (device-wide LU)", w.water_cluster(96, 5), 0.0),
+             ("water96 (several panels and row tiles)", w.water_cluster(96, 5), 0.0),
              ("co_cnx6", (np.array(golden["co_cnx6"]["numbers"]), np.array(golden["co_cnx6"]["positions"])), -3.0),
              ("mindless04", (np.array(golden["mindless04"]["numbers"]), np.array(golden["mindless04"]["positions"])),
               0.0)]
@@ -128,4 +129,35 @@ def test_device_eeq_guess(golden):
         assert abs(qd.sum() - c) <= 1e-10, tag
     ref, tol = g["expect"]["q[0]"]
     assert abs(b.charges(0)[0] - ref) <= tol
+    b.close()
+
+
+def test_device_eeq_guess_of_indefinite_matrices():
+    """Two hydrogens closer than 0.7 bohr make the charge-interaction matrix
+    indefinite (their 2 x 2 block already is): the Cholesky stops in its first
+    panel, in a later one or in the last, and the molecule's matrix is built
+    again and eliminated with pivoting, beside molecules whose Cholesky goes
+    through.  Tolerance as for the other guesses: the elimination's growth is
+    small at 1e-10 / 1e-16."""
+    import math
+    xa = _engine()
+    from xtb_amd import workloads as w
+    gam, alpha, r = -0.35015861, 0.55159092, 0.5   # EEQ hardness and width of hydrogen, distance in bohr
+    assert gam + math.sqrt(2.0 / math.pi) / alpha < math.erf(r / (math.sqrt(2.0) * alpha)) / r
+    h2 = np.array([[0.0, 0.0, 0.0], [0.0, 0.0, r]])
+    cases = []
+    for n, front in ((1, True), (5, False), (12, True), (30, False), (96, False)):
+        z, x = w.water_cluster(n, 5)
+        far = h2 + x.max(axis=0) + 9.0
+        for bad in (False, True):
+            zz = z if not bad else np.concatenate([[1, 1], z] if front else [z, [1, 1]])
+            xx = x if not bad else np.concatenate([far, x] if front else [x, far])
+            cases.append((zz.astype(np.int32), xx, 1.0 if n == 5 else 0.0))
+    b = xa.Batch([(z, x, c, 1 if c else 0) for z, x, c in cases])
+    b.setup()
+    for m, (z, x, c) in enumerate(cases):
+        qd = b.charges(m)
+        d = float(np.max(np.abs(qd - po.eeq(z, x, charge=c))))
+        print(f"{len(z)} atoms: max |q_device - q_oracle| = {d:.2e}", flush=True)
+        assert d <= 1e-10 and abs(qd.sum() - c) <= 1e-10, (len(z), d)
     b.close()
