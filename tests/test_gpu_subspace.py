@@ -172,6 +172,19 @@ def test_blocks_on_the_blocked_eigensolver(monkeypatch, blk_min):
         _check(x, y, f"{len(z)} atoms")
 
 
+@pytest.mark.parametrize("whole,half", [(65, 1 << 30), (1 << 30, 80), (200, 100)])
+def test_lines_of_whole_matrices_and_blocks(monkeypatch, whole, half):
+    """Whole matrices and blocks on the blocked eigensolver from lines of their
+    own."""
+    from xtb_amd import workloads as w
+    monkeypatch.setenv("XTBAMD_EIG_BLK_MIN", str(whole))
+    monkeypatch.setenv("XTBAMD_EIG_BLK_MIN_HALF", str(half))
+    mols = [w.alkane(27, 3), w.alkane(40, 3), w.water_cluster(23, 5)]
+    (a, _), (b, _) = _both(monkeypatch, mols)
+    for (z, _), x, y in zip(mols, a, b):
+        _check(x, y, f"{len(z)} atoms")
+
+
 def test_orthogonalisation_over_the_spectrum():
     """S^(-1/2) from S = I (two atoms far apart: every eigenvalue at one end of
     the interval that the scaled steps expect) to eigenvalues far below it

@@ -417,8 +417,12 @@ class Batch {
   // problems of at least this dimension go to the blocked eigensolver
   // (tridiagonalisation, divide and conquer, back-transformation) instead of
   // the block-Jacobi rounds; register path only.  Off unless the tuning file
-  // or XTBAMD_EIG_BLK_MIN sets it.
+  // or XTBAMD_EIG_BLK_MIN (both) / XTBAMD_EIG_BLK_MIN_HALF sets them.  Whole
+  // matrices start from orbitals of another Fock matrix, the blocks of the
+  // last diagonalisation (k_sub.hip) from nearly their own: their rounds are
+  // fewer, so their line lies higher.
   int eig_blk_min = 1 << 30;
+  int eig_blk_min_half = 1 << 30;
   // the blocked solve as a captured HIP graph (XTBAMD_GRAPH=1); off by
   // default: replaying it measured no faster than the eager launches (one
   // 4200-AO single point 1.523 against 1.514 s, its launches are bound by

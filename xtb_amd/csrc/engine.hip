@@ -867,7 +867,7 @@ static long long* cap_field(Capacity& c, int k) {
 // "off" none): "key value" lines, '#' comments.  Read once per process.
 namespace {
 struct Tuning {
-  int eig_blk_min = -1, eig_blk_iters = -1, jac_lanes = -1, jac_cross = -1, gemm_valu = -1;
+  int eig_blk_min = -1, eig_blk_min_half = -1, eig_blk_iters = -1, jac_lanes = -1, jac_cross = -1, gemm_valu = -1;
 };
 const Tuning& tuning() {
   static const Tuning t = [] {
@@ -893,6 +893,7 @@ const Tuning& tuning() {
       if (line[0] == '#' || std::sscanf(line, "%63s %63s", key, val) != 2) continue;
       const std::string k(key), v(val);
       if (k == "eig_blk_min") r.eig_blk_min = std::atoi(val);
+      else if (k == "eig_blk_min_half") r.eig_blk_min_half = std::atoi(val);
       else if (k == "eig_blk_iters") r.eig_blk_iters = std::atoi(val);
       else if (k == "jac_lanes") r.jac_lanes = std::atoi(val);
       else if (k == "jac_cross") r.jac_cross = std::atoi(val);
@@ -908,7 +909,8 @@ const Tuning& tuning() {
 void Batch::init_common() {
   // the autotuner's choices first; environment variables override them
   const Tuning& tu = tuning();
-  if (tu.eig_blk_min > 0) eig_blk_min = std::max(65, tu.eig_blk_min);
+  if (tu.eig_blk_min > 0) eig_blk_min = eig_blk_min_half = std::max(65, tu.eig_blk_min);
+  if (tu.eig_blk_min_half > 0) eig_blk_min_half = std::max(65, tu.eig_blk_min_half);
   if (tu.eig_blk_iters >= 0) eig_blk_iters = tu.eig_blk_iters;
   if (tu.jac_lanes > 0) jac_lanes = std::min(kMaxLanes, tu.jac_lanes);
   if (tu.jac_cross >= 0) jac_cross = tu.jac_cross != 0;
@@ -933,7 +935,8 @@ void Batch::init_common() {
   trace_rounds = std::getenv("XTBAMD_TRACE_ROUNDS") != nullptr;
   if (const char* r = std::getenv("XTBAMD_JAC_LANES")) jac_lanes = std::min(kMaxLanes, std::max(1, std::atoi(r)));
   if (const char* r = std::getenv("XTBAMD_JAC_SMALL")) jac_small = std::min(64, std::max(32, std::atoi(r)));
-  if (const char* r = std::getenv("XTBAMD_EIG_BLK_MIN")) eig_blk_min = std::max(65, std::atoi(r));
+  if (const char* r = std::getenv("XTBAMD_EIG_BLK_MIN")) eig_blk_min = eig_blk_min_half = std::max(65, std::atoi(r));
+  if (const char* r = std::getenv("XTBAMD_EIG_BLK_MIN_HALF")) eig_blk_min_half = std::max(65, std::atoi(r));
   if (const char* r = std::getenv("XTBAMD_SUBSPACE")) subspace_on = std::atoi(r) != 0;
   if (const char* r = std::getenv("XTBAMD_SUB_WG")) sub_wg = std::atoi(r);
   if (const char* r = std::getenv("XTBAMD_EIG_BLK_ITERS")) eig_blk_iters = std::max(0, std::atoi(r));
@@ -1383,7 +1386,7 @@ void Batch::jac_lists(JacSet& js) {
     p.small = 0;
     // the largest problems also go to the blocked eigensolver, which takes
     // them for the first eig_blk_iters SCC iterations (the lanes after)
-    const bool to_blk = blk_path && p.dim >= eig_blk_min;
+    const bool to_blk = blk_path && p.dim >= (js.half ? eig_blk_min_half : eig_blk_min);
     if (to_blk) blk.push_back(m);
     big.push_back(m);
     js.big_max_dim = std::max(js.big_max_dim, p.dim);

@@ -4,17 +4,21 @@ Times, on the device, the choices the engine leaves open and writes them to a
 tuning file that every batch reads at set-up (``tuning_gfx950.txt`` next to
 ``libxtb_amd.so``; environment variables ``XTBAMD_*`` override it):
 
-* ``eig_blk_min`` and ``eig_blk_iters``: the smallest eigenproblem
-  dimension that goes to the blocked eigensolver (Householder
+* ``eig_blk_iters``: for how many SCC iterations (from the first) large
+  eigenproblems go to the blocked eigensolver (Householder
   tridiagonalisation, divide and conquer, back-transformation) instead of
-  block-Jacobi rounds, and for how many SCC iterations (from the first; the
-  block-Jacobi rounds start from the previous orbitals after that).
-  One-molecule single points per size bin (water clusters and alkanes, up to
-  the 700-water cluster) are timed with block Jacobi, the blocked solver in
-  every iteration and in the first 2 or 4; the cutoff is the smallest bin
-  from which a blocked variant wins in every larger bin, the iteration count
-  that of the largest bin, and both are kept only if the 512-molecule batch
-  is not slower with them.
+  block-Jacobi rounds, which start from the previous orbitals after that: 2, 4
+  or all, timed on the 700-water cluster with a diagonalisation in every
+  iteration (as open shells and small gaps take it).
+* ``eig_blk_min``: the smallest dimension that goes there.  One-molecule
+  single points per size bin (water clusters and alkanes, up to the 700-water
+  cluster) with block Jacobi and with the blocked solver; the cutoff is the
+  smallest bin from which the blocked solver wins in every larger bin, kept
+  only if the 512-molecule batch is not slower with it.
+* ``eig_blk_min_half``: the same for the occupied and virtual blocks of the
+  last diagonalisation, which start nearly diagonal: the larger block of the
+  smallest bin from which the blocked solver wins in every larger bin (whole
+  matrices at their own cutoff).
 * ``jac_lanes`` (1..3) and ``jac_cross`` (0/1): the stream lanes and the
   cross-round schedule of the block-Jacobi rounds, timed on the 512-molecule
   workload.
@@ -39,7 +43,8 @@ if ROOT not in sys.path:
 
 from xtb_amd import workloads  # noqa: E402
 
-KEYS = ("XTBAMD_EIG_BLK_MIN", "XTBAMD_EIG_BLK_ITERS", "XTBAMD_JAC_LANES", "XTBAMD_JAC_CROSS", "XTBAMD_GEMM")
+KEYS = ("XTBAMD_EIG_BLK_MIN", "XTBAMD_EIG_BLK_MIN_HALF", "XTBAMD_EIG_BLK_ITERS", "XTBAMD_JAC_LANES",
+        "XTBAMD_JAC_CROSS", "XTBAMD_GEMM", "XTBAMD_SUBSPACE")
 
 
 def _set(env):
@@ -67,43 +72,62 @@ def _time_batch(mols, env, steps, warmup=1):
 
 
 def tune(steps=3, out=HERE, log=print):
-    rows_bins, rows_batch = [], []
-    # 1. eigensolver path per size bin (one molecule per batch): block Jacobi,
-    # the blocked solver in every SCC iteration, or in the first few only
+    rows_iters, rows_bins, rows_half, rows_batch = [], [], [], []
+    off = 1 << 30
     bins = [("water", 12), ("alkane", 24), ("water", 22), ("alkane", 44), ("water", 43), ("alkane", 86),
-            ("water", 64), ("water", 100), ("water", 170), ("water", 256), ("water", 400), ("water", 700)]
-    hybrid = (2, 4)
-    best_per_bin = []
-    for kind, size in bins:
+            ("water", 64), ("water", 100), ("water", 170), ("alkane", 240), ("water", 256), ("alkane", 300),
+            ("water", 300), ("water", 400), ("alkane", 500), ("water", 500), ("water", 600), ("alkane", 700),
+            ("water", 700)]
+
+    def molecule(kind, size, seed=7):
         if kind == "water" and size == 700:
-            z, x = workloads.large_water_cluster(2024)
-        else:
-            z, x = workloads.water_cluster(size, 7) if kind == "water" else workloads.alkane(size, 7)
+            return workloads.large_water_cluster(2017 + seed)
+        return workloads.water_cluster(size, seed) if kind == "water" else workloads.alkane(size, seed)
+
+    # 1. eigensolver path: the number of iterations, then the cutoff per size
+    # bin (one molecule per batch)
+    big = [molecule("water", 700)]
+    for it in (2, 4, off):
+        t, _ = _time_batch(big, {"XTBAMD_SUBSPACE": 0, "XTBAMD_EIG_BLK_MIN": 65, "XTBAMD_EIG_BLK_ITERS": it}, steps)
+        rows_iters.append((it, t))
+        log(f"tune eig: {'every iteration' if it == off else f'first {it}'} on the blocked solver {1e3 * t:.1f} ms")
+    iters = min(rows_iters, key=lambda r: r[1])[0]
+    whole = {"XTBAMD_EIG_BLK_MIN": 65, "XTBAMD_EIG_BLK_MIN_HALF": off, "XTBAMD_EIG_BLK_ITERS": iters}
+    for kind, size in bins:
+        z, x = molecule(kind, size)
         nao = workloads.ao_count(z)
-        tj, ej = _time_batch([(z, x)], {"XTBAMD_EIG_BLK_MIN": 1 << 30}, steps)
-        tb, eb = _time_batch([(z, x)], {"XTBAMD_EIG_BLK_MIN": 65}, steps)
-        th = []
-        for it in hybrid:
-            t, _ = _time_batch([(z, x)], {"XTBAMD_EIG_BLK_MIN": 65, "XTBAMD_EIG_BLK_ITERS": it}, steps)
-            th.append(t)
+        tj, ej = _time_batch([(z, x)], {"XTBAMD_EIG_BLK_MIN": off}, steps)
+        tb, eb = _time_batch([(z, x)], whole, steps)
         dE = abs(ej[0] - eb[0])
-        rows_bins.append((kind, size, nao, tj, tb, th, dE))
-        opts = {1 << 30: tb}
-        opts.update({it: t for it, t in zip(hybrid, th)})
-        it_best = min(opts, key=lambda k: opts[k])
-        best_per_bin.append((nao, opts[it_best] < tj, it_best, tj, opts))
-        log(f"tune eig: {kind} {size} nao={nao} jacobi {1e3 * tj:.1f} ms blocked {1e3 * tb:.1f} ms "
-            + " ".join(f"first-{it} {1e3 * t:.1f} ms" for it, t in zip(hybrid, th)) + f" dE={dE:.1e}")
-    best_per_bin.sort(key=lambda r: r[0])
-    # one setting for every size from the cut on: the iteration count that
-    # is best for the largest molecule, and the smallest cut from which that
-    # count beats block Jacobi at every size measured
-    cut, iters = 1 << 30, 1 << 30
-    if best_per_bin and best_per_bin[-1][1]:
-        it_l = best_per_bin[-1][2]
-        for i in range(len(best_per_bin)):
-            if all(opts[it_l] < tj for _, _, _, tj, opts in best_per_bin[i:]):
-                cut, iters = best_per_bin[i][0], it_l
+        rows_bins.append((nao, kind, size, tj, tb, dE))
+        log(f"tune eig: {kind} {size} nao={nao} jacobi {1e3 * tj:.1f} ms blocked {1e3 * tb:.1f} ms dE={dE:.1e}")
+    rows_bins.sort()
+    cut = off
+    for i in range(len(rows_bins)):
+        if all(tb < tj for _, _, _, tj, tb, _ in rows_bins[i:]):
+            cut = rows_bins[i][0]
+            break
+    # the blocks of the last diagonalisation, whole matrices at their cutoff
+    # (two geometries each: the rounds of a block differ by up to two times)
+    cut_half = off
+    if cut < off:
+        env = {"XTBAMD_EIG_BLK_MIN": cut, "XTBAMD_EIG_BLK_ITERS": iters}
+        for kind, size in (("water", 170), ("alkane", 300), ("water", 300), ("water", 400), ("alkane", 500),
+                           ("water", 500), ("alkane", 700), ("water", 550), ("water", 600), ("water", 650),
+                           ("alkane", 900), ("water", 700)):
+            tl = th = 0.0
+            for seed in (7, 8):
+                z, x = molecule(kind, size, seed)
+                occ = 4 * size if kind == "water" else 3 * size + 1
+                block = max(occ, workloads.ao_count(z) - occ)
+                tl += 0.5 * _time_batch([(z, x)], dict(env, XTBAMD_EIG_BLK_MIN_HALF=off), steps)[0]
+                th += 0.5 * _time_batch([(z, x)], dict(env, XTBAMD_EIG_BLK_MIN_HALF=block), steps)[0]
+            rows_half.append((block, kind, size, tl, th))
+            log(f"tune blocks: {kind} {size} block of {block} rows: rounds {1e3 * tl:.1f} ms blocked {1e3 * th:.1f} ms")
+        rows_half.sort()
+        for i in range(len(rows_half)):
+            if all(th < tl for *_, tl, th in rows_half[i:]):
+                cut_half = rows_half[i][0]
                 break
     # 2. batch schedule on the 512-molecule workload
     mols = workloads.mixed_batch(512, seed=2024)
@@ -111,20 +135,20 @@ def tune(steps=3, out=HERE, log=print):
     for lanes in (1, 2, 3):
         for cross in (0, 1):
             t, _ = _time_batch(mols, {"XTBAMD_JAC_LANES": lanes, "XTBAMD_JAC_CROSS": cross,
-                                      "XTBAMD_EIG_BLK_MIN": 1 << 30}, steps)
+                                      "XTBAMD_EIG_BLK_MIN": off}, steps)
             rows_batch.append((f"jac_lanes={lanes} jac_cross={cross}", t))
             log(f"tune batch: lanes {lanes} cross {cross}: {1e3 * t:.1f} ms")
             if best is None or t < best[0]:
                 best = (t, lanes, cross)
     _, lanes, cross = best
     base = {"XTBAMD_JAC_LANES": lanes, "XTBAMD_JAC_CROSS": cross}
-    tv, _ = _time_batch(mols, dict(base, XTBAMD_GEMM="valu", XTBAMD_EIG_BLK_MIN=1 << 30), steps)
-    tm, _ = _time_batch(mols, dict(base, XTBAMD_GEMM="mfma", XTBAMD_EIG_BLK_MIN=1 << 30), steps)
+    tv, _ = _time_batch(mols, dict(base, XTBAMD_GEMM="valu", XTBAMD_EIG_BLK_MIN=off), steps)
+    tm, _ = _time_batch(mols, dict(base, XTBAMD_GEMM="mfma", XTBAMD_EIG_BLK_MIN=off), steps)
     rows_batch += [("gemm=valu", tv), ("gemm=mfma", tm)]
     gemm = "valu" if tv < tm else "mfma"
     # the cutoff must not slow the batch down (its largest problems are below
     # it unless the blocked path wins there too)
-    if cut < 1 << 30:
+    if cut < off:
         tc, _ = _time_batch(mols, dict(base, XTBAMD_GEMM=gemm, XTBAMD_EIG_BLK_MIN=cut, XTBAMD_EIG_BLK_ITERS=iters),
                             steps)
         rows_batch.append((f"eig_blk_min={cut}", tc))
@@ -136,25 +160,33 @@ def tune(steps=3, out=HERE, log=print):
     stamp = time.strftime("%Y-%m-%d %H:%M:%S")
     with open(os.path.join(out, "tuning_gfx950.txt"), "w") as f:
         f.write(f"# written by python -m xtb_amd.tune ({stamp}); environment variables XTBAMD_* override\n")
-        f.write(f"eig_blk_min {cut}\neig_blk_iters {iters}\njac_lanes {lanes}\njac_cross {cross}\ngemm {gemm}\n")
+        f.write(f"eig_blk_min {cut}\neig_blk_min_half {cut_half}\neig_blk_iters {iters}\njac_lanes {lanes}\n"
+                f"jac_cross {cross}\ngemm {gemm}\n")
     with open(os.path.join(out, "autotune_gfx950.md"), "w") as f:
         f.write("# Autotuner measurements (one MI355X)\n\n")
         f.write("Command: `python -m xtb_amd.tune --out <dir>` (median of "
                 f"{steps} timed runs after one warm-up per configuration).\n\n")
-        f.write("## Eigensolver path per size (one molecule per batch, whole single point)\n\n")
-        f.write("| molecule | AOs | block Jacobi ms | blocked, every iteration ms | "
-                + " | ".join(f"blocked, first {it} iterations ms" for it in hybrid)
-                + " | dE Jacobi vs blocked (Eh) |\n|---|---:|---:|---:|" + "---:|" * len(hybrid) + "---:|\n")
-        for kind, size, nao, tj, tb, th, dE in rows_bins:
+        f.write("## SCC iterations on the blocked solver ((H2O)700, a diagonalisation in every iteration)\n\n"
+                "| iterations | ms |\n|---|---:|\n")
+        for it, t in rows_iters:
+            f.write(f"| {'all' if it == off else f'first {it}'} | {1e3 * t:.1f} |\n")
+        f.write("\n## Eigensolver path per size (one molecule per batch, whole single point)\n\n")
+        f.write("| molecule | AOs | block Jacobi ms | blocked ms | dE (Eh) |\n|---|---:|---:|---:|---:|\n")
+        for nao, kind, size, tj, tb, dE in rows_bins:
             name = f"(H2O){size}" if kind == "water" else f"C{size}H{2 * size + 2}"
-            f.write(f"| {name} | {nao} | {1e3 * tj:.1f} | {1e3 * tb:.1f} | "
-                    + " | ".join(f"{1e3 * t:.1f}" for t in th) + f" | {dE:.1e} |\n")
+            f.write(f"| {name} | {nao} | {1e3 * tj:.1f} | {1e3 * tb:.1f} | {dE:.1e} |\n")
+        f.write("\n## Blocks of the last diagonalisation (whole matrices at their cutoff; mean of two geometries)\n\n"
+                "| larger block (rows) | molecule | block Jacobi ms | blocked ms |\n|---:|---|---:|---:|\n")
+        for block, kind, size, tl, th in rows_half:
+            name = f"(H2O){size}" if kind == "water" else f"C{size}H{2 * size + 2}"
+            f.write(f"| {block} | {name} | {1e3 * tl:.1f} | {1e3 * th:.1f} |\n")
         f.write("\n## 512-molecule batch (ms per batched step)\n\n| configuration | ms |\n|---|---:|\n")
         for name, t in rows_batch:
             f.write(f"| {name} | {1e3 * t:.1f} |\n")
-        f.write(f"\nChosen: eig_blk_min {cut}, eig_blk_iters {iters}, jac_lanes {lanes}, jac_cross {cross}, "
-                f"gemm {gemm}.\n")
-    return {"eig_blk_min": cut, "eig_blk_iters": iters, "jac_lanes": lanes, "jac_cross": cross, "gemm": gemm}
+        f.write(f"\nChosen: eig_blk_min {cut}, eig_blk_min_half {cut_half}, eig_blk_iters {iters}, "
+                f"jac_lanes {lanes}, jac_cross {cross}, gemm {gemm}.\n")
+    return {"eig_blk_min": cut, "eig_blk_min_half": cut_half, "eig_blk_iters": iters, "jac_lanes": lanes,
+            "jac_cross": cross, "gemm": gemm}
 
 
 def main(argv=None):
