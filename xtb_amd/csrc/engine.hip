@@ -1869,7 +1869,9 @@ void eig_set_build(EigSet& es, const std::vector<int>& dims, EigMem& mem, const 
     es.maxn = std::max(es.maxn, e.n);
     es.maxdepth = std::max(es.maxdepth, depth);
   }
-  es.npanel = (es.maxn - 1 + kEigNb - 1) / kEigNb;
+  // the panels hold all n columns: the last diagonal entry is that of the
+  // row which starts column n - 1, also where that column starts a panel
+  es.npanel = (es.maxn + kEigNb - 1) / kEigNb;
   es.nblk = (es.maxn - 1 + kBtNb - 1) / kBtNb;
   work(es.Aw, 0, lend ? lend->Aw : nullptr, mat);
   work(es.Vh, 1, lend ? lend->Vh : nullptr, mat);
