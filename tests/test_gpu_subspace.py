@@ -172,12 +172,15 @@ def test_blocks_on_the_blocked_eigensolver(monkeypatch, blk_min):
         _check(x, y, f"{len(z)} atoms")
 
 
-@pytest.mark.parametrize("whole,half", [(65, 1 << 30), (1 << 30, 80), (200, 100)])
-def test_lines_of_whole_matrices_and_blocks(monkeypatch, whole, half):
-    """Whole matrices and blocks on the blocked eigensolver from lines of their
-    own."""
+@pytest.mark.parametrize("first,whole,half", [(65, 65, 1 << 30), (1 << 30, 1 << 30, 80), (200, 200, 100),
+                                              (65, 1 << 30, 1 << 30), (1 << 30, 65, 1 << 30), (150, 200, 130)])
+def test_lines_of_whole_matrices_and_blocks(monkeypatch, first, whole, half):
+    """First and later iterations and blocks on the blocked eigensolver from
+    lines of their own; each setting with and without the subspace path, whose
+    absence keeps whole matrices in every iteration."""
     from xtb_amd import workloads as w
     monkeypatch.setenv("XTBAMD_EIG_BLK_MIN", str(whole))
+    monkeypatch.setenv("XTBAMD_EIG_BLK_MIN_FIRST", str(first))
     monkeypatch.setenv("XTBAMD_EIG_BLK_MIN_HALF", str(half))
     mols = [w.alkane(27, 3), w.alkane(40, 3), w.water_cluster(23, 5)]
     (a, _), (b, _) = _both(monkeypatch, mols)

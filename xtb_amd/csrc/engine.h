@@ -169,7 +169,7 @@ struct GemmJob;
 // least Batch::eig_blk_min): work arrays, the divide and conquer trees and
 // the product job lists, built by Batch::rebuild().
 struct EigSet {
-  int np = 0, maxn = 0, npanel = 0, maxdepth = 0;
+  int np = 0, maxn = 0, minn = 0, npanel = 0, maxdepth = 0;
   std::vector<int> mols;                 // Jacobi problem (batch slot) of each problem
   std::vector<int> zfin;                 // buffer (0/1) of each problem's final eigenvectors
   std::vector<long long> v_off;          // each problem's vector block in vec
@@ -208,6 +208,7 @@ struct EigSet {
   bool use_graph = false;
   hipGraphExec_t graph = nullptr;
   const void* graph_key[5] = {};
+  int graph_min_n = 0;
 };
 
 // Device memory, streams, events and a host word buffer lent to a Batch: a
@@ -234,10 +235,11 @@ void eig_set_build(EigSet& es, const std::vector<int>& dims, EigMem& mem, const 
 // the blocked eigensolver on es's problems: problem k's matrix is read from
 // Am at jprobs[es.mols[k]] (a_off, ld), its eigenvalues are written to Am's
 // diagonal and its eigenvectors as rows of Wm (w_off, ld); jstate gets the
-// done / failed flags (kJacState ints per problem); mstate (optional) skips
+// done / failed flags (kJacState ints per problem); problems below min_n rows
+// are left out; mstate (optional) skips
 // molecules that no longer iterate
-void eig_set_run(EigSet& es, const JacobiProb* jprobs, int* jstate, const MolState* mstate, double* Am, double* Wm,
-                 hipStream_t s);
+void eig_set_run(EigSet& es, const JacobiProb* jprobs, int* jstate, const MolState* mstate, int min_n, double* Am,
+                 double* Wm, hipStream_t s);
 
 class Batch {
  public:
@@ -417,11 +419,13 @@ class Batch {
   // problems of at least this dimension go to the blocked eigensolver
   // (tridiagonalisation, divide and conquer, back-transformation) instead of
   // the block-Jacobi rounds; register path only.  Off unless the tuning file
-  // or XTBAMD_EIG_BLK_MIN (both) / XTBAMD_EIG_BLK_MIN_HALF sets them.  Whole
-  // matrices start from orbitals of another Fock matrix, the blocks of the
-  // last diagonalisation (k_sub.hip) from nearly their own: their rounds are
-  // fewer, so their line lies higher.
+  // or XTBAMD_EIG_BLK_MIN (all three), _FIRST and _HALF set them.  The first
+  // SCC iteration diagonalises from unrelated orbitals, the next ones from
+  // the previous orbitals and the blocks of the last diagonalisation
+  // (k_sub.hip) from nearly their own: their rounds are fewer, so their lines
+  // lie higher.
   int eig_blk_min = 1 << 30;
+  int eig_blk_min_first = 1 << 30;
   int eig_blk_min_half = 1 << 30;
   // the blocked solve as a captured HIP graph (XTBAMD_GRAPH=1); off by
   // default: replaying it measured no faster than the eager launches (one
@@ -472,7 +476,7 @@ class Batch {
   void eig_build(EigSet& es, const JacSet& js);
   // the blocked eigensolver on the set's problems: A from Am (Jacobi problem
   // layout), eigenvalues onto Am's diagonal, eigenvector rows into Wm
-  void eig_blocked(EigSet& es, const JacSet& js, double* Am, double* Wm, bool check_active, hipStream_t s);
+  void eig_blocked(EigSet& es, const JacSet& js, double* Am, double* Wm, bool check_active, int min_n, hipStream_t s);
   // returns true when W comes out as rows (row j = eigenvector j)
   void jacobi_lanes(JacSet& js, double* Am, double* Wm);
   bool jacobi(JacSet& js, double* Am, double* Wm, double* evout, bool check_active, bool keep_w = false,

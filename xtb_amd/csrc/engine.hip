@@ -867,7 +867,7 @@ static long long* cap_field(Capacity& c, int k) {
 // "off" none): "key value" lines, '#' comments.  Read once per process.
 namespace {
 struct Tuning {
-  int eig_blk_min = -1, eig_blk_min_half = -1, eig_blk_iters = -1, jac_lanes = -1, jac_cross = -1, gemm_valu = -1;
+  int eig_blk_min = -1, eig_blk_min_first = -1, eig_blk_min_half = -1, eig_blk_iters = -1, jac_lanes = -1, jac_cross = -1, gemm_valu = -1;
 };
 const Tuning& tuning() {
   static const Tuning t = [] {
@@ -893,6 +893,7 @@ const Tuning& tuning() {
       if (line[0] == '#' || std::sscanf(line, "%63s %63s", key, val) != 2) continue;
       const std::string k(key), v(val);
       if (k == "eig_blk_min") r.eig_blk_min = std::atoi(val);
+      else if (k == "eig_blk_min_first") r.eig_blk_min_first = std::atoi(val);
       else if (k == "eig_blk_min_half") r.eig_blk_min_half = std::atoi(val);
       else if (k == "eig_blk_iters") r.eig_blk_iters = std::atoi(val);
       else if (k == "jac_lanes") r.jac_lanes = std::atoi(val);
@@ -909,7 +910,9 @@ const Tuning& tuning() {
 void Batch::init_common() {
   // the autotuner's choices first; environment variables override them
   const Tuning& tu = tuning();
-  if (tu.eig_blk_min > 0) eig_blk_min = eig_blk_min_half = std::max(65, tu.eig_blk_min);
+  auto blk_all = [&](int n) { eig_blk_min = eig_blk_min_first = eig_blk_min_half = std::max(65, n); };
+  if (tu.eig_blk_min > 0) blk_all(tu.eig_blk_min);
+  if (tu.eig_blk_min_first > 0) eig_blk_min_first = std::max(65, tu.eig_blk_min_first);
   if (tu.eig_blk_min_half > 0) eig_blk_min_half = std::max(65, tu.eig_blk_min_half);
   if (tu.eig_blk_iters >= 0) eig_blk_iters = tu.eig_blk_iters;
   if (tu.jac_lanes > 0) jac_lanes = std::min(kMaxLanes, tu.jac_lanes);
@@ -935,7 +938,8 @@ void Batch::init_common() {
   trace_rounds = std::getenv("XTBAMD_TRACE_ROUNDS") != nullptr;
   if (const char* r = std::getenv("XTBAMD_JAC_LANES")) jac_lanes = std::min(kMaxLanes, std::max(1, std::atoi(r)));
   if (const char* r = std::getenv("XTBAMD_JAC_SMALL")) jac_small = std::min(64, std::max(32, std::atoi(r)));
-  if (const char* r = std::getenv("XTBAMD_EIG_BLK_MIN")) eig_blk_min = eig_blk_min_half = std::max(65, std::atoi(r));
+  if (const char* r = std::getenv("XTBAMD_EIG_BLK_MIN")) blk_all(std::atoi(r));
+  if (const char* r = std::getenv("XTBAMD_EIG_BLK_MIN_FIRST")) eig_blk_min_first = std::max(65, std::atoi(r));
   if (const char* r = std::getenv("XTBAMD_EIG_BLK_MIN_HALF")) eig_blk_min_half = std::max(65, std::atoi(r));
   if (const char* r = std::getenv("XTBAMD_SUBSPACE")) subspace_on = std::atoi(r) != 0;
   if (const char* r = std::getenv("XTBAMD_SUB_WG")) sub_wg = std::atoi(r);
@@ -1386,7 +1390,7 @@ void Batch::jac_lists(JacSet& js) {
     p.small = 0;
     // the largest problems also go to the blocked eigensolver, which takes
     // them for the first eig_blk_iters SCC iterations (the lanes after)
-    const bool to_blk = blk_path && p.dim >= (js.half ? eig_blk_min_half : eig_blk_min);
+    const bool to_blk = blk_path && p.dim >= (js.half ? eig_blk_min_half : std::min(eig_blk_min, eig_blk_min_first));
     if (to_blk) blk.push_back(m);
     big.push_back(m);
     js.big_max_dim = std::max(js.big_max_dim, p.dim);
@@ -1674,13 +1678,14 @@ bool Batch::jacobi(JacSet& js, double* Am, double* Wm, double* evout, bool check
   // the largest problems go to the blocked eigensolver on stream3 (after the
   // small ones), beside the lanes
   EigSet& es = js.half ? eig_h_ : eig_;
-  const bool blk = rows && !pivot_lds && es.np > 0 &&
+  const int blk_n = js.half ? eig_blk_min_half : iterations_ == 0 ? eig_blk_min_first : eig_blk_min;
+  const bool blk = rows && !pivot_lds && es.np > 0 && es.maxn >= blk_n &&
                    (iterations_ < eig_blk_iters || (final_ && eig_blk_iters > 0));
   // the blocked path's problems are marked done for the lanes
   if (blk)
-    hipLaunchKernelGGL(k_eig_claim, dim3(1), dim3(256), 0, stream, (const EigProb*)es.d_probs, es.np, js.state);
+    hipLaunchKernelGGL(k_eig_claim, dim3(1), dim3(256), 0, stream, (const EigProb*)es.d_probs, es.np, blk_n, js.state);
   // the lanes test their progress once per period of their largest problem
-  jac_period_ = blk ? std::max(1, js.max_rounds_lanes) : js.max_rounds;
+  jac_period_ = blk && es.minn >= blk_n ? std::max(1, js.max_rounds_lanes) : js.max_rounds;
   const bool forked = lanes || blk;
   // the small problems (one workgroup each, k_jac_small) run
   // on stream3 beside the lanes
@@ -1696,7 +1701,7 @@ bool Batch::jacobi(JacSet& js, double* Am, double* Wm, double* evout, bool check
   if (js.nsmall)
     hipLaunchKernelGGL(k_jac_small, dim3(js.nsmall), dim3(256), 0, forked ? stream3 : stream, js.d_probs, js.d_small,
                        Am, Wm, (const double*)js.scale, js.state, keep_w ? 1 : 0, rows ? 1 : 0, jac_tol);
-  if (blk) eig_blocked(es, js, Am, Wm, check_active, stream3);
+  if (blk) eig_blocked(es, js, Am, Wm, check_active, blk_n, stream3);
   if (forked) {
     if (lanes) jacobi_lanes(js, Am, Wm);
     auto join = [&](hipEvent_t ev, hipStream_t s) {
@@ -1836,6 +1841,7 @@ void eig_set_build(EigSet& es, const std::vector<int>& dims, EigMem& mem, const 
   es.v_off.clear();
   es.ld.clear();
   es.maxn = 0;
+  es.minn = 1 << 30;
   es.maxdepth = 0;
   for (int k = 0; k < es.np; ++k) {
     EigProb& e = probs[k];
@@ -1867,6 +1873,7 @@ void eig_set_build(EigSet& es, const std::vector<int>& dims, EigMem& mem, const 
     while (((e.n + (1 << depth) - 1) >> depth) > kDcLeaf) ++depth;
     e.depth = depth;
     es.maxn = std::max(es.maxn, e.n);
+    es.minn = std::min(es.minn, e.n);
     es.maxdepth = std::max(es.maxdepth, depth);
   }
   // the panels hold all n columns: the last diagonal entry is that of the
@@ -2056,38 +2063,40 @@ void eig_set_build(EigSet& es, const std::vector<int>& dims, EigMem& mem, const 
   HIPCHECK(hipMemset(es.P, 0, (size_t)std::max(1LL, pp) * sizeof(double)));
 }
 
-void Batch::eig_blocked(EigSet& es, const JacSet& js, double* Am, double* Wm, bool check_active, hipStream_t s) {
-  eig_set_run(es, js.d_probs, js.state, check_active ? (const MolState*)d_state : (const MolState*)nullptr, Am, Wm,
-              s);
+void Batch::eig_blocked(EigSet& es, const JacSet& js, double* Am, double* Wm, bool check_active, int min_n,
+                        hipStream_t s) {
+  eig_set_run(es, js.d_probs, js.state, check_active ? (const MolState*)d_state : (const MolState*)nullptr, min_n, Am,
+              Wm, s);
 }
 
-static void eig_set_launch(EigSet& es, const JacobiProb* jprobs, int* jstate, const MolState* mstate, double* Am,
-                           double* Wm, hipStream_t s);
+static void eig_set_launch(EigSet& es, const JacobiProb* jprobs, int* jstate, const MolState* mstate, int min_n,
+                           double* Am, double* Wm, hipStream_t s);
 
-void eig_set_run(EigSet& es, const JacobiProb* jprobs, int* jstate, const MolState* mstate, double* Am, double* Wm,
-                 hipStream_t s) {
+void eig_set_run(EigSet& es, const JacobiProb* jprobs, int* jstate, const MolState* mstate, int min_n, double* Am,
+                 double* Wm, hipStream_t s) {
   if (!es.use_graph || es.np == 0) {
-    eig_set_launch(es, jprobs, jstate, mstate, Am, Wm, s);
+    eig_set_launch(es, jprobs, jstate, mstate, min_n, Am, Wm, s);
     return;
   }
   const void* key[5] = {jprobs, jstate, mstate, Am, Wm};
-  if (!es.graph || !std::equal(key, key + 5, es.graph_key)) {
+  if (!es.graph || !std::equal(key, key + 5, es.graph_key) || es.graph_min_n != min_n) {
     if (es.graph) HIPCHECK(hipGraphExecDestroy(es.graph));
     es.graph = nullptr;
     hipGraph_t g = nullptr;
     HIPCHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-    eig_set_launch(es, jprobs, jstate, mstate, Am, Wm, s);
+    eig_set_launch(es, jprobs, jstate, mstate, min_n, Am, Wm, s);
     HIPCHECK(hipStreamEndCapture(s, &g));
     const hipError_t e = hipGraphInstantiate(&es.graph, g, nullptr, nullptr, 0);
     (void)hipGraphDestroy(g);
     HIPCHECK(e);
     std::copy(key, key + 5, es.graph_key);
+    es.graph_min_n = min_n;
   }
   HIPCHECK(hipGraphLaunch(es.graph, s));
 }
 
-static void eig_set_launch(EigSet& es, const JacobiProb* jprobs, int* jstate, const MolState* mstate, double* Am,
-                           double* Wm, hipStream_t s) {
+static void eig_set_launch(EigSet& es, const JacobiProb* jprobs, int* jstate, const MolState* mstate, int min_n,
+                           double* Am, double* Wm, hipStream_t s) {
   const int np = es.np;
   auto gemm_launch = [&](const EigSet::Launch& L, bool ta, bool tb) {
     if (L.ntile == 0) return;
@@ -2100,7 +2109,7 @@ static void eig_set_launch(EigSet& es, const JacobiProb* jprobs, int* jstate, co
   };
   const long long nn = (long long)es.maxn * es.maxn;
   hipLaunchKernelGGL(k_eig_in, dim3(gstride(nn), np), dim3(256), 0, s, (const EigProb*)es.d_probs, jprobs, mstate,
-                     es.act, (const double*)Am, es.Aw);
+                     min_n, es.act, (const double*)Am, es.Aw);
   // 1. tridiagonalisation
   const int nmax = es.maxn;
   for (int pi = 0; pi < es.npanel; ++pi) {
@@ -3792,7 +3801,7 @@ int xtbamd_eigh(int nprob, const int* n, const double* a, double* evals, double*
     xtbamd::EigSet es;
     for (int k = 0; k < nprob; ++k) es.mols.push_back(k);
     xtbamd::eig_set_build(es, dims, mem);
-    xtbamd::eig_set_run(es, djp, dst, nullptr, dA, dW, nullptr);
+    xtbamd::eig_set_run(es, djp, dst, nullptr, 0, dA, dW, nullptr);
     HIPCHECK(hipDeviceSynchronize());
     std::vector<double> h((size_t)off);
     HIPCHECK(hipMemcpy(h.data(), dA, off * sizeof(double), hipMemcpyDeviceToHost));

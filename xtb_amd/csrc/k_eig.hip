@@ -908,19 +908,21 @@ __global__ void __launch_bounds__(256) k_trd_tblock(const EigProb* __restrict__ 
       for (int b = 0; b < kBtNb; ++b) To[(long long)tid * tw + c * kBtNb + b] = To[(long long)tid * tw + b];
 }
 
-// the blocked path's problems are done for the block-Jacobi lanes
-__global__ void k_eig_claim(const EigProb* __restrict__ probs, int np, int* jstate) {
-  for (int k = threadIdx.x; k < np; k += blockDim.x) jstate[probs[k].mol * kJacState] = 1;
+// the blocked path's problems (of at least min_n rows) are done for the
+// block-Jacobi lanes
+__global__ void k_eig_claim(const EigProb* __restrict__ probs, int np, int min_n, int* jstate) {
+  for (int k = threadIdx.x; k < np; k += blockDim.x)
+    if (probs[k].n >= min_n) jstate[probs[k].mol * kJacState] = 1;
 }
 
 // the problems' matrices into the solver's layout (problems of molecules
-// that are not diagonalised are switched off)
+// that are not diagonalised and those below min_n rows are switched off)
 __global__ void __launch_bounds__(256) k_eig_in(const EigProb* __restrict__ probs, const JacobiProb* __restrict__ jp,
-                                                const MolState* __restrict__ mstate, int* act,
+                                                const MolState* __restrict__ mstate, int min_n, int* act,
                                                 const double* __restrict__ Asrc, double* Aw) {
   const EigProb p = probs[blockIdx.y];
   const JacobiProb q = jp[p.mol];
-  const bool on = !mstate || mstate[q.mol].diag;
+  const bool on = p.n >= min_n && (!mstate || mstate[q.mol].diag);
   if (blockIdx.x == 0 && threadIdx.x == 0) act[blockIdx.y] = on ? 1 : 0;
   if (!on) return;
   const int n = p.n;

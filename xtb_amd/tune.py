@@ -4,21 +4,20 @@ Times, on the device, the choices the engine leaves open and writes them to a
 tuning file that every batch reads at set-up (``tuning_gfx950.txt`` next to
 ``libxtb_amd.so``; environment variables ``XTBAMD_*`` override it):
 
-* ``eig_blk_iters``: for how many SCC iterations (from the first) large
-  eigenproblems go to the blocked eigensolver (Householder
+* the smallest eigenproblems that go to the blocked eigensolver (Householder
   tridiagonalisation, divide and conquer, back-transformation) instead of
-  block-Jacobi rounds, which start from the previous orbitals after that: 2, 4
-  or all, timed on the 700-water cluster with a diagonalisation in every
-  iteration (as open shells and small gaps take it).
-* ``eig_blk_min``: the smallest dimension that goes there.  One-molecule
-  single points per size bin (water clusters and alkanes, up to the 700-water
-  cluster) with block Jacobi and with the blocked solver; the cutoff is the
-  smallest bin from which the blocked solver wins in every larger bin, kept
-  only if the 512-molecule batch is not slower with it.
-* ``eig_blk_min_half``: the same for the occupied and virtual blocks of the
-  last diagonalisation, which start nearly diagonal: the larger block of the
-  smallest bin from which the blocked solver wins in every larger bin (whole
-  matrices at their own cutoff).
+  block-Jacobi rounds; each line is the smallest size from which the blocked
+  solver wins at every larger one:
+  ``eig_blk_min_first``, the first SCC iteration (unrelated orbitals to start
+  from), one-molecule single points of water clusters and alkanes, kept only
+  if the 512-molecule batch is not slower with it;
+  ``eig_blk_min``, the next iterations up to ``eig_blk_iters`` (2 or 4, or
+  all; timed on the 700-water cluster with a diagonalisation in every
+  iteration, as open shells and small gaps take it): the mean of a water
+  cluster and an alkane, with a diagonalisation in every iteration and on the
+  subspace path, which falls back to some;
+  ``eig_blk_min_half``, the occupied and virtual blocks of the last
+  diagonalisation, which start nearly diagonal (the size of the larger block).
 * ``jac_lanes`` (1..3) and ``jac_cross`` (0/1): the stream lanes and the
   cross-round schedule of the block-Jacobi rounds, timed on the 512-molecule
   workload.
@@ -43,8 +42,8 @@ if ROOT not in sys.path:
 
 from xtb_amd import workloads  # noqa: E402
 
-KEYS = ("XTBAMD_EIG_BLK_MIN", "XTBAMD_EIG_BLK_MIN_HALF", "XTBAMD_EIG_BLK_ITERS", "XTBAMD_JAC_LANES",
-        "XTBAMD_JAC_CROSS", "XTBAMD_GEMM", "XTBAMD_SUBSPACE")
+KEYS = ("XTBAMD_EIG_BLK_MIN", "XTBAMD_EIG_BLK_MIN_FIRST", "XTBAMD_EIG_BLK_MIN_HALF", "XTBAMD_EIG_BLK_ITERS",
+        "XTBAMD_JAC_LANES", "XTBAMD_JAC_CROSS", "XTBAMD_GEMM", "XTBAMD_SUBSPACE")
 
 
 def _set(env):
@@ -72,7 +71,7 @@ def _time_batch(mols, env, steps, warmup=1):
 
 
 def tune(steps=3, out=HERE, log=print):
-    rows_iters, rows_bins, rows_half, rows_batch = [], [], [], []
+    rows_iters, rows_next, rows_bins, rows_half, rows_batch = [], [], [], [], []
     off = 1 << 30
     bins = [("water", 12), ("alkane", 24), ("water", 22), ("alkane", 44), ("water", 43), ("alkane", 86),
             ("water", 64), ("water", 100), ("water", 170), ("alkane", 240), ("water", 256), ("alkane", 300),
@@ -84,34 +83,48 @@ def tune(steps=3, out=HERE, log=print):
             return workloads.large_water_cluster(2017 + seed)
         return workloads.water_cluster(size, seed) if kind == "water" else workloads.alkane(size, seed)
 
-    # 1. eigensolver path: the number of iterations, then the cutoff per size
-    # bin (one molecule per batch)
+    def line(rows):
+        """smallest size from which the blocked solver wins in every larger bin"""
+        rows.sort()
+        for i in range(len(rows)):
+            if all(tb < tj for *_, tj, tb in rows[i:]):
+                return rows[i][0]
+        return off
+
+    # 1. eigensolver path: iterations after the first, a diagonalisation in each
     big = [molecule("water", 700)]
     for it in (2, 4, off):
         t, _ = _time_batch(big, {"XTBAMD_SUBSPACE": 0, "XTBAMD_EIG_BLK_MIN": 65, "XTBAMD_EIG_BLK_ITERS": it}, steps)
         rows_iters.append((it, t))
         log(f"tune eig: {'every iteration' if it == off else f'first {it}'} on the blocked solver {1e3 * t:.1f} ms")
     iters = min(rows_iters, key=lambda r: r[1])[0]
-    whole = {"XTBAMD_EIG_BLK_MIN": 65, "XTBAMD_EIG_BLK_MIN_HALF": off, "XTBAMD_EIG_BLK_ITERS": iters}
+    for size in (300, 400, 500, 600, 700):   # 6 AOs per water and per carbon
+        tj = tb = 0.0
+        for kind in ("water", "alkane"):
+            z, x = molecule(kind, size)
+            for sub in (0, 1):
+                env = {"XTBAMD_SUBSPACE": sub, "XTBAMD_EIG_BLK_ITERS": iters, "XTBAMD_EIG_BLK_MIN_FIRST": 65,
+                       "XTBAMD_EIG_BLK_MIN_HALF": off}
+                tj += 0.25 * _time_batch([(z, x)], dict(env, XTBAMD_EIG_BLK_MIN=off), steps)[0]
+                tb += 0.25 * _time_batch([(z, x)], dict(env, XTBAMD_EIG_BLK_MIN=65), steps)[0]
+        rows_next.append((6 * size, tj, tb))
+        log(f"tune eig: {6 * size} AOs first iteration blocked {1e3 * tj:.1f} ms, also the next {1e3 * tb:.1f} ms")
+    cut_next = line(rows_next)
+    # the first iteration (one molecule per batch)
     for kind, size in bins:
         z, x = molecule(kind, size)
-        nao = workloads.ao_count(z)
         tj, ej = _time_batch([(z, x)], {"XTBAMD_EIG_BLK_MIN": off}, steps)
-        tb, eb = _time_batch([(z, x)], whole, steps)
+        tb, eb = _time_batch([(z, x)], {"XTBAMD_EIG_BLK_MIN": off, "XTBAMD_EIG_BLK_MIN_FIRST": 65}, steps)
         dE = abs(ej[0] - eb[0])
-        rows_bins.append((nao, kind, size, tj, tb, dE))
-        log(f"tune eig: {kind} {size} nao={nao} jacobi {1e3 * tj:.1f} ms blocked {1e3 * tb:.1f} ms dE={dE:.1e}")
-    rows_bins.sort()
-    cut = off
-    for i in range(len(rows_bins)):
-        if all(tb < tj for _, _, _, tj, tb, _ in rows_bins[i:]):
-            cut = rows_bins[i][0]
-            break
+        rows_bins.append((workloads.ao_count(z), kind, size, dE, tj, tb))
+        log(f"tune eig: {kind} {size} nao={rows_bins[-1][0]} jacobi {1e3 * tj:.1f} ms blocked {1e3 * tb:.1f} ms "
+            f"dE={dE:.1e}")
+    cut = min(line(rows_bins), cut_next)
     # the blocks of the last diagonalisation, whole matrices at their cutoff
     # (two geometries each: the rounds of a block differ by up to two times)
     cut_half = off
     if cut < off:
-        env = {"XTBAMD_EIG_BLK_MIN": cut, "XTBAMD_EIG_BLK_ITERS": iters}
+        env = {"XTBAMD_EIG_BLK_MIN": cut_next, "XTBAMD_EIG_BLK_MIN_FIRST": cut, "XTBAMD_EIG_BLK_ITERS": iters}
         for kind, size in (("water", 170), ("alkane", 300), ("water", 300), ("water", 400), ("alkane", 500),
                            ("water", 500), ("alkane", 700), ("water", 550), ("water", 600), ("water", 650),
                            ("alkane", 900), ("water", 700)):
@@ -124,11 +137,7 @@ def tune(steps=3, out=HERE, log=print):
                 th += 0.5 * _time_batch([(z, x)], dict(env, XTBAMD_EIG_BLK_MIN_HALF=block), steps)[0]
             rows_half.append((block, kind, size, tl, th))
             log(f"tune blocks: {kind} {size} block of {block} rows: rounds {1e3 * tl:.1f} ms blocked {1e3 * th:.1f} ms")
-        rows_half.sort()
-        for i in range(len(rows_half)):
-            if all(th < tl for *_, tl, th in rows_half[i:]):
-                cut_half = rows_half[i][0]
-                break
+        cut_half = line(rows_half)
     # 2. batch schedule on the 512-molecule workload
     mols = workloads.mixed_batch(512, seed=2024)
     best = None
@@ -149,19 +158,20 @@ def tune(steps=3, out=HERE, log=print):
     # the cutoff must not slow the batch down (its largest problems are below
     # it unless the blocked path wins there too)
     if cut < off:
-        tc, _ = _time_batch(mols, dict(base, XTBAMD_GEMM=gemm, XTBAMD_EIG_BLK_MIN=cut, XTBAMD_EIG_BLK_ITERS=iters),
+        tc, _ = _time_batch(mols, dict(base, XTBAMD_GEMM=gemm, XTBAMD_EIG_BLK_MIN=cut),
                             steps)
-        rows_batch.append((f"eig_blk_min={cut}", tc))
+        rows_batch.append((f"eig_blk_min_first={cut}", tc))
         if tc > min(tv, tm):
-            rows_batch.append((f"eig_blk_min={cut} rejected for the batch", tc))
+            rows_batch.append((f"eig_blk_min_first={cut} rejected for the batch", tc))
             cut = max(cut, 1 + max(workloads.ao_count(z) for z, _ in mols))
     _set({})
     os.environ.pop("XTBAMD_TUNING", None)
     stamp = time.strftime("%Y-%m-%d %H:%M:%S")
     with open(os.path.join(out, "tuning_gfx950.txt"), "w") as f:
         f.write(f"# written by python -m xtb_amd.tune ({stamp}); environment variables XTBAMD_* override\n")
-        f.write(f"eig_blk_min {cut}\neig_blk_min_half {cut_half}\neig_blk_iters {iters}\njac_lanes {lanes}\n"
-                f"jac_cross {cross}\ngemm {gemm}\n")
+        f.write(f"eig_blk_min {cut_next}\neig_blk_min_first {cut}\neig_blk_min_half {cut_half}\n"
+                f"eig_blk_iters {iters}\n"
+                f"jac_lanes {lanes}\njac_cross {cross}\ngemm {gemm}\n")
     with open(os.path.join(out, "autotune_gfx950.md"), "w") as f:
         f.write("# Autotuner measurements (one MI355X)\n\n")
         f.write("Command: `python -m xtb_amd.tune --out <dir>` (median of "
@@ -170,23 +180,27 @@ def tune(steps=3, out=HERE, log=print):
                 "| iterations | ms |\n|---|---:|\n")
         for it, t in rows_iters:
             f.write(f"| {'all' if it == off else f'first {it}'} | {1e3 * t:.1f} |\n")
-        f.write("\n## Eigensolver path per size (one molecule per batch, whole single point)\n\n")
+        name = lambda kind, size: f"(H2O){size}" if kind == "water" else f"C{size}H{2 * size + 2}"
+        f.write("\n## Iterations after the first, up to that number (mean of a water cluster and an alkane, with a\n"
+                "diagonalisation in every iteration and on the subspace path)\n\n"
+                "| AOs | block Jacobi ms | blocked ms |\n|---:|---:|---:|\n")
+        for nao, tj, tb in rows_next:
+            f.write(f"| {nao} | {1e3 * tj:.1f} | {1e3 * tb:.1f} |\n")
+        f.write("\n## First iteration (one molecule per batch, whole single point)\n\n")
         f.write("| molecule | AOs | block Jacobi ms | blocked ms | dE (Eh) |\n|---|---:|---:|---:|---:|\n")
-        for nao, kind, size, tj, tb, dE in rows_bins:
-            name = f"(H2O){size}" if kind == "water" else f"C{size}H{2 * size + 2}"
-            f.write(f"| {name} | {nao} | {1e3 * tj:.1f} | {1e3 * tb:.1f} | {dE:.1e} |\n")
+        for nao, kind, size, dE, tj, tb in rows_bins:
+            f.write(f"| {name(kind, size)} | {nao} | {1e3 * tj:.1f} | {1e3 * tb:.1f} | {dE:.1e} |\n")
         f.write("\n## Blocks of the last diagonalisation (whole matrices at their cutoff; mean of two geometries)\n\n"
                 "| larger block (rows) | molecule | block Jacobi ms | blocked ms |\n|---:|---|---:|---:|\n")
         for block, kind, size, tl, th in rows_half:
-            name = f"(H2O){size}" if kind == "water" else f"C{size}H{2 * size + 2}"
-            f.write(f"| {block} | {name} | {1e3 * tl:.1f} | {1e3 * th:.1f} |\n")
+            f.write(f"| {block} | {name(kind, size)} | {1e3 * tl:.1f} | {1e3 * th:.1f} |\n")
         f.write("\n## 512-molecule batch (ms per batched step)\n\n| configuration | ms |\n|---|---:|\n")
-        for name, t in rows_batch:
-            f.write(f"| {name} | {1e3 * t:.1f} |\n")
-        f.write(f"\nChosen: eig_blk_min {cut}, eig_blk_min_half {cut_half}, eig_blk_iters {iters}, "
+        for conf, t in rows_batch:
+            f.write(f"| {conf} | {1e3 * t:.1f} |\n")
+        f.write(f"\nChosen: eig_blk_min {cut_next}, eig_blk_min_first {cut}, eig_blk_min_half {cut_half}, eig_blk_iters {iters}, "
                 f"jac_lanes {lanes}, jac_cross {cross}, gemm {gemm}.\n")
-    return {"eig_blk_min": cut, "eig_blk_min_half": cut_half, "eig_blk_iters": iters, "jac_lanes": lanes,
-            "jac_cross": cross, "gemm": gemm}
+    return {"eig_blk_min": cut_next, "eig_blk_min_first": cut, "eig_blk_min_half": cut_half, "eig_blk_iters": iters,
+            "jac_lanes": lanes, "jac_cross": cross, "gemm": gemm}
 
 
 def main(argv=None):
