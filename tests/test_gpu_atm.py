@@ -51,3 +51,22 @@ def test_three_body_dispersion_against_oracle(sizes):
         de = abs(r["e_disp"] - o["e_disp"])
         print(f"{len(z)} atoms: dg={dg:.2e} de={de:.2e}", flush=True)
         assert dg <= 1e-9 and de <= 1e-10, (len(z), dg, de)
+
+
+@pytest.mark.parametrize("carbons", [20, 41, 42, 43])
+def test_three_body_dispersion_beyond_the_cutoff(carbons):
+    """Chains longer than the 40 bohr cutoff of a pair, with pairs on either
+    side of it inside a block of 128 atoms and across its end (62, 125, 128 and
+    131 atoms).  With the cutoff at 41.2 bohr the oracle's energy changes by
+    9e-10 Eh for 62 atoms and 8e-7 for 125, its gradient by 4e-8 and 8e-8."""
+    import xtb_amd
+    from xtb_amd import workloads as w
+    z, x = w.alkane(carbons, 5)
+    d = np.linalg.norm(x[:, None] - x[None], axis=-1)
+    assert np.any(d > 40.0) and np.any(d[:, 0] < 40.0)
+    r = xtb_amd.singlepoint(z, x)
+    o = po.singlepoint(z, x)
+    dg = float(np.max(np.abs(r["gradient"] - o["gradient"])))
+    de = abs(r["e_disp"] - o["e_disp"])
+    print(f"{len(z)} atoms: dg={dg:.2e} de={de:.2e}", flush=True)
+    assert r["iterations"] == o["iterations"] and dg <= 1e-9 and de <= 1e-10, (len(z), dg, de)

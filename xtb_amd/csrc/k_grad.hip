@@ -440,7 +440,7 @@ __global__ void __launch_bounds__(64) k_d4_grad2(const MolDesc* __restrict__ des
 }
 
 // 1 / x and 1 / sqrt(x), x > 0, from the hardware approximations by two
-// Newton steps each
+// Newton steps each: below 0.9 eps relative (IEEE: 0.5)
 __device__ __forceinline__ double quick_rcp(double x) {
   double y = __builtin_amdgcn_rcp(x);
   y = fma(y, fma(-x, y, 1.0), y);
@@ -462,7 +462,12 @@ __device__ __forceinline__ double quick_rsqrt(double x) {
 // per pair, so that a triple takes one 1 / sqrt, one 1 / x and products (the
 // square and cube roots and seven divisions per triple took 51 ms for 2100
 // atoms, this takes 15.5; 1.9 ms for the 512-molecule batch).  A lane per atom
-// c, the atoms b < c shared out over the four waves.
+// c, the atoms b < c shared out over the four waves.  The inverse powers of
+// the three distances' product come from one 1 / sqrt of it, the square with
+// a Newton step of its own: the error of a triple against 80 bits is that of
+// IEEE square roots and divisions (2-norm over 4e5 random triples: gradient
+// 9.1e-16 and 9.1e-16, energy 8.0e-16 and 7.1e-16; with a product of three
+// 1 / sqrt 1.1e-15 and 9.1e-16).
 constexpr int kAtmB = 128;   // atoms b per LDS block
 
 __global__ void __launch_bounds__(256) k_d4_atm(const MolDesc* __restrict__ desc, const double* __restrict__ xyz,
@@ -470,7 +475,7 @@ __global__ void __launch_bounds__(256) k_d4_atm(const MolDesc* __restrict__ desc
                                                 const double* __restrict__ damp, double* grad, double* dedcn,
                                                 double* eatm) {
   __shared__ double sh[4];
-  // of the pairs (a, b): vector, r^2, 1 / r, sqrt(C6), damping, CN ratio
+  // of the pairs (a, b): vector, r^2, 1 / r^2, sqrt(C6), damping, CN ratio
   __shared__ double pb[kAtmB][8];
   const MolDesc md = desc[blockIdx.y];
   const int a = blockIdx.x;
@@ -491,7 +496,7 @@ __global__ void __launch_bounds__(256) k_d4_atm(const MolDesc* __restrict__ desc
       if (b < n && b != a) {
         for (int k = 0; k < 3; ++k) v[k] = x[3 * b + k] - ra[k];
         v[3] = v[0] * v[0] + v[1] * v[1] + v[2] * v[2];
-        v[4] = quick_rsqrt(v[3]);
+        v[4] = 1.0 / v[3];
         v[5] = S[(long long)a * n + b];
         v[6] = F[(long long)a * n + b];
         v[7] = Da[b];
@@ -501,12 +506,12 @@ __global__ void __launch_bounds__(256) k_d4_atm(const MolDesc* __restrict__ desc
     __syncthreads();
     for (int c0 = b0 / 64 * 64; c0 < n; c0 += 64) {
       const int c = c0 + lane;
-      double rik[3] = {0, 0, 0}, r2ik = 0.0, ivik = 0.0, sik = 0.0, fik = 0.0, dik = 0.0;
+      double rik[3] = {0, 0, 0}, r2ik = 0.0, iv2ik = 0.0, sik = 0.0, fik = 0.0, dik = 0.0;
       bool on = c < n && c != a;
       if (on) {
         for (int k = 0; k < 3; ++k) rik[k] = x[3 * c + k] - ra[k];
         r2ik = rik[0] * rik[0] + rik[1] * rik[1] + rik[2] * rik[2];
-        ivik = quick_rsqrt(r2ik);
+        iv2ik = 1.0 / r2ik;
         sik = S[(long long)a * n + c];
         fik = F[(long long)a * n + c];
         dik = Da[c];
@@ -521,9 +526,10 @@ __global__ void __launch_bounds__(256) k_d4_atm(const MolDesc* __restrict__ desc
         const double r2jk = d0 * d0 + d1 * d1 + d2 * d2;
         if (!on || b >= c || r2jk > cut2) continue;
         const double sjk = S[(long long)b * n + c], fjk = F[(long long)b * n + c];
-        const double ivij = v[4];
         const double c9 = -(v[5] * sik) * sjk;
-        const double inv1 = (ivij * ivik) * quick_rsqrt(r2jk), inv2 = inv1 * inv1, inv3 = inv1 * inv2;   // 1 / (r r r)^k
+        const double rrr2 = (r2ij * r2ik) * r2jk;
+        const double inv1 = quick_rsqrt(rrr2), sq = inv1 * inv1;   // 1 / (r r r)^k
+        const double inv2 = fma(sq, fma(-rrr2, sq, 1.0), sq), inv3 = inv1 * inv2;
         const double ang_fact = 0.375 * inv2 * inv3;
         const double ang = ang_fact * (r2ij + r2jk - r2ik) * (r2ij - r2jk + r2ik) * (-r2ij + r2jk + r2ik) + inv3;
         const double cralp = (v[6] * fik) * fjk;
@@ -536,8 +542,8 @@ __global__ void __launch_bounds__(256) k_d4_atm(const MolDesc* __restrict__ desc
         const double g2 = r2ik * r2ik * r2ik + r2ik * r2ik * (r2jk + r2ij) +
                           r2ik * (3.0 * r2jk * r2jk + 2.0 * r2jk * r2ij + 3.0 * r2ij * r2ij) -
                           5.0 * (r2jk - r2ij) * (r2jk - r2ij) * (r2jk + r2ij);
-        const double dGr1 = (cf * g1 + da) * (ivij * ivij);
-        const double dGr2 = (cf * g2 + da) * (ivik * ivik);
+        const double dGr1 = (cf * g1 + da) * v[4];
+        const double dGr2 = (cf * g2 + da) * iv2ik;
         for (int k = 0; k < 3; ++k) g[k] += (-dGr1 * v[k] - dGr2 * rik[k]) * kD4s9;
         const double ce = c9 * (ang * fdmp) * kD4s9;
         dcn -= ce * (v[7] + dik);
