@@ -169,16 +169,15 @@ static void sub_contraction() {
 }
 
 // who may take the path in the next iteration: not the molecules that gave up,
-// open shells, filled bases, gaps below the bound and the smallest molecules
+// open shells, filled bases and gaps far below the bound
 static void sub_next() {
   struct {
     int active, off, nopen, nel, nao, phase;
     double gap;
     bool may;
-  } cases[] = {{1, 0, 0, 32, 24, 0, 4.0, true},  {1, 0, 0, 32, 24, 0, 1.0, false}, {1, 0, 0, 32, 24, 2, 1.0, true},
-               {1, 0, 0, 32, 24, 4, 1.0, true},  {1, 1, 0, 32, 24, 3, 4.0, true},  {1, 2, 0, 32, 24, 3, 4.0, false},
-               {0, 0, 0, 32, 24, 4, 4.0, false}, {1, 0, 1, 31, 24, 0, 4.0, false}, {1, 0, 0, 48, 24, 0, 4.0, false},
-               {1, 0, 0, 26, 21, 0, 4.0, true},  {1, 0, 0, 26, 20, 0, 4.0, false}};
+  } cases[] = {{1, 0, 0, 8, 6, 0, 4.0, true},  {1, 0, 0, 8, 6, 0, 1.0, false}, {1, 0, 0, 8, 6, 2, 1.0, true},
+               {1, 0, 0, 8, 6, 4, 1.0, true},  {1, 1, 0, 8, 6, 3, 4.0, true},  {1, 2, 0, 8, 6, 3, 4.0, false},
+               {0, 0, 0, 8, 6, 4, 4.0, false}, {1, 0, 1, 7, 6, 0, 4.0, false}, {1, 0, 0, 12, 6, 0, 4.0, false}};
   for (auto& c : cases) {
     MolDesc md;
     MolState st;

@@ -1215,6 +1215,11 @@ void Batch::grow(T_*& ptr, long long& capv, long long need) {
   ptr = alloc<T_>(capv);
 }
 
+// closed shells with occupied and virtual orbitals
+static bool sub_able(const MolDesc& d) {
+  return d.n > 1 && d.nopen == 0 && (d.nel & 1) == 0 && d.nel >= 2 && d.nel / 2 < d.nao;
+}
+
 // Appends the tiles of a launch (per molecule) to out in an order that keeps
 // a molecule on one XCD: workgroup b of a launch runs on XCD b mod kXcds, so
 // the matrices of a molecule are fetched by one L2 only.  Molecules go to the

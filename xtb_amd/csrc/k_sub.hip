@@ -41,16 +41,6 @@
 namespace xtbamd {
 
 constexpr int kSubSteps = 24;        // steps per SCC iteration at most
-// Molecules of at most this many orbitals keep the full diagonalisation: a
-// k_jac_small of their size is shorter than the path.  On the path one water
-// (6 AOs) took 1.95 ms instead of 1.50 and 1000 of them 4.3 instead of 2.6, two
-// waters (12) 2.19 and 1.99; at 18 and 20 AOs a single molecule takes 2.45
-// and 2.34, 2.75 and 2.67; from 24 on the path is the faster one for single
-// molecules (2.76 and 2.84) and 84 of them (3.15 and 3.23).  (A batch that
-// fills the chip gains from the path from 48 AOs on only: 1000 x 24 AOs 7.8
-// and 6.6 ms, 300 x 48 7.1 and 7.1; the rule cannot look at the batch, whose
-// molecules get the same bits alone and in a mix.)
-constexpr int kSubMinAo = 20;
 // a molecule that gave up gets a fresh basis from its full diagonalisation,
 // which is closer to the next iterations' orbitals (700 waters: given up on
 // the first basis, 8 to 10 steps on the second); after a second time it
@@ -79,11 +69,6 @@ constexpr int kSubSym = 16;   // the tile is one of a symmetric result
 enum SubOp { kSubB = 0, kSubR, kSubM, kSubCY, kSubE1, kSubZ2, kSubE, kSubZ, kSubCYZ, kSubP };
 
 __device__ __forceinline__ int sub_occ(const MolDesc& md) { return md.nel / 2; }
-
-// closed shells with occupied and virtual orbitals
-__host__ __device__ __forceinline__ bool sub_able(const MolDesc& d) {
-  return d.n > 1 && d.nao > kSubMinAo && d.nopen == 0 && (d.nel & 1) == 0 && d.nel >= 2 && d.nel / 2 < d.nao;
-}
 
 // per-molecule doubles: tolerance of max |R|, the contraction allowed and the
 // contraction seen, then the factor w of each step
@@ -599,7 +584,8 @@ __global__ void __launch_bounds__(256) k_sub_next(const MolDesc* __restrict__ de
     const MolDesc& md = desc[m];
     int* si = sub + m * kSubInts;
     const int o = sub_occ(md);
-    bool on = state[m].active && si[kSubOff] < kSubTries && sub_able(md);
+    bool on = state[m].active && si[kSubOff] < kSubTries && md.nopen == 0 && (md.nel & 1) == 0 && md.n > 1 && o >= 1 &&
+              o < md.nao;
     if (on && si[kSubPhase] != 2 && si[kSubPhase] != 4) {
       const double* e = emo + md.o0;
       on = (1.0 - kSubRhoMin) * (e[o] - e[o - 1]) >= min_gap;
