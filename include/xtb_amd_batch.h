@@ -142,7 +142,7 @@ void xtbamd_server_free(xtbamd_server s);
  * forbid hipMalloc).  Computes what xtbamd_batch_new (one molecule, EEQ
  * guess) + xtbamd_batch_run + xtbamd_batch_get compute, with every device
  * array carved from a 64 MiB scratch area that the library holds on each GPU
- * it runs on until the process ends (molecules of up to about 450 AOs; a
+ * it runs on until the process ends (molecules of up to about 500 AOs; a
  * larger one returns -1 with a message naming the limit).  No hipMalloc,
  * hipFree or allocating library call is made; the first call on a device
  * sets up the scratch address and four events; the work runs on the null

@@ -632,7 +632,10 @@ __global__ void __launch_bounds__(256) k_sub_pending(MolState* state, int nmol, 
 // and a quarter of the elements per round each.
 // The inverse square roots start from I - M / 2 + 3 M^2 / 8 (error 5 M^3 / 16)
 // and take one step Q <- Q (3 I - Q^2 (I + M)) / 2 (error e -> 3 e^2 / 4), a
-// second one where M^6 is not below rounding.
+// second one where M^6 is not below rounding.  The error after the second is
+// not looked at: the path admits o max |M^8| up to 1e-8, so ||M|| up to 0.1,
+// whose start of 3e-4 leaves 7e-8 after the first step and 4e-15 after the
+// second, the size of the rounding of the rotation's products.
 constexpr int kRotVirt = 8;   // a kind + kRotVirt: the same for the virtual block (not kRotU)
 enum RotOp { kRotM = 0, kRotQ1, kRotS, kRotG, kRotQ, kRotU };
 constexpr double kRotOne = 1e-10;   // o max |M^4| up to which one step is enough

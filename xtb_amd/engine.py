@@ -231,10 +231,12 @@ class Batch:
         return out
 
     def results(self, matrices=False):
+        """Results of all molecules.  Without matrices the arrays are fetched
+        for the whole batch, one transfer each, and a molecule's are its parts
+        of them: one that is kept keeps the batch's array alive (copy it, or
+        use result(m), whose arrays are its own)."""
         if matrices:
             return [self.result(m, True) for m in range(len(self))]
-        # the arrays of all molecules in one transfer each, handed out as
-        # each molecule's part
         nmol = len(self)
         rs = (Result * nmol)()
         self._check(self._lib.xtbamd_batch_get_all(self._h, rs))   # sizes first

@@ -176,9 +176,9 @@ def single_table(run_dir, n, top=22):
     algorithmic rates of the kernels whose work has a closed count:
     the full-size products (2 n^3 flops per full product), the tridiagonalisation's
     column kernel (8 (n-2-j)^2 bytes of trailing rows for column j), its panel
-    updates (2 (n-j0-32)^2 * 64 flops per 32-column panel) and the Jacobi tile
-    updates (28 n^2 bytes per round if every pair rotates: an upper bound);
-    then the span of each phase of every blocked eigensolve."""
+    updates (2 (n-j0-32)^2 * 64 flops per 32-column panel); then the span of
+    each phase of every blocked eigensolve.  (The Jacobi rounds have none: they
+    may be those of the whole matrix or of a block of it.)"""
     rows = _trace_rows(run_dir)
     agg = {}
     for s, e, name in rows:
@@ -209,9 +209,6 @@ def single_table(run_dir, n, top=22):
         elif name == "k_bgemm<true, false>" and nsolve:
             r = nsolve * upd_flops / sec / 1e12
             rate = f"{r:.1f} TFLOP/s FP64 MFMA (panel updates), {100 * r / 78.6:.0f}% of 78.6"
-        elif name == "k_jac_apply_R":
-            per = 28.0 * n * n
-            rate = f"<= {c * per / sec / 1e12:.2f} TB/s ({per / 1e6:.0f} MB per round if every pair rotates)"
         out.append(f"| `{name}` | {c} | {t / 1e6:.2f} | {t / c / 1e3:.1f} | {100.0 * t / total:.1f} | {rate} |")
     out.append(f"| total | | {total / 1e6:.2f} | | 100.0 | |")
     # blocked eigensolves: a new one starts where the tridiagonalisation follows another phase
