@@ -104,6 +104,32 @@ def test_subspace_at_temperatures_around_the_gap_bound(monkeypatch, ratio):
             assert cs == cf, (cs, cf)
 
 
+def test_one_workgroup_path_bitwise_at_every_workgroup_size(monkeypatch):
+    """Workgroups of 64, 256 and 512 threads (largest molecule of the launch up
+    to 32, 64 and more AOs) share out the same blocks of the same products: 24,
+    30 and 32 AOs alone, beside 62 and 36 AOs, and beside 96 AOs on the path."""
+    xa = _engine()
+    from xtb_amd import workloads as w
+    small = [w.water_cluster(4, 3), w.water_cluster(5, 3), w.alkane(5, 3), w.water_cluster(1, 3)]
+
+    def run(mols):
+        b = xa.Batch([(z, x, 0.0, 0) for z, x in mols])
+        b.run()
+        r = b.results()
+        b.close()
+        return r
+
+    ref = run(small)
+    mixes = [run(small + [w.alkane(10, 3), w.water_cluster(6, 3)])]
+    monkeypatch.setenv("XTBAMD_SUB_WG", "128")
+    mixes.append(run(small + [w.water_cluster(16, 3)]))
+    for r in mixes:
+        for m, a in enumerate(ref):
+            assert a["iterations"] == r[m]["iterations"] and a["energy"] == r[m]["energy"], m
+            for k in ("gradient", "charges", "wbo", "emo", "focc"):
+                assert np.array_equal(a[k], r[m][k]), (m, k)
+
+
 def test_subspace_launches_only_where_a_molecule_can_use_them(monkeypatch, capfd):
     """Steps queued per SCC iteration (XTBAMD_TRACE_ROUNDS): none in the first
     one, whose orbitals the path needs; none at all for open shells, for gaps

@@ -451,7 +451,7 @@ class Batch {
   double* sub_dbl_ = nullptr;
   // molecules of at most sub_wg orbitals take the path in one workgroup each
   int sub_wg = 64;
-  int sub_nwg_ = 0;
+  int sub_nwg_ = 0, sub_wg_threads_ = 64;
   int* d_sub_wg = nullptr;
   static constexpr int kSubCold = 6;   // steps queued for a cold start
   int sub_guess_ = kSubCold;   // steps queued before the first count is read

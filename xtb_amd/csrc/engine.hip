@@ -1325,6 +1325,7 @@ void Batch::rebuild() {
       if (occupied_[m] && sub_able(desc[m]) && desc[m].nao <= sub_wg) wg.push_back(m);
     std::stable_sort(wg.begin(), wg.end(), [&](int x, int y) { return desc[x].nao > desc[y].nao; });
     sub_nwg_ = (int)wg.size();
+    sub_wg_threads_ = wg.empty() ? 64 : sub_wg_threads(desc[wg[0]].nao);
     if (sub_nwg_)
       HIPCHECK(hipMemcpyAsync(d_sub_wg, wg.data(), wg.size() * sizeof(int), hipMemcpyHostToDevice, stream));
     grow(d_sub_tiles, sub_tiles_cap_, std::max<long long>(1, (long long)st.size()));
@@ -2844,7 +2845,7 @@ void Batch::subspace(bool allow) {
       HIPCHECK(hipEventRecord(ev_fork, stream));
       HIPCHECK(hipStreamWaitEvent(stream2, ev_fork, 0));
     }
-    hipLaunchKernelGGL(k_sub_wg, dim3(sub_nwg_), dim3(512), 0, wide ? stream2 : stream, (const int*)d_sub_wg, d_desc,
+    hipLaunchKernelGGL(k_sub_wg, dim3(sub_nwg_), dim3(sub_wg_threads_), 0, wide ? stream2 : stream, (const int*)d_sub_wg, d_desc,
                        bf, d_state, sub_, sub_res_, sub_dbl_);
     if (wide) HIPCHECK(hipEventRecord(ev_join, stream2));
   }

@@ -393,10 +393,16 @@ __global__ void __launch_bounds__(256) k_sub_gemm(const int4* __restrict__ tiles
 }
 
 // The whole of an SCC iteration's subspace path of one molecule in one
-// workgroup of 8 waves (a wave takes every eighth 32 x 32 block of a
-// product): up to sub_wg orbitals a product is shorter than a launch, and a
-// batch has a molecule for every compute unit.  One call site of the product
-// (two with the row-minor C Y) in a loop over the sequence of kinds.
+// workgroup (its waves share out the 32 x 32 blocks of a product): up to
+// sub_wg orbitals a product is shorter than a launch, and a batch has a
+// molecule for every compute unit.  One call site of the product (two with the
+// row-minor C Y) in a loop over the sequence of kinds.  sub_wg_threads: a wave
+// per block of the launch's largest molecule.  With 8 waves for every size the
+// one that works is the first of each workgroup, and those of all workgroups
+// of a compute unit share a SIMD (ms a run of 1000 molecules, with a
+// diagonalisation in every iteration, 8 waves, now: 6 AOs 2.6, 4.3, 2.9; 24
+// AOs 6.6, 7.8, 5.8; 60 AOs 18.5, 18.7, 16.5; one molecule unchanged).
+inline int sub_wg_threads(int max_nao) { return max_nao <= 32 ? 64 : max_nao <= 64 ? 256 : 512; }
 __global__ void __launch_bounds__(512) k_sub_wg(const int* __restrict__ list, const MolDesc* __restrict__ desc,
                                                 SubBufs bf, MolState* state, int* sub, unsigned long long* res,
                                                 double* dbl) {
@@ -409,13 +415,13 @@ __global__ void __launch_bounds__(512) k_sub_wg(const int* __restrict__ list, co
   double* sd = dbl + (long long)m * kSubDbls;
   const MolDesc md = desc[m];
   const int N = md.nao, o = sub_occ(md), v = N - o;
-  const int tid = threadIdx.x, w = tid >> 6;
+  const int tid = threadIdx.x, w = tid >> 6, nw = blockDim.x >> 6;
   const int par0 = si[kSubPar];
   if (si[kSubFresh]) {
     const double* Am = bf.A + md.m0;
     const double* d = bf.diag + md.o0;
     double* X = bf.X + md.m0;
-    for (int t = tid; t < v * o; t += 512) {
+    for (int t = tid; t < v * o; t += blockDim.x) {
       const int i = t / o, j = t % o;
       const double x = -Am[(long long)(o + i) * N + j] / (d[o + i] - d[j]);
       X[t] = x;
@@ -439,11 +445,11 @@ __global__ void __launch_bounds__(512) k_sub_wg(const int* __restrict__ list, co
     const double ws = op == kSubR && step > 0 ? sd[kSubW + step] : 1.0;
     unsigned long long big = 0ull;
     if (op == kSubCY) {
-      for (int t = w; t < nr * nc; t += 8)
+      for (int t = w; t < nr * nc; t += nw)
         sub_block<true>(op, level, sym, md, bf, par, ws, e2, e3, 32 * (t / nc), 32 * (t % nc), big);
     } else {
       // (the two kinds that share a launch run one after the other here)
-      for (int t = w; t < nr * nc; t += 8)
+      for (int t = w; t < nr * nc; t += nw)
         sub_block<false>(op, level, sym, md, bf, par, ws, e2, e3, 32 * (t / nc), 32 * (t % nc), big);
     }
     if (op == kSubR || op == kSubE) {
