@@ -236,8 +236,7 @@ void eig_set_build(EigSet& es, const std::vector<int>& dims, EigMem& mem, const 
 // Am at jprobs[es.mols[k]] (a_off, ld), its eigenvalues are written to Am's
 // diagonal and its eigenvectors as rows of Wm (w_off, ld); jstate gets the
 // done / failed flags (kJacState ints per problem); problems below min_n rows
-// are left out; mstate (optional) skips
-// molecules that no longer iterate
+// are left out; mstate (optional) skips molecules that are not diagonalised
 void eig_set_run(EigSet& es, const JacobiProb* jprobs, int* jstate, const MolState* mstate, int min_n, double* Am,
                  double* Wm, hipStream_t s);
 

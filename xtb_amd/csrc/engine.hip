@@ -867,7 +867,8 @@ static long long* cap_field(Capacity& c, int k) {
 // "off" none): "key value" lines, '#' comments.  Read once per process.
 namespace {
 struct Tuning {
-  int eig_blk_min = -1, eig_blk_min_first = -1, eig_blk_min_half = -1, eig_blk_iters = -1, jac_lanes = -1, jac_cross = -1, gemm_valu = -1;
+  int eig_blk_min = -1, eig_blk_min_first = -1, eig_blk_min_half = -1, eig_blk_iters = -1;
+  int jac_lanes = -1, jac_cross = -1, gemm_valu = -1;
 };
 const Tuning& tuning() {
   static const Tuning t = [] {
@@ -1693,9 +1694,8 @@ bool Batch::jacobi(JacSet& js, double* Am, double* Wm, double* evout, bool check
   // the lanes test their progress once per period of their largest problem
   jac_period_ = blk && es.minn >= blk_n ? std::max(1, js.max_rounds_lanes) : js.max_rounds;
   const bool forked = lanes || blk;
-  // the small problems (one workgroup each, k_jac_small) run
-  // on stream3 beside the lanes
-  // (only the streams that get work are forked and joined: one molecule's
+  // the small problems (one workgroup each, k_jac_small) run on stream3
+  // beside the lanes (only the streams that get work are forked and joined: one molecule's
   // rounds stay on the main stream)
   static_assert(kMaxLanes == 3, "a stream per lane");
   const bool f2 = lanes && js.gpairs[1] < js.gpairs[2], f4 = lanes && js.gpairs[2] < js.gpairs[3];
@@ -2845,8 +2845,8 @@ void Batch::subspace(bool allow) {
       HIPCHECK(hipEventRecord(ev_fork, stream));
       HIPCHECK(hipStreamWaitEvent(stream2, ev_fork, 0));
     }
-    hipLaunchKernelGGL(k_sub_wg, dim3(sub_nwg_), dim3(sub_wg_threads_), 0, wide ? stream2 : stream, (const int*)d_sub_wg, d_desc,
-                       bf, d_state, sub_, sub_res_, sub_dbl_);
+    hipLaunchKernelGGL(k_sub_wg, dim3(sub_nwg_), dim3(sub_wg_threads_), 0, wide ? stream2 : stream,
+                       (const int*)d_sub_wg, d_desc, bf, d_state, sub_, sub_res_, sub_dbl_);
     if (wide) HIPCHECK(hipEventRecord(ev_join, stream2));
   }
   auto product = [&](int list, int step, int level) {

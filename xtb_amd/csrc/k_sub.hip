@@ -30,9 +30,10 @@
 // T is positive definite and every virtual eigenvalue lies above every
 // occupied one by at least (1 - rho) min D.  The path is left unless that is
 // at least kSubGapKt kT, rho being the contraction seen over the last steps
-// (sub_rate during the steps, sub_gap_kept at convergence): the Fermi occupations of the frontier orbitals are
-// then within e^-26 = 5e-12 of 1 and 0, the size of the density error that the
-// tolerance of R admits, and far below the 1e-9 from which entropy counts.
+// (sub_rate during the steps, sub_gap_kept at convergence): the Fermi
+// occupations of the frontier orbitals are then within e^-26 = 5e-12 of 1 and
+// 0, the size of the density error that the tolerance of R admits, and far
+// below the 1e-9 from which entropy counts.
 // The occupations handed back are those of the last diagonalisation.
 #pragma once
 #include "device_util.h"
